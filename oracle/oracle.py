@@ -52,8 +52,8 @@ def build(fast=True):
 
 
 def build_ref(reference="/root/reference"):
-    """Compile the reference's ggml CPU sources in place (only where the checkout exists)."""
-    if not os.path.isdir(reference):
+    """Compile the reference's ggml CPU sources in place (only where the checkout exists: an empty folder is none)."""
+    if not os.path.isdir(reference) or not os.listdir(reference):
         return False
     subprocess.run(["make", "-s", "-j8", "-C", HERE, "ref", f"REF={reference}"], check=True)
     return True
