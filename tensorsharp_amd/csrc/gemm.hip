@@ -5,8 +5,9 @@
 //      magnitude overflows or underflows fp16), written in the k-order in which the weight
 //      format unpacks (so the dequantizer never has to shuffle lanes), zero-padded to a
 //      multiple of the k-tile.  Optionally gathers rows through an index (MoE).
-//   2. gemm_slim_kernel (32 rows per tile: activations in registers, K split over the wavefronts, long K in
-//      chunks; used up to a few hundred rows, see gemm_tile_m) and gemm_kernel (128 / 256 rows per tile):
+//   2. by size (gemm_tile_m) gemm_slim_kernel (32 rows per tile: activations in registers, K split over the wavefronts,
+//      long K in chunks), gemm_wide_kernel (32 .. 128 rows x 256 columns, K in chunks that fill the chip) or
+//      gemm_xw_kernel / gemm_kernel (128 / 256 rows per tile).  gemm_kernel:
 //      BM x 256 x 64 tiles, eight wavefronts, each owning 32 output columns.  The fp16
 //      activation k-tiles and the RAW quantized bytes of 256 weight rows (one 144-byte window per row
 //      covering four k-tiles of Q4_K / MXFP4 or two of Q8_0) are copied from global memory straight
@@ -578,14 +579,16 @@ struct GQ80 {
     static __device__ __forceinline__ void dequant(const uint32_t (&r)[kRegs], int j, int h, uint32_t delta, bool live, uint32_t (&o)[16],
                                                    uint32_t& bad)
     {
+        // the block starts in the lower or the upper half of r[0]: byte picks by selector, not by branch
         const bool odd = ((delta + (uint32_t)(2 * j + h) * 34u) & 2u) != 0;
-        const uint32_t dbits = live ? (odd ? (r[0] >> 16) : (r[0] & 0xffffu)) : 0u;
-        mark2(bad, dbits);
-        const uint32_t d2 = pk_mul(dbits | (dbits << 16), kWUp2);     // fp16 d * 2^kWShift in both halves
+        const uint32_t pick = odd ? 0x07060504u : 0x05040302u;
+        const uint32_t dd = __builtin_amdgcn_perm(r[0], r[0], odd ? 0x03020302u : 0x01000100u) & (live ? 0xffffffffu : 0u);
+        mark2(bad, dd);
+        const uint32_t d2 = pk_mul(dd, kWUp2);                          // fp16 d * 2^kWShift in both halves
         const uint32_t bias = 0xe480e480u;                              // -1152.0 = -(1024 + 128)
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-            const uint32_t q = (odd ? r[i + 1] : __builtin_amdgcn_alignbyte(r[i + 1], r[i], 2)) ^ 0x80808080u;
+            const uint32_t q = __builtin_amdgcn_perm(r[i + 1], r[i], pick) ^ 0x80808080u;
             // bytes u = q + 128 become fp16 1024 + u: (0x64, u) pairs picked with v_perm
             const uint32_t p0 = __builtin_amdgcn_perm(0x64646464u, q, 0x04010400u);   // (u0, u1)
             const uint32_t p1 = __builtin_amdgcn_perm(0x64646464u, q, 0x04030402u);   // (u2, u3)
@@ -1640,6 +1643,513 @@ __global__ void __launch_bounds__(128 * WN) gemm_xw_kernel(const GemmArgs A)
             }
         }
     }
+}
+
+// vector instructions of the unpacking placed behind each of the 2 TM matrix instructions of a k-step
+template <int TM>
+constexpr int kWideValu = (40 + 2 * TM - 1) / (2 * TM);
+
+// ------------------------------------------------------------------------------------------
+// gemm_wide_kernel: tiles of 32 TM rows (TM 1 .. 4) x 256 columns, eight wavefronts = 4 (64 columns each) x 2 halves of the
+// K range of a turn.  A wavefront unpacks the operands of its own 64 columns in registers, and one activation operand read
+// from LDS feeds two matrix instructions; the two halves meet in LDS once, at the end.
+// What bounds it: the lines that a CU takes from its L2 (measured: about 47 GB/s per CU with all CUs reading, 128 bytes
+// for every line touched).  gemm_xw_kernel copies 48 of a Q4_K block's 144 bytes per k-tile and so takes two lines per row
+// and k-tile, 97 KB per 256 x 256 x 64 step; here a row's whole granule is copied at once, 33 KB per 128 x 256 x 64 step of
+// Q4_K.  Then the vector instructions: four to five per matrix instruction are free, each one more costs about five cycles.
+// Measured, whole call, us (the tile and register-resident kernels -> this one):
+//   Q4_K 512 x 14336 x 4096 91 -> 83, 200 x 4096 x 14336 82 -> 50, 333 x 4096 x 14336 116 -> 68, 200 x 4096 x 4096 38 -> 28
+//   Q8_0 512 x 14336 x 4096 104 -> 84, 200 x 4096 x 14336 82 -> 53, 40 x 21504 x 5376 59 -> 45
+//   Q6_K 200 x 4096 x 14336 96 -> 63, 200 x 21504 x 5376 187 -> 126, 128 x 21504 x 5376 121 -> 70
+// ------------------------------------------------------------------------------------------
+// Weight formats as this kernel reads them.  A granule is the raw bytes of kSup consecutive k-tiles of one row, kept in LDS
+// as kRawRow bytes (an odd multiple of four dwords: the dword reads of 32 rows spread over the most banks that 16-byte
+// pieces allow): kPieces pieces of 16 bytes from 16-byte aligned addresses, so that the granule starts `delta` (0 .. 15)
+// bytes into them.  Activations are in natural order: lane (column, h) holds the weights 32 h .. 32 h + 31 of a k-tile,
+// and quarter q of them (eight weights, four registers) is its B operand of k-step q.
+//   part_off(s):         where granule s starts behind the row start
+//   fetch_hdr / prepare: scales of k-tile j of the granule (half: which two quarters the wavefront takes, kSplit only)
+//   fetch / unpack:      quarter q of its weights
+//   kSplit: the two groups of wavefronts split a k-tile (k-steps 0, 1 / 2, 3) instead of taking a k-tile each: half the
+//           activations per turn, for raw rows so large that two k-tiles' worth of both do not fit LDS
+//   kUsBase, kUsRow:     microseconds per k-tile and per 32 rows of it, for pick_wide
+struct WQ4K {
+    static constexpr double kUsBase = 0.53, kUsRow = 0.125;
+    typedef GQ4K G;
+    static constexpr int kSup = 4, kRawRow = 144, kPieces = 9, kHdr = 4, kState = 2, kQ = 2;
+    static constexpr bool kSplit = false, kAligned = true;               // a block is 144 bytes: rows and blocks are 16-byte aligned
+    static __device__ __forceinline__ uint32_t part_off(int s) { return (uint32_t)s * 144u; }
+    static __device__ __forceinline__ void fetch_hdr(const uint8_t* rp, int, int, uint32_t, uint32_t (&r)[kHdr])
+    {
+        const uint4_t v = *reinterpret_cast<const uint4_t*>(rp);
+        r[0] = v.x; r[1] = v.y; r[2] = v.z; r[3] = v.w;
+    }
+    // sub-block 2 j + h: its six-bit scale and minimum
+    static __device__ __forceinline__ void prepare(const uint32_t (&r)[kHdr], int j, int h, uint32_t, bool, int, uint32_t (&st)[kState], uint32_t& bad)
+    {
+        const int sh = (j & 1) * 16 + 8 * h;
+        const uint32_t a = r[1] >> sh, b = r[2] >> sh, c = r[3] >> sh;
+        const uint32_t hi = 0u - (uint32_t)(j >> 1);     // sub-blocks 4 .. 7: all ones (a mask: no branch in the k loop)
+        const uint32_t sc = (((c & 0xfu) | ((a >> 2) & 0x30u)) & hi) | (a & 0x3fu & ~hi);
+        const uint32_t mn = ((((c >> 4) & 0xfu) | ((b >> 2) & 0x30u)) & hi) | (b & 0x3fu & ~hi);
+        H2U dm;
+        dm.u = r[0];
+        mark2(bad, r[0]);
+        st[0] = splat((float)dm.h.x * kWUp * (float)sc);
+        st[1] = splat(-((float)dm.h.y * kWUp * (float)mn));
+    }
+    static __device__ __forceinline__ void fetch(const uint8_t* rp, int j, int, uint32_t, int q, uint32_t (&r)[kQ])
+    {
+        const uint2 v = *reinterpret_cast<const uint2*>(rp + 16 + j * 32 + q * 8);
+        r[0] = v.x; r[1] = v.y;
+    }
+    // nibble h of every byte: a byte 0 .. 15 read as fp8 (E4M3) is that many 2^-9, so the conversion with a scale of 2^9
+    // gives two exact fp16 integers
+    static __device__ __forceinline__ void unpack(const uint32_t (&r)[kQ], const uint32_t (&st)[kState], int, int h, uint32_t, int, uint32_t (&o)[4])
+    {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const uint32_t t = (r[i] >> (4 * h)) & 0x0f0f0f0fu;
+            H2U lo, hi;
+            lo.h = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(t, 512.f, false);
+            hi.h = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(t, 512.f, true);
+            o[2 * i] = pk_fma(lo.u, st[0], st[1]);
+            o[2 * i + 1] = pk_fma(hi.u, st[0], st[1]);
+        }
+    }
+};
+struct WQ80 {
+    static constexpr double kUsBase = 0.68, kUsRow = 0.11;
+    typedef GQ80 G;
+    static constexpr int kSup = 2, kRawRow = 176, kPieces = 10, kHdr = 1, kState = 1, kQ = 3;
+    static constexpr bool kSplit = false, kAligned = false;
+    static __device__ __forceinline__ uint32_t part_off(int s) { return (uint32_t)s * 136u; }
+    // (delta: byte position of the granule inside its pieces, even)
+    static __device__ __forceinline__ void fetch_hdr(const uint8_t* rp, int j, int h, uint32_t d, uint32_t (&r)[kHdr])
+    {
+        r[0] = *reinterpret_cast<const uint32_t*>(rp + ((d + (uint32_t)(2 * j + h) * 34u) & ~3u));
+    }
+    static __device__ __forceinline__ void prepare(const uint32_t (&r)[kHdr], int j, int h, uint32_t d, bool live, int, uint32_t (&st)[kState], uint32_t& bad)
+    {
+        const bool odd = ((d + (uint32_t)(2 * j + h) * 34u) & 2u) != 0;
+        const uint32_t dd = __builtin_amdgcn_perm(r[0], r[0], odd ? 0x03020302u : 0x01000100u) & (live ? 0xffffffffu : 0u);
+        mark2(bad, dd);
+        st[0] = pk_mul(dd, kWUp2);                       // fp16 d * 2^kWShift in both halves
+    }
+    static __device__ __forceinline__ void fetch(const uint8_t* rp, int j, int h, uint32_t d, int q, uint32_t (&r)[kQ])
+    {
+        const uint32_t* p = reinterpret_cast<const uint32_t*>(rp + ((d + (uint32_t)(2 * j + h) * 34u) & ~3u)) + 2 * q;
+        r[0] = p[0]; r[1] = p[1]; r[2] = p[2];
+    }
+    static __device__ __forceinline__ void unpack(const uint32_t (&r)[kQ], const uint32_t (&st)[kState], int j, int h, uint32_t d, int, uint32_t (&o)[4])
+    {
+        const uint32_t pick = ((d + (uint32_t)(2 * j + h) * 34u) & 2u) ? 0x07060504u : 0x05040302u;
+        const uint32_t bias = 0xe480e480u;               // -1152.0 = -(1024 + 128)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const uint32_t q = __builtin_amdgcn_perm(r[i + 1], r[i], pick) ^ 0x80808080u;
+            // bytes u = q + 128 become fp16 1024 + u: (0x64, u) pairs picked with v_perm
+            o[2 * i] = pk_mul(pk_add(__builtin_amdgcn_perm(0x64646464u, q, 0x04010400u), bias), st[0]);
+            o[2 * i + 1] = pk_mul(pk_add(__builtin_amdgcn_perm(0x64646464u, q, 0x04030402u), bias), st[0]);
+        }
+    }
+};
+// Q6_K: a granule is a block (210 bytes, even delta: fourteen pieces)
+struct WQ6K {
+    static constexpr double kUsBase = 1.1, kUsRow = 0.1;
+    typedef GQ6K G;
+    static constexpr int kSup = 4, kRawRow = 240, kPieces = 14, kHdr = 2, kState = 1, kQ = 6;
+    static constexpr bool kSplit = true, kAligned = false;
+    static __device__ __forceinline__ uint32_t part_off(int s) { return (uint32_t)s * 210u; }
+    static __device__ __forceinline__ void fetch_hdr(const uint8_t* rp, int j, int h, uint32_t d, uint32_t (&r)[kHdr])
+    {
+        r[0] = *reinterpret_cast<const uint32_t*>(rp + ((d + 192u + 4u * j + 2u * h) & ~3u));
+        r[1] = *reinterpret_cast<const uint32_t*>(rp + ((d + 208u) & ~3u));
+    }
+    static __device__ __forceinline__ void prepare(const uint32_t (&r)[kHdr], int, int h, uint32_t d, bool live, int half, uint32_t (&st)[kState], uint32_t& bad)
+    {
+        const float sc = (float)(int)(int8_t)(r[0] >> (((d + 2u * h) & 2u) * 8u + 8u * half));
+        H2U dd;
+        dd.u = (r[1] >> ((d & 2u) * 8u)) & (live ? 0xffffu : 0u);
+        mark2(bad, dd.u);
+        st[0] = splat((float)dd.h.x * kWUp * sc);
+    }
+    static __device__ __forceinline__ void fetch(const uint8_t* rp, int j, int h, uint32_t d, int q, uint32_t (&r)[kQ])
+    {
+        const uint8_t* const base = rp + (d & ~3u) + 8 * q;
+        const uint32_t* a = reinterpret_cast<const uint32_t*>(base + 64 * (j >> 1) + 32 * h);
+        const uint32_t* b = reinterpret_cast<const uint32_t*>(base + 128 + 32 * (j >> 1));
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            r[i] = a[i];
+            r[3 + i] = b[i];
+        }
+    }
+    static __device__ __forceinline__ void unpack(const uint32_t (&r)[kQ], const uint32_t (&st)[kState], int j, int h, uint32_t d, int, uint32_t (&o)[4])
+    {
+        const uint32_t sh = d & 2u, sc = st[0];
+        const uint32_t bias = 0xe420e420u;               // -(1024 + 32)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const uint32_t ql = __builtin_amdgcn_alignbyte(r[i + 1], r[i], sh) >> (4 * (j & 1));
+            const uint32_t qh = __builtin_amdgcn_alignbyte(r[4 + i], r[3 + i], sh) >> (4 * (j & 1) + 2 * h);
+            const uint32_t q6 = (ql & 0x0f0f0f0fu) | ((qh & 0x03030303u) << 4);
+            // bytes u = q become fp16 1024 + u; minus 1056 leaves q - 32 exactly
+            o[2 * i] = pk_mul(pk_add(__builtin_amdgcn_perm(0x64646464u, q6, 0x04010400u), bias), sc);
+            o[2 * i + 1] = pk_mul(pk_add(__builtin_amdgcn_perm(0x64646464u, q6, 0x04030402u), bias), sc);
+        }
+    }
+};
+
+template <typename H, int TM>
+struct WideLayout {
+    static constexpr int BM = 32 * TM, BN = 256;
+    static constexpr int kTurn = H::kSplit ? 1 : 2;                       // k-tiles per turn of the loop
+    static constexpr int kXTile = BM * kXRow, kXStage = kTurn * kXTile;
+    static constexpr int RT = BN * H::kRawRow;                            // bytes of one granule of all columns
+    static constexpr int kCopies = 2 * kXStage + 2 * RT;                  // activations, raw granules
+    static constexpr int kReduce = 8 * TM * 16 * 64 * 4;                  // the partial sums of one column block of every wavefront
+    static constexpr int kBuf = kCopies > kReduce ? kCopies : kReduce;
+    static constexpr size_t kLds = (size_t)kBuf + 1024 + BM * 4 + 2 * BN * 4;   // + dump, row scales, column flags
+};
+
+template <typename H, int TM>
+__global__ void __launch_bounds__(512) gemm_wide_kernel(const GemmArgs A)
+{
+    typedef WideLayout<H, TM> L;
+    constexpr int NB = 2, BN = L::BN, BM = L::BM, RT = L::RT, kXTile = L::kXTile;
+    constexpr int kRawRow = H::kRawRow, kRowPieces = kRawRow / 16;
+    constexpr int KT = L::kTurn;
+    constexpr int XN = L::kXStage / 1024, XI = (XN + 7) / 8;  // 1 KiB copies of a turn's activations, per wavefront
+    constexpr int WN = RT / 1024, WI = (WN + 7) / 8;        // and of a granule (the surplus goes to a dump area)
+    extern __shared__ uint8_t smem[];
+    uint8_t* const xbuf = smem;                          // 2 x kXStage
+    uint8_t* const rbuf = smem + 2 * L::kXStage;            // 2 x RT (the unpackers may read a few bytes past a row)
+    uint8_t* const dump = smem + L::kBuf;                // 1 KiB
+    float* const tile_scales = reinterpret_cast<float*>(dump + 1024);                // BM row scales for the epilogue
+    uint32_t* const col_bad = reinterpret_cast<uint32_t*>(tile_scales + BM);          // [2][BN]
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int g = wave >> 2, wn = wave & 3;
+    const int col = lane & 31, h = lane >> 5;
+
+    // tile order as in gemm_kernel: every XCD takes a contiguous run of (K chunk, row tile, column tile)
+    const int tiles = A.m_tiles * A.n_tiles;
+    const int total = tiles * A.k_chunks;
+    int t = blockIdx.x;
+    {
+        const int per = (total + 7) >> 3;
+        const int xcd = t & 7, slot = t >> 3;
+        t = xcd * per + slot;
+        if (slot >= per || t >= total) return;
+    }
+    const int kc = t / tiles;
+    t -= kc * tiles;
+    const int mt = t / A.n_tiles, nt = t - mt * A.n_tiles;
+    const int m0 = mt * BM, m_rows = min(BM, A.M - m0);
+    const int n0 = nt * BN;
+
+    const uintptr_t wa = reinterpret_cast<uintptr_t>(A.w);
+    const uint32_t base_delta = (uint32_t)(wa & 15);
+    const __amdgpu_buffer_rsrc_t wrs = __builtin_amdgcn_make_buffer_rsrc(
+        reinterpret_cast<void*>(wa & ~(uintptr_t)15), 0, (int)(((uint32_t)A.w_bytes + base_delta + 3u) & ~3u), 0x00020000);
+    const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(const_cast<_Float16*>(A.x16), 0, (int)A.x16_bytes, 0x00020000);
+    const uint32_t row_bytes = (uint32_t)((int64_t)A.w_bytes / A.N);
+    const int kt_begin = kc * A.chunk_kt;                               // a multiple of 4: whole granules
+    const int nkt = min(A.Kp / kBK, kt_begin + A.chunk_kt);            // end of this unit's K range
+
+    // per-lane source offsets of the LDS-direct copies
+    uint32_t x_off[XI], w_row[WI], w_piece[WI];
+#pragma unroll
+    for (int i = 0; i < XI; ++i) {
+        const int q = (wave + 8 * i) * 64 + lane;            // LDS chunk slot: k-tile, row, position q % 8
+        const int tile = q / (BM * 8), row = (q >> 3) % BM, chunk = (q & 7) ^ ((row >> 1) & 7);
+        x_off[i] = row < m_rows && tile < KT ? (uint32_t)(m0 + row) * (uint32_t)(A.xld * 2) + (uint32_t)chunk * 16u + (uint32_t)tile * kXRow : kDeadOffset;
+    }
+#pragma unroll
+    for (int i = 0; i < WI; ++i) {
+        const int c = (wave + 8 * i) * 64 + lane;
+        const int row = c / kRowPieces, piece = c - row * kRowPieces;
+        const bool ok = row < BN && n0 + row < A.N && piece < H::kPieces;
+        w_row[i] = ok ? base_delta + (uint32_t)(n0 + row) * row_bytes + (H::kAligned ? 16u * (uint32_t)piece : 0u) : kDeadOffset;
+        w_piece[i] = (uint32_t)piece * 16u;
+    }
+    // k-tiles past the end: the offset gets its top bit set (out of range: zeros arrive)
+    typedef __attribute__((address_space(3))) uint8_t* lds_ptr;
+    const lds_ptr lds = (lds_ptr)smem;
+    auto copy = [&](const __amdgpu_buffer_rsrc_t& rs, lds_ptr dst, uint32_t voffset, uint32_t soffset) {
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)dst, 16, (int)voffset, (int)soffset, 0, 0);
+    };
+    // the turn that begins at k-tile kt; the second k-tile of a pair may lie past the unit (a wavefront copies one of the two)
+    auto issue_x = [&](int kt) {
+#pragma unroll
+        for (int i = 0; i < XI; ++i) {
+            const int id = wave + 8 * i;
+            const uint32_t past = kt + (KT == 2 && id >= 4 * TM ? 1 : 0) < nkt ? 0u : kDeadOffset;
+            copy(xrs, lds + (8 * i + 8 <= XN || id < XN ? ((kt / KT) & 1) * L::kXStage + id * 1024 : L::kBuf), x_off[i] | past, (uint32_t)kt * kXRow);
+        }
+    };
+    auto issue_w = [&](int s) {
+        const uint32_t past = s * H::kSup < nkt ? 0u : kDeadOffset;
+#pragma unroll
+        for (int i = 0; i < WI; ++i) {
+            const int id = wave + 8 * i;
+            const lds_ptr dst = lds + (8 * i + 8 <= WN || id < WN ? 2 * L::kXStage + (s & 1) * RT + id * 1024 : L::kBuf);
+            if constexpr (H::kAligned) {
+                copy(wrs, dst, w_row[i] | past, H::part_off(s));
+            } else {
+                copy(wrs, dst, (((w_row[i] + H::part_off(s)) & ~15u) + w_piece[i]) | past, 0u);
+            }
+        }
+    };
+
+    for (int i = tid; i < BM; i += 512) tile_scales[i] = A.xscale[m0 + min(i, m_rows - 1)];
+    // this lane's weight rows for the matrix pipe
+    const int raw0 = (wn * (32 * NB) + col) * kRawRow;
+    const int my_n0 = n0 + wn * (32 * NB) + col;
+    uint32_t my_row[NB], bad[NB];
+    bool in_n[NB];
+#pragma unroll
+    for (int n = 0; n < NB; ++n) {
+        in_n[n] = my_n0 + 32 * n < A.N;
+        my_row[n] = in_n[n] ? base_delta + (uint32_t)(my_n0 + 32 * n) * row_bytes : 0u;
+        bad[n] = 0u;                                     // a scale of this lane's column does not fit the fp16 operands
+    }
+    float16_t acc[TM][NB];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int n = 0; n < NB; ++n)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][n][r] = 0.f;
+
+    // A operand of k-step ks of this wavefront's k-tile: chunk 2 ks + h of row (32 i + col), at its swizzled position
+    const int sw = (col >> 1) & 7;
+    int a_off[4];                                        // (kSplit: of k-step 2 g + ks, two of them)
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) a_off[ks] = (H::kSplit ? 0 : g * kXTile) + col * kXRow + ((2 * (H::kSplit ? 2 * g + (ks & 1) : ks) + h) ^ sw) * 16;
+    auto load_a = [&](int kt, int ks, half8_t (&a)[TM]) {       // of the pair that begins at kt
+        const uint8_t* const xs = xbuf + ((kt / KT) & 1) * L::kXStage + a_off[ks];
+#pragma unroll
+        for (int i = 0; i < TM; ++i) a[i] = *reinterpret_cast<const half8_t*>(xs + i * 32 * kXRow);
+    };
+    // raw bytes and scales of k-tile kt; its granule, its place in it and the granule's position inside the copied pieces
+    auto row_of = [&](int s, int n) { return rbuf + (s & 1) * RT + raw0 + n * 32 * kRawRow; };
+    auto delta_of = [&](int s, int n) { return H::kAligned ? 0u : (my_row[n] + H::part_off(s)) & 15u; };
+    uint32_t o[NB][16], hdr[NB][H::kHdr], state[NB][H::kState];
+    auto fetch_hdr = [&](int kt) {
+        const int s = kt / H::kSup, j = kt % H::kSup;
+#pragma unroll
+        for (int n = 0; n < NB; ++n) H::fetch_hdr(row_of(s, n), j, h, delta_of(s, n), hdr[n]);
+    };
+    auto fetch = [&](int kt, int q, uint32_t (&r)[NB][H::kQ]) {
+        const int s = kt / H::kSup, j = kt % H::kSup;
+#pragma unroll
+        for (int n = 0; n < NB; ++n) H::fetch(row_of(s, n), j, h, delta_of(s, n), q, r[n]);
+    };
+    auto prepare = [&](int kt) {
+        const int s = kt / H::kSup, j = kt % H::kSup;
+        const bool live_k = (kt < nkt) & ((kt * 2 + h) * 32 < A.K);      // past the unit's end the raw bytes are zeros or stale
+#pragma unroll
+        for (int n = 0; n < NB; ++n) H::prepare(hdr[n], j, h, delta_of(s, n), live_k & in_n[n], g, state[n], bad[n]);
+    };
+    auto unpack = [&](int kt, int q, int slot, uint32_t (&r)[NB][H::kQ]) {
+        const int s = kt / H::kSup, j = kt % H::kSup;
+#pragma unroll
+        for (int n = 0; n < NB; ++n) {
+            uint32_t v[4];
+            H::unpack(r[n], state[n], j, h, delta_of(s, n), q, v);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) o[n][4 * slot + i] = v[i];
+        }
+    };
+    auto mfma = [&](const half8_t (&a)[TM], int ks) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int n = 0; n < NB; ++n) {
+                const uint4_t bb = {o[n][4 * ks], o[n][4 * ks + 1], o[n][4 * ks + 2], o[n][4 * ks + 3]};
+                acc[i][n] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[i], __builtin_bit_cast(half8_t, bb), acc[i][n], 0, 0, 0);
+            }
+    };
+    // a matrix instruction, then a share of the unpacking, throughout the k-step
+    auto interleave = [&]() {
+#pragma unroll
+        for (int q = 0; q < 2 * TM; ++q) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, kWideValu<TM>, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+
+    const int s_begin = kt_begin / H::kSup;
+    issue_w(s_begin);
+    issue_x(kt_begin);
+    issue_w(s_begin + 1);
+    issue_x(kt_begin + KT);
+    wait_copies_and_barrier<0>();
+    uint32_t ra[NB][H::kQ], rb[NB][H::kQ];
+    half8_t a0[TM], a1[TM];
+    if constexpr (H::kSplit) {
+        // One k-tile a turn, two of its k-steps per group.  As below, with the weights of a k-step unpacked two k-steps ahead.
+        fetch_hdr(kt_begin);
+        prepare(kt_begin);
+        fetch(kt_begin, 2 * g, ra);
+        unpack(kt_begin, 2 * g, 0, ra);
+        fetch(kt_begin, 2 * g + 1, rb);
+        load_a(kt_begin, 0, a0);
+        for (int kt = kt_begin; kt < nkt; ++kt) {
+            uint32_t rc[NB][H::kQ];
+            load_a(kt, 1, a1);
+            fetch_hdr(kt + 1);
+            fetch(kt + 1, 2 * g, ra);
+            fetch(kt + 1, 2 * g + 1, rc);
+            __builtin_amdgcn_sched_barrier(0);
+            mfma(a0, 0);
+            unpack(kt, 2 * g + 1, 1, rb);
+            interleave();
+#pragma unroll
+            for (int n = 0; n < NB; ++n)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(o[n][4 + i]));     // (unpacked here, not where they are used)
+            // the granule requested in the last turn may be in flight: its first k-tile is read three turns later
+            if ((kt & 3) == 3)
+                asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(WI) : "memory");
+            else
+                asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+            asm volatile("s_barrier" ::: "memory");
+            load_a(kt + 1, 0, a0);
+            issue_x(kt + 2);
+            if ((kt & 3) == 2) issue_w(kt / 4 + 2);
+            __builtin_amdgcn_sched_barrier(0);
+            mfma(a1, 1);
+            prepare(kt + 1);
+            unpack(kt + 1, 2 * g, 0, ra);
+            interleave();
+#pragma unroll
+            for (int n = 0; n < NB; ++n)
+#pragma unroll
+                for (int i = 0; i < H::kQ; ++i) rb[n][i] = rc[n][i];
+        }
+    } else {
+        fetch_hdr(kt_begin + g);
+        prepare(kt_begin + g);
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            fetch(kt_begin + g, q, ra);
+            unpack(kt_begin + g, q, q, ra);
+        }
+        fetch(kt_begin + g, 3, rb);
+        load_a(kt_begin, 0, a0);
+        if constexpr (H::kSup == 2) {
+            wait_copies_and_barrier<0>();                    // every wavefront has read its first raw bytes
+            issue_w(s_begin + 2);
+        }
+
+        // Two k-tiles a turn, one per group of four wavefronts.  The quarter of the operands that a k-step has used up is
+        // unpacked anew, for the next k-tile, during the k-step after it; everything read from LDS is requested one k-step
+        // before its use.  The one barrier of a turn stands before the last k-step: behind it the activation stage of the turn
+        // and the raw bytes of the next have been read by all and take the copies of two turns later, which have a whole turn
+        // to land.
+        for (int kt = kt_begin; kt < nkt; kt += 2) {
+            const int mine = kt + g;
+            load_a(kt, 1, a1);
+            fetch_hdr(mine + 2);
+            fetch(mine + 2, 0, ra);
+            __builtin_amdgcn_sched_barrier(0);
+            mfma(a0, 0);
+            unpack(mine, 3, 3, rb);
+            interleave();
+            load_a(kt, 2, a0);
+            fetch(mine + 2, 1, rb);
+            __builtin_amdgcn_sched_barrier(0);
+            mfma(a1, 1);
+            prepare(mine + 2);
+            unpack(mine + 2, 0, 0, ra);
+            interleave();
+            load_a(kt, 3, a1);
+            fetch(mine + 2, 2, ra);
+            uint32_t rc[NB][H::kQ];
+            fetch(mine + 2, 3, rc);
+            __builtin_amdgcn_sched_barrier(0);
+            mfma(a0, 2);
+            unpack(mine + 2, 1, 1, rb);
+            interleave();
+#pragma unroll
+            for (int n = 0; n < NB; ++n)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) asm volatile("" : "+v"(o[n][i]));     // (unpacked here, not where they are used)
+            wait_copies_and_barrier<0>();
+            load_a(kt + 2, 0, a0);
+            issue_x(kt + 4);
+            if constexpr (H::kSup == 2) issue_w(kt / 2 + 3);
+            else if ((kt & 2) == 0) issue_w(kt / 4 + 2);
+            __builtin_amdgcn_sched_barrier(0);
+            mfma(a1, 3);
+            unpack(mine + 2, 2, 2, ra);
+            interleave();
+#pragma unroll
+            for (int n = 0; n < NB; ++n)
+#pragma unroll
+                for (int i = 0; i < H::kQ; ++i) rb[n][i] = rc[n][i];
+        }
+    }
+
+    // The sums of even and odd k-tiles meet in LDS: wavefront (g, wn) hands over column block 1 - g and finishes block g.
+    wait_copies_and_barrier<0>();                        // (the copies still in flight have landed, too)
+    float* const sums = reinterpret_cast<float*>(smem);
+#pragma unroll
+    for (int n = 0; n < NB; ++n) {
+        const int mine = H::G::out_of_range(bad[n]) ? 1 : 0;
+        const int both = mine | __shfl_xor(mine, 32);    // the two lanes of a column (k-halves) saw different blocks
+        if (h == 0) col_bad[g * BN + wn * 64 + 32 * n + col] = (uint32_t)both;
+    }
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int r4 = 0; r4 < 4; ++r4) {
+            float4 v;
+            v.x = g ? acc[i][0][4 * r4] : acc[i][1][4 * r4];
+            v.y = g ? acc[i][0][4 * r4 + 1] : acc[i][1][4 * r4 + 1];
+            v.z = g ? acc[i][0][4 * r4 + 2] : acc[i][1][4 * r4 + 2];
+            v.w = g ? acc[i][0][4 * r4 + 3] : acc[i][1][4 * r4 + 3];
+            reinterpret_cast<float4*>(sums)[((wave * TM + i) * 4 + r4) * 64 + lane] = v;
+        }
+    __syncthreads();
+    float16_t out[TM][1];
+    const int my_n = my_n0 + 32 * g;
+    const bool flagged = (col_bad[wn * 64 + 32 * g + col] | col_bad[BN + wn * 64 + 32 * g + col]) != 0;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int r4 = 0; r4 < 4; ++r4) {
+            const float4 v = reinterpret_cast<const float4*>(sums)[(((wave ^ 4) * TM + i) * 4 + r4) * 64 + lane];
+            const float p[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const float sum = (g ? acc[i][1][4 * r4 + q] : acc[i][0][4 * r4 + q]) + p[q];
+                out[i][0][4 * r4 + q] = flagged ? __uint_as_float(kNaNBits) : sum;
+            }
+        }
+    // epilogue: D[row = 32 i + 8 (r / 4) + 4 h + r % 4][column] times the row scale
+    if (A.partial || (!A.c_rows && !A.accumulate)) {
+        float* const dst = A.partial ? A.partial + (int64_t)kc * A.M * A.N : A.c;
+        store_wave_tile<TM, 1, false>(tile_scales, out, dst, A.partial ? A.N : A.ldc, A.N, m0, m_rows, 0, my_n, h);
+        return;
+    }
+    if (my_n >= A.N) return;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int ml = 32 * i + 8 * (r >> 2) + 4 * h + (r & 3);
+            if (ml < m_rows) {
+                float* p = A.c + (int64_t)(A.c_rows ? A.c_rows[m0 + ml] : m0 + ml) * A.ldc + my_n;
+                const float v = out[i][0][r] * tile_scales[ml];
+                *p = A.accumulate ? *p + v : v;
+            }
+        }
 }
 
 // Number of K chunks for a plain launch: with few tiles and a long K, chunks of K fill the CUs that a whole-K launch
@@ -3084,6 +3594,72 @@ bool launch_slim_for(const GemmArgs& a, int ktw, int m_tiles, hipStream_t stream
     return false;
 }
 
+// Rows and K chunks of a plain launch of gemm_wide_kernel, and the microseconds they are expected to take: rounds of
+// workgroups x k-tiles (a round that leaves CUs idle is up to 40 % faster: the kernel waits for the L2), start and end of
+// a workgroup, and for K chunks the second launch with its reads and writes of the chunk sums.
+struct WidePlan {
+    int tm, k_chunks, chunk_kt;
+    double us;
+};
+inline double chunk_sum_us(int k_chunks, int M, int N) { return k_chunks > 1 ? 3.0 + (double)k_chunks * M * N * 8 / 8.0e6 : 0.0; }
+inline WidePlan pick_wide(int M, int N, int nkt, bool chunks, double base, double per_row_block)
+{
+    WidePlan best{0, 1, 0, 0.0};
+    const int cus = device_info().num_cus, n_tiles = (N + 255) / 256;
+    for (int tm = 1; tm <= 4; ++tm) {
+        const int m_tiles = (M + 32 * tm - 1) / (32 * tm);
+        for (int sc = 1; sc <= (chunks ? 8 : 1); ++sc) {
+            const int chunk = ((nkt + sc - 1) / sc + 3) / 4 * 4;
+            const int kc = (nkt + chunk - 1) / chunk;
+            if (sc > 1 && (kc != sc || chunk < 8)) continue;
+            const int64_t units = (int64_t)m_tiles * n_tiles * kc, rounds = (units + cus - 1) / cus;
+            const double fill = (double)units / (double)(rounds * cus);
+            const double us = (double)rounds * (chunk * (base + per_row_block * tm) * (0.6 + 0.4 * fill) + 3.0) + chunk_sum_us(kc, M, N);
+            if (best.tm == 0 || us < best.us) best = WidePlan{tm, kc, chunk, us};
+        }
+    }
+    return best;
+}
+
+template <typename H, int TM>
+bool launch_wide_tm(const GemmArgs& a, hipStream_t stream)
+{
+    constexpr size_t lds = WideLayout<H, TM>::kLds;
+    static_assert(lds <= 160 * 1024, "LDS");
+    auto kern = gemm_wide_kernel<H, TM>;
+    if (!raise_lds_limit(reinterpret_cast<const void*>(kern), lds)) return false;
+    const int grid = (a.m_tiles * a.n_tiles * a.k_chunks + 7) / 8 * 8;          // whole rounds over the 8 XCDs
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(512), lds, stream, a);
+    if (!hip_ok(hipGetLastError(), "gemm launch")) return false;
+    return a.partial ? launch_chunk_sum(a, stream) : true;
+}
+
+template <typename H>
+bool launch_wide(GemmArgs a, hipStream_t stream, const ChunkScratch& cs)
+{
+    const int nkt = a.Kp / kBK;
+    WidePlan p = pick_wide(a.M, a.N, nkt, true, H::kUsBase, H::kUsRow);
+    a.partial = nullptr;
+    if (p.k_chunks > 1) {
+        const size_t need = (size_t)p.k_chunks * a.M * a.N * sizeof(float);
+        if (cs.need_out) *cs.need_out = need;
+        a.partial = chunk_scratch(cs, need);
+        // the caller's scratch is too small for the chunk sums: whole K per tile (slower)
+        if (!a.partial) p = pick_wide(a.M, a.N, nkt, false, H::kUsBase, H::kUsRow);
+    }
+    if (cs.need_out) return true;
+    a.m_tiles = (a.M + 32 * p.tm - 1) / (32 * p.tm);
+    a.n_tiles = (a.N + 255) / 256;
+    a.k_chunks = p.k_chunks;
+    a.chunk_kt = p.chunk_kt;
+    switch (p.tm) {
+    case 1: return launch_wide_tm<H, 1>(a, stream);
+    case 2: return launch_wide_tm<H, 2>(a, stream);
+    case 3: return launch_wide_tm<H, 3>(a, stream);
+    default: return launch_wide_tm<H, 4>(a, stream);
+    }
+}
+
 // 128-row tiles are 128 x 256 (one workgroup per CU) for these formats, 128 x 128 (two per CU) for the others
 template <typename G>
 constexpr bool kWide128 = G::kSup == 2 || G::kRawRow > 144 || std::is_same<G, GQ4K>::value;
@@ -3116,10 +3692,27 @@ bool launch_slim_mx48(GemmArgs a, int m_tiles, hipStream_t stream, const ChunkSc
     return hip_ok(hipGetLastError(), "gemm launch");
 }
 
+// the tile height of a plain launch that gemm_wide_kernel takes (it picks its own)
+constexpr int kWideTiles = 0;
+
 template <typename G>
 bool launch_for_type(const GemmArgs& a, int bm, int m_tiles, hipStream_t stream, const ChunkScratch& cs)
 {
-    if (bm == 32 && !a.x_mx) return launch_slim_for<G>(a, slim_ktw<G>(a.Kp / kBK), m_tiles, stream, cs);
+    if (bm == kWideTiles) {
+        if constexpr (std::is_same<G, GQ4K>::value) return launch_wide<WQ4K>(a, stream, cs);
+        if constexpr (std::is_same<G, GQ80>::value) return launch_wide<WQ80>(a, stream, cs);
+        if constexpr (std::is_same<G, GQ6K>::value) return launch_wide<WQ6K>(a, stream, cs);
+    }
+    if (bm == 32 && !a.x_mx) {
+        const int ktw = slim_ktw<G>(a.Kp / kBK), kc = (a.Kp / kBK + 8 * ktw - 1) / (8 * ktw);
+        // (a plain launch whose chunk sums do not fit the caller's scratch: tiles that need none)
+        const bool fits = cs.need_out || (kc == 1 && !a.accumulate) || chunk_scratch(cs, (size_t)kc * a.M * a.N * sizeof(float));
+        if (fits || a.tile_expert) return launch_slim_for<G>(a, ktw, m_tiles, stream, cs);
+        if constexpr (std::is_same<G, GQ4K>::value) return launch_xw<PQ4K, 256, 4>(a, (a.M + 255) / 256, stream, cs);
+        if constexpr (std::is_same<G, GQ80>::value) return launch_wide<WQ80>(a, stream, cs);
+        if constexpr (std::is_same<G, GQ6K>::value) return launch_wide<WQ6K>(a, stream, cs);
+        return launch_slim_for<G>(a, ktw, m_tiles, stream, cs);
+    }
     // Q4_K and MXFP4: the 2 x 4 wavefront layout with the operand exchange through LDS (gemm_xw_kernel); 128-row tiles are
     // 128 x 256.  Q4_K takes it for every launch, MXFP4 for plain ones: the MXFP4 expert tiles of a MoE prefill (128
     // rows) stay on two 128 x 128 workgroups per CU (926 vs 968 us at 2048 tokens).
@@ -3174,8 +3767,8 @@ size_t gemm_workspace_bytes(int M, int K)
 
 // Rows of activations per tile for a plain (ungrouped) launch.  The 32-row register-resident kernel streams the
 // weights once per 32 rows, but at a much higher rate than the LDS-tiled kernels and mostly out of the memory-side
-// cache, so it wins well past 32 rows (measured crossovers: 4-bit formats about 128 rows, or up to 512 when the
-// big tiles would leave CUs idle; Q8_0 about 64; Q6_K, whose big tiles are limited to 128 rows, about 256).
+// cache, so it wins well past 32 rows (measured crossovers of the formats that gemm_wide_kernel does not serve: about 128
+// rows, MXFP4 up to 512 when the big tiles would leave CUs idle).
 namespace {
 bool wide_128_row_tiles(int type)
 {
@@ -3194,18 +3787,56 @@ bool wide_128_row_tiles(int type)
 }
 }  // namespace
 
-int gemm_tile_m(int type, int M, int N)
+namespace {
+// Expected microseconds of the register-resident kernel: a unit (32 rows x 32 columns x 8 ktw k-tiles) takes 3.0 (ktw 4) to
+// 4.4 us (ktw 8), a workgroup that crosses into another row tile or K chunk loads its activations again.
+template <typename G>
+double slim_us(int M, int N, int nkt)
 {
-    const int slim_rows = type == kTypeQ8_0 ? 64 : type == kTypeQ6_K ? 256 : 128;
-    if (M <= slim_rows) return 32;
-    if ((type == kTypeQ4_K || type == kTypeMXFP4) && M <= 512 && ((M + 127) / 128) * ((N + 127) / 128) <= 128) return 32;
-    // the 128 x 256 tiles of the other formats: up to 128 rows when they would be very few (Q8_0 128 x 4096 x 4096: 48 -> 27 us)
-    if (wide_128_row_tiles(type) && M <= 128 && ((M + 127) / 128) * ((N + 255) / 256) <= 32) return 32;
+    const int ktw = slim_ktw<G>(nkt), kc = (nkt + 8 * ktw - 1) / (8 * ktw), cus = device_info().num_cus;
+    const int64_t segments = (int64_t)((M + 31) / 32) * kc, units = segments * ((N + 31) / 32);
+    const bool crosses = segments > 1 && units > cus && units % cus != 0;
+    return 5.0 + (double)((units + cus - 1) / cus) * (1.6 + 0.35 * ktw) + (crosses ? 8.0 : 0.0) + chunk_sum_us(kc, M, N);
+}
+
+// and of the 256 x 256 tiles of gemm_kernel / gemm_xw_kernel: 2.0 us per k-tile and round with all CUs at work
+double tile256_us(int M, int N, int nkt)
+{
+    const int cus = device_info().num_cus;
+    const int tiles = ((M + 255) / 256) * ((N + 255) / 256), kc = pick_k_chunks(tiles, nkt, cus, (int64_t)M * N, 1.7);
+    const int64_t units = (int64_t)tiles * kc, rounds = (units + cus - 1) / cus;
+    const double fill = (double)units / (double)(rounds * cus);
+    return (double)rounds * (nkt / (double)kc * 2.0 * (0.5 + 0.5 * fill) + 3.0) + chunk_sum_us(kc, M, N);
+}
+
+// Q4_K, Q8_0 and Q6_K: the cheapest of the three by these models, which were fitted to calls of 40 .. 2048 rows on
+// 1024 x 4096, 4096 x 4096, 4096 x 14336, 5120 x 2560, 14336 x 4096 and 21504 x 5376 weights.  The register-resident kernel
+// keeps few rows and narrow weights (Q4_K 64 x 4096 x 4096 18.0 vs 21.8 us, Q6_K 200 x 1024 x 4096 25.2 vs 29.7), the
+// 256-row tiles keep many rows of wide weights (Q4_K 2048 x 21504 x 5376 494 vs 567 us, Q8_0 700 x 14336 x 4096 121 vs 138):
+// they take half as many weight lines per result.
+template <typename G, typename W>
+int cheapest_tiles(int M, int N, int K)
+{
+    const int nkt = (K + kBK - 1) / kBK;
+    const double wide = pick_wide(M, N, nkt, true, W::kUsBase, W::kUsRow).us, slim = slim_us<G>(M, N, nkt);
+    const double tile = std::is_same<G, GQ6K>::value ? wide : tile256_us(M, N, nkt);       // (no 256-row tiles of Q6_K)
+    if (slim <= wide && slim <= tile) return 32;
+    return wide <= tile ? kWideTiles : 256;
+}
+}  // namespace
+
+int gemm_tile_m(int type, int M, int N, int K)
+{
+    if (M > 3) {
+        if (type == kTypeQ4_K) return cheapest_tiles<GQ4K, WQ4K>(M, N, K);
+        if (type == kTypeQ8_0) return cheapest_tiles<GQ80, WQ80>(M, N, K);
+        if (type == kTypeQ6_K) return cheapest_tiles<GQ6K, WQ6K>(M, N, K);
+    }
+    if (M <= 128) return 32;
+    if (type == kTypeMXFP4 && M <= 512 && ((M + 127) / 128) * ((N + 127) / 128) <= 128) return 32;
     // 128- or 256-row tiles by rounds of workgroups x time per k-tile of a round (measured per k-tile: a 256 x 256 tile
     // 2.0 us; two co-resident 128 x 128 tiles of the 4-bit formats 1.37 us; one 128 x 256 tile of the other formats
-    // 1.4 us).  The model reproduces the measured crossovers (Q4_K, us, 128 / 256 rows): 1024 x 14336 x 4096 196 / 160,
-    // 512 x 28672 x 4096 191 / 158, 600 x 21504 x 5376 221 / 198, 512 x 14336 x 4096 94 / 105, MXFP4 512 x 5760 x 2880
-    // 52 / 88.
+    // 1.4 us; MXFP4 512 x 5760 x 2880, us, 128 / 256 rows: 52 / 88).
     const int cus = device_info().num_cus;
     const bool two_per_cu = !wide_128_row_tiles(type);                    // 128 x 128 tiles, two workgroups per CU
     const int64_t tiles256 = (int64_t)((M + 255) / 256) * ((N + 255) / 256);
@@ -3244,6 +3875,7 @@ bool launch_convert(int type, const ConvertSrc& src, int M, int K, void* workspa
                            x_row_halfs(K), chunks, x16, scales);
         return hip_ok(hipGetLastError(), "activation convert launch");
     }
+    if (layout == 2) type = kTypeQ8_0;      // natural order
     // three activation orders: the K-quant nibble order, the split-nibble order of the 32-weight blocks, natural
     switch (type) {
     case kTypeQ4_K: case kTypeQ5_K: launch_convert_typed<kTypeQ4_K, SRC>(src, M, K, kp, x16, scales, stream); break;
@@ -3265,8 +3897,9 @@ bool launch_convert(int type, const ConvertSrc& src, int M, int K, void* workspa
 // 32 x 184320 x 2880 61-67 vs 74-84 us)
 int gemm_x_layout(int type, int M, int N, int K)
 {
+    if (type == kTypeQ4_K) return gemm_tile_m(type, M, N, K) == kWideTiles ? 2 : 0;
     if (type != kTypeMXFP4 || K > 1024 * kCvtHold * 4) return 0;
-    return gemm_tile_m(type, M, N) >= 128 || (int64_t)N * K >= ((int64_t)64 << 20) ? 1 : 0;
+    return gemm_tile_m(type, M, N, K) >= 128 || (int64_t)N * K >= ((int64_t)64 << 20) ? 1 : 0;
 }
 
 bool launch_convert_x(int type, const float* x, int64_t ldx, const int* row_map, int M, int K, void* workspace,
@@ -3333,9 +3966,12 @@ bool gemm_dispatch(int type, const void* w, int64_t w_bytes, const void* workspa
         bm = tiles->bm;
         m_tiles = tiles->count;
     } else {
-        bm = gemm_tile_m(type, M, N);
-        if (type == kTypeQ6_K && bm == 256) bm = 128;     // two raw Q6_K super-tiles of 256 columns do not fit LDS
-        m_tiles = (M + bm - 1) / bm;
+        bm = gemm_tile_m(type, M, N, K);
+        if (type == kTypeQ4_K && (bm == kWideTiles) != (x_layout == 2)) {
+            set_last_error("gemm: the activations are not in the order that this launch reads (gemm_x_layout).");
+            return false;
+        }
+        m_tiles = bm == kWideTiles ? 1 : (M + bm - 1) / bm;
     }
     if (m_tiles == 0) return true;
     switch (type) {

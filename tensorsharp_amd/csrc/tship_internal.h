@@ -146,15 +146,15 @@ bool launch_gemv_group(int type, int count, const GemvArgs* args, hipStream_t st
 // ---- prefill GEMM ---------------------------------------------------------------------------
 // Workspace layout: [M floats of row scales, padded to 256 B][M x Kp fp16 activations].
 size_t gemm_workspace_bytes(int M, int K);
-int gemm_tile_m(int type, int M, int N);   // rows of activations per tile for a plain (ungrouped) launch
+int gemm_tile_m(int type, int M, int N, int K);   // rows of activations per tile for a plain (ungrouped) launch (0: gemm_wide_kernel picks its own)
 
 // fp32 activations -> workspace (fp16 in the weight format's unpack order + per-row scales);
 // row_map (device, optional) gathers source rows.
 // norm_w (device, optional) applies RMSNorm first: x <- x / sqrt(mean(x^2) + eps) * norm_w.
 bool launch_convert_x(int type, const float* x, int64_t ldx, const int* row_map, int M, int K, void* workspace,
                       hipStream_t stream, const float* norm_w = nullptr, float eps = 0.f, int layout = 0);
-// layout of the converted activations the GEMM of this shape reads (plain launches): 0 fp16, 1 MX fp6 pairs (MXFP4 on the
-// block-scaled matrix instruction); pass it to launch_convert_x and to launch_gemm
+// layout of the converted activations the GEMM of this shape reads (plain launches): 0 fp16 in the format's unpack order,
+// 1 MX fp6 pairs (MXFP4 on the block-scaled matrix instruction), 2 fp16 in natural order (Q4_K on gemm_wide_kernel); pass it to launch_convert_x and to launch_gemm
 int gemm_x_layout(int type, int M, int N, int K);
 // The same for the activations of an expert's down projection: row m is SwiGLU-OAI of (gate | up)[m] (+ the bias
 // row of expert_of[m]), formed while it is read.

@@ -484,3 +484,37 @@ def test_narrow_results_are_formed_from_exact_weights(hip, oracle, name, M, N, K
     torch.cuda.synchronize()
     err = inputs.row_l2_err(y.cpu().numpy(), ref)         # fp16 operands would leave 1e-4 ... 1e-3 here
     assert err <= 1e-5, (name, M, N, K, err)
+
+
+@pytest.mark.parametrize("name,M,N,K", [
+    # 32 .. 128 rows per tile with a ragged last one, a ragged last column tile, whole K and K in chunks
+    ("q4_k", 33, 14800, 1024), ("q4_k", 97, 15000, 512), ("q4_k", 129, 8200, 256), ("q4_k", 160, 2100, 1280),
+    ("q4_k", 250, 4099, 2304), ("q4_k", 333, 1500, 4096),
+    # Q8_0 rows that begin at any even byte of a 16-byte piece; the last k-tile a single block; an odd number of k-tiles
+    ("q8_0", 40, 15000, 1056), ("q8_0", 250, 4099, 2080), ("q8_0", 333, 1500, 2592), ("q8_0", 250, 4100, 2112),
+    ("q6_k", 130, 14400, 512), ("q6_k", 250, 9000, 768), ("q6_k", 333, 2100, 2304), ("q6_k", 40, 15001, 1280),
+])
+def test_wide_tiles(hip, oracle, name, M, N, K):
+    # mid-sized calls: product, product added to a residual, and a scale outside the fp16 operands in the last k-tile
+    import torch
+    from tensorsharp_amd import QuantizedWeight
+    from oracle.oracle import Q6_K
+    t = {**T, "q6_k": Q6_K}[name]
+    rng = np.random.default_rng(M + N + K)
+    wq = q6k_weight(N, K, M) if name == "q6_k" else oracle.quantize(t, (rng.standard_normal(N * K) * 0.02).astype(np.float32))
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    y = run_device(hip, t, wq, N, K, x)
+    check(y, oracle.matmul_f64(t, wq, N, K, x), (name, M, N, K))
+    residual = rng.standard_normal((M, N)).astype(np.float32)
+    r = torch.from_numpy(residual).cuda()
+    hip.FusedMatMulQuantAdd(r, torch.from_numpy(x).cuda(), QuantizedWeight(torch.from_numpy(wq).cuda(), t, K, N))
+    # one fp32 addition (and, with K in chunks, the residual added first instead of last): a few ulp of the largest term
+    assert np.abs(r.cpu().numpy() - (residual + y)).max() <= 4e-6 * (np.abs(residual).max() + np.abs(y).max())
+    bad = wq.copy()
+    blocks, size, d_at = {"q4_k": (K // 256, 144, 0), "q8_0": (K // 32, 34, 0), "q6_k": (K // 256, 210, 208)}[name]
+    column = N - 1
+    at = (column * blocks + blocks - 1) * size + d_at
+    bad[at:at + 2] = np.frombuffer(np.float16(1.0).tobytes(), np.uint8)
+    z = run_device(hip, t, bad, N, K, x)
+    assert np.isnan(z[:, column]).all()
+    assert np.array_equal(z[:, :column], y[:, :column])
