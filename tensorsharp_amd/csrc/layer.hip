@@ -117,11 +117,13 @@ __global__ void __launch_bounds__(kAttnWaves * 64) attn_decode_kernel(float* k_c
         if (blockIdx.z == 0) {
             for (int i = (int)threadIdx.x * 4; i < pre_floats; i += kAttnWaves * 64 * 4) {
                 typedef float f4_t __attribute__((ext_vector_type(4)));
-                f4_t a, b;                                     // never used: the loads are for the caches
-                if (pre0) asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(a) : "v"(pre0 + i) : "memory");
-                if (pre1) asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(b) : "v"(pre1 + i) : "memory");
+                // ordinary loads with a use that costs nothing: the compiler owns their registers and waits (written in
+                // asm, a load in flight could land in registers that already hold the next address)
+                f4_t a = {0.f, 0.f, 0.f, 0.f}, b = a;
+                if (pre0) a = *reinterpret_cast<const f4_t*>(pre0 + i);
+                if (pre1) b = *reinterpret_cast<const f4_t*>(pre1 + i);
+                asm volatile("" ::"v"(a), "v"(b));
             }
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         }
         return;
     }
