@@ -386,19 +386,20 @@ __global__ void __launch_bounds__(kAttnWaves * 64) attn_decode_kernel(float* k_c
     }
 }
 
-// one workgroup per head: wavefront w merges splits w, w + 4, ... (four rows in flight), the wavefronts meet in LDS
-__global__ void __launch_bounds__(kAttnWaves * 64) attn_combine_kernel(const float* __restrict__ partial, int splits, int head_dim,
+// one workgroup per head: wavefront w merges splits w, w + WAVES, ... (four rows in flight), the wavefronts meet in LDS
+template <int WAVES>
+__global__ void __launch_bounds__(WAVES * 64) attn_combine_kernel(const float* __restrict__ partial, int splits, int head_dim,
                                                                         float* __restrict__ out)
 {
     constexpr int kPer = kMaxHeadDim / 64, kRow = kMaxHeadDim + 2;
-    __shared__ float sacc[kAttnWaves][kMaxHeadDim], sl[kAttnWaves];
+    __shared__ float sacc[WAVES][kMaxHeadDim], sl[WAVES];
     const int h = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const float* base = partial + (int64_t)h * splits * kRow;
     float ms[4], ls[4], v[4][kPer];
     auto load_rows = [&](int s0) {
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-            const int s = s0 + u * kAttnWaves;
+            const int s = s0 + u * WAVES;
             const bool live = s < splits;
             const float* p = base + (int64_t)(live ? s : s0) * kRow;
             ms[u] = live ? p[0] : -INFINITY;
@@ -410,10 +411,10 @@ __global__ void __launch_bounds__(kAttnWaves * 64) attn_combine_kernel(const flo
             }
         }
     };
-    // When one batch of rows per wavefront covers the splits (up to 1024 positions), it is requested before the maximum
-    // over all splits is worked out (every wavefront computes it: independent loads, one pass), so that the two round
-    // trips overlap: 0.35 us per layer.  (With more batches the early request measured 0.3 us slower.)
-    constexpr int kBatch = 4 * kAttnWaves;
+    // When one batch of rows per wavefront covers the splits (16 of four wavefronts, 64 of sixteen), it is requested before
+    // the maximum over all splits is worked out (every wavefront computes it: independent loads, one pass), so that the two
+    // round trips overlap: 0.35 us per layer.  (With more batches the early request measured 0.3 us slower.)
+    constexpr int kBatch = 4 * WAVES;
     const bool early = splits <= kBatch;
     if (early && wave < splits) load_rows(wave);
     float mm = -INFINITY;
@@ -440,13 +441,13 @@ __global__ void __launch_bounds__(kAttnWaves * 64) attn_combine_kernel(const flo
     if (wave == 0) {
         float lt = 0.f;
 #pragma unroll
-        for (int w = 0; w < kAttnWaves; ++w) lt += sl[w];
+        for (int w = 0; w < WAVES; ++w) lt += sl[w];
 #pragma unroll
         for (int j = 0; j < kPer; ++j) {
             const int d = lane + 64 * j;
             float a = 0.f;
 #pragma unroll
-            for (int w = 0; w < kAttnWaves; ++w) a += sacc[w][d];
+            for (int w = 0; w < WAVES; ++w) a += sacc[w][d];
             if (d < head_dim) out[(int64_t)h * head_dim + d] = a / lt;
         }
     }
@@ -527,7 +528,12 @@ bool launch_attention_decode(const float* qkv, const float* q_norm_w, const floa
 #undef TSHIP_ATTN_LAUNCH
     if (!hip_ok(hipGetLastError(), "attention launch")) return false;
     if (splits == 1) return true;
-    hipLaunchKernelGGL(attn_combine_kernel, dim3(num_heads), dim3(kAttnWaves * 64), 0, stream, partial_ws, splits, head_dim, out);
+    // Four wavefronts request up to 16 splits' rows in one round trip; more splits take sixteen, which cover 64, instead of
+    // further dependent trips (32 splits, 32 heads: three layers at 4001 positions 196.5 -> 194.8 us).
+    if (splits <= 16)
+        hipLaunchKernelGGL(attn_combine_kernel<4>, dim3(num_heads), dim3(4 * 64), 0, stream, partial_ws, splits, head_dim, out);
+    else
+        hipLaunchKernelGGL(attn_combine_kernel<16>, dim3(num_heads), dim3(16 * 64), 0, stream, partial_ws, splits, head_dim, out);
     return hip_ok(hipGetLastError(), "attention combine launch");
 }
 

@@ -167,6 +167,13 @@ def test_head_shapes_groupings_and_split_counts(hip, oracle, heads, kv_heads, he
         assert rel(kd.cpu().numpy()[:, pos], kc[:, pos]) <= 1e-5 and rel(vd.cpu().numpy()[:, pos], vc[:, pos]) <= 1e-5
 
 
+@pytest.mark.parametrize("head_dim,prefix", [(64, 1023), (256, 1023), (128, 8191)])
+def test_split_merge_on_few_and_many_wavefronts(hip, oracle, head_dim, prefix):
+    # the merge takes 4 wavefronts up to 16 splits and 16 beyond (positions 1023 -> 1024), and a second batch of rows from
+    # 65 splits on (positions 8191 -> 8192)
+    test_head_shapes_groupings_and_split_counts(hip, oracle, 2, 1, head_dim, 2, prefix)
+
+
 @pytest.mark.parametrize("head_dim", [64, 80, 96, 128, 192, 256])
 @pytest.mark.parametrize("group,kv_heads,prefix", [(1, 4, 70), (4, 8, 2100), (8, 8, 2100)])
 def test_every_attention_instantiation(hip, oracle, head_dim, group, kv_heads, prefix):
