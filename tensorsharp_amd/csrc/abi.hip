@@ -323,10 +323,14 @@ struct MatmulPlan {
     bool narrow;          // few result columns: fp32 copy of the weight + the dense kernel
     int m_step;           // activation rows per launch
     int64_t n_step;       // weight rows per launch
+    GemmPlan gemm;        // prefill: how a launch over a whole slice runs
     size_t conv_bytes;    // [row scales][fp16 activations] of one slice of rows (prefill), or the RMSNorm rows (decode)
     size_t chunk_bytes;   // sums of K chunks of one launch
     size_t total() const { return conv_bytes + chunk_bytes; }
 };
+
+// norm: RMSNorm prologue on the activations; accumulate: the product is added to the result.  One plan serves the size of a
+// call's workspace, its conversions and its launches.
 
 MatmulPlan plan_matmul(int type, int M, int64_t K, int64_t N, bool norm, bool accumulate)
 {
@@ -367,20 +371,15 @@ MatmulPlan plan_matmul(int type, int M, int64_t K, int64_t N, bool norm, bool ac
     p.m_step = (int)std::min<int64_t>(M, std::max<int64_t>(256, ((kMaxOperandBytes - 1) / (int64_t)(kp * 2)) / 256 * 256));
     p.conv_bytes = al(gemm_workspace_bytes(p.m_step, (int)K));
     // the launches of a call differ only in their last, smaller slices: the first one needs the most
-    p.chunk_bytes = al(gemm_chunk_ws_bytes(type, p.m_step, (int)std::min<int64_t>(N, p.n_step), (int)K, nullptr, accumulate));
+    p.gemm = plan_gemm(type, p.m_step, (int)std::min<int64_t>(N, p.n_step), (int)K, accumulate);
+    p.chunk_bytes = al(p.gemm.chunk_bytes);
     return p;
 }
 
-// bytes of device workspace one matmul needs (norm: RMSNorm prologue on the activations)
-size_t matmul_ws_bytes(int type, int M, int64_t K, int64_t N, bool norm, bool accumulate)
-{
-    return plan_matmul(type, M, K, N, norm, accumulate).total();
-}
-
-// result (+)= f(m1) * W^T with f = identity or RMSNorm(eps) * norm_w.  All pointers are device pointers; `ws` has
-// ws_bytes >= matmul_ws_bytes() bytes (with fewer, the K-chunk sums are given up first: see launch_gemm).
-bool run_matmul_device_ws(const TSHipTensorView2D& result, const TSHipTensorView2D& m1, const void* w, int type, int64_t K,
-                          int64_t N, hipStream_t stream, void* ws, size_t ws_bytes, const float* norm_w, float eps, bool accumulate)
+// result (+)= f(m1) * W^T with f = identity or RMSNorm(eps) * norm_w, as `plan` (of the same call) says.  All pointers are
+// device pointers; `ws` has ws_bytes >= plan.total() bytes (with fewer, the K-chunk sums are given up first: see launch_gemm).
+bool run_matmul_device_ws(const MatmulPlan& plan, const TSHipTensorView2D& result, const TSHipTensorView2D& m1, const void* w, int type,
+                          int64_t K, int64_t N, hipStream_t stream, void* ws, size_t ws_bytes, const float* norm_w, float eps, bool accumulate)
 {
     const size_t rs = row_size(type, K);
     if (!check_device_operands(m1, w, type)) return false;
@@ -389,7 +388,6 @@ bool run_matmul_device_ws(const TSHipTensorView2D& result, const TSHipTensorView
         return false;
     }
     const int M = m1.dim0;
-    const MatmulPlan plan = plan_matmul(type, M, K, N, norm_w != nullptr, accumulate);
     if (plan.conv_bytes > ws_bytes) {
         set_last_error("matmul: the device workspace is too small for the converted activations.");
         return false;
@@ -446,26 +444,27 @@ bool run_matmul_device_ws(const TSHipTensorView2D& result, const TSHipTensorView
         int converted = -1;         // activation layout in the workspace (row slices of an over-large weight may differ)
         for (int64_t n0 = 0; n0 < N; n0 += plan.n_step) {
             const int64_t n = std::min<int64_t>(plan.n_step, N - n0);
-            const int layout = gemm_x_layout(type, m, (int)n, (int)K);
-            if (layout != converted) {
-                if (!launch_convert_x(type, x, m1.stride0, nullptr, m, (int)K, ws, stream, norm_w, eps, layout)) return false;
-                converted = layout;
+            const bool whole = m == plan.m_step && n == std::min<int64_t>(N, plan.n_step);
+            const GemmPlan g = whole ? plan.gemm : plan_gemm(type, m, (int)n, (int)K, accumulate);
+            if (g.x_layout != converted) {
+                if (!launch_convert_x(type, x, m1.stride0, nullptr, m, (int)K, ws, stream, norm_w, eps, g.x_layout)) return false;
+                converted = g.x_layout;
             }
-            if (!launch_gemm(type, wb + (size_t)n0 * rs, (int64_t)(rs * (size_t)n), ws, out + (int64_t)m0 * result.stride0 + n0,
-                             result.stride0, nullptr, m, (int)n, (int)K, nullptr, stream, accumulate, chunk_ws, chunk_bytes, layout))
+            if (!launch_gemm(type, g, wb + (size_t)n0 * rs, (int64_t)(rs * (size_t)n), ws, out + (int64_t)m0 * result.stride0 + n0,
+                             result.stride0, m, (int)n, (int)K, stream, accumulate, chunk_ws, chunk_bytes))
                 return false;
         }
     }
     return true;
 }
 
-bool run_matmul_device(const TSHipTensorView2D& result, const TSHipTensorView2D& m1, const void* w, int type, int64_t K,
-                       int64_t N, hipStream_t stream)
+bool run_matmul_device(const TSHipTensorView2D& result, const TSHipTensorView2D& m1, const void* w, int type, int64_t K, int64_t N,
+                       hipStream_t stream, const float* norm_w = nullptr, float eps = 0.f, bool accumulate = false)
 {
-    const size_t need = matmul_ws_bytes(type, m1.dim0, K, N, false, false);
-    WsLease ws(stream, need);
+    const MatmulPlan plan = plan_matmul(type, m1.dim0, K, N, norm_w != nullptr, accumulate);
+    WsLease ws(stream, plan.total());
     if (!ws.ok()) return false;
-    return run_matmul_device_ws(result, m1, w, type, K, N, stream, ws.ptr(), need, nullptr, 0.f, false);
+    return run_matmul_device_ws(plan, result, m1, w, type, K, N, stream, ws.ptr(), plan.total(), norm_w, eps, accumulate);
 }
 
 // ---- static device scratch of the entry point that allocates nothing ---------------------------
@@ -499,22 +498,31 @@ unsigned char* scratch_ptr()
 
 // FFN of the fused entry points on device operands (ggml_ops_fused.cpp:390-640):
 //   residual += W_down * ( silu(g) * u ),  [g | u] = W_gate_up * (RMSNorm(input) * norm_w)
-// `ws` has ffn_ws_bytes() bytes.
-size_t ffn_ws_bytes(int M, int gu_type, int dn_type, int hidden, int half)
+// `ws` has plan.total bytes.
+struct FfnPlan {
+    MatmulPlan gu, dn;
+    size_t gu_bytes, act_bytes, mm_bytes, total;      // [gate | up rows][gated rows][workspace of either matmul]
+};
+
+FfnPlan plan_ffn(int M, int gu_type, int dn_type, int hidden, int half)
 {
     auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
-    return al((size_t)M * 2 * half * sizeof(float)) + al((size_t)M * half * sizeof(float)) +
-           std::max(matmul_ws_bytes(gu_type, M, hidden, 2 * (int64_t)half, true, false), matmul_ws_bytes(dn_type, M, half, hidden, false, true));
+    FfnPlan p{};
+    p.gu = plan_matmul(gu_type, M, hidden, 2 * (int64_t)half, true, false);
+    p.dn = plan_matmul(dn_type, M, half, hidden, false, true);
+    p.gu_bytes = al((size_t)M * 2 * half * sizeof(float));
+    p.act_bytes = al((size_t)M * half * sizeof(float));
+    p.mm_bytes = std::max(p.gu.total(), p.dn.total());
+    p.total = p.gu_bytes + p.act_bytes + p.mm_bytes;
+    return p;
 }
 
-bool run_ffn_swiglu_device(const TSHipTensorView2D& residual, const TSHipTensorView2D& input, const float* norm_w, float eps,
-                           const void* gate_up, int gu_type, const void* down, int dn_type, int hidden, int half,
+bool run_ffn_swiglu_device(const FfnPlan& plan, const TSHipTensorView2D& residual, const TSHipTensorView2D& input, const float* norm_w,
+                           float eps, const void* gate_up, int gu_type, const void* down, int dn_type, int hidden, int half,
                            hipStream_t stream, char* ws)
 {
     const int M = input.dim0;
-    const size_t gu_bytes = ((size_t)M * 2 * half * sizeof(float) + 255) & ~(size_t)255;
-    const size_t act_bytes = ((size_t)M * half * sizeof(float) + 255) & ~(size_t)255;
-    const size_t mm_bytes = ffn_ws_bytes(M, gu_type, dn_type, hidden, half) - gu_bytes - act_bytes;
+    const size_t gu_bytes = plan.gu_bytes, act_bytes = plan.act_bytes, mm_bytes = plan.mm_bytes;
     float* gu = reinterpret_cast<float*>(ws);
     float* act = reinterpret_cast<float*>(ws + gu_bytes);
     void* mm_ws = ws + gu_bytes + act_bytes;
@@ -543,10 +551,10 @@ bool run_ffn_swiglu_device(const TSHipTensorView2D& residual, const TSHipTensorV
         return true;
     }
     const TSHipTensorView2D gu_view{gu, M, 2 * half, 2 * half, 1, (int64_t)((size_t)M * 2 * half * sizeof(float))};
-    if (!run_matmul_device_ws(gu_view, input, gate_up, gu_type, hidden, 2 * half, stream, mm_ws, mm_bytes, norm_w, eps, false)) return false;
+    if (!run_matmul_device_ws(plan.gu, gu_view, input, gate_up, gu_type, hidden, 2 * half, stream, mm_ws, mm_bytes, norm_w, eps, false)) return false;
     if (!launch_silu_mul(gu, 2 * half, M, half, act, stream)) return false;
     const TSHipTensorView2D act_view{act, M, half, half, 1, (int64_t)((size_t)M * half * sizeof(float))};
-    return run_matmul_device_ws(residual, act_view, down, dn_type, half, hidden, stream, mm_ws, mm_bytes, nullptr, 0.f, true);
+    return run_matmul_device_ws(plan.dn, residual, act_view, down, dn_type, half, hidden, stream, mm_ws, mm_bytes, nullptr, 0.f, true);
 }
 
 // ---- a weighted set of expert FFNs on device operands ------------------------------------------
@@ -604,9 +612,9 @@ ExpertSetLayout expert_set_layout(int M, int n, const ExpertFfn* ex, int H, int 
     L.tmp_off = L.dn_off + (size_t)n * L.dn_stride * sizeof(float);
     L.mm_off = L.tmp_off + al((size_t)M * I * sizeof(float));
     for (int e = 0; e < n; ++e) {
-        if (ex[e].gate) L.mm_bytes = std::max(L.mm_bytes, matmul_ws_bytes(ex[e].gate_type, M, H, I, false, false));
-        L.mm_bytes = std::max(L.mm_bytes, matmul_ws_bytes(ex[e].up_type, M, H, I, false, false));
-        L.mm_bytes = std::max(L.mm_bytes, matmul_ws_bytes(ex[e].down_type, M, I, N, false, false));
+        if (ex[e].gate) L.mm_bytes = std::max(L.mm_bytes, plan_matmul(ex[e].gate_type, M, H, I, false, false).total());
+        L.mm_bytes = std::max(L.mm_bytes, plan_matmul(ex[e].up_type, M, H, I, false, false).total());
+        L.mm_bytes = std::max(L.mm_bytes, plan_matmul(ex[e].down_type, M, I, N, false, false).total());
     }
     L.total = L.mm_off + L.mm_bytes;
     // the tiled form
@@ -639,7 +647,7 @@ ExpertSetLayout expert_set_layout(int M, int n, const ExpertFfn* ex, int H, int 
     const GemmTiles plan_tiles{nullptr, nullptr, nullptr, max_tiles, L.bm, 0};
     for (int e = 0; e < n; ++e) {
         auto need = [&](int type, int nn, int kk) {
-            return gemm_chunk_ws_bytes(type, (int)rows, nn, kk, &plan_tiles, false, expert_tiles_x_layout(type, L.bm, kk, nn));
+            return gemm_tiles_ws_bytes(type, plan_tiles, (int)rows, nn, kk, expert_tiles_x_layout(type, L.bm, kk, nn));
         };
         if (ex[e].gate) L.chunk_bytes = std::max(L.chunk_bytes, need(ex[e].gate_type, I, H));
         L.chunk_bytes = std::max(L.chunk_bytes, need(ex[e].up_type, I, H));
@@ -691,8 +699,8 @@ bool run_expert_linear_tiled(const ExpertSetLayout& L, char* ws, int n, int M, c
         if (!launch_convert_x(t, x, ldx, gather ? row_map : nullptr, rows, K, ws + x_off, stream, nullptr, 0.f, layout)) return false;
         GemmTiles tiles{t_expert, t_row0, t_rows, spec.count * per, L.bm, (int64_t)(row_size(t, K) * (size_t)out_features)};
         tiles.expert_off = offs;
-        if (!launch_gemm(t, reinterpret_cast<const void*>(base), tiles.expert_stride, ws + x_off, c, ldc, nullptr, rows, out_features, K, &tiles,
-                         stream, false, L.chunk_bytes ? ws + L.chunk_off : nullptr, L.chunk_bytes, layout))
+        if (!launch_gemm_tiles(t, tiles, reinterpret_cast<const void*>(base), tiles.expert_stride, ws + x_off, c, ldc, nullptr, rows,
+                               out_features, K, stream, L.chunk_bytes ? ws + L.chunk_off : nullptr, L.chunk_bytes, layout))
             return false;
     }
     return true;
@@ -801,16 +809,16 @@ bool run_expert_set_device(const TSHipTensorView2D& out, const float* base, int6
                 const int64_t span = (int64_t)(((size_t)(M - 1) * 2 * I + I) * sizeof(float));
                 const TSHipTensorView2D g_view{a_e, M, I, 2 * I, 1, span};
                 const TSHipTensorView2D u_view{a_e + I, M, I, 2 * I, 1, span};
-                if (!run_matmul_device_ws(g_view, x, ex[e].gate, ex[e].gate_type, H, I, stream, mm_ws, L.mm_bytes, nullptr, 0.f, false)) return false;
-                if (!run_matmul_device_ws(u_view, x, ex[e].up, ex[e].up_type, H, I, stream, mm_ws, L.mm_bytes, nullptr, 0.f, false)) return false;
+                if (!run_matmul_device_ws(plan_matmul(ex[e].gate_type, M, H, I, false, false), g_view, x, ex[e].gate, ex[e].gate_type, H, I, stream, mm_ws, L.mm_bytes, nullptr, 0.f, false)) return false;
+                if (!run_matmul_device_ws(plan_matmul(ex[e].up_type, M, H, I, false, false), u_view, x, ex[e].up, ex[e].up_type, H, I, stream, mm_ws, L.mm_bytes, nullptr, 0.f, false)) return false;
                 if (!launch_silu_mul(a_e, 2 * I, M, I, tmp, stream)) return false;
                 const TSHipTensorView2D t_view{tmp, M, I, I, 1, (int64_t)((size_t)M * I * sizeof(float))};
-                if (!run_matmul_device_ws(d_view, t_view, ex[e].down, ex[e].down_type, I, N, stream, mm_ws, L.mm_bytes, nullptr, 0.f, false)) return false;
+                if (!run_matmul_device_ws(plan_matmul(ex[e].down_type, M, I, N, false, false), d_view, t_view, ex[e].down, ex[e].down_type, I, N, stream, mm_ws, L.mm_bytes, nullptr, 0.f, false)) return false;
             } else {
                 const TSHipTensorView2D u_view{a_e, M, I, I, 1, (int64_t)((size_t)M * I * sizeof(float))};
-                if (!run_matmul_device_ws(u_view, x, ex[e].up, ex[e].up_type, H, I, stream, mm_ws, L.mm_bytes, nullptr, 0.f, false)) return false;
+                if (!run_matmul_device_ws(plan_matmul(ex[e].up_type, M, H, I, false, false), u_view, x, ex[e].up, ex[e].up_type, H, I, stream, mm_ws, L.mm_bytes, nullptr, 0.f, false)) return false;
                 if (!launch_relu_sqr(a_e, (int64_t)M * I, stream)) return false;
-                if (!run_matmul_device_ws(d_view, u_view, ex[e].down, ex[e].down_type, I, N, stream, mm_ws, L.mm_bytes, nullptr, 0.f, false)) return false;
+                if (!run_matmul_device_ws(plan_matmul(ex[e].down_type, M, I, N, false, false), d_view, u_view, ex[e].down, ex[e].down_type, I, N, stream, mm_ws, L.mm_bytes, nullptr, 0.f, false)) return false;
             }
         }
     }
@@ -1180,17 +1188,23 @@ bool validate_outproj_ffn(const TSHipTensorView2D& residual, const TSHipTensorVi
     return true;
 }
 
-size_t outproj_ffn_ws_bytes(int M, const WeightDesc& out_w, const WeightDesc& gu, const WeightDesc& dn, int hidden, int half)
+struct OutprojFfnPlan {
+    MatmulPlan out;
+    FfnPlan ffn;
+    size_t total() const { return std::max(out.total(), ffn.total); }
+};
+
+OutprojFfnPlan plan_outproj_ffn(int M, const WeightDesc& out_w, const WeightDesc& gu, const WeightDesc& dn, int hidden, int half)
 {
-    return std::max(matmul_ws_bytes(out_w.type, M, out_w.ne0, out_w.ne1, false, true), ffn_ws_bytes(M, gu.type, dn.type, hidden, half));
+    return OutprojFfnPlan{plan_matmul(out_w.type, M, out_w.ne0, out_w.ne1, false, true), plan_ffn(M, gu.type, dn.type, hidden, half)};
 }
 
-bool run_outproj_ffn_device(const TSHipTensorView2D& residual, const TSHipTensorView2D& input, const void* out_w, const WeightDesc& od,
-                            const float* norm_w, float eps, const void* gu, int gu_type, const void* dn, int dn_type, int half,
-                            hipStream_t stream, char* ws, size_t ws_bytes)
+bool run_outproj_ffn_device(const OutprojFfnPlan& plan, const TSHipTensorView2D& residual, const TSHipTensorView2D& input, const void* out_w,
+                            const WeightDesc& od, const float* norm_w, float eps, const void* gu, int gu_type, const void* dn, int dn_type,
+                            int half, hipStream_t stream, char* ws)
 {
-    if (!run_matmul_device_ws(residual, input, out_w, od.type, od.ne0, od.ne1, stream, ws, ws_bytes, nullptr, 0.f, true)) return false;
-    return run_ffn_swiglu_device(residual, residual, norm_w, eps, gu, gu_type, dn, dn_type, residual.dim1, half, stream, ws);
+    if (!run_matmul_device_ws(plan.out, residual, input, out_w, od.type, od.ne0, od.ne1, stream, ws, plan.total(), nullptr, 0.f, true)) return false;
+    return run_ffn_swiglu_device(plan.ffn, residual, residual, norm_w, eps, gu, gu_type, dn, dn_type, residual.dim1, half, stream, ws);
 }
 
 bool validate_outproj_router(const TSHipTensorView2D& residual, const TSHipTensorView2D& input, const WeightDesc& out_w, const void* norm_w,
@@ -1208,26 +1222,32 @@ bool validate_outproj_router(const TSHipTensorView2D& residual, const TSHipTenso
     return true;
 }
 
-size_t outproj_router_ws_bytes(int M, const WeightDesc& out_w, const WeightDesc& router)
+struct OutprojRouterPlan {
+    MatmulPlan out, router;
+    size_t total() const { return std::max(out.total(), router.total()); }
+};
+
+OutprojRouterPlan plan_outproj_router(int M, const WeightDesc& out_w, const WeightDesc& router)
 {
-    return std::max(matmul_ws_bytes(out_w.type, M, out_w.ne0, out_w.ne1, false, true), matmul_ws_bytes(router.type, M, router.ne0, router.ne1, false, false));
+    return OutprojRouterPlan{plan_matmul(out_w.type, M, out_w.ne0, out_w.ne1, false, true), plan_matmul(router.type, M, router.ne0, router.ne1, false, false)};
 }
 
 // residual += input * W_out^T; normed_out = RMSNorm(residual) * norm_w; router_out = normed_out * W_router^T
 // (ggml_ops_fused.cpp:1310-1330).  normed_out must be a contiguous [M x hidden] device view.
-bool run_outproj_router_device(const TSHipTensorView2D& residual, const TSHipTensorView2D& input, const void* out_w, const WeightDesc& od,
-                               const float* norm_w, float eps, const TSHipTensorView2D& normed_out, const void* router_w,
-                               const WeightDesc& rd, const TSHipTensorView2D& router_out, hipStream_t stream, char* ws, size_t ws_bytes)
+bool run_outproj_router_device(const OutprojRouterPlan& plan, const TSHipTensorView2D& residual, const TSHipTensorView2D& input, const void* out_w,
+                               const WeightDesc& od, const float* norm_w, float eps, const TSHipTensorView2D& normed_out, const void* router_w,
+                               const WeightDesc& rd, const TSHipTensorView2D& router_out, hipStream_t stream, char* ws)
 {
     if (normed_out.stride1 != 1 || (normed_out.dim0 > 1 && normed_out.stride0 != normed_out.dim1) || router_out.stride1 != 1) {
         set_last_error("fused_outproj_norm_router: normedOut must be contiguous and routerOut a standard view on the device.");
         return false;
     }
-    if (!run_matmul_device_ws(residual, input, out_w, od.type, od.ne0, od.ne1, stream, ws, ws_bytes, nullptr, 0.f, true)) return false;
+    const size_t ws_bytes = plan.total();
+    if (!run_matmul_device_ws(plan.out, residual, input, out_w, od.type, od.ne0, od.ne1, stream, ws, ws_bytes, nullptr, 0.f, true)) return false;
     if (!launch_rms_norm_rows(static_cast<const float*>(residual.data), residual.stride0, norm_w, eps, residual.dim0, residual.dim1,
                               static_cast<float*>(normed_out.data), stream))
         return false;
-    return run_matmul_device_ws(router_out, normed_out, router_w, rd.type, rd.ne0, rd.ne1, stream, ws, ws_bytes, nullptr, 0.f, false);
+    return run_matmul_device_ws(plan.router, router_out, normed_out, router_w, rd.type, rd.ne0, rd.ne1, stream, ws, ws_bytes, nullptr, 0.f, false);
 }
 
 // ---- weighted expert sets (the bridge's per-token MoE calls) ------------------------------------
@@ -1387,6 +1407,27 @@ int TSHip_SetGemvTimeline(void* device_buffer, int64_t capacity_bytes)
     return 1;
 }
 
+int TSHip_MatmulPlanDevice(int m2_ggml_type, int rows, int64_t m2_ne0, int64_t m2_ne1, int accumulate, int64_t plan[4])
+{
+    return guarded(0, "matmul_plan", [&]() -> int {
+        if (!plan || rows <= 0 || m2_ne0 <= 0 || m2_ne0 > INT32_MAX || m2_ne1 <= 0 || !is_matmul_type(m2_ggml_type) ||
+            row_size(m2_ggml_type, m2_ne0) == 0) {
+            set_last_error("Invalid arguments for matmul_plan.");
+            return 0;
+        }
+        const MatmulPlan p = plan_matmul(m2_ggml_type, rows, m2_ne0, m2_ne1, false, accumulate != 0);
+        const bool dense = is_dense_type(m2_ggml_type) || m2_ggml_type == kTypeQ8_1 || p.narrow;
+        const int64_t sums = (int64_t)p.m_step * std::min<int64_t>(p.n_step, m2_ne1) * (int64_t)sizeof(float);
+        plan[0] = dense ? TSHIP_PLAN_DENSE : p.gemv ? TSHIP_PLAN_GEMV
+                  : p.gemm.bm == 0 ? TSHIP_PLAN_WIDE : p.gemm.bm == 32 ? TSHIP_PLAN_REGISTERS : TSHIP_PLAN_TILES;
+        plan[1] = dense || p.gemv ? 1 : p.gemm.bm == 0 ? 32 * p.gemm.wide_tm : p.gemm.bm;
+        plan[2] = dense || p.gemv ? 1 : std::max<int64_t>(1, (int64_t)p.gemm.chunk_bytes / sums);
+        plan[3] = (int64_t)p.total();
+        clear_last_error();
+        return 1;
+    });
+}
+
 int TSHip_DequantizeToF32Device(int ggml_type, const void* src, int64_t num_elements, float* dst)
 {
     return guarded(-1, "dequantize", [&]() -> int {
@@ -1450,7 +1491,8 @@ int TSHip_AddmmQuantF32DeviceNoAlloc(TSHipTensorView2D result, TSHipTensorView2D
         if (!validate_addmm_quant(result, m1, m2_data, m2_ggml_type, m2_ne0, m2_ne1, m2_raw_bytes)) return 0;
         if (!check_device_views(result, m1)) return 0;
         // [converted activations + row scales][sums of K chunks]: both live in the static array
-        const size_t need = plan_matmul(m2_ggml_type, m1.dim0, m2_ne0, m2_ne1, false, false).conv_bytes;
+        const MatmulPlan plan = plan_matmul(m2_ggml_type, m1.dim0, m2_ne0, m2_ne1, false, false);
+        const size_t need = plan.conv_bytes;
         if (need > kScratchBytes) {
             set_last_error("addmm_quant (no-alloc): the converted activations of this call (" + std::to_string(need) +
                            " bytes) exceed the static scratch buffer of " + std::to_string(kScratchBytes) +
@@ -1460,7 +1502,7 @@ int TSHip_AddmmQuantF32DeviceNoAlloc(TSHipTensorView2D result, TSHipTensorView2D
         unsigned char* ws = scratch_ptr();
         if (!ws) return 0;
         // what the converted activations leave of the array takes the sums of K chunks
-        if (!run_matmul_device_ws(result, m1, m2_data, m2_ggml_type, m2_ne0, m2_ne1, t_stream, ws, kScratchBytes, nullptr, 0.f, false))
+        if (!run_matmul_device_ws(plan, result, m1, m2_data, m2_ggml_type, m2_ne0, m2_ne1, t_stream, ws, kScratchBytes, nullptr, 0.f, false))
             return 0;
         clear_last_error();
         return 1;
@@ -1584,8 +1626,8 @@ int TSHip_MoEExpertsGptOssForwardF32Device(TSHipTensorView2D result, TSHipTensor
         const size_t o_gu = take((size_t)A * 2 * F * 4), o_dn = take((size_t)A * H * 4);
         const GemmTiles plan_tiles{nullptr, nullptr, nullptr, max_tiles, bm, 0};
         const size_t chunk_bytes = small ? 0
-                                         : std::max(gemm_chunk_ws_bytes(ggml_type, A, (int)(2 * F), (int)H, &plan_tiles, false, x_layout),
-                                                    gemm_chunk_ws_bytes(ggml_type, A, (int)H, (int)F, &plan_tiles, false, x_layout));
+                                         : std::max(gemm_tiles_ws_bytes(ggml_type, plan_tiles, A, (int)(2 * F), (int)H, x_layout),
+                                                    gemm_tiles_ws_bytes(ggml_type, plan_tiles, A, (int)H, (int)F, x_layout));
         const size_t o_chunk = take(chunk_bytes);
         WsLease lease(stream, off);
         if (!lease.ok()) return 0;
@@ -1646,8 +1688,8 @@ int TSHip_MoEExpertsGptOssForwardF32Device(TSHipTensorView2D result, TSHipTensor
                 if (!launch_gemm_swiglu_mx(gate_up_w, ws + o_ws1, ws + o_ws2, gu, gate_up_bias, alpha, limit, A, (int)F, (int)H, &tiles, stream))
                     return 0;
             } else {
-                if (!launch_gemm(ggml_type, gate_up_w, gu_bytes, ws + o_ws1, gu, 2 * F, nullptr, A, (int)(2 * F), (int)H, &tiles, stream,
-                                 false, ws + o_chunk, chunk_bytes, x_layout))
+                if (!launch_gemm_tiles(ggml_type, tiles, gate_up_w, gu_bytes, ws + o_ws1, gu, 2 * F, nullptr, A, (int)(2 * F), (int)H, stream,
+                                       ws + o_chunk, chunk_bytes, x_layout))
                     return 0;
                 // bias + SwiGLU-OAI are formed while the down projection's activations are converted
                 if (!launch_convert_x_swiglu(ggml_type, gu, gate_up_bias, maps.expert_of, alpha, limit, A, (int)F, ws + o_ws2, stream,
@@ -1655,8 +1697,8 @@ int TSHip_MoEExpertsGptOssForwardF32Device(TSHipTensorView2D result, TSHipTensor
                     return 0;
             }
             tiles.expert_stride = dn_bytes;
-            if (!launch_gemm(ggml_type, down_w, dn_bytes, ws + o_ws2, dn, H, nullptr, A, (int)H, (int)F, &tiles, stream, false,
-                             ws + o_chunk, chunk_bytes, x_layout))
+            if (!launch_gemm_tiles(ggml_type, tiles, down_w, dn_bytes, ws + o_ws2, dn, H, nullptr, A, (int)H, (int)F, stream, ws + o_chunk,
+                                   chunk_bytes, x_layout))
                 return 0;
             if (!launch_moe_combine(dn, down_bias, ids, weights, maps.pos_of, T, k, E, (int)H, false,
                                     static_cast<float*>(result.data), result.stride0, stream))
@@ -1943,11 +1985,7 @@ int TSHip_FusedRmsNormMatMulQuantF32Device(TSHipTensorView2D result, TSHipTensor
                                    m2_raw_bytes, "fused rms_norm_matmul", "result"))
             return 0;
         if (!check_device_views(result, input)) return 0;
-        const size_t need = matmul_ws_bytes(m2_ggml_type, input.dim0, m2_ne0, m2_ne1, true, false);
-        WsLease ws(t_stream, need);
-        if (!ws.ok()) return 0;
-        if (!run_matmul_device_ws(result, input, m2_data, m2_ggml_type, m2_ne0, m2_ne1, t_stream, ws.ptr(), need, norm_weight, eps, false))
-            return 0;
+        if (!run_matmul_device(result, input, m2_data, m2_ggml_type, m2_ne0, m2_ne1, t_stream, norm_weight, eps, false)) return 0;
         clear_last_error();
         return 1;
     });
@@ -1962,11 +2000,7 @@ int TSHip_FusedMatMulQuantAddF32Device(TSHipTensorView2D residual, TSHipTensorVi
                                    "fused matmul_add", "residual"))
             return 0;
         if (!check_device_views(residual, input)) return 0;
-        const size_t need = matmul_ws_bytes(m2_ggml_type, input.dim0, m2_ne0, m2_ne1, false, true);
-        WsLease ws(t_stream, need);
-        if (!ws.ok()) return 0;
-        if (!run_matmul_device_ws(residual, input, m2_data, m2_ggml_type, m2_ne0, m2_ne1, t_stream, ws.ptr(), need, nullptr, 0.f, true))
-            return 0;
+        if (!run_matmul_device(residual, input, m2_data, m2_ggml_type, m2_ne0, m2_ne1, t_stream, nullptr, 0.f, true)) return 0;
         clear_last_error();
         return 1;
     });
@@ -1984,9 +2018,10 @@ int TSHip_FusedFFNSwiGLUQuantF32Device(TSHipTensorView2D residual, TSHipTensorVi
                           gate_up_ne1, gate_up_raw_bytes, down_data, down_ggml_type, down_ne0, down_ne1, down_raw_bytes, half_dim))
             return 0;
         if (!check_device_views(residual, input)) return 0;
-        WsLease ws(t_stream, ffn_ws_bytes(input.dim0, gate_up_ggml_type, down_ggml_type, input.dim1, half_dim));
+        const FfnPlan plan = plan_ffn(input.dim0, gate_up_ggml_type, down_ggml_type, input.dim1, half_dim);
+        WsLease ws(t_stream, plan.total);
         if (!ws.ok()) return 0;
-        if (!run_ffn_swiglu_device(residual, input, norm_weight, eps, gate_up_data, gate_up_ggml_type, down_data, down_ggml_type,
+        if (!run_ffn_swiglu_device(plan, residual, input, norm_weight, eps, gate_up_data, gate_up_ggml_type, down_data, down_ggml_type,
                                    input.dim1, half_dim, t_stream, ws.ptr()))
             return 0;
         clear_last_error();
@@ -2008,9 +2043,7 @@ int TSHip_FusedRmsNormMatMulQuantF32(TSHipTensorView2D result, TSHipTensorView2D
         if (!w) return 0;
         return with_host_tensors(result, false, input, norm_weight_data, norm_weight_count,
                                  [&](const TSHipTensorView2D& x, const TSHipTensorView2D& y, const float* nw, hipStream_t st) {
-                                     const size_t need = matmul_ws_bytes(m2_ggml_type, x.dim0, m2_ne0, m2_ne1, true, false);
-                                     WsLease ws(st, need);
-                                     return ws.ok() && run_matmul_device_ws(y, x, w, m2_ggml_type, m2_ne0, m2_ne1, st, ws.ptr(), need, nw, eps, false);
+                                     return run_matmul_device(y, x, w, m2_ggml_type, m2_ne0, m2_ne1, st, nw, eps, false);
                                  });
     });
 }
@@ -2028,9 +2061,7 @@ int TSHip_FusedMatMulQuantAddF32(TSHipTensorView2D residual, TSHipTensorView2D i
         if (!w) return 0;
         return with_host_tensors(residual, true, input, nullptr, 0,
                                  [&](const TSHipTensorView2D& x, const TSHipTensorView2D& y, const float*, hipStream_t st) {
-                                     const size_t need = matmul_ws_bytes(m2_ggml_type, x.dim0, m2_ne0, m2_ne1, false, true);
-                                     WsLease ws(st, need);
-                                     return ws.ok() && run_matmul_device_ws(y, x, w, m2_ggml_type, m2_ne0, m2_ne1, st, ws.ptr(), need, nullptr, 0.f, true);
+                                     return run_matmul_device(y, x, w, m2_ggml_type, m2_ne0, m2_ne1, st, nullptr, 0.f, true);
                                  });
     });
 }
@@ -2052,9 +2083,10 @@ int TSHip_FusedFFNSwiGLUQuantF32(TSHipTensorView2D residual, TSHipTensorView2D i
         if (!dn) return 0;
         return with_host_tensors(residual, true, input, norm_weight_data, norm_weight_count,
                                  [&](const TSHipTensorView2D& x, const TSHipTensorView2D& y, const float* nw, hipStream_t st) {
-                                     WsLease ws(st, ffn_ws_bytes(x.dim0, gate_up_ggml_type, down_ggml_type, x.dim1, half_dim));
-                                     return ws.ok() && run_ffn_swiglu_device(y, x, nw, eps, gu, gate_up_ggml_type, dn, down_ggml_type, x.dim1,
-                                                                             half_dim, st, ws.ptr());
+                                     const FfnPlan plan = plan_ffn(x.dim0, gate_up_ggml_type, down_ggml_type, x.dim1, half_dim);
+                                     WsLease ws(st, plan.total);
+                                     return ws.ok() && run_ffn_swiglu_device(plan, y, x, nw, eps, gu, gate_up_ggml_type, dn, down_ggml_type,
+                                                                             x.dim1, half_dim, st, ws.ptr());
                                  });
     });
 }
@@ -2071,11 +2103,11 @@ int TSHip_FusedOutProjFFNQuantF32Device(TSHipTensorView2D residual, TSHipTensorV
         const WeightDesc gd{gu_data, gu_type, gu_ne0, gu_ne1, gu_raw_bytes}, dd{dn_data, dn_type, dn_ne0, dn_ne1, dn_raw_bytes};
         if (!validate_outproj_ffn(residual, input, od, ffn_norm_weight, ffn_norm_count, gd, dd, half_dim)) return 0;
         if (!check_device_views(residual, input)) return 0;
-        const size_t need = outproj_ffn_ws_bytes(input.dim0, od, gd, dd, residual.dim1, half_dim);
-        WsLease ws(t_stream, need);
+        const OutprojFfnPlan plan = plan_outproj_ffn(input.dim0, od, gd, dd, residual.dim1, half_dim);
+        WsLease ws(t_stream, plan.total());
         if (!ws.ok()) return 0;
-        if (!run_outproj_ffn_device(residual, input, out_proj_data, od, ffn_norm_weight, eps, gu_data, gu_type, dn_data, dn_type, half_dim,
-                                    t_stream, ws.ptr(), need))
+        if (!run_outproj_ffn_device(plan, residual, input, out_proj_data, od, ffn_norm_weight, eps, gu_data, gu_type, dn_data, dn_type,
+                                    half_dim, t_stream, ws.ptr()))
             return 0;
         clear_last_error();
         return 1;
@@ -2099,9 +2131,9 @@ int TSHip_FusedOutProjFFNQuantF32(TSHipTensorView2D residual, TSHipTensorView2D 
         if (!dn) return 0;
         const HostTensor io[2] = {{&residual, true, true}, {&input, true, false}};
         return with_host_io(io, 2, ffn_norm_data, ffn_norm_count, [&](const TSHipTensorView2D* dv, const float* nw, hipStream_t st) {
-            const size_t need = outproj_ffn_ws_bytes(dv[1].dim0, od, gd, dd, dv[0].dim1, half_dim);
-            WsLease ws(st, need);
-            return ws.ok() && run_outproj_ffn_device(dv[0], dv[1], ow, od, nw, eps, gu, gu_type, dn, dn_type, half_dim, st, ws.ptr(), need);
+            const OutprojFfnPlan plan = plan_outproj_ffn(dv[1].dim0, od, gd, dd, dv[0].dim1, half_dim);
+            WsLease ws(st, plan.total());
+            return ws.ok() && run_outproj_ffn_device(plan, dv[0], dv[1], ow, od, nw, eps, gu, gu_type, dn, dn_type, half_dim, st, ws.ptr());
         });
     });
 }
@@ -2121,11 +2153,11 @@ int TSHip_FusedOutProjNormRouterQuantF32Device(TSHipTensorView2D residual, TSHip
             set_last_error("Device addmm_quant needs stride1 == 1 views.");
             return 0;
         }
-        const size_t need = outproj_router_ws_bytes(input.dim0, od, rd);
-        WsLease ws(t_stream, need);
+        const OutprojRouterPlan plan = plan_outproj_router(input.dim0, od, rd);
+        WsLease ws(t_stream, plan.total());
         if (!ws.ok()) return 0;
-        if (!run_outproj_router_device(residual, input, out_proj_data, od, norm_weight, eps, normed_out, router_data, rd, router_out,
-                                       t_stream, ws.ptr(), need))
+        if (!run_outproj_router_device(plan, residual, input, out_proj_data, od, norm_weight, eps, normed_out, router_data, rd, router_out,
+                                       t_stream, ws.ptr()))
             return 0;
         clear_last_error();
         return 1;
@@ -2148,9 +2180,9 @@ int TSHip_FusedOutProjNormRouterQuantF32(TSHipTensorView2D residual, TSHipTensor
         if (!rw) return 0;
         const HostTensor io[4] = {{&residual, true, true}, {&input, true, false}, {&normed_out, false, true}, {&router_out, false, true}};
         return with_host_io(io, 4, norm_data, norm_count, [&](const TSHipTensorView2D* dv, const float* nw, hipStream_t st) {
-            const size_t need = outproj_router_ws_bytes(dv[1].dim0, od, rd);
-            WsLease ws(st, need);
-            return ws.ok() && run_outproj_router_device(dv[0], dv[1], ow, od, nw, eps, dv[2], rw, rd, dv[3], st, ws.ptr(), need);
+            const OutprojRouterPlan plan = plan_outproj_router(dv[1].dim0, od, rd);
+            WsLease ws(st, plan.total());
+            return ws.ok() && run_outproj_router_device(plan, dv[0], dv[1], ow, od, nw, eps, dv[2], rw, rd, dv[3], st, ws.ptr());
         });
     });
 }
@@ -2639,9 +2671,11 @@ bool run_layer_decode(float* hidden, const LayerShape& L, const float* attn_norm
     auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
     const size_t b_qkv = al((size_t)qkv_n * 4), b_attn = al((size_t)q_dim * 4);
     const size_t b_part = al(attention_decode_ws_bytes(L.num_heads, position + 1));
-    const size_t b_mm = al(std::max(matmul_ws_bytes(L.qkv_type, 1, L.hidden, qkv_n, true, false), matmul_ws_bytes(L.o_type, 1, q_dim, L.hidden, false, true)));
-    const size_t b_ffn = ffn_ws_bytes(1, L.gu_type, L.down_type, L.hidden, L.intermediate);
-    WsLease lease(stream, b_qkv + b_attn + b_part + b_mm + b_ffn);
+    const MatmulPlan qkv_plan = plan_matmul(L.qkv_type, 1, L.hidden, qkv_n, true, false);
+    const MatmulPlan o_plan = plan_matmul(L.o_type, 1, q_dim, L.hidden, false, true);
+    const FfnPlan ffn_plan = plan_ffn(1, L.gu_type, L.down_type, L.hidden, L.intermediate);
+    const size_t b_mm = al(std::max(qkv_plan.total(), o_plan.total()));
+    WsLease lease(stream, b_qkv + b_attn + b_part + b_mm + ffn_plan.total);
     if (!lease.ok()) return false;
     char* ws = lease.ptr();
     float* qkv_out = reinterpret_cast<float*>(ws);
@@ -2651,14 +2685,14 @@ bool run_layer_decode(float* hidden, const LayerShape& L, const float* attn_norm
     const TSHipTensorView2D h_view{hidden, 1, L.hidden, L.hidden, 1, (int64_t)L.hidden * 4};
     const TSHipTensorView2D qkv_view{qkv_out, 1, qkv_n, qkv_n, 1, (int64_t)qkv_n * 4};
     const TSHipTensorView2D attn_view{attn, 1, q_dim, q_dim, 1, (int64_t)q_dim * 4};
-    if (!run_matmul_device_ws(qkv_view, h_view, qkv, L.qkv_type, L.hidden, qkv_n, stream, mm_ws, b_mm, attn_norm, eps, false)) return false;
+    if (!run_matmul_device_ws(qkv_plan, qkv_view, h_view, qkv, L.qkv_type, L.hidden, qkv_n, stream, mm_ws, b_mm, attn_norm, eps, false)) return false;
     if (!launch_attention_decode(qkv_out, q_norm, k_norm, eps, rope_base, rope_freq_scale, rope_mode, k_cache, v_cache, L.num_heads,
                                  L.num_kv_heads, L.head_dim, L.max_seq_len, position, part, attn, stream, ffn_norm, next_attn_norm, L.hidden))
         return false;
     // hidden += W_o attn
-    if (!run_matmul_device_ws(h_view, attn_view, o, L.o_type, q_dim, L.hidden, stream, mm_ws, b_mm, nullptr, 0.f, true)) return false;
+    if (!run_matmul_device_ws(o_plan, h_view, attn_view, o, L.o_type, q_dim, L.hidden, stream, mm_ws, b_mm, nullptr, 0.f, true)) return false;
     // hidden += W_down(silu(g) * u); the FFN reads hidden (RMSNorm) before its last kernel adds into it
-    return run_ffn_swiglu_device(h_view, h_view, ffn_norm, eps, gu, L.gu_type, down, L.down_type, L.hidden, L.intermediate, stream,
+    return run_ffn_swiglu_device(ffn_plan, h_view, h_view, ffn_norm, eps, gu, L.gu_type, down, L.down_type, L.hidden, L.intermediate, stream,
                                  ws + b_qkv + b_attn + b_part + b_mm);
 }
 

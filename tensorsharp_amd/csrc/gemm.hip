@@ -3635,10 +3635,10 @@ bool launch_wide_tm(const GemmArgs& a, hipStream_t stream)
 }
 
 template <typename H>
-bool launch_wide(GemmArgs a, hipStream_t stream, const ChunkScratch& cs)
+bool launch_wide(GemmArgs a, WidePlan p, hipStream_t stream, const ChunkScratch& cs)
 {
     const int nkt = a.Kp / kBK;
-    WidePlan p = pick_wide(a.M, a.N, nkt, true, H::kUsBase, H::kUsRow);
+    if (p.tm == 0) p = pick_wide(a.M, a.N, nkt, true, H::kUsBase, H::kUsRow);
     a.partial = nullptr;
     if (p.k_chunks > 1) {
         const size_t need = (size_t)p.k_chunks * a.M * a.N * sizeof(float);
@@ -3696,12 +3696,12 @@ bool launch_slim_mx48(GemmArgs a, int m_tiles, hipStream_t stream, const ChunkSc
 constexpr int kWideTiles = 0;
 
 template <typename G>
-bool launch_for_type(const GemmArgs& a, int bm, int m_tiles, hipStream_t stream, const ChunkScratch& cs)
+bool launch_for_type(const GemmArgs& a, int bm, int m_tiles, const WidePlan& wide, hipStream_t stream, const ChunkScratch& cs)
 {
     if (bm == kWideTiles) {
-        if constexpr (std::is_same<G, GQ4K>::value) return launch_wide<WQ4K>(a, stream, cs);
-        if constexpr (std::is_same<G, GQ80>::value) return launch_wide<WQ80>(a, stream, cs);
-        if constexpr (std::is_same<G, GQ6K>::value) return launch_wide<WQ6K>(a, stream, cs);
+        if constexpr (std::is_same<G, GQ4K>::value) return launch_wide<WQ4K>(a, wide, stream, cs);
+        if constexpr (std::is_same<G, GQ80>::value) return launch_wide<WQ80>(a, wide, stream, cs);
+        if constexpr (std::is_same<G, GQ6K>::value) return launch_wide<WQ6K>(a, wide, stream, cs);
     }
     if (bm == 32 && !a.x_mx) {
         const int ktw = slim_ktw<G>(a.Kp / kBK), kc = (a.Kp / kBK + 8 * ktw - 1) / (8 * ktw);
@@ -3709,8 +3709,8 @@ bool launch_for_type(const GemmArgs& a, int bm, int m_tiles, hipStream_t stream,
         const bool fits = cs.need_out || (kc == 1 && !a.accumulate) || chunk_scratch(cs, (size_t)kc * a.M * a.N * sizeof(float));
         if (fits || a.tile_expert) return launch_slim_for<G>(a, ktw, m_tiles, stream, cs);
         if constexpr (std::is_same<G, GQ4K>::value) return launch_xw<PQ4K, 256, 4>(a, (a.M + 255) / 256, stream, cs);
-        if constexpr (std::is_same<G, GQ80>::value) return launch_wide<WQ80>(a, stream, cs);
-        if constexpr (std::is_same<G, GQ6K>::value) return launch_wide<WQ6K>(a, stream, cs);
+        if constexpr (std::is_same<G, GQ80>::value) return launch_wide<WQ80>(a, wide, stream, cs);
+        if constexpr (std::is_same<G, GQ6K>::value) return launch_wide<WQ6K>(a, wide, stream, cs);
         return launch_slim_for<G>(a, ktw, m_tiles, stream, cs);
     }
     // Q4_K and MXFP4: the 2 x 4 wavefront layout with the operand exchange through LDS (gemm_xw_kernel); 128-row tiles are
@@ -3815,22 +3815,23 @@ double tile256_us(int M, int N, int nkt)
 // 256-row tiles keep many rows of wide weights (Q4_K 2048 x 21504 x 5376 494 vs 567 us, Q8_0 700 x 14336 x 4096 121 vs 138):
 // they take half as many weight lines per result.
 template <typename G, typename W>
-int cheapest_tiles(int M, int N, int K)
+int cheapest_tiles(int M, int N, int K, WidePlan* plan)
 {
     const int nkt = (K + kBK - 1) / kBK;
-    const double wide = pick_wide(M, N, nkt, true, W::kUsBase, W::kUsRow).us, slim = slim_us<G>(M, N, nkt);
+    *plan = pick_wide(M, N, nkt, true, W::kUsBase, W::kUsRow);
+    const double wide = plan->us, slim = slim_us<G>(M, N, nkt);
     const double tile = std::is_same<G, GQ6K>::value ? wide : tile256_us(M, N, nkt);       // (no 256-row tiles of Q6_K)
     if (slim <= wide && slim <= tile) return 32;
     return wide <= tile ? kWideTiles : 256;
 }
-}  // namespace
 
-int gemm_tile_m(int type, int M, int N, int K)
+// Rows of activations per tile of a plain launch (kWideTiles: gemm_wide_kernel, as *wide says)
+int gemm_tile_m(int type, int M, int N, int K, WidePlan* wide)
 {
     if (M > 3) {
-        if (type == kTypeQ4_K) return cheapest_tiles<GQ4K, WQ4K>(M, N, K);
-        if (type == kTypeQ8_0) return cheapest_tiles<GQ80, WQ80>(M, N, K);
-        if (type == kTypeQ6_K) return cheapest_tiles<GQ6K, WQ6K>(M, N, K);
+        if (type == kTypeQ4_K) return cheapest_tiles<GQ4K, WQ4K>(M, N, K, wide);
+        if (type == kTypeQ8_0) return cheapest_tiles<GQ80, WQ80>(M, N, K, wide);
+        if (type == kTypeQ6_K) return cheapest_tiles<GQ6K, WQ6K>(M, N, K, wide);
     }
     if (M <= 128) return 32;
     if (type == kTypeMXFP4 && M <= 512 && ((M + 127) / 128) * ((N + 127) / 128) <= 128) return 32;
@@ -3845,8 +3846,6 @@ int gemm_tile_m(int type, int M, int N, int K)
     const double t128 = (double)((tiles128 + (two_per_cu ? 2 : 1) * cus - 1) / ((two_per_cu ? 2 : 1) * cus)) * (two_per_cu ? 1.37 : 1.4);
     return t256 < t128 ? 256 : 128;
 }
-
-namespace {
 
 template <int TYPE, int SRC>
 void launch_convert_typed(const ConvertSrc& src, int M, int K, int kp, _Float16* x16, float* scales, hipStream_t stream)
@@ -3890,18 +3889,6 @@ bool launch_convert(int type, const ConvertSrc& src, int M, int K, void* workspa
 
 }  // namespace
 
-// Which activation layout the GEMM of this shape reads: 0 fp16 in the format's unpack order; 1 two MX fp6 terms for
-// gemm_mx_kernel (plain MXFP4 launches on 128- or 256-row tiles).
-// (rows longer than 32768 stay on the fp16 path, whose tile kernels cut such a K into chunks, and so do small batches
-// over small weights, which gain nothing: 64 x 5760 x 2880 18.2 vs 17.7 us, 16 x 4096 x 14336 26.9 vs 23.0 us, but
-// 32 x 184320 x 2880 61-67 vs 74-84 us)
-int gemm_x_layout(int type, int M, int N, int K)
-{
-    if (type == kTypeQ4_K) return gemm_tile_m(type, M, N, K) == kWideTiles ? 2 : 0;
-    if (type != kTypeMXFP4 || K > 1024 * kCvtHold * 4) return 0;
-    return gemm_tile_m(type, M, N, K) >= 128 || (int64_t)N * K >= ((int64_t)64 << 20) ? 1 : 0;
-}
-
 bool launch_convert_x(int type, const float* x, int64_t ldx, const int* row_map, int M, int K, void* workspace,
                       hipStream_t stream, const float* norm_w, float eps, int layout)
 {
@@ -3928,14 +3915,9 @@ bool launch_convert_x_swiglu(int type, const float* gate_up, const float* bias, 
 }
 
 namespace {
-bool gemm_dispatch(int type, const void* w, int64_t w_bytes, const void* workspace, float* c, int64_t ldc, const int* c_rows,
-                   int M, int N, int K, const GemmTiles* tiles, hipStream_t stream, bool accumulate, const ChunkScratch& cs,
-                   int x_layout)
+// what every launch takes, plain or grouped; false (with the last error) where 32-bit offsets do not reach
+bool gemm_args(GemmArgs* out, const void* w, int64_t w_bytes, const void* workspace, float* c, int64_t ldc, int M, int N, int K, int x_layout)
 {
-    if (w_bytes >= kMaxOperandBytes && !tiles) {
-        set_last_error("gemm: a single weight of 2 GiB or more must be split by rows.");
-        return false;
-    }
     GemmArgs a{};
     a.w = static_cast<const uint8_t*>(w);
     a.w_bytes = w_bytes;
@@ -3943,8 +3925,6 @@ bool gemm_dispatch(int type, const void* w, int64_t w_bytes, const void* workspa
     a.x16 = reinterpret_cast<const _Float16*>(static_cast<const char*>(workspace) + (((size_t)M * sizeof(float) + 255) & ~(size_t)255));
     a.c = c;
     a.ldc = ldc;
-    a.c_rows = c_rows;
-    a.accumulate = accumulate ? 1 : 0;
     a.x_mx = x_layout == 1 ? 1 : 0;
     a.M = M;
     a.N = N;
@@ -3956,46 +3936,93 @@ bool gemm_dispatch(int type, const void* w, int64_t w_bytes, const void* workspa
         set_last_error("gemm: the converted activations of one call must stay below 2 GiB; split the rows.");
         return false;
     }
-    int bm, m_tiles;
-    if (tiles) {
-        a.tile_expert = tiles->expert;
-        a.tile_row0 = tiles->row0;
-        a.tile_rows = tiles->rows;
-        a.expert_stride = tiles->expert_stride;
-        a.expert_off = tiles->expert_off;
-        bm = tiles->bm;
-        m_tiles = tiles->count;
-    } else {
-        bm = gemm_tile_m(type, M, N, K);
-        if (type == kTypeQ4_K && (bm == kWideTiles) != (x_layout == 2)) {
-            set_last_error("gemm: the activations are not in the order that this launch reads (gemm_x_layout).");
-            return false;
-        }
-        m_tiles = bm == kWideTiles ? 1 : (M + bm - 1) / bm;
-    }
+    *out = a;
+    return true;
+}
+
+bool gemm_dispatch(int type, const GemmArgs& a, int bm, int m_tiles, const WidePlan& wide, hipStream_t stream, const ChunkScratch& cs)
+{
     if (m_tiles == 0) return true;
     switch (type) {
-    case kTypeQ4_K: return launch_for_type<GQ4K>(a, bm, m_tiles, stream, cs);
-    case kTypeMXFP4: return launch_for_type<GMXFP4>(a, bm, m_tiles, stream, cs);
-    case kTypeQ8_0: return launch_for_type<GQ80>(a, bm, m_tiles, stream, cs);
-    case kTypeQ6_K: return launch_for_type<GQ6K>(a, bm, m_tiles, stream, cs);
-    case kTypeQ5_K: return launch_for_type<GQ5K>(a, bm, m_tiles, stream, cs);
-    case kTypeQ4_0: return launch_for_type<GLegacy<kTypeQ4_0>>(a, bm, m_tiles, stream, cs);
-    case kTypeQ4_1: return launch_for_type<GLegacy<kTypeQ4_1>>(a, bm, m_tiles, stream, cs);
-    case kTypeQ5_0: return launch_for_type<GLegacy<kTypeQ5_0>>(a, bm, m_tiles, stream, cs);
-    case kTypeQ5_1: return launch_for_type<GLegacy<kTypeQ5_1>>(a, bm, m_tiles, stream, cs);
-    case kTypeIQ4_NL: return launch_for_type<GLegacy<kTypeIQ4_NL>>(a, bm, m_tiles, stream, cs);
+    case kTypeQ4_K: return launch_for_type<GQ4K>(a, bm, m_tiles, wide, stream, cs);
+    case kTypeMXFP4: return launch_for_type<GMXFP4>(a, bm, m_tiles, wide, stream, cs);
+    case kTypeQ8_0: return launch_for_type<GQ80>(a, bm, m_tiles, wide, stream, cs);
+    case kTypeQ6_K: return launch_for_type<GQ6K>(a, bm, m_tiles, wide, stream, cs);
+    case kTypeQ5_K: return launch_for_type<GQ5K>(a, bm, m_tiles, wide, stream, cs);
+    case kTypeQ4_0: return launch_for_type<GLegacy<kTypeQ4_0>>(a, bm, m_tiles, wide, stream, cs);
+    case kTypeQ4_1: return launch_for_type<GLegacy<kTypeQ4_1>>(a, bm, m_tiles, wide, stream, cs);
+    case kTypeQ5_0: return launch_for_type<GLegacy<kTypeQ5_0>>(a, bm, m_tiles, wide, stream, cs);
+    case kTypeQ5_1: return launch_for_type<GLegacy<kTypeQ5_1>>(a, bm, m_tiles, wide, stream, cs);
+    case kTypeIQ4_NL: return launch_for_type<GLegacy<kTypeIQ4_NL>>(a, bm, m_tiles, wide, stream, cs);
     default: set_last_error("gemm: unsupported type."); return false;
     }
 }
+
+bool gemm_dispatch_plan(int type, GemmArgs a, const GemmPlan& plan, hipStream_t stream, bool accumulate, const ChunkScratch& cs)
+{
+    if (plan.bm < 0 || (a.w_bytes >= kMaxOperandBytes)) {
+        set_last_error(plan.bm < 0 ? "gemm: unsupported type." : "gemm: a single weight of 2 GiB or more must be split by rows.");
+        return false;
+    }
+    a.accumulate = accumulate ? 1 : 0;
+    const WidePlan wide{plan.wide_tm, plan.k_chunks, plan.chunk_kt, 0.0};
+    return gemm_dispatch(type, a, plan.bm, plan.bm == kWideTiles ? 1 : (a.M + plan.bm - 1) / plan.bm, wide, stream, cs);
+}
+
+// only tiles->bm and tiles->count matter when nothing is launched
+bool gemm_dispatch_tiles(int type, GemmArgs a, const int* c_rows, const GemmTiles& tiles, hipStream_t stream, const ChunkScratch& cs)
+{
+    a.c_rows = c_rows;
+    a.tile_expert = tiles.expert;
+    a.tile_row0 = tiles.row0;
+    a.tile_rows = tiles.rows;
+    a.expert_stride = tiles.expert_stride;
+    a.expert_off = tiles.expert_off;
+    return gemm_dispatch(type, a, tiles.bm, tiles.count, WidePlan{0, 1, 0, 0.0}, stream, cs);
+}
 }  // namespace
 
-bool launch_gemm(int type, const void* w, int64_t w_bytes, const void* workspace, float* c, int64_t ldc, const int* c_rows,
-                 int M, int N, int K, const GemmTiles* tiles, hipStream_t stream, bool accumulate, void* chunk_ws,
-                 size_t chunk_ws_bytes, int x_layout)
+GemmPlan plan_gemm(int type, int M, int N, int K, bool accumulate)
+{
+    GemmPlan p{};
+    if (!is_quant_type(type)) {
+        p.bm = -1;
+        return p;
+    }
+    WidePlan wide{0, 1, 0, 0.0};
+    p.bm = gemm_tile_m(type, M, N, K, &wide);
+    p.wide_tm = wide.tm;
+    p.k_chunks = wide.k_chunks;
+    p.chunk_kt = wide.chunk_kt;
+    // The activation layout: MXFP4 rows up to 32768 (longer ones stay on the fp16 path, whose tile kernels cut such a K into
+    // chunks) on 128- or 256-row tiles, or in small batches over large weights (small ones gain nothing: 64 x 5760 x 2880 18.2
+    // vs 17.7 us, 16 x 4096 x 14336 26.9 vs 23.0 us, but 32 x 184320 x 2880 61-67 vs 74-84 us), are MX fp6 pairs;
+    // gemm_wide_kernel reads natural order, which for the other two formats it serves is their unpack order anyway
+    if (type == kTypeQ4_K && p.bm == kWideTiles) p.x_layout = 2;
+    if (type == kTypeMXFP4 && K <= 1024 * kCvtHold * 4 && (p.bm >= 128 || (int64_t)N * K >= ((int64_t)64 << 20))) p.x_layout = 1;
+    // a buffer "large enough", so that the launcher makes the choices it would make with the reported bytes at hand
+    const ChunkScratch cs{nullptr, ~(size_t)0, &p.chunk_bytes};
+    GemmArgs a{};
+    const int64_t w_bytes = block_bytes(type) * (K / block_elems(type)) * N;
+    if (!gemm_args(&a, nullptr, w_bytes, nullptr, nullptr, N, M, N, K, p.x_layout) || !gemm_dispatch_plan(type, a, p, nullptr, accumulate, cs))
+        p.chunk_bytes = 0;
+    return p;
+}
+
+bool launch_gemm(int type, const GemmPlan& plan, const void* w, int64_t w_bytes, const void* workspace, float* c, int64_t ldc, int M, int N,
+                 int K, hipStream_t stream, bool accumulate, void* chunk_ws, size_t chunk_ws_bytes)
 {
     const ChunkScratch cs{static_cast<float*>(chunk_ws), chunk_ws ? chunk_ws_bytes : 0, nullptr};
-    return gemm_dispatch(type, w, w_bytes, workspace, c, ldc, c_rows, M, N, K, tiles, stream, accumulate, cs, x_layout);
+    GemmArgs a{};
+    return gemm_args(&a, w, w_bytes, workspace, c, ldc, M, N, K, plan.x_layout) && gemm_dispatch_plan(type, a, plan, stream, accumulate, cs);
+}
+
+bool launch_gemm_tiles(int type, const GemmTiles& tiles, const void* w, int64_t w_bytes, const void* workspace, float* c, int64_t ldc,
+                       const int* c_rows, int M, int N, int K, hipStream_t stream, void* chunk_ws, size_t chunk_ws_bytes, int x_layout)
+{
+    const ChunkScratch cs{static_cast<float*>(chunk_ws), chunk_ws ? chunk_ws_bytes : 0, nullptr};
+    GemmArgs a{};
+    return gemm_args(&a, w, w_bytes, workspace, c, ldc, M, N, K, x_layout) && gemm_dispatch_tiles(type, a, c_rows, tiles, stream, cs);
 }
 
 bool gemm_swiglu_mx_fits(int F, int K)
@@ -4049,16 +4076,12 @@ bool launch_gemm_swiglu_mx(const void* w, const void* workspace, void* workspace
     return a.Kp / kBK <= 32 ? launch_slim_mx<4, 1, 1>(a, tiles->count, stream, cs) : launch_slim_mx<6, 1, 1>(a, tiles->count, stream, cs);
 }
 
-size_t gemm_chunk_ws_bytes(int type, int M, int N, int K, const GemmTiles* tiles, bool accumulate, int x_layout)
+size_t gemm_tiles_ws_bytes(int type, const GemmTiles& tiles, int M, int N, int K, int x_layout)
 {
     size_t need = 0;
-    // a buffer "large enough" so that the launchers make the choices they would make with the reported bytes at hand
     const ChunkScratch cs{nullptr, ~(size_t)0, &need};
-    const int64_t w_bytes = tiles ? 0 : (int64_t)(block_bytes(type) * (K / block_elems(type))) * N;
-    if (!gemm_dispatch(type, nullptr, w_bytes, nullptr, nullptr, N, nullptr, M, N, K, tiles, nullptr, accumulate, cs,
-                       x_layout >= 0 ? x_layout : tiles ? 0 : gemm_x_layout(type, M, N, K)))
-        return 0;
-    return need;
+    GemmArgs a{};
+    return gemm_args(&a, nullptr, 0, nullptr, nullptr, N, M, N, K, x_layout) && gemm_dispatch_tiles(type, a, nullptr, tiles, nullptr, cs) ? need : 0;
 }
 
 }  // namespace tship

@@ -146,16 +146,24 @@ bool launch_gemv_group(int type, int count, const GemvArgs* args, hipStream_t st
 // ---- prefill GEMM ---------------------------------------------------------------------------
 // Workspace layout: [M floats of row scales, padded to 256 B][M x Kp fp16 activations].
 size_t gemm_workspace_bytes(int M, int K);
-int gemm_tile_m(int type, int M, int N, int K);   // rows of activations per tile for a plain (ungrouped) launch (0: gemm_wide_kernel picks its own)
+
+// How a plain (ungrouped) launch runs.  Worked out once per call: the rule prices several kernels and tilings (0.3 us), and the
+// conversion of the activations, the size of the scratch and the launch have to agree on its answer.
+struct GemmPlan {
+    int bm;                              // rows of activations per tile: 32, 128 or 256, 0 where gemm_wide_kernel runs, -1 no kernel
+    int wide_tm, k_chunks, chunk_kt;     // gemm_wide_kernel: rows per tile / 32, K chunks, k-tiles per chunk
+    int x_layout;                        // of the converted activations: 0 fp16 in the format's unpack order, 1 MX fp6 pairs (MXFP4 on
+                                         // the block-scaled matrix instruction), 2 fp16 in natural order (Q4_K on gemm_wide_kernel)
+    size_t chunk_bytes;                  // scratch for the sums of K chunks (0 for most shapes)
+};
+GemmPlan plan_gemm(int type, int M, int N, int K, bool accumulate);
 
 // fp32 activations -> workspace (fp16 in the weight format's unpack order + per-row scales);
 // row_map (device, optional) gathers source rows.
 // norm_w (device, optional) applies RMSNorm first: x <- x / sqrt(mean(x^2) + eps) * norm_w.
+// layout: see GemmPlan::x_layout.
 bool launch_convert_x(int type, const float* x, int64_t ldx, const int* row_map, int M, int K, void* workspace,
                       hipStream_t stream, const float* norm_w = nullptr, float eps = 0.f, int layout = 0);
-// layout of the converted activations the GEMM of this shape reads (plain launches): 0 fp16 in the format's unpack order,
-// 1 MX fp6 pairs (MXFP4 on the block-scaled matrix instruction), 2 fp16 in natural order (Q4_K on gemm_wide_kernel); pass it to launch_convert_x and to launch_gemm
-int gemm_x_layout(int type, int M, int N, int K);
 // The same for the activations of an expert's down projection: row m is SwiGLU-OAI of (gate | up)[m] (+ the bias
 // row of expert_of[m]), formed while it is read.
 bool launch_convert_x_swiglu(int type, const float* gate_up, const float* bias, const int* expert_of, float alpha, float limit,
@@ -182,15 +190,16 @@ bool gemm_swiglu_mx_fits(int F, int K);
 bool launch_gemm_swiglu_mx(const void* w, const void* workspace, void* workspace_out, float* act, const float* bias, float alpha,
                            float limit, int M, int F, int K, const GemmTiles* tiles, hipStream_t stream);
 
-// c[row] (row = c_rows ? c_rows[m] : m) [N] = x16[m] . W^T * scale[m], m < M
-// accumulate: c[row] += ... instead of c[row] = ...
-// chunk_ws (device): where the sums of K chunks go, gemm_chunk_ws_bytes() of them (a shape whose chunk sums do not fit
-// what is passed runs with whole K per tile, or fails when its kernel cannot do without chunks).  Nothing is allocated.
-bool launch_gemm(int type, const void* w, int64_t w_bytes, const void* workspace, float* c, int64_t ldc,
-                 const int* c_rows, int M, int N, int K, const GemmTiles* tiles, hipStream_t stream, bool accumulate = false,
-                 void* chunk_ws = nullptr, size_t chunk_ws_bytes = 0, int x_layout = 0);
-// bytes of chunk_ws the same launch uses (0 for most shapes); only tiles->bm and tiles->count are read
-size_t gemm_chunk_ws_bytes(int type, int M, int N, int K, const GemmTiles* tiles, bool accumulate, int x_layout = -1);
+// c[m] [N] = x16[m] . W^T * scale[m], m < M, as `plan` (of the same shape) says; accumulate: c[m] += ... instead of c[m] = ...
+// chunk_ws (device): where the sums of K chunks go, plan.chunk_bytes of them (a shape whose chunk sums do not fit what is
+// passed runs with whole K per tile, or fails when its kernel cannot do without chunks).  Nothing is allocated.
+bool launch_gemm(int type, const GemmPlan& plan, const void* w, int64_t w_bytes, const void* workspace, float* c, int64_t ldc, int M, int N,
+                 int K, hipStream_t stream, bool accumulate, void* chunk_ws, size_t chunk_ws_bytes);
+// the same by tile tables: c[row] with row = c_rows ? c_rows[m] : m
+bool launch_gemm_tiles(int type, const GemmTiles& tiles, const void* w, int64_t w_bytes, const void* workspace, float* c, int64_t ldc,
+                       const int* c_rows, int M, int N, int K, hipStream_t stream, void* chunk_ws, size_t chunk_ws_bytes, int x_layout);
+// bytes of chunk_ws such a launch uses; only tiles.bm and tiles.count are read
+size_t gemm_tiles_ws_bytes(int type, const GemmTiles& tiles, int M, int N, int K, int x_layout);
 // the kernels address one weight (or one launch's converted activations) with 32-bit offsets
 constexpr int64_t kMaxOperandBytes = ((int64_t)1 << 31) - 64;
 

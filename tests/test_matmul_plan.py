@@ -1,0 +1,49 @@
+"""How products are planned (TSHip_MatmulPlanDevice): CPU tests, no GPU needed - the library assumes 256 CUs without one."""
+import ctypes as C
+
+import pytest
+
+from tensorsharp_amd import hip_native as N
+
+Q4_K, Q5_K, Q6_K, Q8_0, MXFP4, Q8_1, F32 = 12, 13, 14, 8, 39, 9, 0
+GEMV, DENSE, REGISTERS, WIDE, TILES = 1, 2, 3, 4, 5
+
+
+def plan(t, rows, n, k, accumulate=0):
+    """(kernel, rows per tile, K chunks, workspace bytes)"""
+    out = (C.c_int64 * 4)()
+    N.check_result(N.lib().TSHip_MatmulPlanDevice(t, rows, k, n, accumulate, out), "plan")
+    return tuple(out)
+
+
+def converted_bytes(rows, k):
+    """row scales and fp16 activations of a call, 256-byte granules"""
+    al = lambda b: (b + 255) // 256 * 256
+    return al(rows * ((k + 63) // 64 * 64) * 2 + al(rows * 4) + 256)
+
+
+def test_kernels_by_rows_columns_and_type():
+    for t in (Q4_K, Q5_K, Q6_K, Q8_0, MXFP4):
+        for rows in (1, 2, 3):
+            assert plan(t, rows, 4096, 4096) == (GEMV, 1, 1, 0)
+        assert plan(t, 4, 63, 4096)[0] == DENSE and plan(t, 4, 64, 4096)[0] != DENSE
+        assert plan(t, 4096, 4096, 1024)[0] in (WIDE, TILES)
+    assert plan(F32, 100, 4096, 4096) == (DENSE, 1, 1, 0)
+    assert plan(Q8_1, 100, 4096, 4096)[0] == DENSE
+
+
+@pytest.mark.parametrize("t", [Q4_K, Q5_K, Q6_K, Q8_0, MXFP4])
+@pytest.mark.parametrize("rows,n,k", [(4, 4096, 4096), (24, 14336, 4096), (200, 4096, 14336), (700, 1024, 2048), (2048, 21504, 5376)])
+@pytest.mark.parametrize("accumulate", [0, 1])
+def test_workspace_holds_the_converted_rows_and_the_chunk_sums(t, rows, n, k, accumulate):
+    kernel, tile, chunks, ws = plan(t, rows, n, k, accumulate)
+    sums = chunks * rows * n * 4 if chunks > 1 or (accumulate and kernel == REGISTERS) else 0     # the register kernel adds in a second pass
+    assert ws >= converted_bytes(rows, k) + sums
+    assert 1 <= chunks <= (k + 63) // 64 and tile in (32, 64, 96, 128, 256)
+
+
+def test_argument_errors():
+    out = (C.c_int64 * 4)()
+    for args in ((Q4_K, 0, 4096, 4096), (Q4_K, 8, 4000, 4096), (Q4_K, 8, 4096, 0), (77, 8, 4096, 4096)):
+        assert N.lib().TSHip_MatmulPlanDevice(*args, 0, out) == 0
+    assert N.lib().TSHip_MatmulPlanDevice(Q4_K, 8, 4096, 4096, 0, None) == 0
