@@ -601,6 +601,19 @@ int expert_tiles_x_layout(int type, int bm, int K, int out_features)
     return type == kTypeMXFP4 && bm == 32 && K <= 32768 && out_features >= 256 ? 1 : 0;
 }
 
+// The plan of one linear of the experts of a set, whose shape they share: experts of the same type as the one before them take
+// its plan.  (A set of 32 experts had been planned linear by linear, also where it runs as tile-table launches and needs none.)
+struct ExpertLinearPlan {
+    int type = -1;
+    MatmulPlan plan{};
+    const MatmulPlan& of(int t, int M, int64_t K, int64_t N)
+    {
+        if (t != type) plan = plan_matmul(t, M, K, N, false, false);
+        type = t;
+        return plan;
+    }
+};
+
 ExpertSetLayout expert_set_layout(int M, int n, const ExpertFfn* ex, int H, int I, int N)
 {
     auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
@@ -611,12 +624,6 @@ ExpertSetLayout expert_set_layout(int M, int n, const ExpertFfn* ex, int H, int 
     L.dn_off = L.act_off + (size_t)n * L.act_stride * sizeof(float);
     L.tmp_off = L.dn_off + (size_t)n * L.dn_stride * sizeof(float);
     L.mm_off = L.tmp_off + al((size_t)M * I * sizeof(float));
-    for (int e = 0; e < n; ++e) {
-        if (ex[e].gate) L.mm_bytes = std::max(L.mm_bytes, plan_matmul(ex[e].gate_type, M, H, I, false, false).total());
-        L.mm_bytes = std::max(L.mm_bytes, plan_matmul(ex[e].up_type, M, H, I, false, false).total());
-        L.mm_bytes = std::max(L.mm_bytes, plan_matmul(ex[e].down_type, M, I, N, false, false).total());
-    }
-    L.total = L.mm_off + L.mm_bytes;
     // the tiled form
     const int64_t rows = (int64_t)n * M;
     bool tiled = M > 1 && rows <= 65535;
@@ -628,7 +635,16 @@ ExpertSetLayout expert_set_layout(int M, int n, const ExpertFfn* ex, int H, int 
                 (!ex[e].gate || fits(ex[e].gate_type, I, H));
     }
     tiled = tiled && gemm_workspace_bytes((int)rows, std::max(H, I)) < (size_t)kMaxOperandBytes;
-    if (!tiled) return L;
+    if (!tiled) {
+        ExpertLinearPlan gate, up, down;
+        for (int e = 0; e < n; ++e) {
+            if (ex[e].gate) L.mm_bytes = std::max(L.mm_bytes, gate.of(ex[e].gate_type, M, H, I).total());
+            L.mm_bytes = std::max(L.mm_bytes, up.of(ex[e].up_type, M, H, I).total());
+            L.mm_bytes = std::max(L.mm_bytes, down.of(ex[e].down_type, M, I, N).total());
+        }
+        L.total = L.mm_off + L.mm_bytes;
+        return L;
+    }
     L.tiled = true;
     L.bm = M > 160 ? 128 : 32;
     const int ld = ex[0].gate ? 2 * I : I;
@@ -801,6 +817,7 @@ bool run_expert_set_device(const TSHipTensorView2D& out, const float* base, int6
         for (int e = 0; e < n; ++e) lin.w[e] = ex[e].down, lin.type[e] = ex[e].down_type;
         if (!run_expert_linear_tiled(L, ws, n, M, lin, rows_in, I, false, L.x2_off, dn, N, N, I, stream)) return false;
     } else {
+        ExpertLinearPlan gate_plan, up_plan, down_plan;
         for (int e = 0; e < n; ++e) {
             float* a_e = act + (size_t)e * L.act_stride;
             float* d_e = dn + (size_t)e * L.dn_stride;
@@ -809,16 +826,16 @@ bool run_expert_set_device(const TSHipTensorView2D& out, const float* base, int6
                 const int64_t span = (int64_t)(((size_t)(M - 1) * 2 * I + I) * sizeof(float));
                 const TSHipTensorView2D g_view{a_e, M, I, 2 * I, 1, span};
                 const TSHipTensorView2D u_view{a_e + I, M, I, 2 * I, 1, span};
-                if (!run_matmul_device_ws(plan_matmul(ex[e].gate_type, M, H, I, false, false), g_view, x, ex[e].gate, ex[e].gate_type, H, I, stream, mm_ws, L.mm_bytes, nullptr, 0.f, false)) return false;
-                if (!run_matmul_device_ws(plan_matmul(ex[e].up_type, M, H, I, false, false), u_view, x, ex[e].up, ex[e].up_type, H, I, stream, mm_ws, L.mm_bytes, nullptr, 0.f, false)) return false;
+                if (!run_matmul_device_ws(gate_plan.of(ex[e].gate_type, M, H, I), g_view, x, ex[e].gate, ex[e].gate_type, H, I, stream, mm_ws, L.mm_bytes, nullptr, 0.f, false)) return false;
+                if (!run_matmul_device_ws(up_plan.of(ex[e].up_type, M, H, I), u_view, x, ex[e].up, ex[e].up_type, H, I, stream, mm_ws, L.mm_bytes, nullptr, 0.f, false)) return false;
                 if (!launch_silu_mul(a_e, 2 * I, M, I, tmp, stream)) return false;
                 const TSHipTensorView2D t_view{tmp, M, I, I, 1, (int64_t)((size_t)M * I * sizeof(float))};
-                if (!run_matmul_device_ws(plan_matmul(ex[e].down_type, M, I, N, false, false), d_view, t_view, ex[e].down, ex[e].down_type, I, N, stream, mm_ws, L.mm_bytes, nullptr, 0.f, false)) return false;
+                if (!run_matmul_device_ws(down_plan.of(ex[e].down_type, M, I, N), d_view, t_view, ex[e].down, ex[e].down_type, I, N, stream, mm_ws, L.mm_bytes, nullptr, 0.f, false)) return false;
             } else {
                 const TSHipTensorView2D u_view{a_e, M, I, I, 1, (int64_t)((size_t)M * I * sizeof(float))};
-                if (!run_matmul_device_ws(plan_matmul(ex[e].up_type, M, H, I, false, false), u_view, x, ex[e].up, ex[e].up_type, H, I, stream, mm_ws, L.mm_bytes, nullptr, 0.f, false)) return false;
+                if (!run_matmul_device_ws(up_plan.of(ex[e].up_type, M, H, I), u_view, x, ex[e].up, ex[e].up_type, H, I, stream, mm_ws, L.mm_bytes, nullptr, 0.f, false)) return false;
                 if (!launch_relu_sqr(a_e, (int64_t)M * I, stream)) return false;
-                if (!run_matmul_device_ws(plan_matmul(ex[e].down_type, M, I, N, false, false), d_view, u_view, ex[e].down, ex[e].down_type, I, N, stream, mm_ws, L.mm_bytes, nullptr, 0.f, false)) return false;
+                if (!run_matmul_device_ws(down_plan.of(ex[e].down_type, M, I, N), d_view, u_view, ex[e].down, ex[e].down_type, I, N, stream, mm_ws, L.mm_bytes, nullptr, 0.f, false)) return false;
             }
         }
     }
