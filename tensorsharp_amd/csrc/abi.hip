@@ -370,9 +370,18 @@ MatmulPlan plan_matmul(int type, int M, int64_t K, int64_t N, bool norm, bool ac
     const size_t kp = (size_t)((K + 63) / 64) * 64;
     p.m_step = (int)std::min<int64_t>(M, std::max<int64_t>(256, ((kMaxOperandBytes - 1) / (int64_t)(kp * 2)) / 256 * 256));
     p.conv_bytes = al(gemm_workspace_bytes(p.m_step, (int)K));
-    // the launches of a call differ only in their last, smaller slices: the first one needs the most
-    p.gemm = plan_gemm(type, p.m_step, (int)std::min<int64_t>(N, p.n_step), (int)K, accumulate);
-    p.chunk_bytes = al(p.gemm.chunk_bytes);
+    // The last slice of rows and of columns may be smaller, and few tiles want more K chunks than many: the sums of the
+    // hungriest slice have to fit.
+    const int n_full = (int)std::min<int64_t>(N, p.n_step), m_rest = M % p.m_step, n_rest = (int)(N % n_full);
+    p.gemm = plan_gemm(type, p.m_step, n_full, (int)K, accumulate);
+    p.chunk_bytes = p.gemm.chunk_bytes;
+    auto also = [&](int m, int n) {
+        if (m > 0 && n > 0) p.chunk_bytes = std::max(p.chunk_bytes, plan_gemm(type, m, n, (int)K, accumulate).chunk_bytes);
+    };
+    also(m_rest, n_full);
+    also(p.m_step, n_rest);
+    also(m_rest, n_rest);
+    p.chunk_bytes = al(p.chunk_bytes);
     return p;
 }
 

@@ -47,3 +47,17 @@ def test_argument_errors():
     for args in ((Q4_K, 0, 4096, 4096), (Q4_K, 8, 4000, 4096), (Q4_K, 8, 4096, 0), (77, 8, 4096, 4096)):
         assert N.lib().TSHip_MatmulPlanDevice(*args, 0, out) == 0
     assert N.lib().TSHip_MatmulPlanDevice(Q4_K, 8, 4096, 4096, 0, None) == 0
+
+
+@pytest.mark.parametrize("t,rows,n,k,m_step,n_step", [
+    # activations beyond 2 GiB of fp16: 16128 rows at a time, and a rest whose 32-row units need their K-chunk sums
+    (Q5_K, 16128 + 32, 64, 65536, 16128, 64), (MXFP4, 16128 + 9, 300, 65536, 16128, 300), (Q4_K, 16128 + 32, 300, 65536, 16128, 300),
+    # weights beyond 2 GiB: 123136 columns at a time, and a rest of few tiles
+    (Q8_0, 512, 123136 + 300, 16384, 512, 123136), (Q4_K, 700, 232960 + 70, 16384, 700, 232960), (Q6_K, 40, 159744 + 513, 16384, 40, 159744),
+])
+def test_workspace_holds_the_sums_of_every_slice(t, rows, n, k, m_step, n_step):
+    have = plan(t, rows, n, k)[3] - converted_bytes(m_step, k)
+    for m in {m_step, rows % m_step or m_step}:
+        for cols in {n_step, n % n_step or n_step}:
+            need = plan(t, m, cols, k)[3] - converted_bytes(m, k)
+            assert have >= need, (m, cols, have, need)
