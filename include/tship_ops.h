@@ -322,14 +322,15 @@ TSHIP_EXPORT int TSHip_MulMatIdF32Device(TSHipTensorView3D result, TSHipTensorVi
 TSHIP_EXPORT int TSHip_SetGemvTimeline(void* device_buffer, int64_t capacity_bytes);
 
 /* Diagnostics, no counterpart in the reference: how a product of `rows` activation rows with such a weight runs on the device
- * (accumulate: added to the result).  plan[0] kernel (TSHIP_PLAN_*), plan[1] activation rows per tile, plan[2] K chunks
+ * (accumulate: added to the result; max_workspace: at most that many bytes of workspace, 0 for no bound).  plan[0] kernel (TSHIP_PLAN_*), plan[1] activation rows per tile, plan[2] K chunks
  * whose sums meet in the workspace (1: none), plan[3] workspace bytes.  Needs no GPU (256 CUs are assumed without one). */
 #define TSHIP_PLAN_GEMV 1        /* one GEMV per row */
 #define TSHIP_PLAN_DENSE 2       /* dense kernel (dense weights, or an exact fp32 copy of a narrow one) */
 #define TSHIP_PLAN_REGISTERS 3   /* units of 32 rows x 32 columns, activations in registers */
 #define TSHIP_PLAN_WIDE 4        /* 32 .. 128 rows x 256 columns */
 #define TSHIP_PLAN_TILES 5       /* 128- or 256-row tiles */
-TSHIP_EXPORT int TSHip_MatmulPlanDevice(int m2_ggml_type, int rows, int64_t m2_ne0, int64_t m2_ne1, int accumulate, int64_t plan[4]);
+TSHIP_EXPORT int TSHip_MatmulPlanDevice(int m2_ggml_type, int rows, int64_t m2_ne0, int64_t m2_ne1, int accumulate, int64_t max_workspace,
+                                       int64_t plan[4]);
 
 /* replaces TSGgml_AddIdF32 (ggml_ops_matmul.cpp:1123-1290, :1451-1473; GgmlNative.cs:442-448, :1081-1084; managed
  * GgmlBasicOps.AddID :1092-1108): ggml_add_id, the per-expert bias that goes with a mul_mat_id,

@@ -329,10 +329,11 @@ struct MatmulPlan {
     size_t total() const { return conv_bytes + chunk_bytes; }
 };
 
-// norm: RMSNorm prologue on the activations; accumulate: the product is added to the result.  One plan serves the size of a
+// norm: RMSNorm prologue on the activations; accumulate: the product is added to the result; max_ws: the workspace that the
+// call will have - kernels and K chunks are chosen so that their sums fit what the conversions leave of it.  One plan serves the size of a
 // call's workspace, its conversions and its launches.
 
-MatmulPlan plan_matmul(int type, int M, int64_t K, int64_t N, bool norm, bool accumulate)
+MatmulPlan plan_matmul(int type, int M, int64_t K, int64_t N, bool norm, bool accumulate, size_t max_ws = ~(size_t)0)
 {
     auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
     MatmulPlan p{};
@@ -373,20 +374,21 @@ MatmulPlan plan_matmul(int type, int M, int64_t K, int64_t N, bool norm, bool ac
     // The last slice of rows and of columns may be smaller, and few tiles want more K chunks than many: the sums of the
     // hungriest slice have to fit.
     const int n_full = (int)std::min<int64_t>(N, p.n_step), m_rest = M % p.m_step, n_rest = (int)(N % n_full);
-    p.gemm = plan_gemm(type, p.m_step, n_full, (int)K, accumulate);
+    const size_t max_chunk = max_ws > p.conv_bytes ? max_ws - p.conv_bytes : 0;
+    p.gemm = plan_gemm(type, p.m_step, n_full, (int)K, accumulate, max_chunk);
     p.chunk_bytes = p.gemm.chunk_bytes;
     auto also = [&](int m, int n) {
-        if (m > 0 && n > 0) p.chunk_bytes = std::max(p.chunk_bytes, plan_gemm(type, m, n, (int)K, accumulate).chunk_bytes);
+        if (m > 0 && n > 0) p.chunk_bytes = std::max(p.chunk_bytes, plan_gemm(type, m, n, (int)K, accumulate, max_chunk).chunk_bytes);
     };
     also(m_rest, n_full);
     also(p.m_step, n_rest);
     also(m_rest, n_rest);
-    p.chunk_bytes = al(p.chunk_bytes);
+    p.chunk_bytes = std::min(al(p.chunk_bytes), max_chunk);
     return p;
 }
 
 // result (+)= f(m1) * W^T with f = identity or RMSNorm(eps) * norm_w, as `plan` (of the same call) says.  All pointers are
-// device pointers; `ws` has ws_bytes >= plan.total() bytes (with fewer, the K-chunk sums are given up first: see launch_gemm).
+// device pointers; `ws` has ws_bytes >= plan.total() bytes.
 bool run_matmul_device_ws(const MatmulPlan& plan, const TSHipTensorView2D& result, const TSHipTensorView2D& m1, const void* w, int type,
                           int64_t K, int64_t N, hipStream_t stream, void* ws, size_t ws_bytes, const float* norm_w, float eps, bool accumulate)
 {
@@ -454,7 +456,7 @@ bool run_matmul_device_ws(const MatmulPlan& plan, const TSHipTensorView2D& resul
         for (int64_t n0 = 0; n0 < N; n0 += plan.n_step) {
             const int64_t n = std::min<int64_t>(plan.n_step, N - n0);
             const bool whole = m == plan.m_step && n == std::min<int64_t>(N, plan.n_step);
-            const GemmPlan g = whole ? plan.gemm : plan_gemm(type, m, (int)n, (int)K, accumulate);
+            const GemmPlan g = whole ? plan.gemm : plan_gemm(type, m, (int)n, (int)K, accumulate, chunk_bytes);
             if (g.x_layout != converted) {
                 if (!launch_convert_x(type, x, m1.stride0, nullptr, m, (int)K, ws, stream, norm_w, eps, g.x_layout)) return false;
                 converted = g.x_layout;
@@ -1433,7 +1435,7 @@ int TSHip_SetGemvTimeline(void* device_buffer, int64_t capacity_bytes)
     return 1;
 }
 
-int TSHip_MatmulPlanDevice(int m2_ggml_type, int rows, int64_t m2_ne0, int64_t m2_ne1, int accumulate, int64_t plan[4])
+int TSHip_MatmulPlanDevice(int m2_ggml_type, int rows, int64_t m2_ne0, int64_t m2_ne1, int accumulate, int64_t max_workspace, int64_t plan[4])
 {
     return guarded(0, "matmul_plan", [&]() -> int {
         if (!plan || rows <= 0 || m2_ne0 <= 0 || m2_ne0 > INT32_MAX || m2_ne1 <= 0 || !is_matmul_type(m2_ggml_type) ||
@@ -1441,7 +1443,8 @@ int TSHip_MatmulPlanDevice(int m2_ggml_type, int rows, int64_t m2_ne0, int64_t m
             set_last_error("Invalid arguments for matmul_plan.");
             return 0;
         }
-        const MatmulPlan p = plan_matmul(m2_ggml_type, rows, m2_ne0, m2_ne1, false, accumulate != 0);
+        const MatmulPlan p = plan_matmul(m2_ggml_type, rows, m2_ne0, m2_ne1, false, accumulate != 0,
+                                         max_workspace > 0 ? (size_t)max_workspace : ~(size_t)0);
         const bool dense = is_dense_type(m2_ggml_type) || m2_ggml_type == kTypeQ8_1 || p.narrow;
         const int64_t sums = (int64_t)p.m_step * std::min<int64_t>(p.n_step, m2_ne1) * (int64_t)sizeof(float);
         plan[0] = dense ? TSHIP_PLAN_DENSE : p.gemv ? TSHIP_PLAN_GEMV
@@ -1517,7 +1520,7 @@ int TSHip_AddmmQuantF32DeviceNoAlloc(TSHipTensorView2D result, TSHipTensorView2D
         if (!validate_addmm_quant(result, m1, m2_data, m2_ggml_type, m2_ne0, m2_ne1, m2_raw_bytes)) return 0;
         if (!check_device_views(result, m1)) return 0;
         // [converted activations + row scales][sums of K chunks]: both live in the static array
-        const MatmulPlan plan = plan_matmul(m2_ggml_type, m1.dim0, m2_ne0, m2_ne1, false, false);
+        const MatmulPlan plan = plan_matmul(m2_ggml_type, m1.dim0, m2_ne0, m2_ne1, false, false, kScratchBytes);
         const size_t need = plan.conv_bytes;
         if (need > kScratchBytes) {
             set_last_error("addmm_quant (no-alloc): the converted activations of this call (" + std::to_string(need) +

@@ -3601,17 +3601,18 @@ struct WidePlan {
     int tm, k_chunks, chunk_kt;
     double us;
 };
+inline bool chunk_sums_fit(int k_chunks, int M, int N, size_t max_bytes) { return (size_t)k_chunks * M * N * sizeof(float) <= max_bytes; }
 inline double chunk_sum_us(int k_chunks, int M, int N) { return k_chunks > 1 ? 3.0 + (double)k_chunks * M * N * 8 / 8.0e6 : 0.0; }
-inline WidePlan pick_wide(int M, int N, int nkt, bool chunks, double base, double per_row_block)
+inline WidePlan pick_wide(int M, int N, int nkt, size_t max_chunk_bytes, double base, double per_row_block)
 {
     WidePlan best{0, 1, 0, 0.0};
     const int cus = device_info().num_cus, n_tiles = (N + 255) / 256;
     for (int tm = 1; tm <= 4; ++tm) {
         const int m_tiles = (M + 32 * tm - 1) / (32 * tm);
-        for (int sc = 1; sc <= (chunks ? 8 : 1); ++sc) {
+        for (int sc = 1; sc <= 8; ++sc) {
             const int chunk = ((nkt + sc - 1) / sc + 3) / 4 * 4;
             const int kc = (nkt + chunk - 1) / chunk;
-            if (sc > 1 && (kc != sc || chunk < 8)) continue;
+            if (sc > 1 && (kc != sc || chunk < 8 || !chunk_sums_fit(kc, M, N, max_chunk_bytes))) continue;
             const int64_t units = (int64_t)m_tiles * n_tiles * kc, rounds = (units + cus - 1) / cus;
             const double fill = (double)units / (double)(rounds * cus);
             const double us = (double)rounds * (chunk * (base + per_row_block * tm) * (0.6 + 0.4 * fill) + 3.0) + chunk_sum_us(kc, M, N);
@@ -3635,17 +3636,17 @@ bool launch_wide_tm(const GemmArgs& a, hipStream_t stream)
 }
 
 template <typename H>
-bool launch_wide(GemmArgs a, WidePlan p, hipStream_t stream, const ChunkScratch& cs)
+bool launch_wide(GemmArgs a, const WidePlan& p, hipStream_t stream, const ChunkScratch& cs)
 {
-    const int nkt = a.Kp / kBK;
-    if (p.tm == 0) p = pick_wide(a.M, a.N, nkt, true, H::kUsBase, H::kUsRow);
     a.partial = nullptr;
     if (p.k_chunks > 1) {
         const size_t need = (size_t)p.k_chunks * a.M * a.N * sizeof(float);
         if (cs.need_out) *cs.need_out = need;
         a.partial = chunk_scratch(cs, need);
-        // the caller's scratch is too small for the chunk sums: whole K per tile (slower)
-        if (!a.partial) p = pick_wide(a.M, a.N, nkt, false, H::kUsBase, H::kUsRow);
+        if (!a.partial && !cs.need_out) {
+            set_last_error("gemm: the K-chunk sums of this shape do not fit the scratch buffer.");
+            return false;
+        }
     }
     if (cs.need_out) return true;
     a.m_tiles = (a.M + 32 * p.tm - 1) / (32 * p.tm);
@@ -3703,16 +3704,7 @@ bool launch_for_type(const GemmArgs& a, int bm, int m_tiles, const WidePlan& wid
         if constexpr (std::is_same<G, GQ80>::value) return launch_wide<WQ80>(a, wide, stream, cs);
         if constexpr (std::is_same<G, GQ6K>::value) return launch_wide<WQ6K>(a, wide, stream, cs);
     }
-    if (bm == 32 && !a.x_mx) {
-        const int ktw = slim_ktw<G>(a.Kp / kBK), kc = (a.Kp / kBK + 8 * ktw - 1) / (8 * ktw);
-        // (a plain launch whose chunk sums do not fit the caller's scratch: tiles that need none)
-        const bool fits = cs.need_out || (kc == 1 && !a.accumulate) || chunk_scratch(cs, (size_t)kc * a.M * a.N * sizeof(float));
-        if (fits || a.tile_expert) return launch_slim_for<G>(a, ktw, m_tiles, stream, cs);
-        if constexpr (std::is_same<G, GQ4K>::value) return launch_xw<PQ4K, 256, 4>(a, (a.M + 255) / 256, stream, cs);
-        if constexpr (std::is_same<G, GQ80>::value) return launch_wide<WQ80>(a, wide, stream, cs);
-        if constexpr (std::is_same<G, GQ6K>::value) return launch_wide<WQ6K>(a, wide, stream, cs);
-        return launch_slim_for<G>(a, ktw, m_tiles, stream, cs);
-    }
+    if (bm == 32 && !a.x_mx) return launch_slim_for<G>(a, slim_ktw<G>(a.Kp / kBK), m_tiles, stream, cs);
     // Q4_K and MXFP4: the 2 x 4 wavefront layout with the operand exchange through LDS (gemm_xw_kernel); 128-row tiles are
     // 128 x 256.  Q4_K takes it for every launch, MXFP4 for plain ones: the MXFP4 expert tiles of a MoE prefill (128
     // rows) stay on two 128 x 128 workgroups per CU (926 vs 968 us at 2048 tokens).
@@ -3788,22 +3780,27 @@ bool wide_128_row_tiles(int type)
 }  // namespace
 
 namespace {
+constexpr double kNoScratch = 1e30;      // a kernel that cannot do without chunk sums which do not fit
+
 // Expected microseconds of the register-resident kernel: a unit (32 rows x 32 columns x 8 ktw k-tiles) takes 3.0 (ktw 4) to
 // 4.4 us (ktw 8), a workgroup that crosses into another row tile or K chunk loads its activations again.
 template <typename G>
-double slim_us(int M, int N, int nkt)
+double slim_us(int M, int N, int nkt, bool accumulate, size_t max_chunk_bytes)
 {
     const int ktw = slim_ktw<G>(nkt), kc = (nkt + 8 * ktw - 1) / (8 * ktw), cus = device_info().num_cus;
+    if ((kc > 1 || accumulate) && !chunk_sums_fit(kc, M, N, max_chunk_bytes)) return kNoScratch;
     const int64_t segments = (int64_t)((M + 31) / 32) * kc, units = segments * ((N + 31) / 32);
     const bool crosses = segments > 1 && units > cus && units % cus != 0;
     return 5.0 + (double)((units + cus - 1) / cus) * (1.6 + 0.35 * ktw) + (crosses ? 8.0 : 0.0) + chunk_sum_us(kc, M, N);
 }
 
 // and of the 256 x 256 tiles of gemm_kernel / gemm_xw_kernel: 2.0 us per k-tile and round with all CUs at work
-double tile256_us(int M, int N, int nkt)
+double tile256_us(int M, int N, int nkt, size_t max_chunk_bytes)
 {
     const int cus = device_info().num_cus;
-    const int tiles = ((M + 255) / 256) * ((N + 255) / 256), kc = pick_k_chunks(tiles, nkt, cus, (int64_t)M * N, 1.7);
+    const int tiles = ((M + 255) / 256) * ((N + 255) / 256);
+    int kc = pick_k_chunks(tiles, nkt, cus, (int64_t)M * N, 1.7);
+    if (!chunk_sums_fit(kc, M, N, max_chunk_bytes)) kc = 1;       // (as the launchers do)
     const int64_t units = (int64_t)tiles * kc, rounds = (units + cus - 1) / cus;
     const double fill = (double)units / (double)(rounds * cus);
     return (double)rounds * (nkt / (double)kc * 2.0 * (0.5 + 0.5 * fill) + 3.0) + chunk_sum_us(kc, M, N);
@@ -3815,24 +3812,24 @@ double tile256_us(int M, int N, int nkt)
 // 256-row tiles keep many rows of wide weights (Q4_K 2048 x 21504 x 5376 494 vs 567 us, Q8_0 700 x 14336 x 4096 121 vs 138):
 // they take half as many weight lines per result.
 template <typename G, typename W>
-int cheapest_tiles(int M, int N, int K, WidePlan* plan)
+int cheapest_tiles(int M, int N, int K, bool accumulate, size_t max_chunk_bytes, WidePlan* plan)
 {
     const int nkt = (K + kBK - 1) / kBK;
-    *plan = pick_wide(M, N, nkt, true, W::kUsBase, W::kUsRow);
-    const double wide = plan->us, slim = slim_us<G>(M, N, nkt);
-    const double tile = std::is_same<G, GQ6K>::value ? wide : tile256_us(M, N, nkt);       // (no 256-row tiles of Q6_K)
+    const double slim = slim_us<G>(M, N, nkt, accumulate, max_chunk_bytes);
+    if (M <= 3 && slim < kNoScratch) return 32;
+    *plan = pick_wide(M, N, nkt, max_chunk_bytes, W::kUsBase, W::kUsRow);
+    const double wide = plan->us;
+    const double tile = std::is_same<G, GQ6K>::value ? wide : tile256_us(M, N, nkt, max_chunk_bytes);       // (no 256-row tiles of Q6_K)
     if (slim <= wide && slim <= tile) return 32;
     return wide <= tile ? kWideTiles : 256;
 }
 
 // Rows of activations per tile of a plain launch (kWideTiles: gemm_wide_kernel, as *wide says)
-int gemm_tile_m(int type, int M, int N, int K, WidePlan* wide)
+int gemm_tile_m(int type, int M, int N, int K, bool accumulate, size_t max_chunk_bytes, WidePlan* wide)
 {
-    if (M > 3) {
-        if (type == kTypeQ4_K) return cheapest_tiles<GQ4K, WQ4K>(M, N, K, wide);
-        if (type == kTypeQ8_0) return cheapest_tiles<GQ80, WQ80>(M, N, K, wide);
-        if (type == kTypeQ6_K) return cheapest_tiles<GQ6K, WQ6K>(M, N, K, wide);
-    }
+    if (type == kTypeQ4_K) return cheapest_tiles<GQ4K, WQ4K>(M, N, K, accumulate, max_chunk_bytes, wide);
+    if (type == kTypeQ8_0) return cheapest_tiles<GQ80, WQ80>(M, N, K, accumulate, max_chunk_bytes, wide);
+    if (type == kTypeQ6_K) return cheapest_tiles<GQ6K, WQ6K>(M, N, K, accumulate, max_chunk_bytes, wide);
     if (M <= 128) return 32;
     if (type == kTypeMXFP4 && M <= 512 && ((M + 127) / 128) * ((N + 127) / 128) <= 128) return 32;
     // 128- or 256-row tiles by rounds of workgroups x time per k-tile of a round (measured per k-tile: a 256 x 256 tile
@@ -3982,7 +3979,7 @@ bool gemm_dispatch_tiles(int type, GemmArgs a, const int* c_rows, const GemmTile
 }
 }  // namespace
 
-GemmPlan plan_gemm(int type, int M, int N, int K, bool accumulate)
+GemmPlan plan_gemm(int type, int M, int N, int K, bool accumulate, size_t max_chunk_bytes)
 {
     GemmPlan p{};
     if (!is_quant_type(type)) {
@@ -3990,7 +3987,7 @@ GemmPlan plan_gemm(int type, int M, int N, int K, bool accumulate)
         return p;
     }
     WidePlan wide{0, 1, 0, 0.0};
-    p.bm = gemm_tile_m(type, M, N, K, &wide);
+    p.bm = gemm_tile_m(type, M, N, K, accumulate, max_chunk_bytes, &wide);
     p.wide_tm = wide.tm;
     p.k_chunks = wide.k_chunks;
     p.chunk_kt = wide.chunk_kt;
@@ -4000,12 +3997,13 @@ GemmPlan plan_gemm(int type, int M, int N, int K, bool accumulate)
     // gemm_wide_kernel reads natural order, which for the other two formats it serves is their unpack order anyway
     if (type == kTypeQ4_K && p.bm == kWideTiles) p.x_layout = 2;
     if (type == kTypeMXFP4 && K <= 1024 * kCvtHold * 4 && (p.bm >= 128 || (int64_t)N * K >= ((int64_t)64 << 20))) p.x_layout = 1;
-    // a buffer "large enough", so that the launcher makes the choices it would make with the reported bytes at hand
+    // the launcher's own dry run, with no bound, so that it makes the choices it would make with the reported bytes at hand
     const ChunkScratch cs{nullptr, ~(size_t)0, &p.chunk_bytes};
     GemmArgs a{};
     const int64_t w_bytes = block_bytes(type) * (K / block_elems(type)) * N;
     if (!gemm_args(&a, nullptr, w_bytes, nullptr, nullptr, N, M, N, K, p.x_layout) || !gemm_dispatch_plan(type, a, p, nullptr, accumulate, cs))
         p.chunk_bytes = 0;
+    if (p.bm >= 128 && p.chunk_bytes > max_chunk_bytes) p.chunk_bytes = 0;      // these run with whole K then
     return p;
 }
 

@@ -156,7 +156,8 @@ struct GemmPlan {
                                          // the block-scaled matrix instruction), 2 fp16 in natural order (Q4_K on gemm_wide_kernel)
     size_t chunk_bytes;                  // scratch for the sums of K chunks (0 for most shapes)
 };
-GemmPlan plan_gemm(int type, int M, int N, int K, bool accumulate);
+// max_chunk_bytes: what the launch will be given; kernels and K chunks whose sums do not fit are passed over
+GemmPlan plan_gemm(int type, int M, int N, int K, bool accumulate, size_t max_chunk_bytes = ~(size_t)0);
 
 // fp32 activations -> workspace (fp16 in the weight format's unpack order + per-row scales);
 // row_map (device, optional) gathers source rows.
@@ -191,8 +192,8 @@ bool launch_gemm_swiglu_mx(const void* w, const void* workspace, void* workspace
                            float limit, int M, int F, int K, const GemmTiles* tiles, hipStream_t stream);
 
 // c[m] [N] = x16[m] . W^T * scale[m], m < M, as `plan` (of the same shape) says; accumulate: c[m] += ... instead of c[m] = ...
-// chunk_ws (device): where the sums of K chunks go, plan.chunk_bytes of them (a shape whose chunk sums do not fit what is
-// passed runs with whole K per tile, or fails when its kernel cannot do without chunks).  Nothing is allocated.
+// chunk_ws (device): where the sums of K chunks go, plan.chunk_bytes of them (with less, 128- and 256-row tiles run with whole K
+// and the other kernels fail: plan_gemm takes the bound).  Nothing is allocated.
 bool launch_gemm(int type, const GemmPlan& plan, const void* w, int64_t w_bytes, const void* workspace, float* c, int64_t ldc, int M, int N,
                  int K, hipStream_t stream, bool accumulate, void* chunk_ws, size_t chunk_ws_bytes);
 // the same by tile tables: c[row] with row = c_rows ? c_rows[m] : m

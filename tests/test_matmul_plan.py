@@ -9,10 +9,10 @@ Q4_K, Q5_K, Q6_K, Q8_0, MXFP4, Q8_1, F32 = 12, 13, 14, 8, 39, 9, 0
 GEMV, DENSE, REGISTERS, WIDE, TILES = 1, 2, 3, 4, 5
 
 
-def plan(t, rows, n, k, accumulate=0):
+def plan(t, rows, n, k, accumulate=0, max_workspace=0):
     """(kernel, rows per tile, K chunks, workspace bytes)"""
     out = (C.c_int64 * 4)()
-    N.check_result(N.lib().TSHip_MatmulPlanDevice(t, rows, k, n, accumulate, out), "plan")
+    N.check_result(N.lib().TSHip_MatmulPlanDevice(t, rows, k, n, accumulate, max_workspace, out), "plan")
     return tuple(out)
 
 
@@ -45,8 +45,8 @@ def test_workspace_holds_the_converted_rows_and_the_chunk_sums(t, rows, n, k, ac
 def test_argument_errors():
     out = (C.c_int64 * 4)()
     for args in ((Q4_K, 0, 4096, 4096), (Q4_K, 8, 4000, 4096), (Q4_K, 8, 4096, 0), (77, 8, 4096, 4096)):
-        assert N.lib().TSHip_MatmulPlanDevice(*args, 0, out) == 0
-    assert N.lib().TSHip_MatmulPlanDevice(Q4_K, 8, 4096, 4096, 0, None) == 0
+        assert N.lib().TSHip_MatmulPlanDevice(*args, 0, 0, out) == 0
+    assert N.lib().TSHip_MatmulPlanDevice(Q4_K, 8, 4096, 4096, 0, 0, None) == 0
 
 
 @pytest.mark.parametrize("t,rows,n,k,m_step,n_step", [
@@ -61,3 +61,20 @@ def test_workspace_holds_the_sums_of_every_slice(t, rows, n, k, m_step, n_step):
         for cols in {n_step, n % n_step or n_step}:
             need = plan(t, m, cols, k)[3] - converted_bytes(m, k)
             assert have >= need, (m, cols, have, need)
+
+
+@pytest.mark.parametrize("t,rows,n,k", [(Q6_K, 333, 4096, 14336), (Q4_K, 333, 4096, 14336), (Q8_0, 200, 4096, 14336), (Q4_K, 700, 4096, 14336),
+                                        (Q4_K, 64, 4096, 14336), (Q8_0, 16, 4096, 14336), (Q6_K, 20, 9728, 9728)])
+@pytest.mark.parametrize("accumulate", [0, 1])
+def test_a_bounded_workspace_keeps_as_many_chunks_as_fit(t, rows, n, k, accumulate):
+    conv, sums = converted_bytes(rows, k), rows * n * 4
+    kernel, _, free, ws = plan(t, rows, n, k, accumulate)
+    assert free >= 2 and ws >= conv + free * sums
+    assert plan(t, rows, n, k, accumulate, ws) == plan(t, rows, n, k, accumulate)           # just enough
+    last = free
+    for fit in range(free - 1, -1, -1):
+        got = plan(t, rows, n, k, accumulate, conv + fit * sums)
+        assert got[3] <= conv + fit * sums and got[2] <= max(fit, 1) and got[2] <= last
+        assert got[2] >= 2 or fit < 2 or got[0] != WIDE, (fit, got)        # some of the chunks, where the tiles take any number
+        last = got[2]
+    assert plan(t, rows, n, k, accumulate, 1)[2] == 1                       # (refused by the entry points: not even the conversions fit)
