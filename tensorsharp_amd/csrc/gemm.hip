@@ -26,6 +26,7 @@
 
 #include <algorithm>
 #include <mutex>
+#include <numeric>
 #include <type_traits>
 
 namespace tship {
@@ -454,8 +455,6 @@ __global__ void __launch_bounds__(kMxCvtBlocks) convert_x_mx_kernel(const Conver
 // ------------------------------------------------------------------------------------------
 struct GQ4K {
     static constexpr int kRegs = 8;
-    static constexpr int kSup = 4;            // one 256-element super-block
-    static constexpr int kRawRow = 144;       // LDS bytes of one row's super-tile window
     static constexpr int kTileStep = 4;       // a wavefront's K range starts at a multiple of this many k-tiles
     static constexpr uint32_t sup_offset(int s) { return (uint32_t)s * 144u; }            // window start of super-tile s
     static __device__ __forceinline__ uint32_t sup_delta(uint32_t delta, int /*s*/) { return delta; }
@@ -1672,9 +1671,7 @@ constexpr int kWideValu = (40 + 2 * TM - 1) / (2 * TM);
 //   fetch / unpack:      quarter q of its weights
 //   kSplit: the two groups of wavefronts split a k-tile (k-steps 0, 1 / 2, 3) instead of taking a k-tile each: half the
 //           activations per turn, for raw rows so large that two k-tiles' worth of both do not fit LDS
-//   kUsBase, kUsRow:     microseconds per k-tile and per 32 rows of it, for pick_wide
 struct WQ4K {
-    static constexpr double kUsBase = 0.53, kUsRow = 0.125;
     typedef GQ4K G;
     static constexpr int kSup = 4, kRawRow = 144, kPieces = 9, kHdr = 4, kState = 2, kQ = 2;
     static constexpr bool kSplit = false, kAligned = true;               // a block is 144 bytes: rows and blocks are 16-byte aligned
@@ -1719,7 +1716,6 @@ struct WQ4K {
     }
 };
 struct WQ80 {
-    static constexpr double kUsBase = 0.68, kUsRow = 0.11;
     typedef GQ80 G;
     static constexpr int kSup = 2, kRawRow = 176, kPieces = 10, kHdr = 1, kState = 1, kQ = 3;
     static constexpr bool kSplit = false, kAligned = false;
@@ -1756,7 +1752,6 @@ struct WQ80 {
 };
 // Q6_K: a granule is a block (210 bytes, even delta: fourteen pieces)
 struct WQ6K {
-    static constexpr double kUsBase = 1.1, kUsRow = 0.1;
     typedef GQ6K G;
     static constexpr int kSup = 4, kRawRow = 240, kPieces = 14, kHdr = 2, kState = 1, kQ = 6;
     static constexpr bool kSplit = true, kAligned = false;
@@ -3594,33 +3589,9 @@ bool launch_slim_for(const GemmArgs& a, int ktw, int m_tiles, hipStream_t stream
     return false;
 }
 
-// Rows and K chunks of a plain launch of gemm_wide_kernel, and the microseconds they are expected to take: rounds of
-// workgroups x k-tiles (a round that leaves CUs idle is up to 40 % faster: the kernel waits for the L2), start and end of
-// a workgroup, and for K chunks the second launch with its reads and writes of the chunk sums.
 struct WidePlan {
-    int tm, k_chunks, chunk_kt;
-    double us;
+    int tm, k_chunks, chunk_kt;      // rows per tile / 32, K chunks, k-tiles per chunk
 };
-inline bool chunk_sums_fit(int k_chunks, int M, int N, size_t max_bytes) { return (size_t)k_chunks * M * N * sizeof(float) <= max_bytes; }
-inline double chunk_sum_us(int k_chunks, int M, int N) { return k_chunks > 1 ? 3.0 + (double)k_chunks * M * N * 8 / 8.0e6 : 0.0; }
-inline WidePlan pick_wide(int M, int N, int nkt, size_t max_chunk_bytes, double base, double per_row_block)
-{
-    WidePlan best{0, 1, 0, 0.0};
-    const int cus = device_info().num_cus, n_tiles = (N + 255) / 256;
-    for (int tm = 1; tm <= 4; ++tm) {
-        const int m_tiles = (M + 32 * tm - 1) / (32 * tm);
-        for (int sc = 1; sc <= 8; ++sc) {
-            const int chunk = ((nkt + sc - 1) / sc + 3) / 4 * 4;
-            const int kc = (nkt + chunk - 1) / chunk;
-            if (sc > 1 && (kc != sc || chunk < 8 || !chunk_sums_fit(kc, M, N, max_chunk_bytes))) continue;
-            const int64_t units = (int64_t)m_tiles * n_tiles * kc, rounds = (units + cus - 1) / cus;
-            const double fill = (double)units / (double)(rounds * cus);
-            const double us = (double)rounds * (chunk * (base + per_row_block * tm) * (0.6 + 0.4 * fill) + 3.0) + chunk_sum_us(kc, M, N);
-            if (best.tm == 0 || us < best.us) best = WidePlan{tm, kc, chunk, us};
-        }
-    }
-    return best;
-}
 
 template <typename H, int TM>
 bool launch_wide_tm(const GemmArgs& a, hipStream_t stream)
@@ -3663,7 +3634,7 @@ bool launch_wide(GemmArgs a, const WidePlan& p, hipStream_t stream, const ChunkS
 
 // 128-row tiles are 128 x 256 (one workgroup per CU) for these formats, 128 x 128 (two per CU) for the others
 template <typename G>
-constexpr bool kWide128 = G::kSup == 2 || G::kRawRow > 144 || std::is_same<G, GQ4K>::value;
+constexpr bool kWide128 = G::kSup == 2 || G::kRawRow > 144;
 
 // 48-row units (gemm_slim_mx48_kernel): one K chunk
 template <int EPI>
@@ -3757,18 +3728,15 @@ size_t gemm_workspace_bytes(int M, int K)
     return (size_t)M * x_row_halfs(K) * sizeof(_Float16) + (((size_t)M * sizeof(float) + 255) & ~(size_t)255) + 256;
 }
 
-// Rows of activations per tile for a plain (ungrouped) launch.  The 32-row register-resident kernel streams the
-// weights once per 32 rows, but at a much higher rate than the LDS-tiled kernels and mostly out of the memory-side
-// cache, so it wins well past 32 rows (measured crossovers of the formats that gemm_wide_kernel does not serve: about 128
-// rows, MXFP4 up to 512 when the big tiles would leave CUs idle).
+// Rows of activations per tile for a plain (ungrouped) launch of the formats that gemm_wide_kernel does not serve.  The 32-row
+// register-resident kernel streams the weights once per 32 rows, but at a much higher rate than the LDS-tiled kernels and
+// mostly out of the memory-side cache, so it wins well past 32 rows (measured crossovers: about 128 rows, MXFP4 up to 512
+// when the big tiles would leave CUs idle).
 namespace {
 bool wide_128_row_tiles(int type)
 {
     switch (type) {
-    case kTypeQ4_K: return kWide128<GQ4K>;
     case kTypeMXFP4: return true;      // plain launches: gemm_xw_kernel's 128 x 256 tiles
-    case kTypeQ8_0: return kWide128<GQ80>;
-    case kTypeQ6_K: return kWide128<GQ6K>;
     case kTypeQ5_K: return kWide128<GQ5K>;
     case kTypeQ4_0: return kWide128<GLegacy<kTypeQ4_0>>;
     case kTypeQ4_1: return kWide128<GLegacy<kTypeQ4_1>>;
@@ -3780,56 +3748,123 @@ bool wide_128_row_tiles(int type)
 }  // namespace
 
 namespace {
-constexpr double kNoScratch = 1e30;      // a kernel that cannot do without chunk sums which do not fit
+// ---- which kernel serves a plain launch of Q4_K, Q8_0 and Q6_K -----------------------------------
+// The cheapest of the register-resident kernel, gemm_wide_kernel (four tile heights, up to eight K chunks) and the 128- and
+// 256-row tiles, by what they are expected to cost.  The constants (microseconds) were fitted to measured calls, conversion
+// included, with weights that come from HBM: 14 shapes from 1024 x 4096 to 28672 x 4096 with 24 row counts from 4 to 2048, and
+// about 380 random ones per format over 4 .. 2048 rows, 1000 .. 28672 columns and K of 1024 .. 21504, a third of them added to
+// a residual.  On the calls it was fitted to the pick takes 0.4 % (Q4_K), 0.5 % (Q8_0) and 0.2 % (Q6_K) longer than the fastest
+// candidate on average and more than 4 % longer on 25 of 714, 23 of 576 and 1 of 559; on 200 random calls per format that an
+// earlier fit of the same form had not seen 0.9, 1.1 and 0.2 %.  Where the lines lie, us (register-resident / gemm_wide_kernel
+// / 128 rows / 256 rows):
+//   Q4_K  8 x 4096 x 4096 12.4 / 16.3 / - / -,  64 x 4096 x 4096 17.4 / 21.0 / 28.5 / 34.0,  200 x 4096 x 4096 38.5 / 28.3 / 32.2 /
+//         39.8,  1024 x 9728 x 2560 151 / 85.8 / 104.7 / 68.7
+//   Q8_0  8 x 14336 x 4096 23.2 / 24.0 / - / -,  128 x 28672 x 4096 90.7 / 60.0 / 67.0 / 76.6,  400 x 4096 x 4096 - / 39.2 / 37.4 / -
+//   Q6_K  512 x 4096 x 4096 - / 47.5 / 45.1 / -,  2048 x 2560 x 9728 - / 200.8 / 240.7 / -
+struct RuleCosts {
+    // register-resident kernel: a call; its activations, per 32 rows and 8 k-tiles per wavefront; a round of units and per k-tile
+    // of a wavefront in it; a workgroup whose units cross into another row tile or K chunk (it loads activations anew)
+    double slim, slim_rows, unit, unit_kt, cross, cross_kt;
+    // gemm_wide_kernel: a call, a k-tile of a round and per 32 rows in it, the share of that time that an almost empty round
+    // takes, a round
+    double wide, wide_kt, wide_kt_rows, wide_fill, wide_round;
+    double t256, t256_kt, t256_fill, t256_round;      // 256- and 128-row tiles, likewise
+    double t128, t128_kt, t128_fill, t128_round;
+    double sums, sums_rate;                            // the launch that adds K chunks: a call, TB/s of its sums written and read
+    double add;                                        // results added in place, per 1e6 of them
+};
+constexpr RuleCosts kCostsQ4K{6.257, 6.384, 0.284, 0.533, 1.675, 0.777, 4.941, 0.370, 0.165, 0.951, 4.558,
+                              4.514, 1.637, 0.628, 5.768, 0.697, 1.244, 0.892, 5.599, 1.546, 4.218, 3.963};
+constexpr RuleCosts kCostsQ80{5.688, 8.132, 0.854, 0.474, 0.044, 1.016, 4.734, 0.444, 0.168, 0.988, 6.634,
+                              0.000, 1.791, 0.976, 7.753, 3.439, 1.404, 1.040, 2.000, 0.768, 4.952, 3.239};
+constexpr RuleCosts kCostsQ6K{6.557, 4.816, 0.457, 0.662, 1.910, 0.430, 4.096, 1.010, 0.144, 0.948, 8.949,      // (no 256-row tiles)
+                              0.000, 0.000, 0.000, 0.000, 7.308, 1.649, 0.909, 0.727, 3.024, 9.405, 3.810};
+constexpr double kNotServed = 1e30;      // a kernel that a format has not, or whose chunk sums do not fit
 
-// Expected microseconds of the register-resident kernel: a unit (32 rows x 32 columns x 8 ktw k-tiles) takes 3.0 (ktw 4) to
-// 4.4 us (ktw 8), a workgroup that crosses into another row tile or K chunk loads its activations again.
+inline bool chunk_sums_fit(int k_chunks, int M, int N, size_t max_bytes) { return (size_t)k_chunks * M * N * sizeof(float) <= max_bytes; }
+inline double sums_us(const RuleCosts& c, int k_chunks, int M, int N) { return c.sums + (double)k_chunks * M * N * 8e-6 / c.sums_rate; }
+// what follows the tiles of gemm_wide_kernel and of the 128- and 256-row kernels
+inline double finish_us(const RuleCosts& c, int k_chunks, int M, int N, bool accumulate)
+{
+    return k_chunks > 1 ? sums_us(c, k_chunks, M, N) : accumulate ? c.add * M * N * 1e-6 : 0.0;
+}
+
 template <typename G>
-double slim_us(int M, int N, int nkt, bool accumulate, size_t max_chunk_bytes)
+double slim_us(const RuleCosts& c, int M, int N, int nkt, bool accumulate, size_t max_chunk_bytes)
 {
     const int ktw = slim_ktw<G>(nkt), kc = (nkt + 8 * ktw - 1) / (8 * ktw), cus = device_info().num_cus;
-    if ((kc > 1 || accumulate) && !chunk_sums_fit(kc, M, N, max_chunk_bytes)) return kNoScratch;
-    const int64_t segments = (int64_t)((M + 31) / 32) * kc, units = segments * ((N + 31) / 32);
-    const bool crosses = segments > 1 && units > cus && units % cus != 0;
-    return 5.0 + (double)((units + cus - 1) / cus) * (1.6 + 0.35 * ktw) + (crosses ? 8.0 : 0.0) + chunk_sum_us(kc, M, N);
+    const bool two_pass = kc > 1 || accumulate;          // (launch_slim adds to a residual in the second launch only)
+    if (two_pass && !chunk_sums_fit(kc, M, N, max_chunk_bytes)) return kNotServed;
+    const int64_t segments = (int64_t)((M + 31) / 32) * kc, n32 = (N + 31) / 32, units = segments * n32;
+    // Workgroup b takes the units from floor(units b / cus) on.  Segment i ends inside a workgroup's run unless n32 ((-i cus) mod
+    // segments) < cus, and over all i that remainder is at most segments - gcd(segments, cus).
+    const bool crosses = units > cus && n32 * (segments - std::gcd(segments, (int64_t)cus)) >= cus;
+    const double kt = 0.4 * ktw + 0.6 * nkt / (8.0 * kc);      // (wavefronts past the end of K leave theirs to the others)
+    return c.slim + c.slim_rows * std::min(M, 32) * ktw / 256.0 + (double)((units + cus - 1) / cus) * (c.unit + c.unit_kt * kt) +
+           (crosses ? c.cross + c.cross_kt * ktw : 0.0) + (two_pass ? sums_us(c, kc, M, N) : 0.0);
 }
 
-// and of the 256 x 256 tiles of gemm_kernel / gemm_xw_kernel: 2.0 us per k-tile and round with all CUs at work
-double tile256_us(int M, int N, int nkt, size_t max_chunk_bytes)
+// rounds of workgroups x k-tiles; the last round may leave CUs idle
+inline double rounds_us(int64_t units, double tile_us, double fill_share, double round_us)
 {
     const int cus = device_info().num_cus;
-    const int tiles = ((M + 255) / 256) * ((N + 255) / 256);
-    int kc = pick_k_chunks(tiles, nkt, cus, (int64_t)M * N, 1.7);
-    if (!chunk_sums_fit(kc, M, N, max_chunk_bytes)) kc = 1;       // (as the launchers do)
-    const int64_t units = (int64_t)tiles * kc, rounds = (units + cus - 1) / cus;
-    const double fill = (double)units / (double)(rounds * cus);
-    return (double)rounds * (nkt / (double)kc * 2.0 * (0.5 + 0.5 * fill) + 3.0) + chunk_sum_us(kc, M, N);
+    const int64_t rounds = (units + cus - 1) / cus;
+    return (double)rounds * (tile_us * (fill_share + (1.0 - fill_share) * (double)units / (double)(rounds * cus)) + round_us);
 }
 
-// Q4_K, Q8_0 and Q6_K: the cheapest of the three by these models, which were fitted to calls of 40 .. 2048 rows on
-// 1024 x 4096, 4096 x 4096, 4096 x 14336, 5120 x 2560, 14336 x 4096 and 21504 x 5376 weights.  The register-resident kernel
-// keeps few rows and narrow weights (Q4_K 64 x 4096 x 4096 18.0 vs 21.8 us, Q6_K 200 x 1024 x 4096 25.2 vs 29.7), the
-// 256-row tiles keep many rows of wide weights (Q4_K 2048 x 21504 x 5376 494 vs 567 us, Q8_0 700 x 14336 x 4096 121 vs 138):
-// they take half as many weight lines per result.
-template <typename G, typename W>
-int cheapest_tiles(int M, int N, int K, bool accumulate, size_t max_chunk_bytes, WidePlan* plan)
+inline double wide_us(const RuleCosts& c, int M, int N, int nkt, bool accumulate, size_t max_chunk_bytes, WidePlan* plan)
+{
+    double best = kNotServed;
+    const int64_t n_tiles = (N + 255) / 256;
+    for (int sc = 1; sc <= 8; ++sc) {
+        const int chunk = ((nkt + sc - 1) / sc + 3) / 4 * 4;
+        if (sc > 1 && (chunk < 8 || (nkt + chunk - 1) / chunk != sc || !chunk_sums_fit(sc, M, N, max_chunk_bytes))) continue;
+        const double finish = c.wide + finish_us(c, sc, M, N, accumulate);
+        for (int tm = 1; tm <= 4; ++tm) {
+            if (tm > 1 && 32 * (tm - 1) >= M) break;
+            const double us = finish + rounds_us((M + 32 * tm - 1) / (32 * tm) * n_tiles * sc, chunk * (c.wide_kt + c.wide_kt_rows * tm), c.wide_fill, c.wide_round);
+            if (us < best) {
+                best = us;
+                *plan = WidePlan{tm, sc, chunk};
+            }
+        }
+    }
+    return best;
+}
+
+inline double tile_us(const RuleCosts& c, int bm, int M, int N, int nkt, bool accumulate, size_t max_chunk_bytes)
+{
+    const int64_t tiles = (int64_t)((M + bm - 1) / bm) * ((N + 255) / 256);
+    int kc = pick_k_chunks((int)std::min<int64_t>(tiles, 1 << 20), nkt, device_info().num_cus, (int64_t)M * N, 1.7 * bm / 256.0);
+    if (kc > 1 && !chunk_sums_fit(kc, M, N, max_chunk_bytes)) kc = 1;       // (as the launchers do)
+    const int chunk = kc > 1 ? ((nkt + kc - 1) / kc + 3) / 4 * 4 : nkt;
+    if (kc > 1) kc = (nkt + chunk - 1) / chunk;
+    const double finish = finish_us(c, kc, M, N, accumulate);
+    return bm == 256 ? c.t256 + finish + rounds_us(tiles * kc, chunk * c.t256_kt, c.t256_fill, c.t256_round)
+                     : c.t128 + finish + rounds_us(tiles * kc, chunk * c.t128_kt, c.t128_fill, c.t128_round);
+}
+
+// Few rows stay on the register-resident kernel: all of three and less, and of Q8_0 and Q6_K up to 16, where it was the fastest
+// of all measured calls but one (Q8_0 11 x 8441 x 5120, 8 % behind) while the expected costs are too close to tell.
+template <typename G>
+int cheapest_tiles(const RuleCosts& c, int M, int N, int K, bool accumulate, size_t max_chunk_bytes, WidePlan* plan)
 {
     const int nkt = (K + kBK - 1) / kBK;
-    const double slim = slim_us<G>(M, N, nkt, accumulate, max_chunk_bytes);
-    if (M <= 3 && slim < kNoScratch) return 32;
-    *plan = pick_wide(M, N, nkt, max_chunk_bytes, W::kUsBase, W::kUsRow);
-    const double wide = plan->us;
-    const double tile = std::is_same<G, GQ6K>::value ? wide : tile256_us(M, N, nkt, max_chunk_bytes);       // (no 256-row tiles of Q6_K)
-    if (slim <= wide && slim <= tile) return 32;
-    return wide <= tile ? kWideTiles : 256;
+    const double slim = slim_us<G>(c, M, N, nkt, accumulate, max_chunk_bytes);
+    if (M <= (std::is_same<G, GQ4K>::value ? 3 : 16) && slim < kNotServed) return 32;
+    const double wide = wide_us(c, M, N, nkt, accumulate, max_chunk_bytes, plan);
+    const double t128 = tile_us(c, 128, M, N, nkt, accumulate, max_chunk_bytes);
+    const double t256 = std::is_same<G, GQ6K>::value ? kNotServed : tile_us(c, 256, M, N, nkt, accumulate, max_chunk_bytes);
+    const double best = std::min(std::min(slim, wide), std::min(t128, t256));
+    return best == slim ? 32 : best == wide ? kWideTiles : best == t128 ? 128 : 256;
 }
 
 // Rows of activations per tile of a plain launch (kWideTiles: gemm_wide_kernel, as *wide says)
 int gemm_tile_m(int type, int M, int N, int K, bool accumulate, size_t max_chunk_bytes, WidePlan* wide)
 {
-    if (type == kTypeQ4_K) return cheapest_tiles<GQ4K, WQ4K>(M, N, K, accumulate, max_chunk_bytes, wide);
-    if (type == kTypeQ8_0) return cheapest_tiles<GQ80, WQ80>(M, N, K, accumulate, max_chunk_bytes, wide);
-    if (type == kTypeQ6_K) return cheapest_tiles<GQ6K, WQ6K>(M, N, K, accumulate, max_chunk_bytes, wide);
+    if (type == kTypeQ4_K) return cheapest_tiles<GQ4K>(kCostsQ4K, M, N, K, accumulate, max_chunk_bytes, wide);
+    if (type == kTypeQ8_0) return cheapest_tiles<GQ80>(kCostsQ80, M, N, K, accumulate, max_chunk_bytes, wide);
+    if (type == kTypeQ6_K) return cheapest_tiles<GQ6K>(kCostsQ6K, M, N, K, accumulate, max_chunk_bytes, wide);
     if (M <= 128) return 32;
     if (type == kTypeMXFP4 && M <= 512 && ((M + 127) / 128) * ((N + 127) / 128) <= 128) return 32;
     // 128- or 256-row tiles by rounds of workgroups x time per k-tile of a round (measured per k-tile: a 256 x 256 tile
@@ -3962,7 +3997,7 @@ bool gemm_dispatch_plan(int type, GemmArgs a, const GemmPlan& plan, hipStream_t 
         return false;
     }
     a.accumulate = accumulate ? 1 : 0;
-    const WidePlan wide{plan.wide_tm, plan.k_chunks, plan.chunk_kt, 0.0};
+    const WidePlan wide{plan.wide_tm, plan.k_chunks, plan.chunk_kt};
     return gemm_dispatch(type, a, plan.bm, plan.bm == kWideTiles ? 1 : (a.M + plan.bm - 1) / plan.bm, wide, stream, cs);
 }
 
@@ -3975,7 +4010,7 @@ bool gemm_dispatch_tiles(int type, GemmArgs a, const int* c_rows, const GemmTile
     a.tile_rows = tiles.rows;
     a.expert_stride = tiles.expert_stride;
     a.expert_off = tiles.expert_off;
-    return gemm_dispatch(type, a, tiles.bm, tiles.count, WidePlan{0, 1, 0, 0.0}, stream, cs);
+    return gemm_dispatch(type, a, tiles.bm, tiles.count, WidePlan{0, 1, 0}, stream, cs);
 }
 }  // namespace
 
@@ -3986,7 +4021,7 @@ GemmPlan plan_gemm(int type, int M, int N, int K, bool accumulate, size_t max_ch
         p.bm = -1;
         return p;
     }
-    WidePlan wide{0, 1, 0, 0.0};
+    WidePlan wide{0, 1, 0};
     p.bm = gemm_tile_m(type, M, N, K, accumulate, max_chunk_bytes, &wide);
     p.wide_tm = wide.tm;
     p.k_chunks = wide.k_chunks;

@@ -78,3 +78,57 @@ def test_a_bounded_workspace_keeps_as_many_chunks_as_fit(t, rows, n, k, accumula
         assert got[2] >= 2 or fit < 2 or got[0] != WIDE, (fit, got)        # some of the chunks, where the tiles take any number
         last = got[2]
     assert plan(t, rows, n, k, accumulate, 1)[2] == 1                       # (refused by the entry points: not even the conversions fit)
+
+
+# measured us of a call, conversion included, weights from HBM: register-resident kernel, the best tiling of the wide kernel, 128- and
+# 256-row tiles (None: not a candidate, or not measured)
+MEASURED = [
+    (Q4_K, 8, 4096, 4096, 12.44, 16.28, None, None),
+    (Q4_K, 24, 14336, 4096, 21.49, 22.75, 29.53, None),
+    (Q4_K, 64, 4096, 4096, 17.41, 21.03, 28.53, 34.04),
+    (Q4_K, 96, 4096, 4096, 30.29, 22.9, 29.82, 35.6),
+    (Q4_K, 333, 4096, 14336, 115.11, 68.06, 75.84, 90.81),
+    (Q4_K, 512, 14336, 4096, 115.92, 75.75, 82.23, 82.91),
+    (Q4_K, 1024, 9728, 2560, 150.97, 85.79, 104.73, 68.69),
+    (Q4_K, 2048, 21504, 5376, 1369.3, 563.49, 629.79, 474.88),
+    (Q8_0, 4, 4096, 4096, 12.79, 18.09, None, None),
+    (Q8_0, 8, 9728, 2560, 18.02, 18.44, None, None),
+    (Q8_0, 8, 14336, 4096, 23.23, 23.96, None, None),
+    (Q8_0, 64, 4096, 4096, 18.59, 22.1, 29.58, 36.76),
+    (Q8_0, 128, 28672, 4096, 90.74, 60.0, 66.98, 76.55),
+    (Q8_0, 400, 4096, 4096, 55.68, 39.17, 37.37, 44.49),
+    (Q8_0, 512, 14336, 4096, 164.74, 80.42, 87.37, 88.92),
+    (Q8_0, 2048, 21504, 5376, 1408.48, 599.65, 683.56, 522.59),
+    (Q6_K, 8, 4096, 4096, 12.97, 23.46, None, None),
+    (Q6_K, 32, 9728, 2560, 21.68, 25.89, 31.07, None),
+    (Q6_K, 64, 4096, 4096, 19.18, 28.07, 35.66, None),
+    (Q6_K, 128, 14336, 4096, 54.08, 47.4, 44.14, None),
+    (Q6_K, 333, 4096, 14336, 140.48, 94.45, 100.25, None),
+    (Q6_K, 512, 14336, 4096, 181.74, 108.19, 106.67, None),
+    (Q6_K, 1024, 14336, 4096, 374.15, 210.59, 205.78, None),
+    (Q6_K, 2048, 2560, 9728, 351.84, 200.81, 240.7, None),
+    (Q6_K, 512, 4096, 4096, 62.72, 47.51, 45.06, None),
+]
+
+
+@pytest.mark.parametrize("t,rows,n,k,registers,wide,tiles128,tiles256", MEASURED)
+def test_the_pick_is_the_measured_best_or_close(t, rows, n, k, registers, wide, tiles128, tiles256):
+    # few rows that the wide kernel pads to 32, Q6_K on 128-row tiles again, long prompts on 256-row tiles: nothing more than 5 %
+    # behind the fastest
+    kernel, tile, _, _ = plan(t, rows, n, k)
+    took = {REGISTERS: registers, WIDE: wide}[kernel] if kernel != TILES else {128: tiles128, 256: tiles256}[tile]
+    assert took <= 1.05 * min(us for us in (registers, wide, tiles128, tiles256) if us is not None)
+
+
+def test_adding_to_a_residual_counts_the_second_pass_of_the_register_kernel():
+    # it writes its sums to the workspace and adds them in a second launch; the wide kernel adds in place
+    picks = [(plan(Q4_K, m, n, 2304)[0], plan(Q4_K, m, n, 2304, 1)[0]) for m in range(17, 200) for n in (1024, 2048, 4096, 8192, 14336)]
+    assert any(plain == REGISTERS and added == WIDE for plain, added in picks)
+    assert not any(plain == WIDE and added == REGISTERS for plain, added in picks)
+
+
+@pytest.mark.parametrize("t", [Q8_0, Q6_K])
+@pytest.mark.parametrize("rows", [4, 8, 16])
+def test_few_rows_stay_on_the_register_kernel(t, rows):
+    for n, k in ((1024, 4096), (4096, 4096), (9728, 2560), (21504, 5376), (4096, 14336)):
+        assert plan(t, rows, n, k)[0] == REGISTERS and plan(t, rows, n, k, 1)[0] == REGISTERS
