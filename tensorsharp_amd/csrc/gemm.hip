@@ -3752,11 +3752,10 @@ namespace {
 // The cheapest of the register-resident kernel, gemm_wide_kernel (four tile heights, up to eight K chunks) and the 128- and
 // 256-row tiles, by what they are expected to cost.  The constants (microseconds) were fitted to measured calls, conversion
 // included, with weights that come from HBM: 14 shapes from 1024 x 4096 to 28672 x 4096 with 24 row counts from 4 to 2048, and
-// about 380 random ones per format over 4 .. 2048 rows, 1000 .. 28672 columns and K of 1024 .. 21504, a third of them added to
-// a residual.  On the calls it was fitted to the pick takes 0.4 % (Q4_K), 0.5 % (Q8_0) and 0.2 % (Q6_K) longer than the fastest
-// candidate on average and more than 4 % longer on 25 of 714, 23 of 576 and 1 of 559; on 200 random calls per format that an
-// earlier fit of the same form had not seen 0.9, 1.1 and 0.2 %.  Where the lines lie, us (register-resident / gemm_wide_kernel
-// / 128 rows / 256 rows):
+// about 870 random ones per format over 4 .. 2048 rows, 64 .. 28672 columns and K of 256 .. 21504, a third of them added to a
+// residual.  On 300 further random calls per format the pick took 0.4 % (Q4_K), 0.3 % (Q8_0) and 0.2 % (Q6_K) longer than the
+// fastest candidate on average, more than 4 % longer on 11, 8 and 3 of them, 11 % at most.
+// Where the lines lie, us (register-resident / gemm_wide_kernel / 128 rows / 256 rows):
 //   Q4_K  8 x 4096 x 4096 12.4 / 16.3 / - / -,  64 x 4096 x 4096 17.4 / 21.0 / 28.5 / 34.0,  200 x 4096 x 4096 38.5 / 28.3 / 32.2 /
 //         39.8,  1024 x 9728 x 2560 151 / 85.8 / 104.7 / 68.7
 //   Q8_0  8 x 14336 x 4096 23.2 / 24.0 / - / -,  128 x 28672 x 4096 90.7 / 60.0 / 67.0 / 76.6,  400 x 4096 x 4096 - / 39.2 / 37.4 / -
@@ -3771,23 +3770,21 @@ struct RuleCosts {
     double t256, t256_kt, t256_fill, t256_round;      // 256- and 128-row tiles, likewise
     double t128, t128_kt, t128_fill, t128_round;
     double sums, sums_rate;                            // the launch that adds K chunks: a call, TB/s of its sums written and read
-    double add;                                        // results added in place, per 1e6 of them
+    double wide_add, tile_add;                         // results added in place: a round, per 32 rows of a tile (one load after the other)
 };
-constexpr RuleCosts kCostsQ4K{6.257, 6.384, 0.284, 0.533, 1.675, 0.777, 4.941, 0.370, 0.165, 0.951, 4.558,
-                              4.514, 1.637, 0.628, 5.768, 0.697, 1.244, 0.892, 5.599, 1.546, 4.218, 3.963};
-constexpr RuleCosts kCostsQ80{5.688, 8.132, 0.854, 0.474, 0.044, 1.016, 4.734, 0.444, 0.168, 0.988, 6.634,
-                              0.000, 1.791, 0.976, 7.753, 3.439, 1.404, 1.040, 2.000, 0.768, 4.952, 3.239};
-constexpr RuleCosts kCostsQ6K{6.557, 4.816, 0.457, 0.662, 1.910, 0.430, 4.096, 1.010, 0.144, 0.948, 8.949,      // (no 256-row tiles)
-                              0.000, 0.000, 0.000, 0.000, 7.308, 1.649, 0.909, 0.727, 3.024, 9.405, 3.810};
+constexpr RuleCosts kCostsQ4K{6.538, 6.588, 0.471, 0.444, 4.440, 0.000, 5.031, 0.423, 0.153, 0.966, 3.404,
+                              11.108, 1.670, 0.618, 0.032, 4.101, 1.189, 0.725, 6.098,
+                              2.367, 4.806, 3.964, 4.582};
+constexpr RuleCosts kCostsQ80{6.249, 5.523, 1.221, 0.339, 0.590, 0.891, 5.085, 0.495, 0.148, 1.006, 5.151,
+                              3.152, 1.741, 0.926, 4.675, 4.610, 1.247, 1.492, 1.841,
+                              1.697, 5.090, 6.433, 1.591};
+constexpr RuleCosts kCostsQ6K{5.858, 6.414, 0.393, 0.658, 2.025, 0.406, 4.411, 1.047, 0.156, 0.890, 6.472,      // (no 256-row tiles)
+                              0.000, 0.000, 0.000, 0.000, 6.177, 1.561, 0.938, 3.905,
+                              3.284, 7.419, 3.358, 1.187};
 constexpr double kNotServed = 1e30;      // a kernel that a format has not, or whose chunk sums do not fit
 
 inline bool chunk_sums_fit(int k_chunks, int M, int N, size_t max_bytes) { return (size_t)k_chunks * M * N * sizeof(float) <= max_bytes; }
 inline double sums_us(const RuleCosts& c, int k_chunks, int M, int N) { return c.sums + (double)k_chunks * M * N * 8e-6 / c.sums_rate; }
-// what follows the tiles of gemm_wide_kernel and of the 128- and 256-row kernels
-inline double finish_us(const RuleCosts& c, int k_chunks, int M, int N, bool accumulate)
-{
-    return k_chunks > 1 ? sums_us(c, k_chunks, M, N) : accumulate ? c.add * M * N * 1e-6 : 0.0;
-}
 
 template <typename G>
 double slim_us(const RuleCosts& c, int M, int N, int nkt, bool accumulate, size_t max_chunk_bytes)
@@ -3819,10 +3816,11 @@ inline double wide_us(const RuleCosts& c, int M, int N, int nkt, bool accumulate
     for (int sc = 1; sc <= 8; ++sc) {
         const int chunk = ((nkt + sc - 1) / sc + 3) / 4 * 4;
         if (sc > 1 && (chunk < 8 || (nkt + chunk - 1) / chunk != sc || !chunk_sums_fit(sc, M, N, max_chunk_bytes))) continue;
-        const double finish = c.wide + finish_us(c, sc, M, N, accumulate);
+        const double fixed = c.wide + (sc > 1 ? sums_us(c, sc, M, N) : 0.0), add = sc == 1 && accumulate ? c.wide_add : 0.0;
         for (int tm = 1; tm <= 4; ++tm) {
             if (tm > 1 && 32 * (tm - 1) >= M) break;
-            const double us = finish + rounds_us((M + 32 * tm - 1) / (32 * tm) * n_tiles * sc, chunk * (c.wide_kt + c.wide_kt_rows * tm), c.wide_fill, c.wide_round);
+            const double us = fixed + rounds_us((M + 32 * tm - 1) / (32 * tm) * n_tiles * sc, chunk * (c.wide_kt + c.wide_kt_rows * tm), c.wide_fill,
+                                                c.wide_round + add * tm);
             if (us < best) {
                 best = us;
                 *plan = WidePlan{tm, sc, chunk};
@@ -3839,9 +3837,9 @@ inline double tile_us(const RuleCosts& c, int bm, int M, int N, int nkt, bool ac
     if (kc > 1 && !chunk_sums_fit(kc, M, N, max_chunk_bytes)) kc = 1;       // (as the launchers do)
     const int chunk = kc > 1 ? ((nkt + kc - 1) / kc + 3) / 4 * 4 : nkt;
     if (kc > 1) kc = (nkt + chunk - 1) / chunk;
-    const double finish = finish_us(c, kc, M, N, accumulate);
-    return bm == 256 ? c.t256 + finish + rounds_us(tiles * kc, chunk * c.t256_kt, c.t256_fill, c.t256_round)
-                     : c.t128 + finish + rounds_us(tiles * kc, chunk * c.t128_kt, c.t128_fill, c.t128_round);
+    const double sums = kc > 1 ? sums_us(c, kc, M, N) : 0.0, add = kc == 1 && accumulate ? c.tile_add * bm / 32 : 0.0;
+    return sums + (bm == 256 ? c.t256 + rounds_us(tiles * kc, chunk * c.t256_kt, c.t256_fill, c.t256_round + add)
+                             : c.t128 + rounds_us(tiles * kc, chunk * c.t128_kt, c.t128_fill, c.t128_round + add));
 }
 
 // Few rows stay on the register-resident kernel: all of three and less, and of Q8_0 and Q6_K up to 16, where it was the fastest
