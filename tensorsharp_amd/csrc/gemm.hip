@@ -3773,7 +3773,7 @@ struct RuleCosts {
     double wide_add, tile_add;                         // results added in place: a round, per 32 rows of a tile (one load after the other)
 };
 constexpr RuleCosts kCostsQ4K{6.538, 6.588, 0.471, 0.444, 4.440, 0.000, 5.031, 0.423, 0.153, 0.966, 3.404,
-                              11.108, 1.670, 0.618, 0.032, 4.101, 1.189, 0.725, 6.098,
+                              11.108, 1.670, 0.618, 0.032, 0.000, 0.000, 0.000, 0.000,      // (no 128-row tiles)
                               2.367, 4.806, 3.964, 4.582};
 constexpr RuleCosts kCostsQ80{6.249, 5.523, 1.221, 0.339, 0.590, 0.891, 5.085, 0.495, 0.148, 1.006, 5.151,
                               3.152, 1.741, 0.926, 4.675, 4.610, 1.247, 1.492, 1.841,
@@ -3851,7 +3851,8 @@ int cheapest_tiles(const RuleCosts& c, int M, int N, int K, bool accumulate, siz
     const double slim = slim_us<G>(c, M, N, nkt, accumulate, max_chunk_bytes);
     if (M <= (std::is_same<G, GQ4K>::value ? 3 : 16) && slim < kNotServed) return 32;
     const double wide = wide_us(c, M, N, nkt, accumulate, max_chunk_bytes, plan);
-    const double t128 = tile_us(c, 128, M, N, nkt, accumulate, max_chunk_bytes);
+    // (128-row tiles of Q4_K: never the cheapest)
+    const double t128 = std::is_same<G, GQ4K>::value ? kNotServed : tile_us(c, 128, M, N, nkt, accumulate, max_chunk_bytes);
     const double t256 = std::is_same<G, GQ6K>::value ? kNotServed : tile_us(c, 256, M, N, nkt, accumulate, max_chunk_bytes);
     const double best = std::min(std::min(slim, wide), std::min(t128, t256));
     return best == slim ? 32 : best == wide ? kWideTiles : best == t128 ? 128 : 256;

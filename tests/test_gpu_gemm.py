@@ -108,7 +108,8 @@ def test_config3_q4_k_prefill(hip, oracle):
 
 @pytest.mark.parametrize("name,M", [("q4_k", 40), ("mxfp4", 64), ("q8_0", 9)])
 def test_more_tiles_than_workgroups(hip, oracle, name, M):
-    # few rows x very many columns: the persistent workgroups each walk over several tiles
+    # few rows x very many columns: the register-resident kernel's persistent workgroups each walk over several tiles (Q4_K with
+    # 40 rows runs 64-row tiles instead; test_gpu_prefill_kernels.py asserts which kernel serves a shape)
     rng = np.random.default_rng(57 + M)
     N, K = 256 * 300 + 77, 256
     wq = oracle.quantize(T[name], (rng.standard_normal(N * K) * 0.02).astype(np.float32))
@@ -119,7 +120,8 @@ def test_more_tiles_than_workgroups(hip, oracle, name, M):
 
 @pytest.mark.parametrize("name", ["q8_0", "q4_k", "mxfp4"])
 def test_tall_activations(hip, oracle, name):
-    # M > 1024 takes the 256-row tiles; the last tile is ragged in both directions
+    # many rows over few columns, the last tile ragged in both directions: 128-row tiles (MXFP4), 32-row tiles (Q4_K) or the
+    # register-resident kernel (Q8_0); ragged 256-row tiles are in test_gpu_prefill_kernels.py
     rng = np.random.default_rng(59)
     M, N, K = 1100, 300, 768
     wq = oracle.quantize(T[name], (rng.standard_normal(N * K) * 0.02).astype(np.float32))
@@ -219,7 +221,8 @@ def test_q6_k_rows_two_bytes_off(hip, oracle, M):
                                        # chunks of 12 and 16 k-tiles
                                        ("q4_k", 1024, 520, 2048), ("q8_0", 520, 600, 3072), ("q4_k", 700, 520, 3072)])
 def test_128_row_tiles(hip, oracle, name, M, N, K):
-    # row counts past the register-resident kernel's range: 128-row tiles, ragged last tile
+    # up to 1100 rows over few columns, ragged last tile: 128-row tiles for MXFP4; Q4_K and Q8_0 run what is planned for so few
+    # columns (32- and 64-row tiles, the register-resident kernel), their 128-row tiles are in test_gpu_prefill_kernels.py
     rng = np.random.default_rng(M + N + K)
     wq = oracle.quantize(T[name], (rng.standard_normal(N * K) * 0.02).astype(np.float32))
     x = rng.standard_normal((M, K)).astype(np.float32)
@@ -365,6 +368,8 @@ def test_mxfp4_block_scaled_small_batch_48_row_units(hip, oracle, M):
 
 
 def test_q6_k_128_row_tiles(hip, oracle):
+    # (named for the kernel that served it; 300 rows over 520 columns run the register-resident kernel, ragged 128-row tiles are
+    # in test_gpu_prefill_kernels.py)
     from oracle.oracle import Q6_K
     rng = np.random.default_rng(77)
     M, N, K = 300, 520, 1024
@@ -487,7 +492,7 @@ def test_narrow_results_are_formed_from_exact_weights(hip, oracle, name, M, N, K
 
 
 @pytest.mark.parametrize("name,M,N,K", [
-    # 32 .. 128 rows per tile with a ragged last one, a ragged last column tile, whole K and K in chunks
+    # a ragged last row tile, a ragged last column tile, whole K and K in chunks
     ("q4_k", 33, 14800, 1024), ("q4_k", 97, 15000, 512), ("q4_k", 129, 8200, 256), ("q4_k", 160, 2100, 1280),
     ("q4_k", 250, 4099, 2304), ("q4_k", 333, 1500, 4096),
     # Q8_0 rows that begin at any even byte of a 16-byte piece; the last k-tile a single block; an odd number of k-tiles
@@ -495,7 +500,9 @@ def test_narrow_results_are_formed_from_exact_weights(hip, oracle, name, M, N, K
     ("q6_k", 130, 14400, 512), ("q6_k", 250, 9000, 768), ("q6_k", 333, 2100, 2304), ("q6_k", 40, 15001, 1280),
 ])
 def test_wide_tiles(hip, oracle, name, M, N, K):
-    # mid-sized calls: product, product added to a residual, and a scale outside the fp16 operands in the last k-tile
+    # mid-sized calls (32- to 96-row tiles; Q4_K 33, Q8_0 and Q6_K 40 rows stay on the register-resident kernel; every tile height,
+    # asserted, is in test_gpu_prefill_kernels.py): product, product added to a residual, and a scale outside the fp16
+    # operands in the last k-tile
     import torch
     from tensorsharp_amd import QuantizedWeight
     from oracle.oracle import Q6_K

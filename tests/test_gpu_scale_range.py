@@ -69,7 +69,7 @@ def check_columns(oracle, t, raw, N, K, x, y, tag):
     assert worst <= 1.0, (tag, "per-column error / bound", worst)
 
 
-# rows that reach: the GEMV, the 32-row register-resident kernel, 128-row tiles, 256-row tiles
+# rows that reach the GEMV and, by type and shape, the register-resident kernel, the 32- to 96-row tiles and the 128-row tiles
 ROWS = [1, 3, 8, 100, 160, 300]
 
 

@@ -30,8 +30,7 @@ def _both(hip, t, wq, N, K, x):
 @pytest.mark.parametrize("t", [Q4_K, Q8_0, MXFP4])
 def test_two_calls_in_a_row_second_smaller(hip, oracle, t):
     rng = np.random.default_rng(7100 + t)
-    # first: 300 rows on the 128-row tiles with a long K (K chunks in use for the 4-bit formats); second: 40 rows
-    # (register-resident kernel) of a shorter K, whose scratch overlaps the first call's
+    # first: 300 rows with a long K, in K chunks; second: 40 rows of a shorter K, whose scratch overlaps the first call's
     for (M, N, K) in [(300, 512, 8192), (40, 200, 1024)]:
         wq = oracle.quantize(t, (rng.standard_normal(N * K) * 0.02).astype(np.float32))
         x = rng.standard_normal((M, K)).astype(np.float32)
