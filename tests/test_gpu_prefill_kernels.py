@@ -34,7 +34,7 @@ def weight(name, w, N, K):
 # (format, kernel, rows per tile, K in chunks, rows, columns, K): M and N ragged in the last tile; K of Q8_0 an odd number of blocks
 # (the last k-tile holds one) and, chunked, an odd number of k-tiles; every K has several granules
 PLAIN = [
-    ("q4_k", WIDE, 32, False, 521, 485, 768), ("q4_k", WIDE, 32, True, 28, 79, 2304), ("q4_k", WIDE, 64, False, 1348, 1287, 768),
+    ("q4_k", WIDE, 32, False, 521, 485, 768), ("q4_k", WIDE, 32, True, 45, 487, 2304), ("q4_k", WIDE, 64, False, 1348, 1287, 768),
     ("q4_k", WIDE, 64, True, 899, 551, 1280), ("q4_k", WIDE, 96, False, 1795, 2051, 768), ("q4_k", WIDE, 96, True, 907, 517, 2816),
     ("q4_k", WIDE, 128, False, 1834, 3115, 768), ("q4_k", WIDE, 128, True, 971, 513, 4096),
     ("q4_k", TILES, 256, False, 1537, 4965, 768), ("q4_k", TILES, 256, True, 1800, 2079, 5120),
@@ -51,7 +51,7 @@ PLAIN = [
     ("q4_k", REGISTERS, 32, False, 60, 9001, 768), ("q8_0", REGISTERS, 32, False, 70, 4501, 1312), ("q6_k", REGISTERS, 32, False, 70, 4501, 1280),
 ]
 ADDED = [
-    ("q4_k", WIDE, 32, False, 1038, 783, 768), ("q4_k", WIDE, 32, True, 17, 79, 2304), ("q4_k", WIDE, 64, False, 1414, 1533, 768),
+    ("q4_k", WIDE, 32, False, 1038, 783, 768), ("q4_k", WIDE, 32, True, 77, 487, 4352), ("q4_k", WIDE, 64, False, 1414, 1533, 768),
     ("q4_k", WIDE, 64, True, 897, 517, 1280), ("q4_k", WIDE, 96, False, 1795, 2051, 768), ("q4_k", WIDE, 96, True, 1794, 525, 1280),
     ("q4_k", WIDE, 128, False, 1834, 3115, 768), ("q4_k", WIDE, 128, True, 971, 513, 4096),
     ("q4_k", TILES, 256, False, 1928, 6157, 768), ("q4_k", TILES, 256, True, 1613, 2315, 2048),
