@@ -578,7 +578,8 @@ struct GQ80 {
     static __device__ __forceinline__ void dequant(const uint32_t (&r)[kRegs], int j, int h, uint32_t delta, bool live, uint32_t (&o)[16],
                                                    uint32_t& bad)
     {
-        // the block starts in the lower or the upper half of r[0]: byte picks by selector, not by branch
+        // the block starts in the lower or the upper half of r[0]: byte picks by selector, not by two results and a select
+        // (7 % fewer vector instructions: 2048 x 21504 x 5376 539 -> 526 us)
         const bool odd = ((delta + (uint32_t)(2 * j + h) * 34u) & 2u) != 0;
         const uint32_t pick = odd ? 0x07060504u : 0x05040302u;
         const uint32_t dd = __builtin_amdgcn_perm(r[0], r[0], odd ? 0x03020302u : 0x01000100u) & (live ? 0xffffffffu : 0u);
@@ -1652,14 +1653,16 @@ constexpr int kWideValu = (40 + 2 * TM - 1) / (2 * TM);
 // gemm_wide_kernel: tiles of 32 TM rows (TM 1 .. 4) x 256 columns, eight wavefronts = 4 (64 columns each) x 2 halves of the
 // K range of a turn.  A wavefront unpacks the operands of its own 64 columns in registers, and one activation operand read
 // from LDS feeds two matrix instructions; the two halves meet in LDS once, at the end.
-// What bounds it: the lines that a CU takes from its L2 (measured: about 47 GB/s per CU with all CUs reading, 128 bytes
-// for every line touched).  gemm_xw_kernel copies 48 of a Q4_K block's 144 bytes per k-tile and so takes two lines per row
-// and k-tile, 97 KB per 256 x 256 x 64 step; here a row's whole granule is copied at once, 33 KB per 128 x 256 x 64 step of
-// Q4_K.  Then the vector instructions: four to five per matrix instruction are free, each one more costs about five cycles.
-// Measured, whole call, us (the tile and register-resident kernels -> this one):
-//   Q4_K 512 x 14336 x 4096 91 -> 83, 200 x 4096 x 14336 82 -> 50, 333 x 4096 x 14336 116 -> 68, 200 x 4096 x 4096 38 -> 28
-//   Q8_0 512 x 14336 x 4096 104 -> 84, 200 x 4096 x 14336 82 -> 53, 40 x 21504 x 5376 59 -> 45
-//   Q6_K 200 x 4096 x 14336 96 -> 63, 200 x 21504 x 5376 187 -> 126, 128 x 21504 x 5376 121 -> 70
+// Why: the 128- and 256-row kernels wait for the L2, which answers whole 128-byte lines.  gemm_xw_kernel copies 48 of a Q4_K
+// block's 144 bytes per k-tile and takes two lines per row for them, by the counters 73 KB per 128 x 256 x 64 step (92 KB per
+// 256 x 256 x 64) at 50 (43) GB/s per CU; here a row's whole granule is copied at once: 37 KB per 128 x 256 x 64 step.  What
+// bounds it now: of Q4_K 512 x 14336 x 4096 (77.6 us) the matrix pipe is busy 34 % of the cycles, 8 vector instructions
+// stand beside each matrix instruction, wavefronts wait 35 % of their time; Q6_K (333 x 4096 x 14336) has 16 vector
+// instructions per matrix instruction and bank conflicts in 62 % of its LDS cycles (dword reads of 210-byte blocks).
+// Measured, whole call, us (the best of the other kernels -> this one):
+//   Q4_K 512 x 14336 x 4096 82.2 -> 75.8, 333 x 4096 x 14336 75.8 -> 68.1, 200 x 4096 x 14336 69.7 -> 49.7, 200 x 4096 x 4096 32.2 -> 28.3
+//   Q8_0 512 x 14336 x 4096 87.4 -> 80.4, 200 x 4096 x 14336 77.7 -> 52.6, 48 x 21504 x 5376 56.1 -> 45.5
+//   Q6_K 333 x 4096 x 14336 100.3 -> 94.5, 200 x 4096 x 14336 95.7 -> 64.1, 200 x 21504 x 5376 141.2 -> 125.5
 // ------------------------------------------------------------------------------------------
 // Weight formats as this kernel reads them.  A granule is the raw bytes of kSup consecutive k-tiles of one row, kept in LDS
 // as kRawRow bytes (an odd multiple of four dwords: the dword reads of 32 rows spread over the most banks that 16-byte
