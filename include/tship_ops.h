@@ -145,9 +145,10 @@ TSHIP_EXPORT int TSHip_AddmmQuantF32Device(TSHipTensorView2D result, TSHipTensor
  * results, but the scratch of the prefill path (fp16 activations + row scales, sums of K chunks) lives in a static
  * device array of TSHIP_NO_ALLOC_SCRATCH_BYTES that every GPU the library runs on holds until the process ends; the
  * call makes no hipMalloc / hipFree.  A call whose converted activations (about 2 bytes per activation + 4 per row)
- * exceed the array fails with an error; when only the sums of K chunks do not fit, the launch runs with whole K per
- * tile (results then agree with TSHip_AddmmQuantF32Device to fp32 summation order) or, for the shapes that cannot
- * do without chunks (at most 128 rows with K > 4096 ... 32768 depending on the format), fails with an error.
+ * exceed the array fails with an error; when only the sums of K chunks do not fit, Q4_K, Q8_0 and Q6_K run fewer chunks
+ * or another kernel, and 128- and 256-row tiles of the other formats whole K (results then agree with
+ * TSHip_AddmmQuantF32Device to fp32 summation order), while their shapes that cannot do without chunks (at most 128
+ * rows with K > 4096 ... 32768 depending on the format) fail with an error.
  * All calls on one GPU share the array: calls that overlap on one GPU (two streams, two threads) race. */
 #define TSHIP_NO_ALLOC_SCRATCH_BYTES (64u << 20)
 TSHIP_EXPORT int TSHip_AddmmQuantF32DeviceNoAlloc(TSHipTensorView2D result, TSHipTensorView2D m1, const void* m2_data,
@@ -322,8 +323,9 @@ TSHIP_EXPORT int TSHip_MulMatIdF32Device(TSHipTensorView3D result, TSHipTensorVi
 TSHIP_EXPORT int TSHip_SetGemvTimeline(void* device_buffer, int64_t capacity_bytes);
 
 /* Diagnostics, no counterpart in the reference: how a product of `rows` activation rows with such a weight runs on the device
- * (accumulate: added to the result; max_workspace: at most that many bytes of workspace, 0 for no bound).  plan[0] kernel (TSHIP_PLAN_*), plan[1] activation rows per tile, plan[2] K chunks
- * whose sums meet in the workspace (1: none), plan[3] workspace bytes.  Needs no GPU (256 CUs are assumed without one). */
+ * (accumulate: added to the result; max_workspace: at most that many bytes of workspace, 0 for no bound).  plan[0] kernel
+ * (TSHIP_PLAN_*), plan[1] activation rows per tile, plan[2] K chunks whose sums meet in the workspace (1: none), plan[3]
+ * workspace bytes.  Needs no GPU (256 CUs are assumed without one). */
 #define TSHIP_PLAN_GEMV 1        /* one GEMV per row */
 #define TSHIP_PLAN_DENSE 2       /* dense kernel (dense weights, or an exact fp32 copy of a narrow one) */
 #define TSHIP_PLAN_REGISTERS 3   /* units of 32 rows x 32 columns, activations in registers */

@@ -330,9 +330,8 @@ struct MatmulPlan {
 };
 
 // norm: RMSNorm prologue on the activations; accumulate: the product is added to the result; max_ws: the workspace that the
-// call will have - kernels and K chunks are chosen so that their sums fit what the conversions leave of it.  One plan serves the size of a
-// call's workspace, its conversions and its launches.
-
+// call will have - kernels and K chunks are chosen so that their sums fit what the conversions leave of it.  One plan serves
+// the size of a call's workspace, its conversions and its launches.
 MatmulPlan plan_matmul(int type, int M, int64_t K, int64_t N, bool norm, bool accumulate, size_t max_ws = ~(size_t)0)
 {
     auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
@@ -829,6 +828,9 @@ bool run_expert_set_device(const TSHipTensorView2D& out, const float* base, int6
         if (!run_expert_linear_tiled(L, ws, n, M, lin, rows_in, I, false, L.x2_off, dn, N, N, I, stream)) return false;
     } else {
         ExpertLinearPlan gate_plan, up_plan, down_plan;
+        auto linear = [&](const MatmulPlan& plan, const TSHipTensorView2D& y, const TSHipTensorView2D& v, const void* w, int type, int64_t wk, int64_t wn) {
+            return run_matmul_device_ws(plan, y, v, w, type, wk, wn, stream, mm_ws, L.mm_bytes, nullptr, 0.f, false);
+        };
         for (int e = 0; e < n; ++e) {
             float* a_e = act + (size_t)e * L.act_stride;
             float* d_e = dn + (size_t)e * L.dn_stride;
@@ -837,16 +839,16 @@ bool run_expert_set_device(const TSHipTensorView2D& out, const float* base, int6
                 const int64_t span = (int64_t)(((size_t)(M - 1) * 2 * I + I) * sizeof(float));
                 const TSHipTensorView2D g_view{a_e, M, I, 2 * I, 1, span};
                 const TSHipTensorView2D u_view{a_e + I, M, I, 2 * I, 1, span};
-                if (!run_matmul_device_ws(gate_plan.of(ex[e].gate_type, M, H, I), g_view, x, ex[e].gate, ex[e].gate_type, H, I, stream, mm_ws, L.mm_bytes, nullptr, 0.f, false)) return false;
-                if (!run_matmul_device_ws(up_plan.of(ex[e].up_type, M, H, I), u_view, x, ex[e].up, ex[e].up_type, H, I, stream, mm_ws, L.mm_bytes, nullptr, 0.f, false)) return false;
+                if (!linear(gate_plan.of(ex[e].gate_type, M, H, I), g_view, x, ex[e].gate, ex[e].gate_type, H, I)) return false;
+                if (!linear(up_plan.of(ex[e].up_type, M, H, I), u_view, x, ex[e].up, ex[e].up_type, H, I)) return false;
                 if (!launch_silu_mul(a_e, 2 * I, M, I, tmp, stream)) return false;
                 const TSHipTensorView2D t_view{tmp, M, I, I, 1, (int64_t)((size_t)M * I * sizeof(float))};
-                if (!run_matmul_device_ws(down_plan.of(ex[e].down_type, M, I, N), d_view, t_view, ex[e].down, ex[e].down_type, I, N, stream, mm_ws, L.mm_bytes, nullptr, 0.f, false)) return false;
+                if (!linear(down_plan.of(ex[e].down_type, M, I, N), d_view, t_view, ex[e].down, ex[e].down_type, I, N)) return false;
             } else {
                 const TSHipTensorView2D u_view{a_e, M, I, I, 1, (int64_t)((size_t)M * I * sizeof(float))};
-                if (!run_matmul_device_ws(up_plan.of(ex[e].up_type, M, H, I), u_view, x, ex[e].up, ex[e].up_type, H, I, stream, mm_ws, L.mm_bytes, nullptr, 0.f, false)) return false;
+                if (!linear(up_plan.of(ex[e].up_type, M, H, I), u_view, x, ex[e].up, ex[e].up_type, H, I)) return false;
                 if (!launch_relu_sqr(a_e, (int64_t)M * I, stream)) return false;
-                if (!run_matmul_device_ws(down_plan.of(ex[e].down_type, M, I, N), d_view, u_view, ex[e].down, ex[e].down_type, I, N, stream, mm_ws, L.mm_bytes, nullptr, 0.f, false)) return false;
+                if (!linear(down_plan.of(ex[e].down_type, M, I, N), d_view, u_view, ex[e].down, ex[e].down_type, I, N)) return false;
             }
         }
     }
