@@ -34,6 +34,7 @@
 #include <algorithm>
 #include <cstdlib>
 #include <cstring>
+#include <type_traits>
 
 namespace tship {
 namespace {
@@ -84,6 +85,7 @@ struct GemvGroup {
     int wg_begin[kMaxGroup + 1];
     int count;
     int strict;     // at most one step in flight per wavefront (launches long enough to saturate HBM)
+    int split;      // > 0: a launch of one problem on the split build, row groups per workgroup
 };
 
 union H2U {
@@ -900,7 +902,7 @@ constexpr int kTimelineSlots = 8;
 // in order), then every step of the wavefront's group at once, and the steps are consumed as they arrive.  Measured on
 // one box against the streaming build: MXFP4 5760 x 2880 7.0 -> 6.0 us, 2880 x 2880 5.7 -> 5.0 us, Q4_K 4096 x 4096
 // 5.9 -> 5.5 us; Q8_0 9728 x 2560 loses (9.9 -> 10.8 us) and has no eager build.
-template <typename F, int ACT, bool TL, int EAGER>
+template <typename F, int ACT, bool TL, int EAGER, bool SPLIT = false>
 __device__ __forceinline__ void gemv_body(const GemvProblem& P, int wg, int nwg, int mode, uint32_t* lds, uint64_t* tl, int prob)
 {
     const int lane = threadIdx.x & 63;
@@ -927,7 +929,9 @@ __device__ __forceinline__ void gemv_body(const GemvProblem& P, int wg, int nwg,
     const int lane_row = routed ? 0 : pair ? osub + (sub / (HALF > 0 ? HALF : 1)) * pair : sub;   // its weight row relative to the group's first
     const uint32_t row_bytes = (uint32_t)F::row_bytes(K);
     const int wave_stride = nwg * kWaves;
-    const int gw = __builtin_amdgcn_readfirstlane(wg * kWaves + (int)(threadIdx.x >> 6));
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    // SPLIT: `mode` row groups per workgroup, whose steps the wavefronts share evenly (see gemv_split_kernel)
+    const int gw = SPLIT ? wg * mode : wg * kWaves + wave;
     // The expert id is requested here and looked at after the activations have been requested: between the two lies a
     // memory round trip (a probe with a constant id: 2.2 us of a GPT-OSS token), which the activations' own then overlaps.
     const int eid_raw = P.expert_id ? P.expert_id[0] : 0;
@@ -1076,9 +1080,23 @@ __device__ __forceinline__ void gemv_body(const GemvProblem& P, int wg, int nwg,
     // function of two operands while staging uses it (their staging takes longer, and they are the short dependent
     // launches of a decode step: fused FFN 33.9 -> 32.2 us in an A/B on one box); plain launches lose (4096 x 14336
     // 12.7 -> 14.2 us) and so does the RMSNorm mode, whose staging is as short as the plain one (28672 x 4096 17.2 vs 16.0 us).
-    const bool strict = mode == 1, deep = ACT == kActSiluMul && !strict;
+    // SPLIT: the steps of the workgroup's row groups, numbered group-major, are dealt to its wavefronts in turn
+    const int split_groups = SPLIT ? min(mode, ngroups - gw) : 0;
+    int split_group = 0, split_step = wave;
+    auto split_fetch = [&](Step<F>& st) {
+        while (split_step >= nsteps) {
+            split_step -= nsteps;
+            ++split_group;
+        }
+        fetch(split_group < split_groups ? gw + split_group : ngroups, split_step, st);
+        split_step += kWaves;
+    };
+    const bool strict = !SPLIT && mode == 1, deep = ACT == kActSiluMul && !strict;
     Step<F> eager[EAGER > 0 ? EAGER : 1];
-    if constexpr (EAGER > 0) {
+    if constexpr (SPLIT) {
+#pragma unroll
+        for (int d = 0; d < EAGER; ++d) split_fetch(eager[d]);
+    } else if constexpr (EAGER > 0) {
 #pragma unroll
         for (int s = 0; s < EAGER; ++s) fetch(s < nsteps ? gw : ngroups, s, eager[s]);
     } else {
@@ -1124,44 +1142,48 @@ __device__ __forceinline__ void gemv_body(const GemvProblem& P, int wg, int nwg,
     }
 
     float acc = 0.f, slot_b = 0.f;
+    // t: the row sum of the lane's row of the group, in every lane of the row
+    auto finish = [&](float t, int group) {
+        if (act == kActRmsNorm) t *= out_scale;
+        const int row = group * gstep + osub;
+        bool writer = l16 == 0 && group < ngroups && row < N;
+        if (routed) {
+            // slot values sit in the leader lanes 0, LPR, 2 LPR, ...; the weighted sum runs in slot order
+            const float v = t + slot_b;
+            float o = 0.f;
+#pragma unroll
+            for (int sl = 0; sl < RPG; ++sl) {
+                const float vs = __shfl(v, sl * LPR);
+                const int id = slot_id4[sl & 3];                  // uniform
+                if (id >= 0 && id < P.n_experts) o = fmaf(slot_w4[sl & 3], vs, o);
+            }
+            t = o;
+            writer = lane == 0 && group < ngroups;
+        }
+        if (pair) {
+            const float up = __shfl_xor(t, 32);       // the up value sits 32 lanes above its gate value
+            if (P.pair_kind == 0) {
+                // ggml_silu then ggml_mul (ggml-cpu/vec.h:958-960) on the fp32 sums
+                t = (t / (1.0f + expf(-t))) * up;
+            } else {
+                // GptOssModel.cs:901-934: x = min(g + b_g, limit), y = clamp(u + b_u), x * sigmoid(alpha x) * (y + 1)
+                const bool biased = P.norm_w != nullptr && !bad_expert && writer;
+                const float* pb = P.norm_w + (int64_t)(P.expert_id ? eid : 0) * 2 * pair;
+                const float x = fminf(t + (biased ? pb[row] : 0.f), P.limit);
+                const float y = fminf(fmaxf(up + (biased ? pb[pair + row] : 0.f), -P.limit), P.limit);
+                t = (x / (1.0f + expf(P.eps * (-x)))) * (y + 1.0f);
+            }
+            writer = writer && lane < 32;
+        }
+        if (writer) P.y[row] = P.add ? P.add[row] + t : t;
+    };
     auto consume = [&](const Step<F>& st) {
         // lanes past the end of a row (and steps past the last group) hold zeros, zero scales included
         const uint32_t* xu = lds + lds_lane + (uint32_t)st.step * (uint32_t)(LPR * F::kLdsDwords);
         acc += F::dot(st.w, L, st.aux, xu);
         if (routed && st.step == 0) slot_b = st.extra;
-        if (st.step == nsteps - 1) {   // uniform: the 4 rows of the group are complete
-            float t = act == kActRmsNorm ? row_sum<LPR>(acc) * out_scale : row_sum<LPR>(acc);
-            const int row = st.group * gstep + osub;
-            bool writer = l16 == 0 && st.group < ngroups && row < N;
-            if (routed) {
-                // slot values sit in the leader lanes 0, LPR, 2 LPR, ...; the weighted sum runs in slot order
-                const float v = t + slot_b;
-                float o = 0.f;
-#pragma unroll
-                for (int sl = 0; sl < RPG; ++sl) {
-                    const float vs = __shfl(v, sl * LPR);
-                    const int id = slot_id4[sl & 3];                  // uniform
-                    if (id >= 0 && id < P.n_experts) o = fmaf(slot_w4[sl & 3], vs, o);
-                }
-                t = o;
-                writer = lane == 0 && st.group < ngroups;
-            }
-            if (pair) {
-                const float up = __shfl_xor(t, 32);       // the up value sits 32 lanes above its gate value
-                if (P.pair_kind == 0) {
-                    // ggml_silu then ggml_mul (ggml-cpu/vec.h:958-960) on the fp32 sums
-                    t = (t / (1.0f + expf(-t))) * up;
-                } else {
-                    // GptOssModel.cs:901-934: x = min(g + b_g, limit), y = clamp(u + b_u), x * sigmoid(alpha x) * (y + 1)
-                    const bool biased = P.norm_w != nullptr && !bad_expert && writer;
-                    const float* pb = P.norm_w + (int64_t)(P.expert_id ? eid : 0) * 2 * pair;
-                    const float x = fminf(t + (biased ? pb[row] : 0.f), P.limit);
-                    const float y = fminf(fmaxf(up + (biased ? pb[pair + row] : 0.f), -P.limit), P.limit);
-                    t = (x / (1.0f + expf(P.eps * (-x)))) * (y + 1.0f);
-                }
-                writer = writer && lane < 32;
-            }
-            if (writer) P.y[row] = P.add ? P.add[row] + t : t;
+        if (!SPLIT && st.step == nsteps - 1) {   // uniform: the 4 rows of the group are complete
+            finish(row_sum<LPR>(acc), st.group);
             acc = 0.f;
         }
     };
@@ -1183,7 +1205,38 @@ __device__ __forceinline__ void gemv_body(const GemvProblem& P, int wg, int nwg,
             advance(fgroup, fstep);
         }
     };
-    if constexpr (EAGER > 0) {
+    if constexpr (SPLIT) {
+        // sums of the wavefront's share of a row group -> parts[group][wavefront][row]
+        float* parts = reinterpret_cast<float*>(red + kWaves);
+        int open = -1;
+        auto leave = [&]() {
+            const float t = row_sum<LPR>(acc);
+            if (open >= 0 && l16 == 0) parts[((open - gw) * kWaves + wave) * RPG + sub] = t;
+            acc = 0.f;
+        };
+        while (eager[0].group < ngroups) {
+#pragma unroll
+            for (int d = 0; d < EAGER; ++d) {
+                if (eager[d].group < ngroups) {       // uniform
+                    if (eager[d].group != open) {
+                        leave();
+                        open = eager[d].group;
+                    }
+                    consume(eager[d]);
+                }
+                split_fetch(eager[d]);
+            }
+        }
+        leave();
+        __syncthreads();
+        // wavefront g finishes row group g: the parts in order
+        for (int g = wave; g < split_groups; g += kWaves) {
+            // (the wavefronts that took one of its nsteps consecutive steps, from the one that took the first on)
+            float sum = 0.f;
+            for (int j = 0; j < min(nsteps, kWaves); ++j) sum += parts[(g * kWaves + ((g * nsteps + j) & (kWaves - 1))) * RPG + sub];
+            finish(sum, gw + g);
+        }
+    } else if constexpr (EAGER > 0) {
 #pragma unroll
         for (int s = 0; s < EAGER; ++s) {
             if (s < nsteps) consume(eager[s]);       // uniform
@@ -1331,6 +1384,28 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4
     else gemv_body<FmtQ80, ACT, TL, EAGER>(Pv, wg, nwg, strict, lds, tl, 0);
 }
 
+// One problem whose rows are long and few (see the rule in launch_gemv_group): `groups` consecutive row groups per workgroup,
+// whose steps are dealt to its 8 wavefronts in turn, so that every CU has a workgroup and every wavefront kSplitDepth steps
+// in flight; the wavefronts' parts of a row meet in LDS and are added in step order.  Bound: HBM, as far as the 16 wavefronts'
+// requests of a CU reach (Q8_0 4096 x 14336 4.0 TB/s).  Dealing the steps in contiguous runs instead measured the same on
+// most shapes and up to 0.2 us more where a workgroup has two groups.
+template <typename F>
+constexpr int kSplitDepth = F::kRegs <= 6 ? 6 : 4;
+template <typename F, int ACT>
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) gemv_split_kernel(
+    const uint8_t* w, const float* x, float* y, int N, int K, int w_bytes, int groups, const float* add, const float* norm_w, float eps)
+{
+    extern __shared__ uint32_t lds[];
+    GemvProblem Pv;
+    Pv.w = w, Pv.x = x, Pv.y = y, Pv.N = N, Pv.K = K, Pv.w_bytes = (int64_t)(uint32_t)w_bytes, Pv.add = add, Pv.norm_w = norm_w;
+    Pv.act = ACT;
+    Pv.eps = eps, Pv.limit = 0.f;
+    Pv.expert_id = nullptr, Pv.expert_stride = 0, Pv.n_experts = 0;
+    Pv.pair_rows = 0, Pv.pair_kind = 0;
+    Pv.slot_ids = nullptr, Pv.slot_w = nullptr, Pv.slot_bias = nullptr;
+    gemv_body<F, ACT, false, kSplitDepth<F>, true>(Pv, (int)blockIdx.x, (int)gridDim.x, groups, lds, nullptr, 0);
+}
+
 // The routed sum of one token (MoE decode: down projections + weighted sum) as a launch of its own argument list: the
 // stack of expert matrices, the staged activation vectors, the slot tables and the geometry are the preloaded scalars; the
 // result pointer and the bias are read where the code reaches them.
@@ -1452,9 +1527,25 @@ int eager_steps(int type)
     return type == kTypeQ4_K ? kEagerSteps<kTypeQ4_K> : type == kTypeMXFP4 ? kEagerSteps<kTypeMXFP4> : 0;
 }
 
+// the format of a split launch
+template <int TYPE>
+struct SplitFmt {
+    using type = std::conditional_t<TYPE == kTypeQ8_0, FmtQ80, std::conditional_t<TYPE == kTypeMXFP4, FmtMXFP4, FmtLegacy<TYPE>>>;
+};
+
 template <int TYPE, int ACT>
 bool launch_type(const GemvGroup& g, int grid, size_t lds, hipStream_t stream)
 {
+    if constexpr (TYPE != kTypeQ4_K && TYPE != kTypeQ5_K && TYPE != kTypeQ6_K && ACT != kActSiluMul) {
+        if (g.split > 0) {
+            const GemvProblem& p = g.p[0];
+            auto kern = gemv_split_kernel<typename SplitFmt<TYPE>::type, ACT>;
+            if (!raise_lds_limit(reinterpret_cast<const void*>(kern), lds)) return false;
+            hipLaunchKernelGGL(kern, dim3(grid), dim3(kThreads), lds, stream, p.w, p.x, p.y, p.N, p.K, (int)(uint32_t)p.w_bytes, g.split,
+                               p.add, p.norm_w, p.eps);
+            return hip_ok(hipGetLastError(), "gemv launch");
+        }
+    }
     // (the timeline build stamps launches of plain problems only)
     bool plain = true;
     for (int i = 0; i < g.count; ++i) plain = plain && !g.p[i].expert_id && !g.p[i].pair_rows && !g.p[i].slot_ids;
@@ -1639,6 +1730,24 @@ bool launch_gemv_group(int type, int count, const GemvArgs* args, hipStream_t st
             ok = ok && groups <= waves && steps <= eager_steps(type) && args[i].K <= kThreads * 32 && !args[i].slot_ids;
         }
         if (ok) g.strict = 2;
+    }
+    // The split build (gemv_split_kernel) for one problem of a 16-lane format with few and long rows.  Unsplit, a wavefront
+    // takes a row group's steps one after the other, about 0.65 us each, while most CUs have no workgroup; split, a
+    // workgroup of every CU shares per_wg groups among its 8 wavefronts, for 1 us more of start (two barriers, the parts).
+    // So the line lies where the steps saved, steps * (1 - per_wg / 8), are five of Q8_0 and six of the 17- to 24-byte
+    // blocks.  Measured unsplit / split, us: Q8_0 1024 x 14336 16.5 / 6.6, 2048 x 8192 10.6 / 7.1, 2560 x 9728 12.4 / 8.6,
+    // 2560 x 4096 6.7 / 5.7, 4096 x 14336 21.7 / 15.5, on the line 3072 x 3072 5.37 / 5.31 and 6144 x 8192 13.6 / 13.5, past
+    // it 4096 x 2560 5.2 / 5.5; with RMSNorm staging 2560 x 4096 7.6 / 6.8; MXFP4 2560 x 9728 10.7 / 7.6, 1024 x 4096
+    // 4.7 / 4.3, past the line 2560 x 4096 4.79 / 4.84.  (The 32-lane formats have twice the wavefronts per row and lose:
+    // Q4_K 4096 x 14336 8.9 / 10.4, Q6_K 2560 x 9728 9.0 / 9.4.)
+    if (count == 1 && lpr == 16 && !args[0].expert_id && !args[0].slot_ids && !args[0].pair_rows && act != kActSiluMul && !g_timeline) {
+        const int groups = (args[0].N + rpg - 1) / rpg, steps = (args[0].K / unit_elems(type) + lpr - 1) / lpr;
+        const int per_wg = (groups + di.num_cus - 1) / di.num_cus;
+        if (per_wg < kWaves && steps * (kWaves - per_wg) >= kWaves * (type == kTypeQ8_0 ? 5 : 6)) {
+            g.split = per_wg;
+            begin = (groups + per_wg - 1) / per_wg;
+            lds += kWaves * kWaves * 4 * sizeof(float);       // the parts: fewer than kWaves row groups of 4 rows
+        }
     }
     for (int i = 1; i < count; ++i)
         if (args[i].act != act) {

@@ -245,6 +245,36 @@ def test_few_rows_long_k_split_over_wavefronts(hip, oracle, name, N, K):
     assert np.max(np.abs(got - ref)) <= 1e-3 * np.linalg.norm(ref) + 1e-6 * np.max(np.abs(resid)), name
 
 
+@pytest.mark.parametrize("name", ["q8_0", "mxfp4", "q4_0", "q4_1", "q5_0", "q5_1", "iq4_nl"])
+@pytest.mark.parametrize("N,K", [(1, 4096), (1021, 3584 + 32), (1028, 4128), (2050, 4608 + 32), (4094, 6176)])
+def test_split_rows_at_the_edges_of_their_groups(hip, oracle, name, N, K):
+    """Few and long rows of the 16-lane formats: the wavefronts of a workgroup share its row groups (one group per workgroup
+    up to 1024 rows, two and four beyond), also added to a residual and with the RMSNorm in the staging.  A row count that
+    leaves the last group and the last workgroup partly empty, K that ends inside a step and inside a round of eight."""
+    import torch
+    from tensorsharp_amd import QuantizedWeight
+    rng = np.random.default_rng(N * 3 + K)
+    t, wq = host_case_weight(oracle, name, N, K, rng)
+    kind = name if name in RMS_TOL else "q4_k"
+    x = rng.standard_normal((1, K)).astype(np.float32)
+    ref = oracle.matmul_f64(t, wq, N, K, x)
+    w, xd = QuantizedWeight(torch.from_numpy(wq).cuda(), t, K, N), torch.from_numpy(x).cuda()
+    if N > 1:          # (one number has no row to be small against)
+        check(kind, hip.LinearForward(xd, w).cpu().numpy(), ref)
+    resid = rng.standard_normal((1, N)).astype(np.float32)
+    r = torch.from_numpy(resid).cuda()
+    hip.FusedMatMulQuantAdd(r, xd, w)
+    scale = np.linalg.norm(ref) if N > 1 else np.linalg.norm(x) * np.linalg.norm(oracle.dequantize(t, wq, K)) / np.sqrt(K)
+    assert np.max(np.abs(r.cpu().numpy().astype(np.float64) - resid - ref)) <= 1e-3 * scale + 1e-6 * np.max(np.abs(resid))
+    nw = (1 + 0.1 * rng.standard_normal(K)).astype(np.float32)
+    xn = x.astype(np.float64)
+    xn = (xn / np.sqrt(np.mean(xn * xn) + 1e-6) * nw).astype(np.float32)
+    y = torch.full((1, N), float("nan"), device="cuda")
+    hip.FusedRmsNormMatMulQuant(y, xd, torch.from_numpy(nw).cuda(), 1e-6, w)
+    want = oracle.matmul_f64(t, wq, N, K, xn)
+    assert np.max(np.abs(y.cpu().numpy() - want)) <= 1e-3 * (np.linalg.norm(want) if N > 1 else 1.2 * scale)
+
+
 # ---- Q6_K (output matrix and some projections of Q4_K_M files): 210-byte blocks, 2-byte aligned ----
 def q6k_weight(N, K, seed, std=0.02):
     import torch
