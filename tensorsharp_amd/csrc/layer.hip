@@ -8,22 +8,34 @@
 //                        (written by the workgroup of the last split, which uses them from LDS) - then computes
 //                        softmax(q . K^T / sqrt(head_dim)) V over positions 0..position (what ggml_flash_attn_ext
 //                        computes for one query row); a workgroup serves the query heads that share a KV head, so K / V
-//                        rows are loaded once per group; the positions are cut into splits of 64 or 128, each split
+//                        rows are loaded once per group; the positions are cut into splits of 64 or 128 (attn_rows), each split
 //                        leaves (max, sum, weighted V) behind (a single split writes the result itself)
 //   attn_combine_kernel  merges the splits of a head
 //
 // HBM-bound on the KV cache: 2 * num_kv_heads * (position + 1) * head_dim * 4 bytes per call.
 #include "tship_internal.h"
 
+#include <algorithm>
+
 namespace tship {
 namespace {
 
 constexpr int kMaxHeadDim = 256;
-// positions per workgroup of the attention kernel: one trip of the 16 groups x kInFlight rows while the context is
-// short (the kernel is latency bound: more, shorter workgroups), two trips beyond
-int attn_split_len(int total) { return total <= 2048 ? 64 : 128; }
-constexpr int kInFlight = 4;         // K / V rows a 16-lane group loads before it uses the first
-constexpr int kAttnWaves = 4;
+constexpr int kAttnWaves = 8;
+constexpr int kAttnGroups = 4 * kAttnWaves;      // 16-lane groups of a workgroup
+// K / V rows per 16-lane group, all requested at once; a workgroup's split is kAttnGroups times as many positions.  The kernel
+// is latency bound: two rows (more and shorter workgroups) while every CU has at most one workgroup per KV head's split and the
+// merge takes one batch of 64 splits, four beyond and where that leaves a single split and no merge.  Measured us per small
+// layer, two / four rows (query x KV heads): 32 x 8 64 positions 22.7 / 23.7, 100 25.2 / 23.6, 512 25.2 / 26.3, 2048 27.7 / 28.4,
+// 3000 32.0 / 30.8; 8 x 2 4001 24.8 / 26.2, 8192 27.7 / 27.2; 16 x 2 6000 29.1 / 26.9; 32 x 32 512 26.8 / 27.4, 700 29.8 / 29.4.
+constexpr int kFewSplits = 64;
+int attn_rows(int num_kv_heads, int total)
+{
+    if (total <= 2 * kAttnGroups) return 2;
+    if (total <= 4 * kAttnGroups) return 4;
+    const int splits = (total + 2 * kAttnGroups - 1) / (2 * kAttnGroups);
+    return splits <= kFewSplits && (int64_t)num_kv_heads * splits <= device_info().num_cus ? 2 : 4;
+}
 
 __device__ __forceinline__ float wave_sum(float v)
 {
@@ -67,35 +79,86 @@ struct AttnFront {
     float* v_cache;
 };
 
-// Merge of two online-softmax states (max, sum, weighted values).
-template <int N>
-__device__ __forceinline__ void softmax_merge(float& m, float& l, float (&acc)[N], float m2, float l2, const float (&acc2)[N])
+// x of the lane whose number differs in bit B (and, for the mirrors, in the lower ones) inside a row of 16 lanes
+template <int B>
+__device__ __forceinline__ float other16(float x)
 {
-    const float mm = fmaxf(m, m2);
-    const float f1 = m == -INFINITY ? 0.f : expf(m - mm), f2 = m2 == -INFINITY ? 0.f : expf(m2 - mm);
-    l = l * f1 + l2 * f2;
-#pragma unroll
-    for (int j = 0; j < N; ++j) acc[j] = acc[j] * f1 + acc2[j] * f2;
-    m = mm;
+    constexpr int kCtrl = B == 0 ? 0xb1 : B == 1 ? 0x4e : B == 2 ? 0x141 : 0x140;    // quad_perm [1,0,3,2], [2,3,0,1], mirrors of 8 and 16
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), kCtrl, 0xf, 0xf, true));
+}
+// x of lane L of the row of 16, in all its lanes
+template <int L>
+__device__ __forceinline__ float bcast16(float x)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x150 + L, 0xf, 0xf, true));    // row_newbcast
+}
+typedef uint32_t lane_pair_t __attribute__((ext_vector_type(2)));
+// one step of a sum over the four 16-lane rows of a wavefront that leaves a different value behind in each: rows 0 | 1 and 2 | 3
+// (the halves of the wavefront) get a and b
+__device__ __forceinline__ float rows_sum16(float a, float b)
+{
+    const lane_pair_t r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(r.x) + __uint_as_float(r.y);
+}
+__device__ __forceinline__ float rows_sum32(float a, float b)
+{
+    const lane_pair_t r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(r.x) + __uint_as_float(r.y);
+}
+__device__ __forceinline__ float rows_max(float x)
+{
+    lane_pair_t r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    x = fmaxf(__uint_as_float(r.x), __uint_as_float(r.y));
+    r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return fmaxf(__uint_as_float(r.x), __uint_as_float(r.y));
 }
 
-// Sum over the 16 lanes of a group, every lane gets it: four register permutations (pairs inside a quad, quads, mirrored
-// eights, mirrored sixteen) instead of four trips through the LDS crossbar.
-__device__ __forceinline__ float sum16(float v)
+constexpr int log2_of(int n) { return n <= 1 ? 0 : 1 + log2_of(n / 2); }
+
+// Sums over the 16 lanes of a row, NV of them at once, that leave value i only in the lanes that go on with it: at the step
+// of lane bit B a lane keeps the half of the values that its bit names and hands the other half to its neighbour.  Value i
+// ends in the lanes lane / 2^(4 - log2 NV) == i (NV = 32: values 2 lane and 2 lane + 1).  Sixteen sums cost 45 instructions
+// instead of 64, and what follows (maximum, exponential, sum) runs once per value instead of once per value and lane.
+template <int B, int NV>
+__device__ __forceinline__ void scatter_sums(float (&v)[NV], int lane, int count)
 {
-    auto moved = [](float x, auto perm) { return __int_as_float(perm(__float_as_int(x))); };
-    v += moved(v, [](int x) { return __builtin_amdgcn_update_dpp(0, x, 0xb1, 0xf, 0xf, true); });     // quad_perm [1,0,3,2]
-    v += moved(v, [](int x) { return __builtin_amdgcn_update_dpp(0, x, 0x4e, 0xf, 0xf, true); });     // quad_perm [2,3,0,1]
-    v += moved(v, [](int x) { return __builtin_amdgcn_update_dpp(0, x, 0x141, 0xf, 0xf, true); });    // lane i <-> 7 - i of each 8
-    v += moved(v, [](int x) { return __builtin_amdgcn_update_dpp(0, x, 0x140, 0xf, 0xf, true); });    // lane i <-> 15 - i of each 16
-    return v;
+    if constexpr (B >= 0) {
+        if (count > 1) {
+            const bool up = (lane >> B) & 1;
+#pragma unroll
+            for (int i = 0; i < count / 2; ++i) {
+                const float keep = up ? v[i + count / 2] : v[i], give = up ? v[i] : v[i + count / 2];
+                v[i] = keep + other16<B>(give);
+            }
+            scatter_sums<B - 1, NV>(v, lane, count / 2);
+        } else {
+            v[0] += other16<B>(v[0]);
+            scatter_sums<B - 1, NV>(v, lane, 1);
+        }
+    }
 }
+
+template <int L, int N>
+__device__ __forceinline__ float bcast_step(float x, int l)
+{
+    if constexpr (L + 1 < N) return l == L ? bcast16<L>(x) : bcast_step<L + 1, N>(x, l);
+    else return bcast16<L>(x);
+}
+// x of lane l of the row of 16; l is a constant once the loops around are unrolled
+__device__ __forceinline__ float bcast16_at(float x, int l) { return bcast_step<0, 16>(x, l); }
 
 // grid (num_kv_heads, splits, q-head chunks): one workgroup serves G query heads that share a KV head, so every K / V
-// row is loaded once for all of them.  4 wavefronts x 4 groups of 16 lanes; a group takes positions g, g + 16, ... of
-// the split, kInFlight at a time (all their loads are issued before the first is used: the loop is latency bound), lane l of
-// a group holds the head dimensions l, l + 16, ... (PER of them).  Groups, then wavefronts, merge their softmax states.
-template <int PER, int G>
+// row is loaded once for all of them.  8 wavefronts x 4 groups of 16 lanes; a group takes positions g, g + 32, ... of the
+// split, U of them, all requested before the first is used (a split is 32 U positions, there is no second trip), lane l of a
+// group holds the head dimensions l, l + 16, ... (PER of them).  The scores of a group's G x U (head, position) pairs are
+// summed over its lanes by scatter_sums, so that every pair's exponential is evaluated in one lane (or in a few) and reaches
+// the others by row_newbcast; a wavefront has one maximum per head, so that its groups' results add up without further factors;
+// the wavefronts merge their softmax states in LDS.
+// Bound: latency (launch, preparation of the heads, one trip to the caches), then HBM.  Against four wavefronts whose groups took
+// the positions four at a time with one sum, exponential and running maximum per pair: 32 x 8 heads of 128 at 512 positions
+// 6.6 -> 5.2 us, at 4001 positions (33 MB) 13.6 -> 10.6 us by the kernel trace; three Q8_0 layers and a head 182.1 -> 175.2.
+// (K / V rows as 16-byte loads: the same on every shape.)
+template <int PER, int G, int U>
 __global__ void __launch_bounds__(kAttnWaves * 64) attn_decode_kernel(float* k_cache, float* v_cache, const float* qkv, int group,
                                                                        int max_seq_len, int total, int split_len, float scale, int splits,
                                                                        int num_heads, float* __restrict__ partial, const AttnFront F,
@@ -118,8 +181,8 @@ __global__ void __launch_bounds__(kAttnWaves * 64) attn_decode_kernel(float* k_c
             for (int i = (int)threadIdx.x * 4; i < pre_floats; i += kAttnWaves * 64 * 4) {
                 typedef float f4_t __attribute__((ext_vector_type(4)));
                 // Ordinary loads with an empty use: the compiler owns their registers (written in asm, a load in flight could
-                // land in registers that already hold the next address) and waits for them on every trip, four trips of
-                // 1024 floats at a hidden size of 4096.  The trips hide behind the other workgroups' K / V rows: with all
+                // land in registers that already hold the next address) and waits for them on every trip, two trips of
+                // 2048 floats at a hidden size of 4096.  The trips hide behind the other workgroups' K / V rows: with all
                 // eight requests of a thread in flight at once the launch took 6.5 instead of 6.35 us (32 heads, 60 and 200
                 // positions, four runs each).
                 f4_t a = {0.f, 0.f, 0.f, 0.f}, b = a;
@@ -132,28 +195,25 @@ __global__ void __launch_bounds__(kAttnWaves * 64) attn_decode_kernel(float* k_c
     }
     const int h0 = kvh * group + blockIdx.z * G;                     // first query head of this workgroup
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int lg = lane & 15, grp = (wave << 2) | (lane >> 4);       // 16 groups per workgroup
+    const int lg = lane & 15, grp = (wave << 2) | (lane >> 4);
     const float* kb = k_cache + (int64_t)kvh * max_seq_len * HD;
     const float* vb = v_cache + (int64_t)kvh * max_seq_len * HD;
     const int position = total - 1;
     const bool last = split == splits - 1;                           // the split that holds the new position
-    // kInFlight rows of K and of V per group, all requested before the first is used; the first set is requested
-    // here, ahead of the work on the projections below, which does not depend on it
+    // U rows of K and of V per group, all requested before the first is used and ahead of the work on the projections below,
+    // which does not depend on them
     const int t_end = min(total, (split + 1) * split_len);
-    float kr[kInFlight][PER], vr[kInFlight][PER];
-    auto load_rows = [&](int t0) {
+    const int t0 = split * split_len + grp;
+    float kr[U][PER], vr[U][PER];
 #pragma unroll
-        for (int u = 0; u < kInFlight; ++u) {
-            const int64_t row = (int64_t)min(t0 + 16 * u, t_end - 1) * HD + lg;      // rows past the split: a valid row, unused
+    for (int u = 0; u < U; ++u) {
+        const int64_t row = (int64_t)min(t0 + kAttnGroups * u, t_end - 1) * HD + lg;      // rows past the split: a valid row, unused
 #pragma unroll
-            for (int j = 0; j < PER; ++j) {
-                kr[u][j] = kb[row + 16 * j];
-                vr[u][j] = vb[row + 16 * j];
-            }
+        for (int j = 0; j < PER; ++j) {
+            kr[u][j] = kb[row + 16 * j];
+            vr[u][j] = vb[row + 16 * j];
         }
-    };
-    int t0 = split * split_len + grp;
-    load_rows(t0);
+    }
 
     // ---- the projections' last steps, per head: RMSNorm over the head (ggml_rms_norm, then * weight), RoPE at
     // `position` (ggml_rope_ext with n_dims = head_dim: ggml-cpu/ops.cpp:5549-5563, :5636-5652).  Every workgroup
@@ -226,6 +286,7 @@ __global__ void __launch_bounds__(kAttnWaves * 64) attn_decode_kernel(float* k_c
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
             float* dst = is_q ? sq[hh] : sk;
+            const float by = is_q ? scale : 1.0f;
             float* cache = (!is_q && blockIdx.z == 0) ? k_cache + ((int64_t)kvh * max_seq_len + position) * HD : nullptr;
 #pragma unroll
             for (int j = 0; j < kPairs; ++j) {
@@ -234,8 +295,8 @@ __global__ void __launch_bounds__(kAttnWaves * 64) attn_decode_kernel(float* k_c
                     const int i0 = F.neox ? p : 2 * p, i1 = F.neox ? p + half : 2 * p + 1;
                     const float x0 = tmp[wave][i0], x1 = tmp[wave][i1];
                     const float r0 = x0 * cs[j] - x1 * sn[j], r1 = x0 * sn[j] + x1 * cs[j];
-                    dst[i0] = r0;
-                    dst[i1] = r1;
+                    dst[i0] = r0 * by;
+                    dst[i1] = r1 * by;
                     if (cache) {
                         cache[i0] = r0;
                         cache[i1] = r1;
@@ -256,114 +317,103 @@ __global__ void __launch_bounds__(kAttnWaves * 64) attn_decode_kernel(float* k_c
         }
         __syncthreads();
     }
-    float qr[G][PER], acc[G][PER], m[G], l[G];
+    if (last) {       // uniform: the new position's row is not in the caches yet (another workgroup may be writing it)
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            // Slots past the split hold a clamped row (the row being written by this very launch, or whatever the cache memory
+            // held): their values must not reach the sums, not even multiplied by a zero weight (0 * NaN), so they are
+            // replaced, not scaled (the scores below).
+            const int t = t0 + kAttnGroups * u;
+#pragma unroll
+            for (int j = 0; j < PER; ++j) {
+                kr[u][j] = t == position ? sk[lg + 16 * j] : kr[u][j];
+                vr[u][j] = t == position ? sv[lg + 16 * j] : t < t_end ? vr[u][j] : 0.f;
+            }
+        }
+    }
+    // scores: value g U + u is head g, position u of the group
+    constexpr int NV = G * U;
+    constexpr int kPerLane = NV > 16 ? NV / 16 : 1;                  // values a lane ends with
+    constexpr int kShift = NV > 16 ? 0 : 4 - log2_of(NV);            // lane >> kShift: the (first) value of a lane, / kPerLane
+    constexpr int kUInLane = kPerLane;                               // positions of a head that share a lane
+    constexpr int kULanes = log2_of(U / kUInLane);                   // lane bits kShift .. that number a head's positions
+    float sc[NV];
 #pragma unroll
     for (int g = 0; g < G; ++g) {
-        m[g] = -INFINITY;
-        l[g] = 0.f;
+        float qr[PER];
+#pragma unroll
+        for (int j = 0; j < PER; ++j) qr[j] = sq[g][lg + 16 * j];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            float d = 0.f;
+#pragma unroll
+            for (int j = 0; j < PER; ++j) d += qr[j] * kr[u][j];
+            sc[g * U + u] = d;
+        }
+    }
+    scatter_sums<3, NV>(sc, lg, NV);
+    if (last) {
+#pragma unroll
+        for (int r = 0; r < kPerLane; ++r) {
+            const int u = ((lg >> kShift) * kPerLane + r) & (U - 1);
+            if (t0 + kAttnGroups * u >= t_end) sc[r] = -INFINITY;
+        }
+    }
+    auto over_positions = [&](float x, auto op) {                    // of the lane's head, inside the group
+        if constexpr (kULanes > 0) x = op(x, other16<kShift>(x));
+        if constexpr (kULanes > 1) x = op(x, other16<kShift + 1>(x));
+        return x;
+    };
+    float m = sc[0];
+#pragma unroll
+    for (int r = 1; r < kPerLane; ++r) m = fmaxf(m, sc[r]);
+    m = rows_max(over_positions(m, [](float a, float b) { return fmaxf(a, b); }));
+    const float mref = m == -INFINITY ? 0.f : m;                     // a wavefront without a live position: weights of zero
+    float l = 0.f;
+#pragma unroll
+    for (int r = 0; r < kPerLane; ++r) {
+        sc[r] = expf(sc[r] - mref);
+        l += sc[r];
+    }
+    l = over_positions(l, [](float a, float b) { return a + b; });
+    l = rows_sum16(l, l);
+    l = rows_sum32(l, l);
+    // the lane that holds value i (NV = 32: two values per lane)
+    auto lane_of = [&](int i) { return (i / kPerLane) << kShift; };
+    if (lane < 16 && (lane & ((1 << (kShift + kULanes)) - 1)) == 0) {
+        const int g = lane >> (kShift + kULanes);
+        if (g < G) {
+            sm[wave][g] = m;
+            sl[wave][g] = l;
+        }
+    }
+    constexpr int NF = (G * PER + 3) / 4 * 4;
+    float acc[NF];
+#pragma unroll
+    for (int f = G * PER; f < NF; ++f) acc[f] = 0.f;
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+        float pw[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) pw[u] = bcast16_at(sc[(g * U + u) % kPerLane], lane_of(g * U + u));
 #pragma unroll
         for (int j = 0; j < PER; ++j) {
-            qr[g][j] = sq[g][lg + 16 * j] * scale;
-            acc[g][j] = 0.f;
+            float a = 0.f;
+#pragma unroll
+            for (int u = 0; u < U; ++u) a += pw[u] * vr[u][j];
+            acc[g * PER + j] = a;
         }
     }
-    for (; t0 < t_end; t0 += 16 * kInFlight) {
-        bool live[kInFlight];
+    // the four groups of the wavefront: row r of it ends with the sums of acc[4 q + r]
+    float* const my_acc = &sacc[wave][0][0];
 #pragma unroll
-        for (int u = 0; u < kInFlight; ++u) live[u] = t0 + 16 * u < t_end;
-        if (last) {       // uniform: the new position's row is not in the caches yet (another workgroup may be writing it)
-#pragma unroll
-            for (int u = 0; u < kInFlight; ++u) {
-                const bool fresh = t0 + 16 * u == position;
-#pragma unroll
-                for (int j = 0; j < PER; ++j) {
-                    kr[u][j] = fresh ? sk[lg + 16 * j] : kr[u][j];
-                    vr[u][j] = fresh ? sv[lg + 16 * j] : vr[u][j];
-                }
-            }
-        }
-        // Slots past the split hold a clamped row (in the last split the row being written by this very launch, or
-        // whatever the cache memory held): their values must not reach the sums, not even multiplied by a zero
-        // weight (0 * NaN), so they are replaced, not scaled.
-#pragma unroll
-        for (int u = 0; u < kInFlight; ++u)
-#pragma unroll
-            for (int j = 0; j < PER; ++j) {
-                kr[u][j] = live[u] ? kr[u][j] : 0.f;
-                vr[u][j] = live[u] ? vr[u][j] : 0.f;
-            }
-#pragma unroll
-        for (int g = 0; g < G; ++g) {
-            float d[kInFlight];
-#pragma unroll
-            for (int u = 0; u < kInFlight; ++u) {
-                d[u] = 0.f;
-#pragma unroll
-                for (int j = 0; j < PER; ++j) d[u] += qr[g][j] * kr[u][j];
-            }
-#pragma unroll
-            for (int u = 0; u < kInFlight; ++u) d[u] = sum16(d[u]);
-            float mn = m[g];
-#pragma unroll
-            for (int u = 0; u < kInFlight; ++u) {
-                if (!live[u]) d[u] = -INFINITY;
-                mn = fmaxf(mn, d[u]);
-            }
-            const float corr = expf(m[g] - mn);                    // exp(-inf) = 0 on the first rows
-            float p[kInFlight], psum = 0.f;
-#pragma unroll
-            for (int u = 0; u < kInFlight; ++u) {
-                p[u] = expf(d[u] - mn);
-                psum += p[u];
-            }
-            l[g] = l[g] * corr + psum;
-#pragma unroll
-            for (int j = 0; j < PER; ++j) {
-                float a = acc[g][j] * corr;
-#pragma unroll
-                for (int u = 0; u < kInFlight; ++u) a += p[u] * vr[u][j];
-                acc[g][j] = a;
-            }
-            m[g] = mn;
-        }
-        if (t0 + 16 * kInFlight < t_end) load_rows(t0 + 16 * kInFlight);
-    }
-    // the four groups of a wavefront
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-        // rows 0 | 1 and 2 | 3 of the wavefront, then the two halves: a lane gets the state of the even and of the odd
-        // member of its pair (register swaps between rows) and merges them, so every lane ends with the same result
-#pragma unroll
-        for (int level = 0; level < 2; ++level) {
-            typedef uint32_t u2_t __attribute__((ext_vector_type(2)));
-            auto both = [&](float x, float& even, float& odd) {
-                const u2_t r = level == 0 ? __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false)
-                                          : __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-                even = __uint_as_float(r.x);
-                odd = __uint_as_float(r.y);
-            };
-            float m1, m2, l1, l2, a1[PER], a2[PER];
-            both(m[g], m1, m2);
-            both(l[g], l1, l2);
-#pragma unroll
-            for (int j = 0; j < PER; ++j) both(acc[g][j], a1[j], a2[j]);
-            softmax_merge<PER>(m1, l1, a1, m2, l2, a2);
-            m[g] = m1;
-            l[g] = l1;
-#pragma unroll
-            for (int j = 0; j < PER; ++j) acc[g][j] = a1[j];
-        }
-        if (lane < 16) {
-            if (lane == 0) {
-                sm[wave][g] = m[g];
-                sl[wave][g] = l[g];
-            }
-#pragma unroll
-            for (int j = 0; j < PER; ++j) sacc[wave][g][lg + 16 * j] = acc[g][j];
-        }
+    for (int q = 0; q < NF / 4; ++q) {
+        const float t = rows_sum32(rows_sum16(acc[4 * q], acc[4 * q + 1]), rows_sum16(acc[4 * q + 2], acc[4 * q + 3]));
+        const int f = 4 * q + (lane >> 4), g = f / PER, j = f - g * PER;
+        if (G * PER % 4 == 0 || f < G * PER) my_acc[g * HD + lg + 16 * j] = t;
     }
     __syncthreads();
-    // the four wavefronts: thread (g, d) of the first G * HD threads
+    // the wavefronts: thread (g, d) of the first G * HD threads
     for (int i = threadIdx.x; i < G * HD; i += kAttnWaves * 64) {
         const int g = i / HD, d = i - g * HD;
         float mm = -INFINITY;
@@ -458,10 +508,10 @@ __global__ void __launch_bounds__(WAVES * 64) attn_combine_kernel(const float* _
 
 }  // namespace
 
+// (at least what any shorter context takes, so that a workspace that served one position serves the next)
 size_t attention_decode_ws_bytes(int num_heads, int total)
 {
-    const int split_len = attn_split_len(total);
-    const int splits = (total + split_len - 1) / split_len;
+    const int splits = std::max((total + 4 * kAttnGroups - 1) / (4 * kAttnGroups), kFewSplits);
     return (size_t)num_heads * splits * (kMaxHeadDim + 2) * sizeof(float);
 }
 
@@ -491,7 +541,7 @@ bool launch_attention_decode(const float* qkv, const float* q_norm_w, const floa
     front.num_kv_heads = num_kv_heads;
     front.k_cache = k_cache;
     front.v_cache = v_cache;
-    const int split_len = attn_split_len(total);
+    const int rows = attn_rows(num_kv_heads, total), split_len = kAttnGroups * rows;
     const int splits = (total + split_len - 1) / split_len;
     if (splits > 65535) {
         set_last_error("layer decode: context too long for one launch.");
@@ -507,10 +557,13 @@ bool launch_attention_decode(const float* qkv, const float* q_norm_w, const floa
     const bool pre = (prefetch0 || prefetch1) && prefetch_floats > 0 && prefetch_floats % 4 == 0 && splits < 65535 &&
                      ((reinterpret_cast<uintptr_t>(prefetch0) | reinterpret_cast<uintptr_t>(prefetch1)) & 15) == 0;
     const dim3 grid(num_kv_heads, splits + (pre ? 1 : 0), group / g), block(kAttnWaves * 64);
-#define TSHIP_ATTN_LAUNCH(PER, GG)                                                                                              \
-    hipLaunchKernelGGL((attn_decode_kernel<PER, GG>), grid, block, 0, stream, front.k_cache, front.v_cache, front.qkv, group,     \
+#define TSHIP_ATTN_LAUNCH_U(PER, GG, U)                                                                                         \
+    hipLaunchKernelGGL((attn_decode_kernel<PER, GG, U>), grid, block, 0, stream, front.k_cache, front.v_cache, front.qkv, group,     \
                        max_seq_len, total, split_len, scale, splits, num_heads, partial_ws, front, splits == 1 ? out : nullptr,           \
                        pre ? prefetch0 : nullptr, pre ? prefetch1 : nullptr, pre ? prefetch_floats : 0)
+#define TSHIP_ATTN_LAUNCH(PER, GG)                                           \
+    if (rows == 2)          TSHIP_ATTN_LAUNCH_U(PER, GG, 2);              \
+    else TSHIP_ATTN_LAUNCH_U(PER, GG, 4)
 #define TSHIP_ATTN_G(PER)                                                    \
     switch (g) {                                                             \
     case 8: TSHIP_ATTN_LAUNCH(PER, 8); break;                                \
@@ -529,6 +582,7 @@ bool launch_attention_decode(const float* qkv, const float* q_norm_w, const floa
     }
 #undef TSHIP_ATTN_G
 #undef TSHIP_ATTN_LAUNCH
+#undef TSHIP_ATTN_LAUNCH_U
     if (!hip_ok(hipGetLastError(), "attention launch")) return false;
     if (splits == 1) return true;
     // Four wavefronts request up to 16 splits' rows in one round trip; more splits take sixteen, which cover 64, instead of
