@@ -604,11 +604,11 @@ bool has_tile_gemm(int type)
     }
 }
 
-// activation layout of a tile-table launch over expert pointers: MXFP4 on 32-row units reads MX fp6 pairs (rows of at least
-// 256 outputs: the error of fp6 pairs against a short row's norm is too close to the 1e-3 bound)
+// activation layout (GemmPlan::x_layout) of a tile-table launch over expert pointers: MXFP4 on 32-row units reads MX fp6 pairs
+// (rows of at least 256 outputs: the error of fp6 pairs against a short row's norm is too close to the 1e-3 bound)
 int expert_tiles_x_layout(int type, int bm, int K, int out_features)
 {
-    return type == kTypeMXFP4 && bm == 32 && K <= 32768 && out_features >= 256 ? 1 : 0;
+    return type == kTypeMXFP4 && bm == 32 && K <= 32768 && out_features >= 256 ? 1 : bm == 32 ? 3 : 0;
 }
 
 // The plan of one linear of the experts of a set, whose shape they share: experts of the same type as the one before them take
@@ -1644,8 +1644,8 @@ int TSHip_MoEExpertsGptOssForwardF32Device(TSHipTensorView2D result, TSHipTensor
         const bool mx_type = ggml_type == kTypeMXFP4 && H <= 32768 && F <= 32768 && H >= 256 && F >= 128;
         const bool rows48 = mx_type && per_expert > 20 && H <= 3072 && F <= 3072;
         const bool mx = mx_type && (rows48 || per_expert <= 160);
-        const int x_layout = mx ? 1 : 0;
         const int bm = rows48 ? 48 : per_expert > 160 ? 128 : 32;
+        const int x_layout = mx ? 1 : bm == 32 ? 3 : 0;
         const int max_tiles = A / bm + E;
         // carve the workspace
         size_t off = 0;

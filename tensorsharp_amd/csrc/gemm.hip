@@ -151,9 +151,15 @@ __device__ __forceinline__ float swiglu_oai(float gate, float up, float alpha, f
     return x / (1.0f + expf(alpha * (-x))) * (y + 1.0f);
 }
 
+// Activations for gemm_slim_kernel: the rows in blocks of 32 (the last one of what is left), a block's pieces of eight halfs -
+// the A operand of one lane in one k-step - ordered by piece and then by row.  Halfs from a row's piece to its next one, and
+// where its first one starts; the rows take the same bytes as rows that follow one another.
+__device__ __forceinline__ int piece_halfs(int row, int rows) { return 8 * min(32, rows - (row & ~31)); }
+__device__ __forceinline__ int64_t piece_start(int row, int ld) { return (int64_t)(row & ~31) * ld + (row & 31) * 8; }
+
 template <int TYPE, int THREADS, int SRC>
 __global__ void __launch_bounds__(THREADS) convert_x_kernel(const ConvertSrc S, int K, int Kp, int ldo, _Float16* __restrict__ out,
-                                                            float* __restrict__ scales)
+                                                            float* __restrict__ scales, int piece_rows)
 {
     const int m = blockIdx.x;
     const int tid = threadIdx.x;
@@ -235,8 +241,11 @@ __global__ void __launch_bounds__(THREADS) convert_x_kernel(const ConvertSrc S, 
     const float inv = __uint_as_float((uint32_t)(254 - se) << 23);
     // the weight operands carry 2^kWShift (see kWShift), the row scale takes it back
     if (tid == 0) scales[m] = __uint_as_float((uint32_t)se << 23) * (1.0f / kWUp);
-    _Float16* dst = out + (int64_t)m * ldo;
-    auto put = [&](int k, float v) { dst[(k & ~(kBK - 1)) | k_slot<TYPE>(k & (kBK - 1))] = (_Float16)(v * inv); };
+    // piece_rows (the number of rows): pieces of eight halfs, row by row within 32 rows (see gemm_slim_kernel); 0: whole rows
+    const int pitch = piece_rows ? piece_halfs(m, piece_rows) : 8;
+    _Float16* dst = out + (piece_rows ? piece_start(m, ldo) : (int64_t)m * ldo);
+    auto at = [&](int pos) { return dst + (pos >> 3) * pitch + (pos & 7); };
+    auto put = [&](int k, float v) { *at((k & ~(kBK - 1)) | k_slot<TYPE>(k & (kBK - 1))) = (_Float16)(v * inv); };
     // Four consecutive activations land in one aligned 8-byte piece of the k-tile: in the K-quant order as
     // (x0, x2, x1, x3), in the natural order as they are, and in the split-nibble order interleaved with the four
     // activations 16 further on, which the lane four to the right (left) holds - the pair swaps them and each stores
@@ -263,10 +272,10 @@ __global__ void __launch_bounds__(THREADS) convert_x_kernel(const ConvertSrc S, 
             o.y = pack2(v.z, v.w);
             slot = k_slot<TYPE>((4 * q) & (kBK - 1));
         }
-        if (q < k4) *reinterpret_cast<uint2*>(dst + (((4 * q) & ~(kBK - 1)) | slot)) = o;
+        if (q < k4) *reinterpret_cast<uint2*>(at(((4 * q) & ~(kBK - 1)) | slot)) = o;
     }
     for (int k = kHeld + tid; k < K; k += THREADS) put(k, tail_value(k));
-    for (int k = K + tid; k < Kp; k += THREADS) dst[(k & ~(kBK - 1)) | k_slot<TYPE>(k & (kBK - 1))] = (_Float16)0.f;
+    for (int k = K + tid; k < Kp; k += THREADS) *at((k & ~(kBK - 1)) | k_slot<TYPE>(k & (kBK - 1))) = (_Float16)0.f;
 }
 
 // ------------------------------------------------------------------------------------------
@@ -819,6 +828,7 @@ struct GemmArgs {
     float* partial;          // null: one chunk, results go straight to c
     int k_chunks;
     int chunk_kt;            // k-tiles per chunk (8 wavefronts x KTW)
+    int x_pieces;            // the activations are in pieces, row by row (piece_start): gemm_slim_kernel
     int x_mx;                // the activations are MX fp6 pairs in gemm_mx_kernel's layout (convert_x_mx_kernel)
     // gemm_slim_mx_kernel<.., .., 1>: bias + SwiGLU-OAI of (gate, up) column pairs, written as MX activation rows
     const float* epi_bias;   // optional [experts x 2 F]
@@ -2661,17 +2671,25 @@ __global__ void __launch_bounds__(512) gemm_slim_kernel(const GemmArgs A)
         const __amdgpu_buffer_rsrc_t wrs = __builtin_amdgcn_make_buffer_rsrc(
             reinterpret_cast<void*>(wa & ~(uintptr_t)3), 0, (int)(((uint32_t)A.w_bytes + base_delta + 3u) & ~3u), 0x00020000);
 
-        // MFMA A operands of this wavefront's K range: row `col`, k-half h of every k-step
+        // MFMA A operands of this wavefront's K range: row `col`, k-half h of every k-step.  Pieces of eight halfs lie row by
+        // row (piece_start), so that a load is one or two contiguous kilobytes: from rows that followed one another each
+        // was 64 pieces of 16 bytes in 32 lines, and the 256 loads of a workgroup took
+        // the address unit about 3 us.  Measured, whole call, us: Q4_K 32 x 14336 x 4096 23.2 -> 19.9, 32 x 4096 x 14336 26.4 -> 23.8,
+        // Q8_0 32 x 2560 x 9728 24.3 -> 21.2, Q5_K 32 x 21504 x 5376 44.4 -> 41.0, MXFP4 32 x 14336 x 4096 21.9 -> 18.2; up to eight
+        // rows the same (the lanes of the missing rows read the last one).
         half8_t a[KTW][4];
         {
-            const _Float16* xr = A.x16 + (int64_t)(m0 + min(col, m_rows - 1)) * A.xld + h * 8;
+            const int row = m0 + min(col, m_rows - 1);
+            const uint32_t piece = 2u * (uint32_t)piece_halfs(row, A.M);              // bytes to the row's next piece
+            const uint32_t first = 2u * (uint32_t)piece_start(row, A.xld) + (uint32_t)h * piece;
+            const uint8_t* const xb = reinterpret_cast<const uint8_t*>(A.x16);
             const half8_t zero = {0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
             for (int t = 0; t < KTW; ++t) {
                 const int kt = min(kt0 + t, nkt - 1);
 #pragma unroll
                 for (int ks = 0; ks < 4; ++ks) {
-                    const half8_t v = *reinterpret_cast<const half8_t*>(xr + kt * kBK + ks * 16);
+                    const half8_t v = *reinterpret_cast<const half8_t*>(xb + (first + (uint32_t)(kt * 8 + 2 * ks) * piece));
                     a[t][ks] = (col < m_rows && t < kcnt) ? v : zero;
                 }
             }
@@ -3678,6 +3696,10 @@ bool launch_for_type(const GemmArgs& a, int bm, int m_tiles, const WidePlan& wid
         if constexpr (std::is_same<G, GQ80>::value) return launch_wide<WQ80>(a, wide, stream, cs);
         if constexpr (std::is_same<G, GQ6K>::value) return launch_wide<WQ6K>(a, wide, stream, cs);
     }
+    if (a.x_pieces != (bm == 32 && !a.x_mx ? 1 : 0)) {
+        set_last_error("gemm: activations in pieces serve the 32-row units of fp16 operands, and these take no others.");
+        return false;
+    }
     if (bm == 32 && !a.x_mx) return launch_slim_for<G>(a, slim_ktw<G>(a.Kp / kBK), m_tiles, stream, cs);
     // Q4_K and MXFP4: the 2 x 4 wavefront layout with the operand exchange through LDS (gemm_xw_kernel); 128-row tiles are
     // 128 x 256.  Q4_K takes it for every launch, MXFP4 for plain ones: the MXFP4 expert tiles of a MoE prefill (128
@@ -3758,15 +3780,19 @@ namespace {
 // about 870 random ones per format over 4 .. 2048 rows, 64 .. 28672 columns and K of 256 .. 21504, a third of them added to a
 // residual.  On 300 further random calls per format the pick took 0.4 % (Q4_K), 0.3 % (Q8_0) and 0.2 % (Q6_K) longer than the
 // fastest candidate on average, more than 4 % longer on 11, 8 and 3 of them, 11 % at most.
+// slim_rows was measured again with the activations in pieces (see gemm_slim_kernel), on 350 (300) calls per format of 2 .. 150
+// rows, 512 .. 21504 columns and K of 1024 .. 14336: with the first fit's value, slim_rows_far, the pick would now be 2.8 / 0.4 /
+// 0.2 % behind (Q4_K / Q8_0 / Q6_K), with this one 0.5 / 0.2 / 0.1 %.
 // Where the lines lie, us (register-resident / gemm_wide_kernel / 128 rows / 256 rows):
 //   Q4_K  8 x 4096 x 4096 12.4 / 16.3 / - / -,  64 x 4096 x 4096 17.4 / 21.0 / 28.5 / 34.0,  200 x 4096 x 4096 38.5 / 28.3 / 32.2 /
 //         39.8,  1024 x 9728 x 2560 151 / 85.8 / 104.7 / 68.7
 //   Q8_0  8 x 14336 x 4096 23.2 / 24.0 / - / -,  128 x 28672 x 4096 90.7 / 60.0 / 67.0 / 76.6,  400 x 4096 x 4096 - / 39.2 / 37.4 / -
 //   Q6_K  512 x 4096 x 4096 - / 47.5 / 45.1 / -,  2048 x 2560 x 9728 - / 200.8 / 240.7 / -
 struct RuleCosts {
-    // register-resident kernel: a call; its activations, per 32 rows and 8 k-tiles per wavefront; a round of units and per k-tile
-    // of a wavefront in it; a workgroup whose units cross into another row tile or K chunk (it loads activations anew)
-    double slim, slim_rows, unit, unit_kt, cross, cross_kt;
+    // register-resident kernel: a call; its activations, per 32 rows and 8 k-tiles per wavefront (and beyond the
+    // calls that slim_rows was fitted to); a round of units and per k-tile of a wavefront in it; a workgroup whose units cross into another
+    // row tile or K chunk (it loads activations anew)
+    double slim, slim_rows, slim_rows_far, unit, unit_kt, cross, cross_kt;
     // gemm_wide_kernel: a call, a k-tile of a round and per 32 rows in it, the share of that time that an almost empty round
     // takes, a round
     double wide, wide_kt, wide_kt_rows, wide_fill, wide_round;
@@ -3775,13 +3801,13 @@ struct RuleCosts {
     double sums, sums_rate;                            // the launch that adds K chunks: a call, TB/s of its sums written and read
     double wide_add, tile_add;                         // results added in place: a round, per 32 rows of a tile (one load after the other)
 };
-constexpr RuleCosts kCostsQ4K{6.538, 6.588, 0.471, 0.444, 4.440, 0.000, 5.031, 0.423, 0.153, 0.966, 3.404,
+constexpr RuleCosts kCostsQ4K{6.538, 3.000, 6.000, 0.471, 0.444, 4.440, 0.000, 5.031, 0.423, 0.153, 0.966, 3.404,
                               11.108, 1.670, 0.618, 0.032, 0.000, 0.000, 0.000, 0.000,      // (no 128-row tiles)
                               2.367, 4.806, 3.964, 4.582};
-constexpr RuleCosts kCostsQ80{6.249, 5.523, 1.221, 0.339, 0.590, 0.891, 5.085, 0.495, 0.148, 1.006, 5.151,
+constexpr RuleCosts kCostsQ80{6.249, 2.500, 5.523, 1.221, 0.339, 0.590, 0.891, 5.085, 0.495, 0.148, 1.006, 5.151,
                               3.152, 1.741, 0.926, 4.675, 4.610, 1.247, 1.492, 1.841,
                               1.697, 5.090, 6.433, 1.591};
-constexpr RuleCosts kCostsQ6K{5.858, 6.414, 0.393, 0.658, 2.025, 0.406, 4.411, 1.047, 0.156, 0.890, 6.472,      // (no 256-row tiles)
+constexpr RuleCosts kCostsQ6K{5.858, 2.500, 6.414, 0.393, 0.658, 2.025, 0.406, 4.411, 1.047, 0.156, 0.890, 6.472,      // (no 256-row tiles)
                               0.000, 0.000, 0.000, 0.000, 6.177, 1.561, 0.938, 3.905,
                               3.284, 7.419, 3.358, 1.187};
 constexpr double kNotServed = 1e30;      // a kernel that a format has not, or whose chunk sums do not fit
@@ -3800,7 +3826,8 @@ double slim_us(const RuleCosts& c, int M, int N, int nkt, bool accumulate, size_
     // segments) < cus, and over all i that remainder is at most segments - gcd(segments, cus).
     const bool crosses = units > cus && n32 * (segments - std::gcd(segments, (int64_t)cus)) >= cus;
     const double kt = 0.4 * ktw + 0.6 * nkt / (8.0 * kc);      // (wavefronts past the end of K leave theirs to the others)
-    return c.slim + c.slim_rows * std::min(M, 32) * ktw / 256.0 + (double)((units + cus - 1) / cus) * (c.unit + c.unit_kt * kt) +
+    const double rows = M <= 32 || (M <= 160 && N >= 1024) ? c.slim_rows : c.slim_rows_far;
+    return c.slim + rows * std::min(M, 32) * ktw / 256.0 + (double)((units + cus - 1) / cus) * (c.unit + c.unit_kt * kt) +
            (crosses ? c.cross + c.cross_kt * ktw : 0.0) + (two_pass ? sums_us(c, kc, M, N) : 0.0);
 }
 
@@ -3884,14 +3911,14 @@ int gemm_tile_m(int type, int M, int N, int K, bool accumulate, size_t max_chunk
 }
 
 template <int TYPE, int SRC>
-void launch_convert_typed(const ConvertSrc& src, int M, int K, int kp, _Float16* x16, float* scales, hipStream_t stream)
+void launch_convert_typed(const ConvertSrc& src, int M, int K, int kp, _Float16* x16, float* scales, hipStream_t stream, int layout)
 {
-    const int ldo = x_row_halfs(K);
+    const int ldo = x_row_halfs(K), piece_rows = layout == 3 ? M : 0;
     // short rows: 256 threads hold the whole row and eight workgroups share a CU
     if (K <= 256 * kCvtHold * 4)
-        hipLaunchKernelGGL((convert_x_kernel<TYPE, 256, SRC>), dim3(M), dim3(256), 0, stream, src, K, kp, ldo, x16, scales);
+        hipLaunchKernelGGL((convert_x_kernel<TYPE, 256, SRC>), dim3(M), dim3(256), 0, stream, src, K, kp, ldo, x16, scales, piece_rows);
     else
-        hipLaunchKernelGGL((convert_x_kernel<TYPE, 1024, SRC>), dim3(M), dim3(1024), 0, stream, src, K, kp, ldo, x16, scales);
+        hipLaunchKernelGGL((convert_x_kernel<TYPE, 1024, SRC>), dim3(M), dim3(1024), 0, stream, src, K, kp, ldo, x16, scales, piece_rows);
 }
 
 template <int SRC>
@@ -3913,11 +3940,11 @@ bool launch_convert(int type, const ConvertSrc& src, int M, int K, void* workspa
     if (layout == 2) type = kTypeQ8_0;      // natural order
     // three activation orders: the K-quant nibble order, the split-nibble order of the 32-weight blocks, natural
     switch (type) {
-    case kTypeQ4_K: case kTypeQ5_K: launch_convert_typed<kTypeQ4_K, SRC>(src, M, K, kp, x16, scales, stream); break;
+    case kTypeQ4_K: case kTypeQ5_K: launch_convert_typed<kTypeQ4_K, SRC>(src, M, K, kp, x16, scales, stream, layout); break;
     case kTypeMXFP4: case kTypeQ4_0: case kTypeQ4_1: case kTypeQ5_0: case kTypeQ5_1: case kTypeIQ4_NL:
-        launch_convert_typed<kTypeMXFP4, SRC>(src, M, K, kp, x16, scales, stream);
+        launch_convert_typed<kTypeMXFP4, SRC>(src, M, K, kp, x16, scales, stream, layout);
         break;
-    case kTypeQ8_0: case kTypeQ6_K: launch_convert_typed<kTypeQ8_0, SRC>(src, M, K, kp, x16, scales, stream); break;
+    case kTypeQ8_0: case kTypeQ6_K: launch_convert_typed<kTypeQ8_0, SRC>(src, M, K, kp, x16, scales, stream, layout); break;
     default: set_last_error("gemm: unsupported type."); return false;
     }
     return hip_ok(hipGetLastError(), "activation convert launch");
@@ -3962,6 +3989,7 @@ bool gemm_args(GemmArgs* out, const void* w, int64_t w_bytes, const void* worksp
     a.c = c;
     a.ldc = ldc;
     a.x_mx = x_layout == 1 ? 1 : 0;
+    a.x_pieces = x_layout == 3 ? 1 : 0;
     a.M = M;
     a.N = N;
     a.K = K;
@@ -4036,6 +4064,7 @@ GemmPlan plan_gemm(int type, int M, int N, int K, bool accumulate, size_t max_ch
     // gemm_wide_kernel reads natural order, which for the other two formats it serves is their unpack order anyway
     if (type == kTypeQ4_K && p.bm == kWideTiles) p.x_layout = 2;
     if (type == kTypeMXFP4 && K <= 1024 * kCvtHold * 4 && (p.bm >= 128 || (int64_t)N * K >= ((int64_t)64 << 20))) p.x_layout = 1;
+    if (p.bm == 32 && p.x_layout == 0) p.x_layout = 3;
     // the launcher's own dry run, with no bound, so that it makes the choices it would make with the reported bytes at hand
     const ChunkScratch cs{nullptr, ~(size_t)0, &p.chunk_bytes};
     GemmArgs a{};

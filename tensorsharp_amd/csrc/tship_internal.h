@@ -153,7 +153,8 @@ struct GemmPlan {
     int bm;                              // rows of activations per tile: 32, 128 or 256, 0 where gemm_wide_kernel runs, -1 no kernel
     int wide_tm, k_chunks, chunk_kt;     // gemm_wide_kernel: rows per tile / 32, K chunks, k-tiles per chunk
     int x_layout;                        // of the converted activations: 0 fp16 in the format's unpack order, 1 MX fp6 pairs (MXFP4 on
-                                         // the block-scaled matrix instruction), 2 fp16 in natural order (Q4_K on gemm_wide_kernel)
+                                         // the block-scaled matrix instruction), 2 fp16 in natural order (Q4_K on gemm_wide_kernel),
+                                         // 3 as 0 in pieces of eight, row by row (the 32-row units of fp16 operands)
     size_t chunk_bytes;                  // scratch for the sums of K chunks (0 for most shapes)
 };
 // max_chunk_bytes: what the launch will be given; kernels and K chunks whose sums do not fit are passed over

@@ -392,6 +392,21 @@ def test_more_formats_matmul(hip, oracle, name, M, N, K):
     check(y, oracle.matmul_f64(t, wq, N, K, x), (name, M, N, K))
 
 
+@pytest.mark.parametrize("name", ["q5_k", "q4_1", "mxfp4"])
+@pytest.mark.parametrize("M", [4, 31, 32, 33, 63, 65, 127])
+@pytest.mark.parametrize("K", [256, 4352])
+def test_32_row_units_with_a_short_last_block_of_rows(hip, oracle, name, M, K):
+    """The activations of the register-resident kernel lie in blocks of 32 rows, the last one of what is left: rows on both
+    sides of a block's end, one k-tile per wavefront and K in chunks.  The bar is check()'s."""
+    from oracle.oracle import MORE_TYPES
+    N = 161
+    t = MORE_TYPES[name] if name in MORE_TYPES else T[name]
+    rng = np.random.default_rng(M + K + t)
+    wq = inputs.random_blocks(name, N, K, rng) if name in MORE_TYPES else oracle.quantize(t, (rng.standard_normal(N * K) * 0.02).astype(np.float32))
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    check(run_device(hip, t, wq, N, K, x), oracle.matmul_f64(t, wq, N, K, x), (name, M, N, K))
+
+
 @pytest.mark.parametrize("name", ["q4_0", "q4_1", "q5_0", "q5_1", "iq4_nl", "q5_k", "mxfp4"])
 def test_256_row_tiles_of_the_other_formats(hip, oracle, name):
     # 1024 x 8448: more 128-row tiles than one round of workgroups, so the launcher takes 256-row tiles
