@@ -246,19 +246,33 @@ def _host_view(a, standard):
     return N.TensorView2D(a.ctypes.data, a.shape[0], a.shape[1], s0, s1, span)
 
 
+_torch_module = None
+
+
+def _torch():
+    """torch, imported with the first call that meets device tensors.  The host path of a call is written for its length: a
+    GEMV of one token takes 8 us on the device, and an import statement, a stream object or a shape read three times over
+    cost up to a microsecond each (one Q8_0 9728 x 2560 linear after another: 12.7 -> 9.1 us of host time per call)."""
+    global _torch_module
+    if _torch_module is None:
+        import torch
+        _torch_module = torch
+    return _torch_module
+
+
 def _device_view(t):
-    import torch
+    torch = _torch()
     if not isinstance(t, torch.Tensor) or t.dim() != 2:
         raise ValueError("AddmmQuant requires 2D tensors for result and m1.")
     if t.dtype != torch.float32:
         raise ValueError("AddmmQuant requires Float32 tensors for result and m1.")
     if not t.is_cuda:
         raise ValueError("device AddmmQuant requires tensors in GPU memory.")
+    rows, cols = t.shape
     s0, s1 = t.stride()
-    if s1 != 1 and t.shape[1] > 1:
+    if s1 != 1 and cols > 1:
         raise NotImplementedError("HIP AddmmQuant requires tensors with supported row-contiguous layouts.")
-    span = ((t.shape[0] - 1) * s0 + (t.shape[1] - 1) + 1) * 4
-    return N.TensorView2D(t.data_ptr(), t.shape[0], t.shape[1], s0, 1, span)
+    return N.TensorView2D(t.data_ptr(), rows, cols, s0, 1, ((rows - 1) * s0 + cols) * 4)
 
 
 class HipBasicOps:
@@ -508,8 +522,7 @@ class HipBasicOps:
         """Same contract with every pointer in device memory; asynchronous on the current stream."""
         rv = _device_view(result)
         mv = _device_view(m1)
-        ok = N.lib().TSHip_AddmmQuantF32Device(rv, mv, C.c_void_p(weight_data), int(ggml_type), int(ne0), int(ne1),
-                                               int(raw_bytes))
+        ok = N.lib().TSHip_AddmmQuantF32Device(rv, mv, weight_data, int(ggml_type), int(ne0), int(ne1), int(raw_bytes))
         N.check_result(ok, "addmm_quant")
 
     @staticmethod
@@ -583,7 +596,7 @@ class HipBasicOps:
     @staticmethod
     def MoERoute(logits, k):
         """logits [T x E] (CUDA fp32) -> (weights [T x k] fp32, ids [T x k] int32)."""
-        import torch
+        torch = _torch()
         T = logits.shape[0]
         ids = torch.empty((T, k), dtype=torch.int32, device=logits.device)
         wts = torch.empty((T, k), dtype=torch.float32, device=logits.device)
@@ -596,7 +609,7 @@ class HipBasicOps:
     def MoEExpertsGptOssForward(hidden, ids, weights, gate_up_w, gate_up_b, down_w, down_b, ggml_type, n_experts, H, F,
                           alpha=1.702, limit=7.0):
         """Expert stage of GptOssModel.MoEForward for routed tokens; all tensors on the device."""
-        import torch
+        torch = _torch()
         out = torch.empty((hidden.shape[0], H), dtype=torch.float32, device=hidden.device)
         HipBasicOps.UseCurrentStream()
         ok = N.lib().TSHip_MoEExpertsGptOssForwardF32Device(
@@ -671,7 +684,7 @@ class HipBasicOps:
     @staticmethod
     def LinearForward(m1, qw: QuantizedWeight):
         if qw.is_device:
-            import torch
+            torch = _torch()
             result = torch.empty((m1.shape[0], qw.ne1), dtype=torch.float32, device=m1.device)
             HipBasicOps.UseCurrentStream()
             HipBasicOps.AddmmQuantDevice(result, m1, qw.ptr, qw.ggml_type, qw.ne0, qw.ne1, qw.raw_bytes)
@@ -683,5 +696,10 @@ class HipBasicOps:
     @staticmethod
     def UseCurrentStream():
         """Launch the *Device entry points on torch's current stream."""
-        import torch
-        N.lib().TSHip_SetStream(C.c_void_p(torch.cuda.current_stream().cuda_stream))
+        torch = _torch()
+        raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+        if raw_stream is not None and torch.cuda.is_initialized():
+            handle = raw_stream(torch._C._cuda_getDevice())     # current_stream().cuda_stream without the stream object
+        else:
+            handle = torch.cuda.current_stream().cuda_stream
+        N.lib().TSHip_SetStream(handle)
