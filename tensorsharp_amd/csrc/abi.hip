@@ -898,6 +898,15 @@ const void* resolve_weight_range(void* base, size_t offset, size_t bytes)
     return resolve_weight(static_cast<char*>(base) + offset, bytes);
 }
 
+// Up to this many bytes of activations the conversion kernel reads them over the link from pinned memory, where the packing left
+// them; more reach it sooner through the copy engine (us a call, read / copied, results written the same way: Q4_K 4096 x 4096
+// with 16 rows 46.9 / 54.6, 64 rows - 1 MiB - 111.0 / 118.0, 96 rows 167.3 / 166.0, 128 rows 207.0 / 201.4).
+constexpr size_t kReadPinnedBytes = (size_t)1 << 20;
+// Results of a call of up to this many bytes are stored to pinned memory by the kernels themselves (with the copy engine
+// after them, activations copied in both: 16 rows 62.4 -> 54.6, 256 rows 373.5 -> 364.8); larger calls keep one pinned
+// region for both directions.
+constexpr size_t kStorePinnedBytes = (size_t)32 << 20;
+
 // w_dev_given: the device copy when the caller has resolved the weight already (sub-weights of a stack)
 int addmm_quant_host(const TSHipTensorView2D& result, const TSHipTensorView2D& m1, void* m2_data, int type, int64_t ne0,
                      int64_t ne1, int64_t raw_bytes, const void* w_dev_given = nullptr)
@@ -916,31 +925,38 @@ int addmm_quant_host(const TSHipTensorView2D& result, const TSHipTensorView2D& m
     if (!w_dev) return 0;
     const size_t x_bytes = (size_t)M * K * sizeof(float);
     const size_t y_bytes = (size_t)M * N * sizeof(float);
-    const size_t x_off = 0, y_off = (x_bytes + 255) & ~(size_t)255;
-    if (!ws_reserve(y_off + y_bytes, std::max(x_bytes, y_bytes))) return 0;
-    float* x_dev = reinterpret_cast<float*>(static_cast<char*>(g_ws.dev) + x_off);
-    float* y_dev = reinterpret_cast<float*>(static_cast<char*>(g_ws.dev) + y_off);
+    const size_t y_off = (x_bytes + 255) & ~(size_t)255;
+    // The dense kernels read activations many times; a GEMV's workgroups read them one and all.  What a conversion reads, and
+    // what the GEMV and GEMM kernels store, is touched once.
+    const MatmulPlan plan = plan_matmul(type, M, K, N, false, false);
+    const bool quantized = !is_dense_type(type) && type != kTypeQ8_1 && !plan.narrow;
+    const bool y_pinned = quantized && y_off + y_bytes <= kStorePinnedBytes;
+    const bool x_pinned = y_pinned && !plan.gemv && x_bytes <= kReadPinnedBytes;
+    if (!ws_reserve(x_pinned ? 0 : y_pinned ? x_bytes : y_off + y_bytes, y_pinned ? y_off + y_bytes : std::max(x_bytes, y_bytes))) return 0;
+    float* const x_stage = static_cast<float*>(g_ws.pinned);
+    float* const y_stage = y_pinned ? reinterpret_cast<float*>(static_cast<char*>(g_ws.pinned) + y_off) : x_stage;
+    float* const x_dev = x_pinned ? x_stage : static_cast<float*>(g_ws.dev);
+    float* const y_dev = y_pinned ? y_stage : reinterpret_cast<float*>(static_cast<char*>(g_ws.dev) + y_off);
 
-    // pack the (possibly strided) activation view into pinned memory, then one H2D copy
-    float* stage = static_cast<float*>(g_ws.pinned);
+    // pack the (possibly strided) activation view into pinned memory
     const float* src = static_cast<const float*>(m1.data);
     if (m1.stride1 == 1) {
-        for (int m = 0; m < M; ++m) std::memcpy(stage + (size_t)m * K, src + (size_t)m * m1.stride0, (size_t)K * sizeof(float));
+        for (int m = 0; m < M; ++m) std::memcpy(x_stage + (size_t)m * K, src + (size_t)m * m1.stride0, (size_t)K * sizeof(float));
     } else {
         for (int m = 0; m < M; ++m)
-            for (int64_t k = 0; k < K; ++k) stage[(size_t)m * K + k] = src[(size_t)m * m1.stride0 + (size_t)k * m1.stride1];
+            for (int64_t k = 0; k < K; ++k) x_stage[(size_t)m * K + k] = src[(size_t)m * m1.stride0 + (size_t)k * m1.stride1];
     }
     hipStream_t stream = nullptr;
-    if (!hip_ok(hipMemcpyAsync(x_dev, stage, x_bytes, hipMemcpyHostToDevice, stream), "hipMemcpy(activations)")) return 0;
+    if (!x_pinned && !hip_ok(hipMemcpyAsync(x_dev, x_stage, x_bytes, hipMemcpyHostToDevice, stream), "hipMemcpy(activations)")) return 0;
 
     TSHipTensorView2D r_dev{y_dev, M, (int)N, (int)N, 1, (int64_t)y_bytes};
     TSHipTensorView2D x_desc{x_dev, M, (int)K, (int)K, 1, (int64_t)x_bytes};
     if (!run_matmul_device(r_dev, x_desc, w_dev, type, K, N, stream)) return 0;
 
-    if (!hip_ok(hipMemcpyAsync(stage, y_dev, y_bytes, hipMemcpyDeviceToHost, stream), "hipMemcpy(result)")) return 0;
+    if (!y_pinned && !hip_ok(hipMemcpyAsync(y_stage, y_dev, y_bytes, hipMemcpyDeviceToHost, stream), "hipMemcpy(result)")) return 0;
     if (!hip_ok(hipStreamSynchronize(stream), "hipStreamSynchronize")) return 0;
     float* dst = static_cast<float*>(result.data);
-    for (int m = 0; m < M; ++m) std::memcpy(dst + (size_t)m * result.stride0, stage + (size_t)m * N, (size_t)N * sizeof(float));
+    for (int m = 0; m < M; ++m) std::memcpy(dst + (size_t)m * result.stride0, y_stage + (size_t)m * N, (size_t)N * sizeof(float));
     clear_last_error();
     return 1;
 }

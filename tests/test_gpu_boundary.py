@@ -179,3 +179,32 @@ def test_device_gather_of_more_than_65535_indices(hip, oracle):
     torch.cuda.synchronize()
     deq = oracle.dequantize(Q8_0, wq).reshape(N, K)
     assert np.array_equal(out.cpu().numpy().view(np.uint32), deq[idx].view(np.uint32))
+
+
+@pytest.mark.parametrize("name,M,N,K", [
+    ("q8_0", 1, 1001, 96), ("mxfp4", 3, 333, 2592),      # GEMV: copied activations, results stored to pinned memory
+    ("q8_0", 5, 1001, 96), ("q4_k", 64, 515, 4096),       # read from pinned memory: the smallest, exactly 1 MiB
+    ("q4_k", 65, 515, 4096),                              # copied
+    ("q8_0", 8, 40, 256),                                 # narrow: the dense kernel
+    ("mxfp4", 580, 14500, 256),                           # results beyond 32 MiB: copied both ways
+])
+def test_host_call_stages_as_the_device_call(hip, oracle, name, M, N, K):
+    """A linear on host tensors gives the bytes of the same linear on device tensors, whichever way its activations and results
+    cross the link; rows of a wider array, twice with other activations (the staging memory is kept)."""
+    import torch
+    from oracle.oracle import MXFP4, Q4_K, Q8_0
+    from tensorsharp_amd import QuantizedWeight, synth
+    t = {"q8_0": Q8_0, "q4_k": Q4_K, "mxfp4": MXFP4}[name]
+    wd = synth.random_weight(t, N, K, "cuda", M + N)
+    wh = wd.cpu().numpy()
+    rng = np.random.default_rng(M + K)
+    try:
+        for _ in range(2):
+            x = rng.standard_normal((M, K + 8)).astype(np.float32)
+            out = np.full((M, N + 3), 7.0, dtype=np.float32)
+            hip.AddmmQuant(out[:, :N], x[:, 4:K + 4], wh.ctypes.data, t, K, N, wh.size)
+            ref = hip.LinearForward(torch.from_numpy(np.ascontiguousarray(x[:, 4:K + 4])).cuda(), QuantizedWeight(wd, t, K, N))
+            assert np.array_equal(out[:, :N], ref.cpu().numpy())
+            assert (out[:, N:] == 7.0).all()
+    finally:
+        hip.InvalidateHostBuffer(wh.ctypes.data)
