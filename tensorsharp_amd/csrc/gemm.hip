@@ -1667,12 +1667,14 @@ constexpr int kWideValu = (40 + 2 * TM - 1) / (2 * TM);
 // block's 144 bytes per k-tile and takes two lines per row for them, by the counters 73 KB per 128 x 256 x 64 step (92 KB per
 // 256 x 256 x 64) at 50 (43) GB/s per CU; here a row's whole granule is copied at once: 37 KB per 128 x 256 x 64 step.  What
 // bounds it now: of Q4_K 512 x 14336 x 4096 (77.6 us) the matrix pipe is busy 34 % of the cycles, 8 vector instructions
-// stand beside each matrix instruction, wavefronts wait 35 % of their time; Q6_K (333 x 4096 x 14336) has 16 vector
-// instructions per matrix instruction and bank conflicts in 62 % of its LDS cycles (dword reads of 210-byte blocks).
+// stand beside each matrix instruction, wavefronts wait 35 % of their time; Q6_K (333 x 4096 x 14336) had 16 vector
+// instructions per matrix instruction and bank conflicts in 62 % of its LDS cycles (dword reads of 210-byte blocks): its loop,
+// with the addresses and shifts of a block worked out once for its four k-tiles, has 8.
 // Measured, whole call, us (the best of the other kernels -> this one):
 //   Q4_K 512 x 14336 x 4096 82.2 -> 75.8, 333 x 4096 x 14336 75.8 -> 68.1, 200 x 4096 x 14336 69.7 -> 49.7, 200 x 4096 x 4096 32.2 -> 28.3
 //   Q8_0 512 x 14336 x 4096 87.4 -> 80.4, 200 x 4096 x 14336 77.7 -> 52.6, 48 x 21504 x 5376 56.1 -> 45.5
-//   Q6_K 333 x 4096 x 14336 100.3 -> 94.5, 200 x 4096 x 14336 95.7 -> 64.1, 200 x 21504 x 5376 141.2 -> 125.5
+//   Q6_K 333 x 4096 x 14336 100.3 -> 94.5, 200 x 4096 x 14336 95.7 -> 64.1, 200 x 21504 x 5376 141.2 -> 125.5;
+//        with the unrolled loop 333 x 4096 x 14336 80.9, FFN of 200 rows with a Q6_K down projection 185.7 -> 177.4
 // ------------------------------------------------------------------------------------------
 // Weight formats as this kernel reads them.  A granule is the raw bytes of kSup consecutive k-tiles of one row, kept in LDS
 // as kRawRow bytes (an odd multiple of four dwords: the dword reads of 32 rows spread over the most banks that 16-byte
@@ -1763,44 +1765,63 @@ struct WQ80 {
         }
     }
 };
-// Q6_K: a granule is a block (210 bytes, even delta: fourteen pieces)
+// Q6_K: a granule is a block (210 bytes, even delta: fourteen pieces).  The loop over its four k-tiles is unrolled, so what depends
+// on where the block lies (Row) is worked out once for it and the reads have constant offsets (229 vector instructions per k-tile
+// of 128 rows before, 119 now); the two quarters of a wavefront are one read of five dwords each of low and of high bits.
 struct WQ6K {
     typedef GQ6K G;
-    static constexpr int kSup = 4, kRawRow = 240, kPieces = 14, kHdr = 2, kState = 1, kQ = 6;
+    static constexpr int kSup = 4, kRawRow = 240, kPieces = 14;
     static constexpr bool kSplit = true, kAligned = false;
     static __device__ __forceinline__ uint32_t part_off(int s) { return (uint32_t)s * 210u; }
-    static __device__ __forceinline__ void fetch_hdr(const uint8_t* rp, int j, int h, uint32_t d, uint32_t (&r)[kHdr])
+    struct Row {
+        const uint8_t *lo, *hi, *sc;         // dwords that hold the low bits, the high bits and the scale of k-tile 0
+        uint32_t shift_lo, shift_hi, shift_sc;
+    };
+    struct Raw {
+        uint32_t lo[5], hi[5], sc;
+    };
+    // half: which two quarters the wavefront takes.  (Rows 32 apart, 64 times as many bytes as half words, lie alike in their
+    // pieces: a Row serves both columns of a lane, `off` bytes on.)
+    static __device__ __forceinline__ void open(Row& r, const uint8_t* rp, uint32_t d, int h, int half)
     {
-        r[0] = *reinterpret_cast<const uint32_t*>(rp + ((d + 192u + 4u * j + 2u * h) & ~3u));
-        r[1] = *reinterpret_cast<const uint32_t*>(rp + ((d + 208u) & ~3u));
+        const uint32_t odd = d & 2u, at = odd + 2u * (uint32_t)h;
+        const uint8_t* const p = rp + (d & ~3u);
+        r.lo = p + 32 * h + 16 * half;
+        r.hi = p + 128 + 16 * half;
+        r.sc = p + 192 + (at & 4u);
+        r.shift_lo = 8u * odd;
+        r.shift_hi = 8u * odd + 2u * (uint32_t)h;
+        r.shift_sc = 8u * (at & 2u) + 8u * (uint32_t)half;
     }
-    static __device__ __forceinline__ void prepare(const uint32_t (&r)[kHdr], int, int h, uint32_t d, bool live, int half, uint32_t (&st)[kState], uint32_t& bad)
+    static __device__ __forceinline__ uint32_t fetch_d(const uint8_t* rp, uint32_t d) { return *reinterpret_cast<const uint32_t*>(rp + (d & ~3u) + 208); }
+    static __device__ __forceinline__ float scale(uint32_t dword, uint32_t shift_lo, bool live, uint32_t& bad)
     {
-        const float sc = (float)(int)(int8_t)(r[0] >> (((d + 2u * h) & 2u) * 8u + 8u * half));
         H2U dd;
-        dd.u = (r[1] >> ((d & 2u) * 8u)) & (live ? 0xffffu : 0u);
+        dd.u = (dword >> shift_lo) & (live ? 0xffffu : 0u);
         mark2(bad, dd.u);
-        st[0] = splat((float)dd.h.x * kWUp * sc);
+        return (float)dd.h.x * kWUp;
     }
-    static __device__ __forceinline__ void fetch(const uint8_t* rp, int j, int h, uint32_t d, int q, uint32_t (&r)[kQ])
+    static __device__ __forceinline__ void fetch(const Row& r, int off, int j, Raw& w)
     {
-        const uint8_t* const base = rp + (d & ~3u) + 8 * q;
-        const uint32_t* a = reinterpret_cast<const uint32_t*>(base + 64 * (j >> 1) + 32 * h);
-        const uint32_t* b = reinterpret_cast<const uint32_t*>(base + 128 + 32 * (j >> 1));
+        const uint32_t* a = reinterpret_cast<const uint32_t*>(r.lo + off + 64 * (j >> 1));
+        const uint32_t* b = reinterpret_cast<const uint32_t*>(r.hi + off + 32 * (j >> 1));
 #pragma unroll
-        for (int i = 0; i < 3; ++i) {
-            r[i] = a[i];
-            r[3 + i] = b[i];
+        for (int i = 0; i < 5; ++i) {
+            w.lo[i] = a[i];
+            w.hi[i] = b[i];
         }
+        w.sc = *reinterpret_cast<const uint32_t*>(r.sc + off + 4 * j);
     }
-    static __device__ __forceinline__ void unpack(const uint32_t (&r)[kQ], const uint32_t (&st)[kState], int j, int h, uint32_t d, int, uint32_t (&o)[4])
+    static __device__ __forceinline__ uint32_t prepare(const Row& r, float d, const Raw& w) { return splat(d * (float)(int)(int8_t)(w.sc >> r.shift_sc)); }
+    // quarter q (0, 1) of the wavefront's two of k-tile j
+    static __device__ __forceinline__ void unpack(const Raw& w, uint32_t shift_lo, uint32_t shift_hi, uint32_t sc, int j, int q, uint32_t* o)
     {
-        const uint32_t sh = d & 2u, sc = st[0];
         const uint32_t bias = 0xe420e420u;               // -(1024 + 32)
+        const uint32_t nibble = 4u * (uint32_t)(j & 1);
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
-            const uint32_t ql = __builtin_amdgcn_alignbyte(r[i + 1], r[i], sh) >> (4 * (j & 1));
-            const uint32_t qh = __builtin_amdgcn_alignbyte(r[4 + i], r[3 + i], sh) >> (4 * (j & 1) + 2 * h);
+            const uint32_t ql = __builtin_amdgcn_alignbit(w.lo[2 * q + i + 1], w.lo[2 * q + i], shift_lo + nibble);
+            const uint32_t qh = __builtin_amdgcn_alignbit(w.hi[2 * q + i + 1], w.hi[2 * q + i], shift_hi + nibble);
             const uint32_t q6 = (ql & 0x0f0f0f0fu) | ((qh & 0x03030303u) << 4);
             // bytes u = q become fp16 1024 + u; minus 1056 leaves q - 32 exactly
             o[2 * i] = pk_mul(pk_add(__builtin_amdgcn_perm(0x64646464u, q6, 0x04010400u), bias), sc);
@@ -1868,7 +1889,7 @@ __global__ void __launch_bounds__(512) gemm_wide_kernel(const GemmArgs A)
     const int nkt = min(A.Kp / kBK, kt_begin + A.chunk_kt);            // end of this unit's K range
 
     // per-lane source offsets of the LDS-direct copies
-    uint32_t x_off[XI], w_row[WI], w_piece[WI];
+    uint32_t x_off[XI], w_off[WI];
 #pragma unroll
     for (int i = 0; i < XI; ++i) {
         const int q = (wave + 8 * i) * 64 + lane;            // LDS chunk slot: k-tile, row, position q % 8
@@ -1880,8 +1901,7 @@ __global__ void __launch_bounds__(512) gemm_wide_kernel(const GemmArgs A)
         const int c = (wave + 8 * i) * 64 + lane;
         const int row = c / kRowPieces, piece = c - row * kRowPieces;
         const bool ok = row < BN && n0 + row < A.N && piece < H::kPieces;
-        w_row[i] = ok ? base_delta + (uint32_t)(n0 + row) * row_bytes + (H::kAligned ? 16u * (uint32_t)piece : 0u) : kDeadOffset;
-        w_piece[i] = (uint32_t)piece * 16u;
+        w_off[i] = ok ? base_delta + (uint32_t)(n0 + row) * row_bytes + 16u * (uint32_t)piece : kDeadOffset;
     }
     // k-tiles past the end: the offset gets its top bit set (out of range: zeros arrive)
     typedef __attribute__((address_space(3))) uint8_t* lds_ptr;
@@ -1905,9 +1925,9 @@ __global__ void __launch_bounds__(512) gemm_wide_kernel(const GemmArgs A)
             const int id = wave + 8 * i;
             const lds_ptr dst = lds + (8 * i + 8 <= WN || id < WN ? 2 * L::kXStage + (s & 1) * RT + id * 1024 : L::kBuf);
             if constexpr (H::kAligned) {
-                copy(wrs, dst, w_row[i] | past, H::part_off(s));
+                copy(wrs, dst, w_off[i] | past, H::part_off(s));
             } else {
-                copy(wrs, dst, (((w_row[i] + H::part_off(s)) & ~15u) + w_piece[i]) | past, 0u);
+                copy(wrs, dst, ((w_off[i] + H::part_off(s)) & ~15u) | past, 0u);
             }
         }
     };
@@ -1916,6 +1936,7 @@ __global__ void __launch_bounds__(512) gemm_wide_kernel(const GemmArgs A)
     // this lane's weight rows for the matrix pipe
     const int raw0 = (wn * (32 * NB) + col) * kRawRow;
     const int my_n0 = n0 + wn * (32 * NB) + col;
+    const uint32_t my_row0 = base_delta + (uint32_t)my_n0 * row_bytes;
     uint32_t my_row[NB], bad[NB];
     bool in_n[NB];
 #pragma unroll
@@ -1945,33 +1966,7 @@ __global__ void __launch_bounds__(512) gemm_wide_kernel(const GemmArgs A)
     // raw bytes and scales of k-tile kt; its granule, its place in it and the granule's position inside the copied pieces
     auto row_of = [&](int s, int n) { return rbuf + (s & 1) * RT + raw0 + n * 32 * kRawRow; };
     auto delta_of = [&](int s, int n) { return H::kAligned ? 0u : (my_row[n] + H::part_off(s)) & 15u; };
-    uint32_t o[NB][16], hdr[NB][H::kHdr], state[NB][H::kState];
-    auto fetch_hdr = [&](int kt) {
-        const int s = kt / H::kSup, j = kt % H::kSup;
-#pragma unroll
-        for (int n = 0; n < NB; ++n) H::fetch_hdr(row_of(s, n), j, h, delta_of(s, n), hdr[n]);
-    };
-    auto fetch = [&](int kt, int q, uint32_t (&r)[NB][H::kQ]) {
-        const int s = kt / H::kSup, j = kt % H::kSup;
-#pragma unroll
-        for (int n = 0; n < NB; ++n) H::fetch(row_of(s, n), j, h, delta_of(s, n), q, r[n]);
-    };
-    auto prepare = [&](int kt) {
-        const int s = kt / H::kSup, j = kt % H::kSup;
-        const bool live_k = (kt < nkt) & ((kt * 2 + h) * 32 < A.K);      // past the unit's end the raw bytes are zeros or stale
-#pragma unroll
-        for (int n = 0; n < NB; ++n) H::prepare(hdr[n], j, h, delta_of(s, n), live_k & in_n[n], g, state[n], bad[n]);
-    };
-    auto unpack = [&](int kt, int q, int slot, uint32_t (&r)[NB][H::kQ]) {
-        const int s = kt / H::kSup, j = kt % H::kSup;
-#pragma unroll
-        for (int n = 0; n < NB; ++n) {
-            uint32_t v[4];
-            H::unpack(r[n], state[n], j, h, delta_of(s, n), q, v);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) o[n][4 * slot + i] = v[i];
-        }
-    };
+    uint32_t o[NB][16];
     auto mfma = [&](const half8_t (&a)[TM], int ks) {
 #pragma unroll
         for (int i = 0; i < TM; ++i)
@@ -1997,50 +1992,103 @@ __global__ void __launch_bounds__(512) gemm_wide_kernel(const GemmArgs A)
     issue_w(s_begin + 1);
     issue_x(kt_begin + KT);
     wait_copies_and_barrier<0>();
-    uint32_t ra[NB][H::kQ], rb[NB][H::kQ];
     half8_t a0[TM], a1[TM];
     if constexpr (H::kSplit) {
         // One k-tile a turn, two of its k-steps per group.  As below, with the weights of a k-step unpacked two k-steps ahead.
-        fetch_hdr(kt_begin);
-        prepare(kt_begin);
-        fetch(kt_begin, 2 * g, ra);
-        unpack(kt_begin, 2 * g, 0, ra);
-        fetch(kt_begin, 2 * g + 1, rb);
+        // K is whole granules; a granule's turns are unrolled.
+        constexpr int kNext = 32 * kRawRow;              // bytes from a column's raw row to its next one's
+        typename H::Row row;
+        typename H::Raw raw[2][NB];
+        uint32_t dword[NB], sc[NB];
+        float d[NB];
+        auto open = [&](int s) {
+            const uint32_t delta = (my_row0 + H::part_off(s)) & 15u;
+            H::open(row, row_of(s, 0), delta, h, g);
+#pragma unroll
+            for (int n = 0; n < NB; ++n) dword[n] = H::fetch_d(row_of(s, n), delta);
+        };
+        auto unpack_q = [&](int j, int q, const typename H::Raw (&w)[NB], uint32_t sl, uint32_t sh) {
+#pragma unroll
+            for (int n = 0; n < NB; ++n) H::unpack(w[n], sl, sh, sc[n], j, q, &o[n][4 * q]);
+        };
+        open(s_begin);
+        uint32_t shift_lo = row.shift_lo, shift_hi = row.shift_hi;      // of the k-tile whose second quarter is still to be unpacked
+#pragma unroll
+        for (int n = 0; n < NB; ++n) {
+            H::fetch(row, n * kNext, 0, raw[0][n]);
+            d[n] = H::scale(dword[n], row.shift_lo, in_n[n], bad[n]);
+            sc[n] = H::prepare(row, d[n], raw[0][n]);
+        }
+        unpack_q(0, 0, raw[0], shift_lo, shift_hi);
         load_a(kt_begin, 0, a0);
-        for (int kt = kt_begin; kt < nkt; ++kt) {
-            uint32_t rc[NB][H::kQ];
-            load_a(kt, 1, a1);
-            fetch_hdr(kt + 1);
-            fetch(kt + 1, 2 * g, ra);
-            fetch(kt + 1, 2 * g + 1, rc);
-            __builtin_amdgcn_sched_barrier(0);
-            mfma(a0, 0);
-            unpack(kt, 2 * g + 1, 1, rb);
-            interleave();
+        for (int s = s_begin; s * 4 < nkt; ++s) {
 #pragma unroll
-            for (int n = 0; n < NB; ++n)
+            for (int j = 0; j < 4; ++j) {
+                const int kt = 4 * s + j, next = (j + 1) & 3;
+                load_a(kt, 1, a1);
+                if (next == 0) open(s + 1);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(o[n][4 + i]));     // (unpacked here, not where they are used)
-            // the granule requested in the last turn may be in flight: its first k-tile is read three turns later
-            if ((kt & 3) == 3)
-                asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(WI) : "memory");
-            else
-                asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-            asm volatile("s_barrier" ::: "memory");
-            load_a(kt + 1, 0, a0);
-            issue_x(kt + 2);
-            if ((kt & 3) == 2) issue_w(kt / 4 + 2);
-            __builtin_amdgcn_sched_barrier(0);
-            mfma(a1, 1);
-            prepare(kt + 1);
-            unpack(kt + 1, 2 * g, 0, ra);
-            interleave();
+                for (int n = 0; n < NB; ++n) H::fetch(row, n * kNext, next, raw[next & 1][n]);
+                __builtin_amdgcn_sched_barrier(0);
+                mfma(a0, 0);
+                unpack_q(j, 1, raw[j & 1], shift_lo, shift_hi);
+                interleave();
 #pragma unroll
-            for (int n = 0; n < NB; ++n)
+                for (int n = 0; n < NB; ++n)
 #pragma unroll
-                for (int i = 0; i < H::kQ; ++i) rb[n][i] = rc[n][i];
+                    for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(o[n][4 + i]));     // (unpacked here, not where they are used)
+                // the granule requested in the last turn may be in flight: its first k-tile is read three turns later
+                if (j == 3)
+                    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(WI) : "memory");
+                else
+                    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+                asm volatile("s_barrier" ::: "memory");
+                load_a(kt + 1, 0, a0);
+                issue_x(kt + 2);
+                if (j == 2) issue_w(s + 2);
+                __builtin_amdgcn_sched_barrier(0);
+                mfma(a1, 1);
+                if (next == 0) {
+                    shift_lo = row.shift_lo;
+                    shift_hi = row.shift_hi;
+                }
+#pragma unroll
+                for (int n = 0; n < NB; ++n) {
+                    if (next == 0) d[n] = H::scale(dword[n], shift_lo, in_n[n] && 4 * (s + 1) < nkt, bad[n]);
+                    sc[n] = H::prepare(row, d[n], raw[next & 1][n]);
+                }
+                unpack_q(next, 0, raw[next & 1], shift_lo, shift_hi);
+                interleave();
+            }
         }
     } else {
+        uint32_t ra[NB][H::kQ], rb[NB][H::kQ], hdr[NB][H::kHdr], state[NB][H::kState];
+        auto fetch_hdr = [&](int kt) {
+            const int s = kt / H::kSup, j = kt % H::kSup;
+    #pragma unroll
+            for (int n = 0; n < NB; ++n) H::fetch_hdr(row_of(s, n), j, h, delta_of(s, n), hdr[n]);
+        };
+        auto fetch = [&](int kt, int q, uint32_t (&r)[NB][H::kQ]) {
+            const int s = kt / H::kSup, j = kt % H::kSup;
+    #pragma unroll
+            for (int n = 0; n < NB; ++n) H::fetch(row_of(s, n), j, h, delta_of(s, n), q, r[n]);
+        };
+        auto prepare = [&](int kt) {
+            const int s = kt / H::kSup, j = kt % H::kSup;
+            const bool live_k = (kt < nkt) & ((kt * 2 + h) * 32 < A.K);      // past the unit's end the raw bytes are zeros or stale
+    #pragma unroll
+            for (int n = 0; n < NB; ++n) H::prepare(hdr[n], j, h, delta_of(s, n), live_k & in_n[n], g, state[n], bad[n]);
+        };
+        auto unpack = [&](int kt, int q, int slot, uint32_t (&r)[NB][H::kQ]) {
+            const int s = kt / H::kSup, j = kt % H::kSup;
+    #pragma unroll
+            for (int n = 0; n < NB; ++n) {
+                uint32_t v[4];
+                H::unpack(r[n], state[n], j, h, delta_of(s, n), q, v);
+    #pragma unroll
+                for (int i = 0; i < 4; ++i) o[n][4 * slot + i] = v[i];
+            }
+        };
         fetch_hdr(kt_begin + g);
         prepare(kt_begin + g);
 #pragma unroll
