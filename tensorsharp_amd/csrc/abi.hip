@@ -321,6 +321,7 @@ constexpr int kNarrowColumns = 64;
 struct MatmulPlan {
     bool gemv;            // decode / tiny batch: one bandwidth-bound GEMV per activation row
     bool narrow;          // few result columns: fp32 copy of the weight + the dense kernel
+    bool converts;        // prefill: activations converted to the workspace, then the GEMM (neither of the above, no dense weight)
     int m_step;           // activation rows per launch
     int64_t n_step;       // weight rows per launch
     GemmPlan gemm;        // prefill: how a launch over a whole slice runs
@@ -367,6 +368,7 @@ MatmulPlan plan_matmul(int type, int M, int64_t K, int64_t N, bool norm, bool ac
         p.conv_bytes = norm && K > gemv_rms_max_k() ? al((size_t)M * (size_t)K * sizeof(float)) : 0;
         return p;
     }
+    p.converts = true;
     const size_t kp = (size_t)((K + 63) / 64) * 64;
     p.m_step = (int)std::min<int64_t>(M, std::max<int64_t>(256, ((kMaxOperandBytes - 1) / (int64_t)(kp * 2)) / 256 * 256));
     p.conv_bytes = al(gemm_workspace_bytes(p.m_step, (int)K));
@@ -387,9 +389,11 @@ MatmulPlan plan_matmul(int type, int M, int64_t K, int64_t N, bool norm, bool ac
 }
 
 // result (+)= f(m1) * W^T with f = identity or RMSNorm(eps) * norm_w, as `plan` (of the same call) says.  All pointers are
-// device pointers; `ws` has ws_bytes >= plan.total() bytes.
+// device pointers; `ws` has ws_bytes >= plan.total() bytes.  silu (calls that convert their activations only): the rows of m1 are
+// (gate | up) of 2 K floats, f(m1) = silu(gate) * up.
 bool run_matmul_device_ws(const MatmulPlan& plan, const TSHipTensorView2D& result, const TSHipTensorView2D& m1, const void* w, int type,
-                          int64_t K, int64_t N, hipStream_t stream, void* ws, size_t ws_bytes, const float* norm_w, float eps, bool accumulate)
+                          int64_t K, int64_t N, hipStream_t stream, void* ws, size_t ws_bytes, const float* norm_w, float eps, bool accumulate,
+                          bool silu = false)
 {
     const size_t rs = row_size(type, K);
     if (!check_device_operands(m1, w, type)) return false;
@@ -457,7 +461,7 @@ bool run_matmul_device_ws(const MatmulPlan& plan, const TSHipTensorView2D& resul
             const bool whole = m == plan.m_step && n == std::min<int64_t>(N, plan.n_step);
             const GemmPlan g = whole ? plan.gemm : plan_gemm(type, m, (int)n, (int)K, accumulate, chunk_bytes);
             if (g.x_layout != converted) {
-                if (!launch_convert_x(type, x, m1.stride0, nullptr, m, (int)K, ws, stream, norm_w, eps, g.x_layout)) return false;
+                if (!launch_convert_x(type, x, m1.stride0, nullptr, m, (int)K, ws, stream, norm_w, eps, g.x_layout, silu)) return false;
                 converted = g.x_layout;
             }
             if (!launch_gemm(type, g, wb + (size_t)n0 * rs, (int64_t)(rs * (size_t)n), ws, out + (int64_t)m0 * result.stride0 + n0,
@@ -562,6 +566,10 @@ bool run_ffn_swiglu_device(const FfnPlan& plan, const TSHipTensorView2D& residua
     }
     const TSHipTensorView2D gu_view{gu, M, 2 * half, 2 * half, 1, (int64_t)((size_t)M * 2 * half * sizeof(float))};
     if (!run_matmul_device_ws(plan.gu, gu_view, input, gate_up, gu_type, hidden, 2 * half, stream, mm_ws, mm_bytes, norm_w, eps, false)) return false;
+    if (plan.dn.converts && M <= 65535) {              // (more rows are refused below)
+        const TSHipTensorView2D gate_view{gu, M, half, 2 * half, 1, gu_view.raw_bytes};
+        return run_matmul_device_ws(plan.dn, residual, gate_view, down, dn_type, half, hidden, stream, mm_ws, mm_bytes, nullptr, 0.f, true, true);
+    }
     if (!launch_silu_mul(gu, 2 * half, M, half, act, stream)) return false;
     const TSHipTensorView2D act_view{act, M, half, half, 1, (int64_t)((size_t)M * half * sizeof(float))};
     return run_matmul_device_ws(plan.dn, residual, act_view, down, dn_type, half, hidden, stream, mm_ws, mm_bytes, nullptr, 0.f, true);
@@ -686,14 +694,14 @@ ExpertSetLayout expert_set_layout(int M, int n, const ExpertFfn* ex, int H, int 
 }
 
 // One linear of a tiled expert set: per block type one tile-table GEMM over the members whose weight has that type.
-// x: fp32 source rows (ldx), gathered through row_map when given; the members' results go to rows slot * M .. of c.
+// x: fp32 source rows (ldx; silu: (gate | up) rows of 2 K floats), gathered through row_map when given; the members' results go to rows slot * M .. of c.
 struct ExpertLinear {
     const void* w[kMaxExpertSet];
     int type[kMaxExpertSet];
 };
 
 bool run_expert_linear_tiled(const ExpertSetLayout& L, char* ws, int n, int M, const ExpertLinear& lin, const float* x, int64_t ldx,
-                             bool gather, size_t x_off, float* c, int64_t ldc, int out_features, int K, hipStream_t stream)
+                             bool gather, size_t x_off, float* c, int64_t ldc, int out_features, int K, hipStream_t stream, bool silu = false)
 {
     auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
     const int per = (M + L.bm - 1) / L.bm;
@@ -722,7 +730,7 @@ bool run_expert_linear_tiled(const ExpertSetLayout& L, char* ws, int n, int M, c
         }
         const int layout = expert_tiles_x_layout(t, L.bm, K, out_features);
         if (!launch_expert_tiles(spec, M, L.bm, t_expert, t_row0, t_rows, offs, gather ? row_map : nullptr, rows, stream)) return false;
-        if (!launch_convert_x(t, x, ldx, gather ? row_map : nullptr, rows, K, ws + x_off, stream, nullptr, 0.f, layout)) return false;
+        if (!launch_convert_x(t, x, ldx, gather ? row_map : nullptr, rows, K, ws + x_off, stream, nullptr, 0.f, layout, silu)) return false;
         GemmTiles tiles{t_expert, t_row0, t_rows, spec.count * per, L.bm, (int64_t)(row_size(t, K) * (size_t)out_features)};
         tiles.expert_off = offs;
         if (!launch_gemm_tiles(t, tiles, reinterpret_cast<const void*>(base), tiles.expert_stride, ws + x_off, c, ldc, nullptr, rows,
@@ -817,15 +825,9 @@ bool run_expert_set_device(const TSHipTensorView2D& out, const float* base, int6
         }
         for (int e = 0; e < n; ++e) lin.w[e] = ex[e].up, lin.type[e] = ex[e].up_type;
         if (!run_expert_linear_tiled(L, ws, n, M, lin, xv, x.stride0, true, L.x1_off, gated ? act + I : act, ld, I, H, stream)) return false;
-        const float* rows_in = act;
-        if (gated) {
-            if (!launch_silu_mul(act, ld, n * M, I, tmp, stream)) return false;
-            rows_in = tmp;
-        } else if (!launch_relu_sqr(act, (int64_t)n * M * I, stream)) {
-            return false;
-        }
+        if (!gated && !launch_relu_sqr(act, (int64_t)n * M * I, stream)) return false;
         for (int e = 0; e < n; ++e) lin.w[e] = ex[e].down, lin.type[e] = ex[e].down_type;
-        if (!run_expert_linear_tiled(L, ws, n, M, lin, rows_in, I, false, L.x2_off, dn, N, N, I, stream)) return false;
+        if (!run_expert_linear_tiled(L, ws, n, M, lin, act, ld, false, L.x2_off, dn, N, N, I, stream, gated)) return false;
     } else {
         ExpertLinearPlan gate_plan, up_plan, down_plan;
         auto linear = [&](const MatmulPlan& plan, const TSHipTensorView2D& y, const TSHipTensorView2D& v, const void* w, int type, int64_t wk, int64_t wn) {

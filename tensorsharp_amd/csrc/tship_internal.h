@@ -163,9 +163,10 @@ GemmPlan plan_gemm(int type, int M, int N, int K, bool accumulate, size_t max_ch
 // fp32 activations -> workspace (fp16 in the weight format's unpack order + per-row scales);
 // row_map (device, optional) gathers source rows.
 // norm_w (device, optional) applies RMSNorm first: x <- x / sqrt(mean(x^2) + eps) * norm_w.
+// silu: the rows are (gate | up) of 2 K floats and the activations silu(gate) * up (no norm_w then).
 // layout: see GemmPlan::x_layout.
 bool launch_convert_x(int type, const float* x, int64_t ldx, const int* row_map, int M, int K, void* workspace,
-                      hipStream_t stream, const float* norm_w = nullptr, float eps = 0.f, int layout = 0);
+                      hipStream_t stream, const float* norm_w = nullptr, float eps = 0.f, int layout = 0, bool silu = false);
 // The same for the activations of an expert's down projection: row m is SwiGLU-OAI of (gate | up)[m] (+ the bias
 // row of expert_of[m]), formed while it is read.
 bool launch_convert_x_swiglu(int type, const float* gate_up, const float* bias, const int* expert_of, float alpha, float limit,

@@ -260,3 +260,34 @@ def test_ffn_decode_paired_store_every_gemv_format(hip, oracle, gu_type, M):
     torch.cuda.synchronize()
     tol = 2e-3 * np.linalg.norm(mm, axis=1, keepdims=True)
     assert np.all(np.abs(r.cpu().numpy() - (resid + mm)) <= tol), (gu_type, M)
+
+
+@pytest.mark.parametrize("down,H,F", [
+    ("q8_0", 192, 96),            # natural order; half a k-tile past the end of K
+    ("q4_k", 256, 512), ("q6_k", 256, 256), ("mxfp4", 256, 160),
+    ("q8_0", 128, 32768 + 96),    # rows longer than the conversion holds in registers
+    ("mxfp4", 32768, 2048),       # 64 M weights: the MX fp6 pairs
+])
+@pytest.mark.parametrize("M", [4, 33])
+def test_gated_rows_are_formed_by_the_conversion(hip, down, H, F, M):
+    """The down projection of several rows converts silu(gate) * up as it reads [gate | up].  Against the same products one by
+    one with the gated rows formed by torch in between: its exponential may differ in the last bit and move an activation by
+    one rounding of its 16-bit (MX: 10-bit block) form, at most 2^-10 of it, so no row by more than that."""
+    import torch
+    from oracle.oracle import Q6_K
+    from tensorsharp_amd import QuantizedWeight, synth
+    t = dict(T_, q6_k=Q6_K)[down]
+    gu = QuantizedWeight(synth.random_weight(Q8_0, 2 * F, H, "cuda", 3), Q8_0, H, 2 * F)
+    dn = QuantizedWeight(synth.random_weight(t, H, F, "cuda", 4), t, F, H)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(M + F)
+    x = torch.randn((M, H), generator=g, device="cuda")
+    nw = torch.rand(H, generator=g, device="cuda") + 0.5
+    got = torch.zeros((M, H), device="cuda")
+    hip.FusedFFNSwiGLUQuant(got, x, nw, EPS, gu, dn, F)
+    both = torch.empty((M, 2 * F), device="cuda")
+    hip.FusedRmsNormMatMulQuant(both, x, nw, EPS, gu)
+    gate, up = both[:, :F], both[:, F:]
+    ref = hip.LinearForward(((gate / (1.0 + torch.exp(-gate))) * up).contiguous(), dn)
+    err = (got.double() - ref.double()).norm(dim=1) / ref.double().norm(dim=1)
+    assert float(err.max()) <= 2.0 ** -10, (down, H, F, M, float(err.max()))
