@@ -111,10 +111,16 @@ __device__ __forceinline__ float dot2(uint32_t a, uint32_t b, float acc)
 {
     return __builtin_amdgcn_fdot2(as_half2(a), as_half2(b), acc, false);
 }
+// bytes 0, 2 and 1, 3 as the low bytes of two halves
+__device__ __forceinline__ uint32_t even_bytes(uint32_t v) { return __builtin_amdgcn_perm(0u, v, 0x0c020c00u); }
+__device__ __forceinline__ uint32_t odd_bytes(uint32_t v) { return __builtin_amdgcn_perm(0u, v, 0x0c030c01u); }
 
+#define TSHIP_DPP_U(v, ctrl) ((uint32_t)__builtin_amdgcn_update_dpp(0, (int)(v), ctrl, 0xf, 0xf, true))
 #define TSHIP_DPP_F(v, ctrl) __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), ctrl, 0xf, 0xf, true))
 constexpr int kDppXor1 = 0xb1;         // quad_perm [1,0,3,2]
 constexpr int kDppXor2 = 0x4e;         // quad_perm [2,3,0,1]
+constexpr int kDppNext = 0x39;         // quad_perm [1,2,3,0]
+constexpr int kDppThird = 0xaa;        // quad_perm [2,2,2,2]
 constexpr int kDppHalfMirror = 0x141;  // lane i <-> 7-i inside each 8
 constexpr int kDppMirror = 0x140;      // lane i <-> 15-i inside each 16
 
@@ -326,17 +332,20 @@ struct FmtQ5K : FmtQ4K {
     {
         const uint4* xu = reinterpret_cast<const uint4*>(xu_dw);
         float lo = 0.f, hi = 0.f;
-        constexpr uint32_t kNib = 0x000f000fu, kFifth = 0x00100010u;
+        constexpr uint32_t kNib = 0x0f0f0f0fu, kFifth = 0x10101010u;
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
             const uint4 xv = xu[j];
             const uint32_t q = w[12 + j];
             const uint32_t h = w[4 + j] >> L.hsh;      // bit 0 of every byte: low-nibble weight, bit 1: high-nibble weight
-            // a 5-bit value left in the low bits of an fp16 is the subnormal v * 2^-24
-            lo = dot2((q & kNib) | ((h << 4) & kFifth), xv.x, lo);
-            lo = dot2(((q >> 8) & kNib) | ((h >> 4) & kFifth), xv.y, lo);
-            hi = dot2(((q >> 4) & kNib) | ((h << 3) & kFifth), xv.z, hi);
-            hi = dot2(((q >> 12) & kNib) | ((h >> 5) & kFifth), xv.w, hi);
+            // four values put together as bytes, then the even and the odd ones picked into halves (as FmtQ6K: 16
+            // instructions for 8 weights with their products instead of 20); a 5-bit value left in the low bits of an fp16
+            // is the subnormal v * 2^-24
+            const uint32_t vl = (q & kNib) | ((h << 4) & kFifth), vh = ((q >> 4) & kNib) | ((h << 3) & kFifth);
+            lo = dot2(even_bytes(vl), xv.x, lo);
+            lo = dot2(odd_bytes(vl), xv.y, lo);
+            hi = dot2(even_bytes(vh), xv.z, hi);
+            hi = dot2(odd_bytes(vh), xv.w, hi);
         }
         const uint4 tail = xu[8];
         const float s1 = __uint_as_float(tail.x), s2 = __uint_as_float(tail.y), xscale = __uint_as_float(tail.z);
@@ -588,10 +597,10 @@ struct FmtLegacy {
                 nl = (__builtin_amdgcn_perm(t3, t2, sl) & ml) | (__builtin_amdgcn_perm(t1, t0, sl) & ~ml);
                 nh = (__builtin_amdgcn_perm(t3, t2, sh) & mh2) | (__builtin_amdgcn_perm(t1, t0, sh) & ~mh2);
                 // bytes (0, 2) and (1, 3) into the low bytes of the two halves: subnormals (value + 128) * 2^-24
-                lo = dot2(__builtin_amdgcn_perm(0u, nl, 0x0c020c00u), xv.x, lo);
-                lo = dot2(__builtin_amdgcn_perm(0u, nl, 0x0c030c01u), xv.y, lo);
-                hi = dot2(__builtin_amdgcn_perm(0u, nh, 0x0c020c00u), xv.z, hi);
-                hi = dot2(__builtin_amdgcn_perm(0u, nh, 0x0c030c01u), xv.w, hi);
+                lo = dot2(even_bytes(nl), xv.x, lo);
+                lo = dot2(odd_bytes(nl), xv.y, lo);
+                hi = dot2(even_bytes(nh), xv.z, hi);
+                hi = dot2(odd_bytes(nh), xv.w, hi);
             } else {
                 const uint32_t q8 = q >> 8;
                 uint32_t a = q & 0x000f000fu, b = q8 & 0x000f000fu, c = q & 0x00f000f0u, e = q8 & 0x00f000f0u;
@@ -708,7 +717,7 @@ struct FmtQ6K {
     static constexpr int kLPR = 32;
     static constexpr int kUnitElems = 64;
     static constexpr int kLdsDwords = 44;
-    static constexpr int kRegs = 19;
+    static constexpr int kRegs = 16;
 
     static __device__ __forceinline__ int64_t row_bytes(int K) { return (int64_t)(K >> 8) * 210; }
 
@@ -754,7 +763,7 @@ struct FmtQ6K {
         uint32_t voff;    // the lane's block: its row inside the group + inside the step
         uint32_t off_a;   // piece A inside the block (piece B is 32 bytes on)
         uint32_t off_h;   // piece H
-        uint32_t off_s;   // the 8 scales of the lane's half
+        uint32_t off_s;   // sixteen bytes with the 8 scales of the lane's half
         int sc_shift;     // bit position of the scales of runs 0 and 2 inside their dwords (runs 1 and 3: 16 bits on)
     };
     static __device__ __forceinline__ Lane lane_setup(int sub, int l16, uint32_t row_bytes)
@@ -764,7 +773,7 @@ struct FmtQ6K {
         L.voff = (uint32_t)sub * row_bytes + (uint32_t)(l16 >> 2) * 210u;
         L.off_a = 64u * n + 16u * j;
         L.off_h = 128u + 32u * n + 16u * j;
-        L.off_s = 192u + 8u * n;
+        L.off_s = 192u + 4u * n;
         L.sc_shift = (int)j * 8;
         return L;
     }
@@ -776,46 +785,53 @@ struct FmtQ6K {
         const uint32_t p = L.voff + row_delta;
         const uint32_t al = live ? (p & ~3u) : kDeadOffset;
         buf_load4(rs, al + L.off_a, soff, &w[0]);
-        w[4] = buf_load1(rs, al + L.off_a + 16u, soff);
-        buf_load4(rs, al + L.off_a + 32u, soff, &w[5]);
-        w[9] = buf_load1(rs, al + L.off_a + 48u, soff);
-        buf_load4(rs, al + L.off_h, soff, &w[10]);
-        w[14] = buf_load1(rs, al + L.off_h + 16u, soff);
-        w[15] = buf_load1(rs, al + L.off_s, soff);
-        w[16] = buf_load1(rs, al + L.off_s + 4u, soff);
-        w[17] = buf_load1(rs, al + L.off_s + 8u, soff);
-        w[18] = buf_load1(rs, al + 208u, soff);
+        buf_load4(rs, al + L.off_a + 32u, soff, &w[4]);
+        buf_load4(rs, al + L.off_h, soff, &w[8]);
+        buf_load4(rs, al + L.off_s, soff, &w[12]);       // (of the upper half: from four bytes before its scales to d)
         return p & 3u;
     }
 
     static __device__ __forceinline__ float dot(const uint32_t (&w)[kRegs], const Lane& L, uint32_t o, const uint32_t* xu_dw)
     {
-        const bool odd = (o & 2u) != 0;       // the block starts at byte 2 of its aligned window
+        const uint32_t at = o & 2u;           // the block's byte position inside its aligned window
         const uint4* xu = reinterpret_cast<const uint4*>(xu_dw);
         float a0 = 0.f, a1 = 0.f, a2 = 0.f, a3 = 0.f;
-        constexpr uint32_t kNib = 0x000f000fu, kTop = 0x00300030u;
+        constexpr uint32_t kNib = 0x0f0f0f0fu, kTop = 0x30303030u;
+        // Four values of a run are put together as bytes, then the even and the odd ones picked into halves: 32 instructions
+        // for 16 weights with their products, where masks and shifts of halves took 43 (no gain by itself: 89.4 -> 89.2 us for
+        // 128256 x 4096, the loads being the limit then, see below).
+        // The quad holds the block, and the dword behind a lane's piece is one that another lane has loaded.  Loading it again,
+        // and scales and d dword by dword, made nine load instructions of what are now four, and the address unit was what
+        // the launch waited for: 128256 x 4096 91.1 -> 77.1 us (4.7 -> 5.6 TB/s), 14336 x 4096 14.2 -> 11.4.
+        const bool j = L.sc_shift != 0, n = L.off_s != 192u;
+        const uint32_t a4 = TSHIP_DPP_U(j ? w[0] : w[4], kDppXor1);                      // 16 bytes on: the other half, the other piece
+        const uint32_t b4 = TSHIP_DPP_U(j ? w[4] : n ? w[0] : w[8], kDppNext);           // piece B: the next lane's B, A of n = 1, H of lane 0
+        const uint32_t h4 = TSHIP_DPP_U(j || n ? w[8] : w[12], kDppNext);                // piece H: the next lane's H, the scales
+        const uint32_t wa[5] = {w[0], w[1], w[2], w[3], a4}, wb[5] = {w[4], w[5], w[6], w[7], b4}, wh[5] = {w[8], w[9], w[10], w[11], h4};
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const uint32_t qa = odd ? __builtin_amdgcn_alignbyte(w[i + 1], w[i], 2) : w[i];
-            const uint32_t qb = odd ? __builtin_amdgcn_alignbyte(w[i + 6], w[i + 5], 2) : w[i + 5];
-            const uint32_t h = odd ? __builtin_amdgcn_alignbyte(w[i + 11], w[i + 10], 2) : w[i + 10];
+            const uint32_t qa = __builtin_amdgcn_alignbyte(wa[i + 1], wa[i], at);
+            const uint32_t qb = __builtin_amdgcn_alignbyte(wb[i + 1], wb[i], at);
+            const uint32_t h = __builtin_amdgcn_alignbyte(wh[i + 1], wh[i], at);
             const uint4 xa = xu[i], xb = xu[4 + i];
-            a0 = dot2((qa & kNib) | ((h << 4) & kTop), xa.x, a0);
-            a0 = dot2(((qa >> 8) & kNib) | ((h >> 4) & kTop), xa.y, a0);
-            a2 = dot2(((qa >> 4) & kNib) | (h & kTop), xa.z, a2);
-            a2 = dot2(((qa >> 12) & kNib) | ((h >> 8) & kTop), xa.w, a2);
-            a1 = dot2((qb & kNib) | ((h << 2) & kTop), xb.x, a1);
-            a1 = dot2(((qb >> 8) & kNib) | ((h >> 6) & kTop), xb.y, a1);
-            a3 = dot2(((qb >> 4) & kNib) | ((h >> 2) & kTop), xb.z, a3);
-            a3 = dot2(((qb >> 12) & kNib) | ((h >> 10) & kTop), xb.w, a3);
+            const uint32_t v0 = (qa & kNib) | ((h << 4) & kTop), v2 = ((qa >> 4) & kNib) | (h & kTop);
+            const uint32_t v1 = (qb & kNib) | ((h << 2) & kTop), v3 = ((qb >> 4) & kNib) | ((h >> 2) & kTop);
+            a0 = dot2(even_bytes(v0), xa.x, a0);
+            a0 = dot2(odd_bytes(v0), xa.y, a0);
+            a2 = dot2(even_bytes(v2), xa.z, a2);
+            a2 = dot2(odd_bytes(v2), xa.w, a2);
+            a1 = dot2(even_bytes(v1), xb.x, a1);
+            a1 = dot2(odd_bytes(v1), xb.y, a1);
+            a3 = dot2(even_bytes(v3), xb.z, a3);
+            a3 = dot2(odd_bytes(v3), xb.w, a3);
         }
         // the half's 8 scale bytes: runs 0, 1 in bytes j, j + 2 of the first dword, runs 2, 3 of the second
-        const uint32_t s01 = odd ? __builtin_amdgcn_alignbyte(w[16], w[15], 2) : w[15];
-        const uint32_t s23 = odd ? __builtin_amdgcn_alignbyte(w[17], w[16], 2) : w[16];
+        const uint32_t sa = n ? w[13] : w[12], sb = n ? w[14] : w[13], se = n ? w[15] : w[14];
+        const uint32_t s01 = __builtin_amdgcn_alignbyte(sb, sa, at), s23 = __builtin_amdgcn_alignbyte(se, sb, at);
         const float sc0 = (float)(int8_t)(s01 >> L.sc_shift), sc1 = (float)(int8_t)(s01 >> (L.sc_shift + 16));
         const float sc2 = (float)(int8_t)(s23 >> L.sc_shift), sc3 = (float)(int8_t)(s23 >> (L.sc_shift + 16));
         H2U dh;
-        dh.u = odd ? (w[18] >> 16) : (w[18] & 0xffffu);
+        dh.u = (TSHIP_DPP_U(w[15], kDppThird) >> (8u * at)) & 0xffffu;
         const float d = (float)dh.h.x;
         const uint4 sums = xu[8], scl = xu[9];
         // a_r carries v * 2^-24; the stored value is v - 32
