@@ -13,7 +13,38 @@ namespace {
 constexpr int kMaxK = 16;
 constexpr int kGroupLdsIds = 8192;     // assignments whose ids the grouping kernel keeps in LDS (32 KiB)
 
-// one wavefront per token
+// The larger value of a wavefront and its index (of equals the lowest), in every lane: register permutations, no LDS.
+template <int CTRL>
+__device__ __forceinline__ void best_of_dpp(float& best, int& bi)
+{
+    const float ov = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(best), CTRL, 0xf, 0xf, true));
+    const int oi = __builtin_amdgcn_update_dpp(0, bi, CTRL, 0xf, 0xf, true);
+    const bool other = ov > best || (ov == best && oi < bi);
+    best = other ? ov : best;
+    bi = other ? oi : bi;
+}
+__device__ __forceinline__ void wave_best(float& best, int& bi)
+{
+    typedef uint32_t u2_t __attribute__((ext_vector_type(2)));
+    best_of_dpp<0xb1>(best, bi);      // quad_perm [1,0,3,2]
+    best_of_dpp<0x4e>(best, bi);      // quad_perm [2,3,0,1]
+    best_of_dpp<0x141>(best, bi);     // half mirror: the other quad of eight lanes
+    best_of_dpp<0x140>(best, bi);     // mirror: the other eight of sixteen
+    // rows of 16, then halves of 32, swapped with themselves: a lane holds both sides
+    auto both = [&](u2_t v, u2_t i) {
+        const float a = __uint_as_float(v.x), b = __uint_as_float(v.y);
+        const bool second = b > a || (b == a && (int)i.y < (int)i.x);
+        best = second ? b : a;
+        bi = second ? (int)i.y : (int)i.x;
+    };
+    both(__builtin_amdgcn_permlane16_swap(__float_as_uint(best), __float_as_uint(best), false, false),
+         __builtin_amdgcn_permlane16_swap((uint32_t)bi, (uint32_t)bi, false, false));
+    both(__builtin_amdgcn_permlane32_swap(__float_as_uint(best), __float_as_uint(best), false, false),
+         __builtin_amdgcn_permlane32_swap((uint32_t)bi, (uint32_t)bi, false, false));
+}
+
+// One wavefront per token.  Latency bound: up to 64 experts a lane keeps its logit (the row was read once per selection), and
+// the selections reduce in registers instead of twelve trips each through the LDS crossbar (4 of 32 experts: one token 4.8 -> 3.6 us, 256 tokens 6.2 -> 5.4).
 __global__ void __launch_bounds__(64) moe_route_kernel(const float* __restrict__ logits, int64_t ld, int E, int k,
                                                        int* __restrict__ ids, float* __restrict__ weights)
 {
@@ -26,12 +57,19 @@ __global__ void __launch_bounds__(64) moe_route_kernel(const float* __restrict__
         sel[s] = -1;
         val[s] = 0.f;
     }
+    const bool held = E <= 64;
+    bool open = held && lane < E;           // this lane's expert has not been taken
+    const float own = open ? row[lane] : 0.f;
 #pragma unroll
     for (int s = 0; s < kMaxK; ++s) {
         if (s < k) {
             float best = -INFINITY;
             int bi = 0x7fffffff;
-            for (int i = lane; i < E; i += 64) {
+            if (open && own > best) {
+                best = own;
+                bi = lane;
+            }
+            for (int i = lane; !held && i < E; i += 64) {
                 bool taken = false;
 #pragma unroll
                 for (int j = 0; j < kMaxK; ++j) taken = taken || (j < s && sel[j] == i);
@@ -41,20 +79,14 @@ __global__ void __launch_bounds__(64) moe_route_kernel(const float* __restrict__
                     bi = i;
                 }
             }
-            for (int o = 32; o > 0; o >>= 1) {
-                const float ov = __shfl_xor(best, o);
-                const int oi = __shfl_xor(bi, o);
-                if (ov > best || (ov == best && oi < bi)) {
-                    best = ov;
-                    bi = oi;
-                }
-            }
+            wave_best(best, bi);
             if (bi == 0x7fffffff) {   // nothing comparable left (all -inf / NaN): the reference keeps index 0
                 bi = 0;
                 best = row[0];
             }
             sel[s] = bi;
             val[s] = best;
+            open = open && bi != lane;
         }
     }
     float mx = -INFINITY;

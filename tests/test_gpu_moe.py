@@ -30,6 +30,24 @@ def test_route_matches_reference_semantics(hip, oracle):
         np.testing.assert_allclose(w2.cpu().numpy(), rw, rtol=2e-6, atol=1e-7)
 
 
+@pytest.mark.parametrize("E,k", [(1, 1), (2, 2), (17, 16), (33, 4), (63, 5), (64, 16), (65, 4), (200, 8)])
+def test_route_of_few_many_tied_and_infinite_logits(hip, oracle, E, k):
+    """Up to 64 experts a lane of the token's wavefront holds a logit, beyond it reads them anew: ties across lanes and halves
+    of the wavefront, rows with fewer finite logits than selections, infinities.  Ids exact; weights: one division and one
+    exponential apart, as above."""
+    import torch
+    rng = np.random.default_rng(E * 31 + k)
+    lg = np.round(rng.standard_normal((40, E)) * 2).astype(np.float32) / 2      # many ties
+    lg[5, :] = -1.5
+    lg[6, 1:] = -np.inf
+    lg[7, : E // 2] = -np.inf
+    lg[8, E - 1] = 40.0
+    w, i = hip.MoERoute(torch.from_numpy(lg).cuda(), k)
+    ri, rw = oracle.moe_route(lg, k)
+    assert np.array_equal(i.cpu().numpy(), ri)
+    np.testing.assert_allclose(w.cpu().numpy(), rw, rtol=2e-6, atol=1e-7)
+
+
 def make_experts(oracle, t, E, H, F, rng, sigma=0.05):
     gu = oracle.quantize(t, (rng.standard_normal(E * 2 * F * H) * sigma).astype(np.float32))
     dn = oracle.quantize(t, (rng.standard_normal(E * H * F) * sigma).astype(np.float32))
