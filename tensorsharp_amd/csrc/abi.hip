@@ -949,13 +949,18 @@ int addmm_quant_host(const TSHipTensorView2D& result, const TSHipTensorView2D& m
             for (int64_t k = 0; k < K; ++k) x_stage[(size_t)m * K + k] = src[(size_t)m * m1.stride0 + (size_t)k * m1.stride1];
     }
     hipStream_t stream = nullptr;
+    // What a failing call has queued may still read or store the pinned memory, which the next call packs its rows into.
+    auto abandon = [&]() -> int {
+        (void)hipStreamSynchronize(stream);
+        return 0;
+    };
     if (!x_pinned && !hip_ok(hipMemcpyAsync(x_dev, x_stage, x_bytes, hipMemcpyHostToDevice, stream), "hipMemcpy(activations)")) return 0;
 
     TSHipTensorView2D r_dev{y_dev, M, (int)N, (int)N, 1, (int64_t)y_bytes};
     TSHipTensorView2D x_desc{x_dev, M, (int)K, (int)K, 1, (int64_t)x_bytes};
-    if (!run_matmul_device(r_dev, x_desc, w_dev, type, K, N, stream)) return 0;
+    if (!run_matmul_device(r_dev, x_desc, w_dev, type, K, N, stream)) return abandon();
 
-    if (!y_pinned && !hip_ok(hipMemcpyAsync(y_stage, y_dev, y_bytes, hipMemcpyDeviceToHost, stream), "hipMemcpy(result)")) return 0;
+    if (!y_pinned && !hip_ok(hipMemcpyAsync(y_stage, y_dev, y_bytes, hipMemcpyDeviceToHost, stream), "hipMemcpy(result)")) return abandon();
     if (!hip_ok(hipStreamSynchronize(stream), "hipStreamSynchronize")) return 0;
     float* dst = static_cast<float*>(result.data);
     for (int m = 0; m < M; ++m) std::memcpy(dst + (size_t)m * result.stride0, y_stage + (size_t)m * N, (size_t)N * sizeof(float));

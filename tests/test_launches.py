@@ -1,0 +1,73 @@
+"""Which kernels a call launches, and what it does when one of them fails: the library on a HIP runtime without a device
+(hip_stub.cpp, preloaded into a process of its own).  CPU tests; nothing is computed."""
+import json
+import os
+import subprocess
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+PRELUDE = """
+import ctypes as C, json, sys
+import numpy as np
+sys.path.insert(0, {root!r})
+from tensorsharp_amd import hip_native as N
+stub = C.CDLL({stub!r})
+stub.stub_log.restype = C.c_char_p
+N._lib = L = C.CDLL(N.LIB_PATH)
+for name, (res, args) in N.SIGNATURES.items():
+    getattr(L, name).restype = res
+    getattr(L, name).argtypes = args
+def view(a, rows, cols, stride=None):
+    s = cols if stride is None else stride
+    return N.TensorView2D(a.ctypes.data, rows, cols, s, 1, ((rows - 1) * s + cols) * 4)
+def space(nbytes):
+    a = np.zeros(nbytes + 64, dtype=np.uint8)
+    return a[-a.ctypes.data % 64:][:nbytes]
+def log():
+    text = stub.stub_log().decode()
+    stub.stub_clear()
+    return [l.split() for l in text.splitlines()]
+out = []
+"""
+
+
+@pytest.fixture(scope="module")
+def stub(tmp_path_factory):
+    lib = str(tmp_path_factory.mktemp("stub") / "libhip_stub.so")
+    subprocess.run(["g++", "-O1", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-Wno-deprecated-declarations",
+                    os.path.join(ROOT, "tests", "hip_stub.cpp"), "-o", lib], check=True)
+
+    def run(code, **values):
+        text = PRELUDE.format(root=ROOT, stub=lib) + "".join(f"{k} = {v!r}\n" for k, v in values.items()) + code + "\nprint(json.dumps(out))"
+        p = subprocess.run([sys.executable, "-c", text], env=dict(os.environ, LD_PRELOAD=lib), capture_output=True, text=True, timeout=300)
+        assert p.returncode == 0, p.stderr[-2000:]
+        return json.loads(p.stdout.splitlines()[-1])
+    return run
+
+
+def launches(log, name):
+    return [l for l in log if l[0] == "launch" and name in l[1]]
+
+
+HOST_LINEAR = """
+x, w, y = np.zeros((M, K), np.float32), space(N_ * K // 256 * 144), np.zeros((M, N_), np.float32)
+for n in fails:
+    stub.stub_fail_launch(n)
+    ok = L.TSHip_AddmmQuantF32(view(y, M, N_), view(x, M, K), w.ctypes.data, 12, K, N_, w.size)
+    out.append([ok, log()])
+"""
+
+
+@pytest.mark.parametrize("M,N,K", [(32, 4096, 4096), (2, 512, 4096)])
+def test_a_host_linear_that_fails_waits_for_what_it_launched(stub, M, N, K):
+    """Kernels read and store the pinned staging memory themselves: after a failed launch the earlier ones have to have ended
+    before the next call packs its activations there."""
+    for n, (ok, log) in enumerate(stub(HOST_LINEAR, M=M, K=K, N_=N, fails=[0, 2, 1, 2])):
+        if n == 0:
+            assert ok == 1 and log[-1][0] == "wait"
+            continue
+        assert ok == 0 and any(l[0] == "failed" for l in log), log
+        assert log[-1][0] == "wait", log
