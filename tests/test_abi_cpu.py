@@ -161,3 +161,12 @@ def test_managed_pinvoke_declarations_match_the_header():
 
 def test_struct_layout_3d_view():
     assert C.sizeof(N.TensorView3D) == 40 and N.TensorView3D.raw_bytes.offset == 32
+
+
+@pytest.mark.parametrize("weight", [b"blocks", "blocks", (C.c_uint8 * 64)(), C.c_void_p(4096), np.zeros(64, np.uint8)])
+def test_a_device_linear_takes_an_address_only(monkeypatch, weight):
+    """A bytes object, a string or a ctypes array as the weight would reach the kernel as host memory."""
+    from tensorsharp_amd import HipBasicOps, hip_basic_ops
+    monkeypatch.setattr(hip_basic_ops, "_device_view", lambda t: N.TensorView2D(4096, 1, 256, 256, 1, 1024))
+    with pytest.raises(TypeError):
+        HipBasicOps.AddmmQuantDevice(None, None, weight, N.TYPE_Q4_K, 256, 256, 256 * 144)
