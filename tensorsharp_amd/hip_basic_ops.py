@@ -522,9 +522,9 @@ class HipBasicOps:
         """Same contract with every pointer in device memory; asynchronous on the current stream."""
         rv = _device_view(result)
         mv = _device_view(m1)
-        if type(weight_data) is not int:                # (an address as it is: 0.2 us less than through c_void_p, which refuses
-            weight_data = C.c_void_p(weight_data)       # bytes, strings and arrays that the bare argument would pass as host memory)
-        ok = N.lib().TSHip_AddmmQuantF32Device(rv, mv, weight_data, int(ggml_type), int(ne0), int(ne1), int(raw_bytes))
+        # (c_void_p refuses bytes, strings and arrays, which the bare argument would pass as host memory)
+        ok = N.lib().TSHip_AddmmQuantF32Device(rv, mv, C.c_void_p(weight_data), int(ggml_type), int(ne0), int(ne1),
+                                               int(raw_bytes))
         N.check_result(ok, "addmm_quant")
 
     @staticmethod
