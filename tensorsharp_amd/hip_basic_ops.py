@@ -700,8 +700,9 @@ class HipBasicOps:
         """Launch the *Device entry points on torch's current stream."""
         torch = _torch()
         raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
-        if raw_stream is not None and torch.cuda.is_initialized():
-            handle = raw_stream(torch._C._cuda_getDevice())     # current_stream().cuda_stream without the stream object
+        get_device = getattr(torch._C, "_cuda_getDevice", None)
+        if raw_stream is not None and get_device is not None and torch.cuda.is_initialized():
+            handle = raw_stream(get_device())                   # current_stream().cuda_stream without the stream object
         else:
             handle = torch.cuda.current_stream().cuda_stream
         N.lib().TSHip_SetStream(handle)

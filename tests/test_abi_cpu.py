@@ -170,3 +170,19 @@ def test_a_device_linear_takes_an_address_only(monkeypatch, weight):
     monkeypatch.setattr(hip_basic_ops, "_device_view", lambda t: N.TensorView2D(4096, 1, 256, 256, 1, 1024))
     with pytest.raises(TypeError):
         HipBasicOps.AddmmQuantDevice(None, None, weight, N.TYPE_Q4_K, 256, 256, 256 * 144)
+
+
+@pytest.mark.parametrize("absent", ["_cuda_getCurrentRawStream", "_cuda_getDevice"])
+def test_current_stream_without_torchs_private_names(monkeypatch, absent):
+    """Either name may be missing from a torch build: the stream object serves then."""
+    import types
+    from tensorsharp_amd import HipBasicOps, hip_basic_ops
+    private = {"_cuda_getCurrentRawStream": lambda dev: 1, "_cuda_getDevice": lambda: 0}
+    del private[absent]
+    fake = types.SimpleNamespace(_C=types.SimpleNamespace(**private), cuda=types.SimpleNamespace(
+        is_initialized=lambda: True, current_stream=lambda: types.SimpleNamespace(cuda_stream=77)))
+    seen = []
+    monkeypatch.setattr(hip_basic_ops, "_torch", lambda: fake)
+    monkeypatch.setattr(N, "lib", lambda: types.SimpleNamespace(TSHip_SetStream=seen.append))
+    HipBasicOps.UseCurrentStream()
+    assert seen == [77]
