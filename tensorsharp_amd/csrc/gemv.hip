@@ -1759,10 +1759,12 @@ bool launch_gemv_group(int type, int count, const GemvArgs* args, hipStream_t st
     if (count == 1 && lpr == 16 && !args[0].expert_id && !args[0].slot_ids && !args[0].pair_rows && act != kActSiluMul && !g_timeline) {
         const int groups = (args[0].N + rpg - 1) / rpg, steps = (args[0].K / unit_elems(type) + lpr - 1) / lpr;
         const int per_wg = (groups + di.num_cus - 1) / di.num_cus;
-        if (per_wg < kWaves && steps * (kWaves - per_wg) >= kWaves * (type == kTypeQ8_0 ? 5 : 6)) {
+        const size_t parts = kWaves * kWaves * 4 * sizeof(float);       // fewer than kWaves row groups of 4 rows
+        // (the longest rows, 65024 of the 32-weight formats but Q8_0, leave 192 bytes more than the parts take; gemv_max_k does not know of them)
+        if (per_wg < kWaves && steps * (kWaves - per_wg) >= kWaves * (type == kTypeQ8_0 ? 5 : 6) && lds + parts <= 160 * 1024) {
             g.split = per_wg;
             begin = (groups + per_wg - 1) / per_wg;
-            lds += kWaves * kWaves * 4 * sizeof(float);       // the parts: fewer than kWaves row groups of 4 rows
+            lds += parts;
         }
     }
     for (int i = 1; i < count; ++i)

@@ -275,6 +275,26 @@ def test_split_rows_at_the_edges_of_their_groups(hip, oracle, name, N, K):
     assert np.max(np.abs(y.cpu().numpy() - want)) <= 1e-3 * (np.linalg.norm(want) if N > 1 else 1.2 * scale)
 
 
+@pytest.mark.parametrize("name,K", [("q8_0", 35840), ("mxfp4", 65024), ("q5_1", 65024)])
+def test_split_rows_of_the_longest_k(hip, oracle, name, K):
+    """As many activations as a workgroup stages (more go through the matrix cores), with the parts of the split rows above
+    them; plain and with the RMSNorm, which is staged in more than one pass."""
+    import torch
+    from tensorsharp_amd import QuantizedWeight
+    rng = np.random.default_rng(K)
+    N = 70
+    t, wq = host_case_weight(oracle, name, N, K, rng)
+    x = rng.standard_normal((1, K)).astype(np.float32)
+    check(name if name in RMS_TOL else "q4_k", run_device(hip, t, wq, N, K, x), oracle.matmul_f64(t, wq, N, K, x))
+    nw = (1 + 0.1 * rng.standard_normal(K)).astype(np.float32)
+    xn = x.astype(np.float64)
+    xn = (xn / np.sqrt(np.mean(xn * xn) + 1e-6) * nw).astype(np.float32)
+    y = torch.full((1, N), float("nan"), device="cuda")
+    hip.FusedRmsNormMatMulQuant(y, torch.from_numpy(x).cuda(), torch.from_numpy(nw).cuda(), 1e-6, QuantizedWeight(torch.from_numpy(wq).cuda(), t, K, N))
+    want = oracle.matmul_f64(t, wq, N, K, xn)
+    assert np.max(np.abs(y.cpu().numpy() - want)) <= 1e-3 * np.linalg.norm(want)
+
+
 # ---- Q6_K (output matrix and some projections of Q4_K_M files): 210-byte blocks, 2-byte aligned ----
 def q6k_weight(N, K, seed, std=0.02):
     import torch

@@ -71,3 +71,30 @@ def test_a_host_linear_that_fails_waits_for_what_it_launched(stub, M, N, K):
             continue
         assert ok == 0 and any(l[0] == "failed" for l in log), log
         assert log[-1][0] == "wait", log
+
+
+GEMV_LINEAR = """
+for t, per, size, rows, k, norm, add in cases:
+    w, x, y = space(rows * (k // per) * size), np.zeros((1, k + 16), np.float32), np.zeros((1, rows), np.float32)
+    xv = N.TensorView2D(x.ctypes.data + -x.ctypes.data % 16, 1, k, k, 1, k * 4)
+    if norm:
+        nw = space(4 * k)
+        ok = L.TSHip_FusedRmsNormMatMulQuantF32Device(view(y, 1, rows), xv, nw.ctypes.data, k, 1e-6, w.ctypes.data, t, k, rows, w.size)
+    elif add:
+        ok = L.TSHip_FusedMatMulQuantAddF32Device(view(y, 1, rows), xv, w.ctypes.data, t, k, rows, w.size)
+    else:
+        ok = L.TSHip_AddmmQuantF32Device(view(y, 1, rows), xv, w.ctypes.data, t, k, rows, w.size)
+    assert ok, L.TSHip_GetLastError()
+    out.append(log())
+"""
+BLOCKS = {"q8_0": (8, 32, 34), "mxfp4": (39, 32, 17), "q4_0": (2, 32, 18), "q4_1": (3, 32, 20), "q5_0": (6, 32, 22), "q5_1": (7, 32, 24), "iq4_nl": (20, 32, 18)}
+LONGEST = {"q8_0": 35840}           # of the formats of 80 LDS bytes per block: 65024
+
+
+@pytest.mark.parametrize("name", BLOCKS)
+def test_the_longest_rows_of_a_split_launch_fit_into_lds(stub, name):
+    k = LONGEST.get(name, 65024)
+    cases = [(*BLOCKS[name], 40, k, norm, 0) for norm in (0, 1)]
+    for log in stub(GEMV_LINEAR, cases=cases):
+        (split,) = launches(log, "gemv_split_kernel")
+        assert int(split[6]) <= 160 * 1024
