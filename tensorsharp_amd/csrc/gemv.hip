@@ -1748,20 +1748,27 @@ bool launch_gemv_group(int type, int count, const GemvArgs* args, hipStream_t st
         if (ok) g.strict = 2;
     }
     // The split build (gemv_split_kernel) for one problem of a 16-lane format with few and long rows.  Unsplit, a wavefront
-    // takes a row group's steps one after the other, about 0.65 us each, while most CUs have no workgroup; split, a
-    // workgroup of every CU shares per_wg groups among its 8 wavefronts, for 1 us more of start (two barriers, the parts).
-    // So the line lies where the steps saved, steps * (1 - per_wg / 8), are five of Q8_0 and six of the 17- to 24-byte
-    // blocks.  Measured unsplit / split, us: Q8_0 1024 x 14336 16.5 / 6.6, 2048 x 8192 10.6 / 7.1, 2560 x 9728 12.4 / 8.6,
-    // 2560 x 4096 6.7 / 5.7, 4096 x 14336 21.7 / 15.5, on the line 3072 x 3072 5.37 / 5.31 and 6144 x 8192 13.6 / 13.5, past
-    // it 4096 x 2560 5.2 / 5.5; with RMSNorm staging 2560 x 4096 7.6 / 6.8; MXFP4 2560 x 9728 10.7 / 7.6, 1024 x 4096
-    // 4.7 / 4.3, past the line 2560 x 4096 4.79 / 4.84.  (The 32-lane formats have twice the wavefronts per row and lose:
-    // Q4_K 4096 x 14336 8.9 / 10.4, Q6_K 2560 x 9728 9.0 / 9.4.)
+    // takes a row group's steps one after the other, 0.4 us each from the cache and 0.6 from HBM, while most CUs have no workgroup;
+    // split, a workgroup of every CU shares per_wg groups among its 8 wavefronts, for 1 us more of start (two barriers, the
+    // parts).  kSplitSteps: the steps from which that pays, by per_wg.  The lines are those of weights that come from HBM, as a
+    // model's do (110 random shapes per format, 8 to 64 weights of 700 MB in turn; plain, with RMSNorm staging, added to a residual).
+    // us, unsplit / split: Q8_0 3072 x 5376 8.9 / 7.8, 4096 x 6144 10.5 / 9.1, 2560 x 7968 11.2 / 8.4, 5120 x 11008 17.4 / 15.1,
+    // 3072 x 14336 18.7 / 12.7, past the line 6144 x 14336 22.0 / 21.5 (RMSNorm 22.8 / 23.8), 5120 x 2560 6.1 / 6.6.
+    // From the 256 MB cache (four weights in turn) the few-step end of three to six groups loses: 3072 x 5376 7.2 / 7.5, 4096 x 6144
+    // 7.7 / 8.3, 5120 x 8192 9.8 / 11.2; 1024 x 14720 13.5 / 6.9 there too.  The cheap blocks of 17 to 20 bytes start later (Q4_0
+    // 1024 x 3264, past the line, 4.6 / 4.9, added to a residual 4.7 / 5.4; 8 steps, on it, 1.00 to 1.05), the others earlier.
+    // (The 32-lane formats have twice the wavefronts per row and lose: Q4_K 4096 x 14336 8.9 / 10.4, Q6_K 2560 x 9728 9.0 / 9.4.)
+    static constexpr int kSplitSteps[3][kWaves - 1] = {{6, 7, 8, 10, 14, 30, 40},        // Q8_0
+                                                       {8, 9, 10, 12, 16, 24, 48},      // MXFP4, Q4_0, Q4_1
+                                                       {7, 8, 10, 12, 16, 24, 48}};     // Q5_0, Q5_1, IQ4_NL
     if (count == 1 && lpr == 16 && !args[0].expert_id && !args[0].slot_ids && !args[0].pair_rows && act != kActSiluMul && !g_timeline) {
         const int groups = (args[0].N + rpg - 1) / rpg, steps = (args[0].K / unit_elems(type) + lpr - 1) / lpr;
         const int per_wg = (groups + di.num_cus - 1) / di.num_cus;
+        const int cls = type == kTypeQ8_0 ? 0 : type == kTypeMXFP4 || type == kTypeQ4_0 || type == kTypeQ4_1 ? 1 : 2;
         const size_t parts = kWaves * kWaves * 4 * sizeof(float);       // fewer than kWaves row groups of 4 rows
-        // (the longest rows, 65024 of the 32-weight formats but Q8_0, leave 192 bytes more than the parts take; gemv_max_k does not know of them)
-        if (per_wg < kWaves && steps * (kWaves - per_wg) >= kWaves * (type == kTypeQ8_0 ? 5 : 6) && lds + parts <= 160 * 1024) {
+        // (the longest rows, 65024 of the 32-weight formats but Q8_0, leave 192 bytes more than the parts take; gemv_max_k
+        // does not know of them)
+        if (per_wg < kWaves && steps >= kSplitSteps[cls][per_wg - 1] && lds + parts <= 160 * 1024) {
             g.split = per_wg;
             begin = (groups + per_wg - 1) / per_wg;
             lds += parts;

@@ -98,3 +98,15 @@ def test_the_longest_rows_of_a_split_launch_fit_into_lds(stub, name):
     for log in stub(GEMV_LINEAR, cases=cases):
         (split,) = launches(log, "gemv_split_kernel")
         assert int(split[6]) <= 160 * 1024
+
+
+@pytest.mark.parametrize("name,rows,steps,split", [
+    ("q8_0", 1024, 6, 1), ("q8_0", 1024, 5, 0), ("q8_0", 2048, 7, 1), ("q8_0", 2048, 6, 0), ("q8_0", 4096, 10, 1), ("q8_0", 4096, 9, 0),
+    ("q8_0", 6144, 30, 1), ("q8_0", 6144, 28, 0), ("q8_0", 7172, 42, 0),
+    ("q4_0", 1024, 8, 1), ("q4_0", 1024, 7, 0), ("q4_1", 1745, 9, 1), ("q4_1", 1745, 8, 0), ("mxfp4", 1318, 8, 0), ("mxfp4", 3072, 10, 1),
+    ("q5_0", 1024, 7, 1), ("iq4_nl", 2048, 8, 1), ("q5_1", 5120, 15, 0),
+])
+def test_rows_are_split_where_that_was_measured_faster(stub, name, rows, steps, split):
+    for norm, add in ((0, 0), (1, 0), (0, 1)):
+        (log,) = stub(GEMV_LINEAR, cases=[(*BLOCKS[name], rows, 512 * steps, norm, add)])
+        assert len(launches(log, "gemv_split_kernel")) == split and len(launches(log, "gemv")) == 1, log
