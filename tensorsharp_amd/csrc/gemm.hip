@@ -165,7 +165,11 @@ template <int TYPE, int THREADS, int SRC>
 __global__ void __launch_bounds__(THREADS) convert_x_kernel(const ConvertSrc S, int K, int Kp, int ldo, _Float16* __restrict__ out,
                                                             float* __restrict__ scales, int piece_rows)
 {
-    const int m = blockIdx.x;
+    // Activations in pieces: the rows of an XCD follow one another, so that its L2 puts whole lines of their pieces together.  With
+    // neighbouring rows on different XCDs each wrote its 16 bytes of a line to memory by itself: 512 x 14336 17.2 -> 12.3 us
+    // (whole rows 11.0), 256 x 11776 11.1 -> 9.2, 2048 x 2048 (16 experts of 128 rows) 8.0 -> 5.9.
+    const int xcd = (int)blockIdx.x & 7;
+    const int m = piece_rows ? xcd * (piece_rows >> 3) + min(xcd, piece_rows & 7) + ((int)blockIdx.x >> 3) : (int)blockIdx.x;
     const int tid = threadIdx.x;
     const float* src = S.x + (int64_t)(S.row_map ? S.row_map[m] : m) * S.ldx;
     const float* norm_w = SRC == kSrcPlain ? S.norm_w : nullptr;
