@@ -28,12 +28,15 @@ constexpr int kAttnGroups = 4 * kAttnWaves;      // 16-lane groups of a workgrou
 // merge takes one batch of 64 splits, four beyond and where that leaves a single split and no merge.  Measured us per small
 // layer, two / four rows (query x KV heads): 32 x 8 64 positions 22.7 / 23.7, 100 25.2 / 23.6, 512 25.2 / 26.3, 2048 27.7 / 28.4,
 // 3000 32.0 / 30.8; 8 x 2 4001 24.8 / 26.2, 8192 27.7 / 27.2; 16 x 2 6000 29.1 / 26.9; 32 x 32 512 26.8 / 27.4, 700 29.8 / 29.4.
-constexpr int kFewSplits = 64;
-int attn_rows(int num_kv_heads, int total)
+// One query head per KV head takes two rows somewhat longer, its small workgroups fit four to a CU (two small layers, two / four
+// rows: 32 x 32 heads at 2049 positions 66.8 / 69.6, 2400 68.2 / 69.7, 2600 71.2 / 70.4, 16 x 16 at 2049 53.7 / 56.5, 2400 54.3 / 56.3).
+constexpr int kFewSplits = 64, kFewSplitsOneHead = 40;
+int attn_rows(int num_heads, int num_kv_heads, int total)
 {
     if (total <= 2 * kAttnGroups) return 2;
     if (total <= 4 * kAttnGroups) return 4;
     const int splits = (total + 2 * kAttnGroups - 1) / (2 * kAttnGroups);
+    if (num_heads == num_kv_heads && splits <= kFewSplitsOneHead) return 2;
     return splits <= kFewSplits && (int64_t)num_kv_heads * splits <= device_info().num_cus ? 2 : 4;
 }
 
@@ -158,8 +161,14 @@ __device__ __forceinline__ float bcast16_at(float x, int l) { return bcast_step<
 // the positions four at a time with one sum, exponential and running maximum per pair: 32 x 8 heads of 128 at 512 positions
 // 6.6 -> 5.2 us, at 4001 positions (33 MB) 13.6 -> 10.6 us by the kernel trace; three Q8_0 layers and a head 182.1 -> 175.2.
 // (K / V rows as 16-byte loads: the same on every shape.)
+// Where a KV head has 3, 5, 6 or 7 query heads, a workgroup of the next power of two serves them all, the last one in the places
+// that are left over (nothing of those is stored).
+// Wavefronts per SIMD that the registers have to leave room for: two workgroups per CU for head dimensions of 192 (131 -> 128
+// registers; 12 x 2 heads at 16000 and 32000 positions 102 -> 91 and 149 -> 132 us per two small layers).
+template <int PER, int G>
+constexpr int kAttnMinWaves = PER == 12 && G <= 4 ? 4 : 1;
 template <int PER, int G, int U>
-__global__ void __launch_bounds__(kAttnWaves * 64) attn_decode_kernel(float* k_cache, float* v_cache, const float* qkv, int group,
+__global__ void __launch_bounds__(kAttnWaves * 64, (kAttnMinWaves<PER, G>)) attn_decode_kernel(float* k_cache, float* v_cache, const float* qkv, int group,
                                                                        int max_seq_len, int total, int split_len, float scale, int splits,
                                                                        int num_heads, float* __restrict__ partial, const AttnFront F,
                                                                        float* __restrict__ out_direct, const float* pre0, const float* pre1,
@@ -194,6 +203,7 @@ __global__ void __launch_bounds__(kAttnWaves * 64) attn_decode_kernel(float* k_c
         return;
     }
     const int h0 = kvh * group + blockIdx.z * G;                     // first query head of this workgroup
+    const int heads = min(G, group - (int)blockIdx.z * G);           // of its places, how many hold a head of their own
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int lg = lane & 15, grp = (wave << 2) | (lane >> 4);
     const float* kb = k_cache + (int64_t)kvh * max_seq_len * HD;
@@ -223,7 +233,7 @@ __global__ void __launch_bounds__(kAttnWaves * 64) attn_decode_kernel(float* k_c
         constexpr int kPer = (HD + 63) / 64, kPairs = (HD / 2 + 63) / 64;
         constexpr int half = HD / 2;
         const int nprep = G + (last ? 1 : 0);
-        auto head_src = [&](int hh) { return qkv + (int64_t)(hh < G ? h0 + hh : num_heads + kvh) * HD; };
+        auto head_src = [&](int hh) { return qkv + (int64_t)(hh < G ? h0 + min(hh, heads - 1) : num_heads + kvh) * HD; };
         // the wavefront's first head is requested before the angles are worked out
         float xv[kPer];
 #pragma unroll
@@ -413,8 +423,8 @@ __global__ void __launch_bounds__(kAttnWaves * 64) attn_decode_kernel(float* k_c
         if (G * PER % 4 == 0 || f < G * PER) my_acc[g * HD + lg + 16 * j] = t;
     }
     __syncthreads();
-    // the wavefronts: thread (g, d) of the first G * HD threads
-    for (int i = threadIdx.x; i < G * HD; i += kAttnWaves * 64) {
+    // the wavefronts: thread (g, d) of the first heads * HD threads
+    for (int i = threadIdx.x; i < heads * HD; i += kAttnWaves * 64) {
         const int g = i / HD, d = i - g * HD;
         float mm = -INFINITY;
 #pragma unroll
@@ -541,7 +551,7 @@ bool launch_attention_decode(const float* qkv, const float* q_norm_w, const floa
     front.num_kv_heads = num_kv_heads;
     front.k_cache = k_cache;
     front.v_cache = v_cache;
-    const int rows = attn_rows(num_kv_heads, total), split_len = kAttnGroups * rows;
+    const int rows = attn_rows(num_heads, num_kv_heads, total), split_len = kAttnGroups * rows;
     const int splits = (total + split_len - 1) / split_len;
     if (splits > 65535) {
         set_last_error("layer decode: context too long for one launch.");
@@ -550,13 +560,21 @@ bool launch_attention_decode(const float* qkv, const float* q_norm_w, const floa
     const float scale = 1.0f / sqrtf((float)head_dim);
     const int group = num_heads / num_kv_heads;
     // query heads per workgroup: as many as share the KV head (its rows are then loaded once), fewer while that leaves
-    // the launch with too few workgroups to hide its latency
+    // the launch with too few workgroups to hide its latency (64 or 256 as the line: 1 to 22 % longer at the contexts between, per
+    // two small layers: 8 x 1 heads of 256 at 6000 positions 57 / 61 / 58 us with 128 / 64 / 256, at 12000 71 / 75 / 84)
     int g = group % 8 == 0 ? 8 : group % 4 == 0 ? 4 : group % 2 == 0 ? 2 : 1;
     while (g > 2 && num_kv_heads * splits * (group / g) < 128) g >>= 1;
+    // Groups of 3, 5, 6 and 7 heads in one workgroup with places left over, once that makes 184 workgroups; with one or two
+    // heads each, every row was loaded two to seven times, and a workgroup of eight wavefronts took up to 8 % longer for it than
+    // the four of a former build.  us per two small layers, g of the rule above / all heads: 40 x 8 heads of 128 at 1500 positions (192
+    // workgroups) 53.8 / 53.9, 2047 59.8 / 55.8, 6000 101.8 / 75.6, 16000 232 / 106, 28 x 4 at 8191 107 / 62, 24 x 8 at 4000
+    // 61.9 / 55.6, 28 x 4 of 64 at 3000 (188) 49.2 / 45.9, 24 x 4 of 256 69.2 / 68.2; short of the line 40 x 8 at 1023 (136) 49.4 / 51.4, 24 x 4 of 256 at 2048 (132) 59 / 66.
+    constexpr int kEnough = 184;
+    if (group < 8 && (group & (group - 1)) != 0 && num_kv_heads * splits >= kEnough) g = group == 3 ? 4 : 8;
     // (vectors to prefetch: whole float4s at 16-byte aligned addresses, else none)
     const bool pre = (prefetch0 || prefetch1) && prefetch_floats > 0 && prefetch_floats % 4 == 0 && splits < 65535 &&
                      ((reinterpret_cast<uintptr_t>(prefetch0) | reinterpret_cast<uintptr_t>(prefetch1)) & 15) == 0;
-    const dim3 grid(num_kv_heads, splits + (pre ? 1 : 0), group / g), block(kAttnWaves * 64);
+    const dim3 grid(num_kv_heads, splits + (pre ? 1 : 0), (group + g - 1) / g), block(kAttnWaves * 64);
 #define TSHIP_ATTN_LAUNCH_U(PER, GG, U)                                                                                         \
     hipLaunchKernelGGL((attn_decode_kernel<PER, GG, U>), grid, block, 0, stream, front.k_cache, front.v_cache, front.qkv, group,     \
                        max_seq_len, total, split_len, scale, splits, num_heads, partial_ws, front, splits == 1 ? out : nullptr,           \

@@ -232,6 +232,14 @@ def test_attention_rows_per_group_at_their_borders(hip, oracle, head_dim, group,
         assert rel(kd.cpu().numpy()[:, pos], kc[:, pos]) <= 1e-5 and rel(vd.cpu().numpy()[:, pos], vc[:, pos]) <= 1e-5
 
 
+@pytest.mark.parametrize("head_dim,group,kv_heads,prefix", [(128, 3, 8, 1600), (128, 5, 8, 1600), (128, 6, 8, 1407), (128, 7, 4, 6200),
+                                                            (64, 7, 8, 1600), (80, 3, 8, 1600), (96, 5, 8, 1600), (192, 6, 8, 1600), (192, 3, 8, 1600), (256, 5, 8, 1600)])
+def test_a_group_of_heads_that_leaves_places_of_its_workgroup_over(hip, oracle, head_dim, group, kv_heads, prefix):
+    """3, 5, 6 and 7 query heads of a KV head in a workgroup of 4 or 8, once there are 184 workgroups (1408 -> 1409 positions
+    with 8 KV heads); two and four cache rows per group of lanes."""
+    test_attention_rows_per_group_at_their_borders(hip, oracle, head_dim, group, kv_heads, prefix)
+
+
 def to_host_layer(layer, QuantizedWeight, dims):
     d = {k: (None if layer[k] is None else np.ascontiguousarray(layer[k])) for k in ("attn_norm", "q_norm", "k_norm", "ffn_norm")}
     for k, (ne0, ne1) in dims.items():

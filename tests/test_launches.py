@@ -110,3 +110,37 @@ def test_rows_are_split_where_that_was_measured_faster(stub, name, rows, steps, 
     for norm, add in ((0, 0), (1, 0), (0, 1)):
         (log,) = stub(GEMV_LINEAR, cases=[(*BLOCKS[name], rows, 512 * steps, norm, add)])
         assert len(launches(log, "gemv_split_kernel")) == split and len(launches(log, "gemv")) == 1, log
+
+
+LAYER = """
+for heads, kv, d, position in cases:
+    h, cap = 256, position + 1
+    q, n = heads * d, kv * d
+    f = lambda m: space(4 * m).ctypes.data_as(C.c_void_p)
+    w = lambda rows, k: (space(rows * k // 32 * 34).ctypes.data_as(C.c_void_p), 8, k, rows, rows * k // 32 * 34)
+    cache = space(4 * kv * cap * d)
+    ok = L.TSHip_TransformerLayerDecodeDevice(f(h), h, f(h), *w(q + 2 * n, h), None, None, d, *w(h, q), f(h), *w(512, h), *w(h, 256),
+                                              cache.ctypes.data, cache.ctypes.data, heads, kv, cap, position, 1e-6, 1e4, 1.0, 256, 2)
+    assert ok, L.TSHip_GetLastError()
+    out.append(log())
+"""
+
+
+@pytest.mark.parametrize("heads,kv,head_dim,position,places,chunks", [
+    (40, 8, 128, 6000, 8, 1), (28, 4, 128, 8191, 8, 1), (24, 8, 128, 4000, 4, 1), (12, 2, 192, 32000, 8, 1),       # the rows of a KV head loaded once
+    (40, 8, 128, 1000, 1, 5), (24, 4, 256, 2047, 2, 3),                                                            # too few workgroups for that
+    (40, 8, 128, 1407, 1, 5), (40, 8, 128, 1408, 8, 1),
+    (32, 8, 128, 4000, 4, 1), (64, 8, 128, 4000, 8, 1), (48, 4, 128, 8000, 4, 3), (8, 8, 128, 8000, 1, 1),
+])
+def test_query_heads_per_attention_workgroup(stub, heads, kv, head_dim, position, places, chunks):
+    (log,) = stub(LAYER, cases=[(heads, kv, head_dim, position)])
+    (attention,) = launches(log, "attn_decode_kernel")
+    assert f"attn_decode_kernelILi{head_dim // 16}ELi{places}E" in attention[1] and int(attention[4]) == chunks, attention
+
+
+@pytest.mark.parametrize("heads,kv,position,rows", [(32, 32, 2559, 2), (32, 32, 2560, 4), (16, 16, 2048, 2), (32, 8, 2048, 4), (32, 8, 2047, 2),
+                                                    (8, 2, 4095, 2), (8, 2, 4096, 4), (32, 32, 63, 2), (32, 32, 64, 4), (32, 32, 128, 2)])
+def test_cache_rows_per_group_of_lanes(stub, heads, kv, position, rows):
+    (log,) = stub(LAYER, cases=[(heads, kv, 64, position)])
+    (attention,) = launches(log, "attn_decode_kernel")
+    assert f"ELi{rows}EEEvP" in attention[1], attention
