@@ -904,10 +904,11 @@ const void* resolve_weight_range(void* base, size_t offset, size_t bytes)
 // them; more reach it sooner through the copy engine (us a call, read / copied, results written the same way: Q4_K 4096 x 4096
 // with 16 rows 46.9 / 54.6, 64 rows - 1 MiB - 111.0 / 118.0, 96 rows 167.3 / 166.0, 128 rows 207.0 / 201.4).
 constexpr size_t kReadPinnedBytes = (size_t)1 << 20;
-// Results of a call of up to this many bytes are stored to pinned memory by the kernels themselves (with the copy engine
-// after them, activations copied in both: 16 rows 62.4 -> 54.6, 256 rows 373.5 -> 364.8); larger calls keep one pinned
-// region for both directions.
-constexpr size_t kStorePinnedBytes = (size_t)32 << 20;
+// Calls of up to this many bytes of activations and results have the kernels store the results to pinned memory.  Larger ones send them
+// through the copy engine: one pinned region serves both directions then, and what the processor packs and unpacks stays in its
+// cache (us a call, copied / stored, activations copied in both: Q4_K 16 x 4096 x 4096 62 / 50, 128 rows 202 / 198, 400 - 13 MB -
+// 538 / 535, 600 820 / 891, 1600 2659 / 2714; 600 x 2560 x 2560 514 / 506, 800 - 16 MB - 663 / 685, 300 x 4096 x 9728 656 / 703).
+constexpr size_t kStorePinnedBytes = (size_t)12 << 20;
 
 // w_dev_given: the device copy when the caller has resolved the weight already (sub-weights of a stack)
 int addmm_quant_host(const TSHipTensorView2D& result, const TSHipTensorView2D& m1, void* m2_data, int type, int64_t ne0,
@@ -928,8 +929,9 @@ int addmm_quant_host(const TSHipTensorView2D& result, const TSHipTensorView2D& m
     const size_t x_bytes = (size_t)M * K * sizeof(float);
     const size_t y_bytes = (size_t)M * N * sizeof(float);
     const size_t y_off = (x_bytes + 255) & ~(size_t)255;
-    // The dense kernels read activations many times; a GEMV's workgroups read them one and all.  What a conversion reads, and
-    // what the GEMV and GEMM kernels store, is touched once.
+    // The dense kernels read activations many times; a GEMV's workgroups read them one and all.  What the GEMV and GEMM kernels
+    // store is touched once, and so is what a conversion reads, but for the part of a row beyond 32768 (four rows of 65536 from
+    // pinned memory still 121 us, copied 123).
     const MatmulPlan plan = plan_matmul(type, M, K, N, false, false);
     const bool quantized = !is_dense_type(type) && type != kTypeQ8_1 && !plan.narrow;
     const bool y_pinned = quantized && y_off + y_bytes <= kStorePinnedBytes;

@@ -73,6 +73,14 @@ def test_a_host_linear_that_fails_waits_for_what_it_launched(stub, M, N, K):
         assert log[-1][0] == "wait", log
 
 
+@pytest.mark.parametrize("M,N,K,copies", [(64, 4096, 4096, 0), (65, 4096, 4096, 1), (380, 4096, 4096, 1), (400, 4096, 4096, 2), (600, 4096, 4096, 2),
+                                          (700, 4096, 256, 0), (800, 4096, 256, 2), (2, 4096, 4096, 1)])
+def test_which_way_a_host_linear_takes_over_the_link(stub, M, N, K, copies):
+    """Up to 1 MiB of activations are read from pinned memory (not by a GEMV); results are stored to it while both take up to 12 MiB."""
+    ((ok, log),) = stub(HOST_LINEAR, M=M, K=K, N_=N, fails=[0])
+    assert ok == 1 and sum(l[0] == "copy" for l in log) == copies, log
+
+
 GEMV_LINEAR = """
 for t, per, size, rows, k, norm, add in cases:
     w, x, y = space(rows * (k // per) * size), np.zeros((1, k + 16), np.float32), np.zeros((1, rows), np.float32)
