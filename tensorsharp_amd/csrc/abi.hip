@@ -515,8 +515,12 @@ unsigned char* scratch_ptr()
 // `ws` has plan.total bytes.
 struct FfnPlan {
     MatmulPlan gu, dn;
-    size_t gu_bytes, act_bytes, mm_bytes, total;      // [gate | up rows][gated rows][workspace of either matmul]
+    size_t gu_bytes, act_bytes, mm_bytes, total;      // [gate | up rows][gated rows, where they are formed][workspace of either matmul]
 };
+
+// silu(gate) * up is formed by the conversion of the down projection's activations (more rows are refused by the kernel that forms
+// the gated rows otherwise)
+bool gates_in_conversion(const FfnPlan& p, int M) { return p.dn.converts && M <= 65535; }
 
 FfnPlan plan_ffn(int M, int gu_type, int dn_type, int hidden, int half)
 {
@@ -525,7 +529,7 @@ FfnPlan plan_ffn(int M, int gu_type, int dn_type, int hidden, int half)
     p.gu = plan_matmul(gu_type, M, hidden, 2 * (int64_t)half, true, false);
     p.dn = plan_matmul(dn_type, M, half, hidden, false, true);
     p.gu_bytes = al((size_t)M * 2 * half * sizeof(float));
-    p.act_bytes = al((size_t)M * half * sizeof(float));
+    p.act_bytes = gates_in_conversion(p, M) ? 0 : al((size_t)M * half * sizeof(float));
     p.mm_bytes = std::max(p.gu.total(), p.dn.total());
     p.total = p.gu_bytes + p.act_bytes + p.mm_bytes;
     return p;
@@ -566,7 +570,7 @@ bool run_ffn_swiglu_device(const FfnPlan& plan, const TSHipTensorView2D& residua
     }
     const TSHipTensorView2D gu_view{gu, M, 2 * half, 2 * half, 1, (int64_t)((size_t)M * 2 * half * sizeof(float))};
     if (!run_matmul_device_ws(plan.gu, gu_view, input, gate_up, gu_type, hidden, 2 * half, stream, mm_ws, mm_bytes, norm_w, eps, false)) return false;
-    if (plan.dn.converts && M <= 65535) {              // (more rows are refused below)
+    if (gates_in_conversion(plan, M)) {
         const TSHipTensorView2D gate_view{gu, M, half, 2 * half, 1, gu_view.raw_bytes};
         return run_matmul_device_ws(plan.dn, residual, gate_view, down, dn_type, half, hidden, stream, mm_ws, mm_bytes, nullptr, 0.f, true, true);
     }
@@ -673,7 +677,7 @@ ExpertSetLayout expert_set_layout(int M, int n, const ExpertFfn* ex, int H, int 
     auto take = [&](size_t b) { const size_t o = off; off += al(b); return o; };
     L.act_off = take((size_t)rows * ld * sizeof(float));
     L.dn_off = take((size_t)rows * N * sizeof(float));
-    L.tmp_off = take((size_t)rows * I * sizeof(float));
+    L.tmp_off = 0;                   // (the gated rows are formed by the conversion of the down projections' activations)
     L.x1_off = take(gemm_workspace_bytes((int)rows, H));
     L.x2_off = take(gemm_workspace_bytes((int)rows, I));
     L.tbl_bytes = al((size_t)max_tiles * 4) * 3 + al((size_t)n * 8) + al((size_t)rows * 4);

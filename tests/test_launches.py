@@ -152,3 +152,34 @@ def test_cache_rows_per_group_of_lanes(stub, heads, kv, position, rows):
     (log,) = stub(LAYER, cases=[(heads, kv, 64, position)])
     (attention,) = launches(log, "attn_decode_kernel")
     assert f"ELi{rows}EEEvP" in attention[1], attention
+
+
+SCRATCH = """
+def blocks(rows, k): return space(rows * k // 32 * 34)
+x, r, nw = np.zeros((M, H), np.float32), np.zeros((M, H), np.float32), space(4 * H)
+plan = (C.c_int64 * 4)()
+def workspace(rows, n, k, add):
+    assert L.TSHip_MatmulPlanDevice(8, rows, k, n, add, 0, plan)
+    return plan[3]
+gu, dn = blocks(2 * F, H), blocks(H, F)
+x16 = N.TensorView2D(x.ctypes.data & ~15, M, H, H, 1, 4 * M * H)
+r16 = N.TensorView2D(r.ctypes.data & ~15, M, H, H, 1, 4 * M * H)
+assert L.TSHip_FusedFFNSwiGLUQuantF32Device(r16, x16, nw.ctypes.data, H, 1e-6, gu.ctypes.data, 8, H, 2 * F, gu.size, dn.ctypes.data, 8, F, H, dn.size, F)
+out.append([log(), 8 * M * F + max(workspace(M, 2 * F, H, 0), workspace(M, H, F, 1))])
+n = 3
+w = (C.c_void_p * n)(*[gu.ctypes.data] * n)
+d = (C.c_void_p * n)(*[dn.ctypes.data] * n)
+up = (8, H, F, F * H // 32 * 34)
+stream = C.c_void_p(1 << 20)                    # (a buffer of its own)
+L.TSHip_SetStream(stream)
+assert L.TSHip_MoEExpertsSwiGLUForwardF32Device(r16, x16, n, w, w, d, *up, *up, 8, F, H, dn.size, (C.c_float * n)(1, 1, 1)), L.TSHip_GetLastError()
+out.append([log(), n * M * (8 * F + 4 * H + 2 * H + 2 * F)])
+"""
+
+
+def test_scratch_of_gated_rows_is_not_reserved_where_the_conversion_forms_them(stub):
+    """[gate | up], the results and the converted activations, but no M x F floats of gated rows."""
+    M, H, F = 64, 1024, 1024
+    for log, need in stub(SCRATCH, M=M, H=H, F=F):
+        (got,) = [int(l[1]) for l in log if l[0] == "malloc"]
+        assert need <= got / 1.25 < need + 4 * M * F, (got / 1.25, need)
