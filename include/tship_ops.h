@@ -318,7 +318,9 @@ TSHIP_EXPORT int TSHip_MulMatIdF32Device(TSHipTensorView3D result, TSHipTensorVi
  * activation mode run a build of the kernel in which every wavefront writes 64-bit words at byte offset
  * 64 * (workgroup * 8 + wavefront) of the buffer: the 100 MHz constant-clock times of [0] its entry, [1] the arrival of its
  * activations, [2] the barrier behind the staging, [3] the end of its first weight step, [4] its exit, and [5] (XCC id |
- * problem index << 8 | wavefront index << 16).  Launches with more wavefronts than capacity_bytes / 64 run the normal kernel.  Pass a null buffer to switch it off.  For profiling runs only
+ * problem index << 8 | wavefront index << 16).  Launches with more wavefronts than capacity_bytes / 64 run the normal kernel.
+ * Few and long rows, whose steps the wavefronts of a workgroup share otherwise, are stamped wavefront by row group (their sums then
+ * differ in the last bit).  Pass a null buffer to switch it off.  For profiling runs only
  * (bench.py --timeline); not thread-safe. */
 TSHIP_EXPORT int TSHip_SetGemvTimeline(void* device_buffer, int64_t capacity_bytes);
 

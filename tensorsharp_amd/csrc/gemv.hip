@@ -1761,7 +1761,8 @@ bool launch_gemv_group(int type, int count, const GemvArgs* args, hipStream_t st
     static constexpr int kSplitSteps[3][kWaves - 1] = {{6, 7, 8, 10, 14, 30, 40},        // Q8_0
                                                        {8, 9, 10, 12, 16, 24, 48},      // MXFP4, Q4_0, Q4_1
                                                        {7, 8, 10, 12, 16, 24, 48}};     // Q5_0, Q5_1, IQ4_NL
-    if (count == 1 && lpr == 16 && !args[0].expert_id && !args[0].slot_ids && !args[0].pair_rows && act != kActSiluMul && !g_timeline) {
+    if (count == 1 && lpr == 16 && !args[0].expert_id && !args[0].slot_ids && !args[0].pair_rows && act != kActSiluMul &&
+        (act != kActPlain || !g_timeline)) {          // (stamped launches run unsplit)
         const int groups = (args[0].N + rpg - 1) / rpg, steps = (args[0].K / unit_elems(type) + lpr - 1) / lpr;
         const int per_wg = (groups + di.num_cus - 1) / di.num_cus;
         const int cls = type == kTypeQ8_0 ? 0 : type == kTypeMXFP4 || type == kTypeQ4_0 || type == kTypeQ4_1 ? 1 : 2;

@@ -183,3 +183,12 @@ def test_scratch_of_gated_rows_is_not_reserved_where_the_conversion_forms_them(s
     for log, need in stub(SCRATCH, M=M, H=H, F=F):
         (got,) = [int(l[1]) for l in log if l[0] == "malloc"]
         assert need <= got / 1.25 < need + 4 * M * F, (got / 1.25, need)
+
+
+def test_only_stamped_launches_leave_the_split_kernel(stub):
+    """While a timeline buffer is set, plain launches of few and long rows run unsplit; those with the RMSNorm are not stamped."""
+    on = "assert L.TSHip_SetGemvTimeline(C.c_void_p(4096), 1 << 20)\n"
+    cases = [(*BLOCKS["q8_0"], 512, 8192, norm, 0) for norm in (0, 1)]
+    for plain, norm in (stub(GEMV_LINEAR, cases=cases), stub(on + GEMV_LINEAR, cases=cases)):
+        assert len(launches(norm, "gemv_split_kernel")) == 1
+    assert not launches(plain, "gemv_split_kernel")
