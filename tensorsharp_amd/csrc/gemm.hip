@@ -1694,6 +1694,7 @@ constexpr int kWideValu = (40 + 2 * TM - 1) / (2 * TM);
 //   Q8_0 512 x 14336 x 4096 87.4 -> 80.4, 200 x 4096 x 14336 77.7 -> 52.6, 48 x 21504 x 5376 56.1 -> 45.5
 //   Q6_K 333 x 4096 x 14336 100.3 -> 94.5, 200 x 4096 x 14336 95.7 -> 64.1, 200 x 21504 x 5376 141.2 -> 125.5;
 //        with the unrolled loop 333 x 4096 x 14336 80.9, FFN of 200 rows with a Q6_K down projection 185.7 -> 177.4
+//        (tiles of 128 rows: 256 registers, 6 more in scratch memory)
 // ------------------------------------------------------------------------------------------
 // Weight formats as this kernel reads them.  A granule is the raw bytes of kSup consecutive k-tiles of one row, kept in LDS
 // as kRawRow bytes (an odd multiple of four dwords: the dword reads of 32 rows spread over the most banks that 16-byte
@@ -2084,27 +2085,27 @@ __global__ void __launch_bounds__(512) gemm_wide_kernel(const GemmArgs A)
         uint32_t ra[NB][H::kQ], rb[NB][H::kQ], hdr[NB][H::kHdr], state[NB][H::kState];
         auto fetch_hdr = [&](int kt) {
             const int s = kt / H::kSup, j = kt % H::kSup;
-    #pragma unroll
+#pragma unroll
             for (int n = 0; n < NB; ++n) H::fetch_hdr(row_of(s, n), j, h, delta_of(s, n), hdr[n]);
         };
         auto fetch = [&](int kt, int q, uint32_t (&r)[NB][H::kQ]) {
             const int s = kt / H::kSup, j = kt % H::kSup;
-    #pragma unroll
+#pragma unroll
             for (int n = 0; n < NB; ++n) H::fetch(row_of(s, n), j, h, delta_of(s, n), q, r[n]);
         };
         auto prepare = [&](int kt) {
             const int s = kt / H::kSup, j = kt % H::kSup;
             const bool live_k = (kt < nkt) & ((kt * 2 + h) * 32 < A.K);      // past the unit's end the raw bytes are zeros or stale
-    #pragma unroll
+#pragma unroll
             for (int n = 0; n < NB; ++n) H::prepare(hdr[n], j, h, delta_of(s, n), live_k & in_n[n], g, state[n], bad[n]);
         };
         auto unpack = [&](int kt, int q, int slot, uint32_t (&r)[NB][H::kQ]) {
             const int s = kt / H::kSup, j = kt % H::kSup;
-    #pragma unroll
+#pragma unroll
             for (int n = 0; n < NB; ++n) {
                 uint32_t v[4];
                 H::unpack(r[n], state[n], j, h, delta_of(s, n), q, v);
-    #pragma unroll
+#pragma unroll
                 for (int i = 0; i < 4; ++i) o[n][4 * slot + i] = v[i];
             }
         };
@@ -3087,11 +3088,11 @@ __global__ void __launch_bounds__(512) gemm_slim_mx_kernel(const GemmArgs A)
                 asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");    // the reads are done: the buffers may be written again
             }
         } else {
-    #pragma unroll
+#pragma unroll
             for (int rb = 0; rb < RB; ++rb) {
                 const int ml = col + 32 * rb;
                 const uint32_t xrow = (uint32_t)(m0 + min(ml, m_rows - 1)) * (uint32_t)(A.xld * 2);
-    #pragma unroll
+#pragma unroll
                 for (int t = 0; t < KTW; ++t) {
                     const bool on = ml < m_rows && t < kcnt;
                     const uint32_t xt = on ? xrow + (uint32_t)(kt0 + t) * 128u : kDeadOffset;
@@ -3848,17 +3849,22 @@ namespace {
 // residual.  On 300 further random calls per format the pick took 0.4 % (Q4_K), 0.3 % (Q8_0) and 0.2 % (Q6_K) longer than the
 // fastest candidate on average, more than 4 % longer on 11, 8 and 3 of them, 11 % at most.
 // slim_rows was measured again with the activations in pieces (see gemm_slim_kernel), on 350 (300) calls per format of 2 .. 150
-// rows, 512 .. 21504 columns and K of 1024 .. 14336: with the first fit's value, slim_rows_far, the pick would now be 2.8 / 0.4 /
-// 0.2 % behind (Q4_K / Q8_0 / Q6_K), with this one 0.5 / 0.2 / 0.1 %.
-// Where the lines lie, us (register-resident / gemm_wide_kernel / 128 rows / 256 rows):
-//   Q4_K  8 x 4096 x 4096 12.4 / 16.3 / - / -,  64 x 4096 x 4096 17.4 / 21.0 / 28.5 / 34.0,  200 x 4096 x 4096 38.5 / 28.3 / 32.2 /
-//         39.8,  1024 x 9728 x 2560 151 / 85.8 / 104.7 / 68.7
-//   Q8_0  8 x 14336 x 4096 23.2 / 24.0 / - / -,  128 x 28672 x 4096 90.7 / 60.0 / 67.0 / 76.6,  400 x 4096 x 4096 - / 39.2 / 37.4 / -
-//   Q6_K  512 x 4096 x 4096 - / 47.5 / 45.1 / -,  2048 x 2560 x 9728 - / 200.8 / 240.7 / -
+// rows, 512 .. 21504 columns and K of 1024 .. 14336: with the first fit's value (6.588 / 5.523 / 6.414 for Q4_K / Q8_0 / Q6_K) the
+// pick would be 2.8 / 0.4 / 0.2 % behind there, with this one 0.5 / 0.2 / 0.1 %.  Above 160 rows and under 1024 columns slim_rows_far
+// still serves, the first fit's value or near it: the kernels do not cross at these edges, more had not been measured.  On 3600
+// calls per format since then, 4 .. 2048 rows and 64 columns on, the pick is 1.6 / 0.4 / 1.2 % behind the fastest candidate (Q4_K 1.9
+// with 6.588); slim_rows throughout with a term for the conversion, and gemm_wide_kernel of Q6_K at 0.84 of its k-tile, would make that
+// 0.3 / 0.2 / 0.1 %.
+// The candidates now, us (register-resident / gemm_wide_kernel / 128 rows / 256 rows):
+//   Q4_K  8 x 4096 x 5376 15.8 / 20.6 / - / -,  64 x 828 x 2560 12.4 / 15.9 / - / 28.5,  64 x 9728 x 9728 47.6 / 42.3 / - / 72.6,
+//         200 x 4096 x 2560 28.3 / 28.0 / - / 34.8,  257 x 512 x 14336 39.2 / 32.0 / - / 84.9,  480 x 9728 x 9728 (added) - / 142 / - / 124
+//   Q8_0  24 x 14336 x 4096 26.4 / 29.5 / - / -,  64 x 14336 x 4096 33.3 / 34.7 / 39.7 / 46.3,  128 x 9728 x 5376 54.8 / 45.1 / 56.2 / 64.6,
+//         400 x 4096 x 4096 - / 41.1 / 41.5 / 48.5,  400 x 9728 x 9728 - / 146 / 173 / 125
+//   Q6_K  64 x 9728 x 9728 54.8 / 52.3 / 78.3 / -,  240 x 9728 x 14336 (added) 230 / 121 / 145 / -,  480 x 14336 x 4096 - / 94.8 / 114 / -
 struct RuleCosts {
-    // register-resident kernel: a call; its activations, per 32 rows and 8 k-tiles per wavefront (and beyond the
-    // calls that slim_rows was fitted to); a round of units and per k-tile of a wavefront in it; a workgroup whose units cross into another
-    // row tile or K chunk (it loads activations anew)
+    // register-resident kernel: a call; its activations, per 32 rows and 8 k-tiles per wavefront (slim_rows_far: above 160 rows, or 32
+    // under 1024 columns); a round of units and per k-tile of a wavefront in it; a workgroup whose units cross into another row
+    // tile or K chunk (it loads activations anew)
     double slim, slim_rows, slim_rows_far, unit, unit_kt, cross, cross_kt;
     // gemm_wide_kernel: a call, a k-tile of a round and per 32 rows in it, the share of that time that an almost empty round
     // takes, a round
@@ -3963,6 +3969,7 @@ int gemm_tile_m(int type, int M, int N, int K, bool accumulate, size_t max_chunk
     if (type == kTypeQ4_K) return cheapest_tiles<GQ4K>(kCostsQ4K, M, N, K, accumulate, max_chunk_bytes, wide);
     if (type == kTypeQ8_0) return cheapest_tiles<GQ80>(kCostsQ80, M, N, K, accumulate, max_chunk_bytes, wide);
     if (type == kTypeQ6_K) return cheapest_tiles<GQ6K>(kCostsQ6K, M, N, K, accumulate, max_chunk_bytes, wide);
+    // (drawn while the register-resident kernel read its activations from whole rows; not measured since)
     if (M <= 128) return 32;
     if (type == kTypeMXFP4 && M <= 512 && ((M + 127) / 128) * ((N + 127) / 128) <= 128) return 32;
     // 128- or 256-row tiles by rounds of workgroups x time per k-tile of a round (measured per k-tile: a 256 x 256 tile

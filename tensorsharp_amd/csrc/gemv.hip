@@ -802,7 +802,7 @@ struct FmtQ6K {
         // 128256 x 4096, the loads being the limit then, see below).
         // The quad holds the block, and the dword behind a lane's piece is one that another lane has loaded.  Loading it again,
         // and scales and d dword by dword, made nine load instructions of what are now four, and the address unit was what
-        // the launch waited for: 128256 x 4096 91.1 -> 77.1 us (4.7 -> 5.6 TB/s), 14336 x 4096 14.2 -> 11.4.
+        // the launch waited for: 128256 x 4096 91.1 -> 77.1 us (4.7 -> 5.6 TB/s), 14336 x 4096 13.1 -> 11.4.
         const bool j = L.sc_shift != 0, n = L.off_s != 192u;
         const uint32_t a4 = TSHIP_DPP_U(j ? w[0] : w[4], kDppXor1);                      // 16 bytes on: the other half, the other piece
         const uint32_t b4 = TSHIP_DPP_U(j ? w[4] : n ? w[0] : w[8], kDppNext);           // piece B: the next lane's B, A of n = 1, H of lane 0
@@ -1675,8 +1675,8 @@ bool launch_gemv_group(int type, int count, const GemvArgs* args, hipStream_t st
     const int budget = di.num_cus * per_cu;
     // (More workgroups than the CUs hold at once, so that later ones start while earlier ones stream, was measured slower:
     // the 123 MB grouped launch 28.0 us with 1.5 x and 2 x the workgroups against 24.3 us.)
-    // (Cutting the K range of a row group over several wavefronts when a matrix has few rows was measured slower on
-    // every shape: 4096 x 14336 Q4_K 13.7 vs 10.9 us, MXFP4 5760 x 2880 7.8 vs 6.7 us.  Requesting more up front - two extra
+    // (Cutting the K range of a row group over several wavefronts is slower for the 32-lane formats, and for the 16-lane ones short
+    // of the line of the split build below: 4096 x 14336 Q4_K 13.7 vs 10.9 us, MXFP4 5760 x 2880 7.8 vs 6.7 us.  Requesting more up front - two extra
     // steps before x is staged, or a ring of four steps per wavefront - was slower too, the 123 MB grouped launch
     // included: 24.5 vs 24.2 us.)
 

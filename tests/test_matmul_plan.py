@@ -82,6 +82,8 @@ def test_a_bounded_workspace_keeps_as_many_chunks_as_fit(t, rows, n, k, accumula
 
 # measured us of a call, conversion included, weights from HBM: register-resident kernel, the best tiling of the wide kernel, 128- and
 # 256-row tiles (None: not a candidate, or not measured)
+# (of the kernels that the rule's constants were first fitted to: the register-resident kernel with whole rows of activations, the wide
+# kernel of Q6_K before its loop was unrolled; both are faster now, the picks asserted here are those of that fit)
 MEASURED = [
     (Q4_K, 8, 4096, 4096, 12.44, 16.28, None, None),
     (Q4_K, 24, 14336, 4096, 21.49, 22.75, 29.53, None),
