@@ -699,10 +699,10 @@ class HipBasicOps:
     def UseCurrentStream():
         """Launch the *Device entry points on torch's current stream."""
         torch = _torch()
-        raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
-        get_device = getattr(torch._C, "_cuda_getDevice", None)
-        if raw_stream is not None and get_device is not None and torch.cuda.is_initialized():
-            handle = raw_stream(get_device())                   # current_stream().cuda_stream without the stream object
-        else:
+        try:                                    # current_stream().cuda_stream without the stream object
+            handle = torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice()) if torch.cuda.is_initialized() else None
+        except AttributeError:                  # (private names, which a torch build may lack)
+            handle = None
+        if handle is None:
             handle = torch.cuda.current_stream().cuda_stream
         N.lib().TSHip_SetStream(handle)
