@@ -5,7 +5,7 @@
 //      magnitude overflows or underflows fp16), written in the k-order in which the weight
 //      format unpacks (so the dequantizer never has to shuffle lanes), zero-padded to a
 //      multiple of the k-tile.  Optionally gathers rows through an index (MoE).
-//   2. by size (gemm_tile_m) gemm_slim_kernel (32 rows per tile: activations in registers, K split over the wavefronts,
+//   2. by size (gemm_tile_m) gemm_slim_kernel / gemm_slim32_kernel (32 rows per tile: activations in registers, K split over the wavefronts,
 //      long K in chunks), gemm_wide_kernel (32 .. 128 rows x 256 columns, K in chunks that fill the chip) or
 //      gemm_xw_kernel / gemm_kernel (128 / 256 rows per tile).  gemm_kernel:
 //      BM x 256 x 64 tiles, eight wavefronts, each owning 32 output columns.  The fp16
@@ -114,12 +114,12 @@ __device__ __forceinline__ int k_slot(int k)
         const int idx = sub * 8 + 2 * (c >> 2) + (b & 1);
         return (idx >> 2) * 16 + hh * 8 + 2 * (idx & 3) + (b >> 1);
     }
-    if (TYPE == kTypeMXFP4) {     // also the order of Q4_0, Q4_1, Q5_0, Q5_1, IQ4_NL
+    if (TYPE == kTypeMXFP4) {     // also the order of Q5_0, Q5_1, IQ4_NL
         // block k/32; quant byte i = k%16 holds elements i (low nibble) and i + 16 (high nibble)
         const int hh = k >> 5, i = k & 15, hi = (k >> 4) & 1;
         return (i >> 2) * 16 + hh * 8 + 2 * (i & 3) + hi;
     }
-    // Q8_0 and Q6_K: 32-element group k/32, natural order
+    // Q8_0, Q6_K, Q4_0, Q4_1 and Q4_K on the register-resident and the wide kernel: 32-element group k/32, natural order
     const int hh = k >> 5, tt = k & 31;
     return (tt >> 3) * 16 + hh * 8 + (tt & 7);
 }
@@ -481,50 +481,49 @@ __global__ void __launch_bounds__(kMxCvtBlocks) convert_x_mx_kernel(const Conver
 //              the delta inside that window; window_bytes() / tile_offset(): the same for windows of any number
 //              of k-tiles (the register-resident kernel)
 // ------------------------------------------------------------------------------------------
+// Q4_K for the register-resident kernel, in natural order: k-half h is sub-block 2 j + h, the nibbles h of a k-tile's 32 quant bytes.
+// A byte 0 .. 15 read as fp8 (E4M3) is that many 2^-9, so the conversion with a scale of 2^9 gives two exact fp16 integers: six vector
+// instructions per four weights where masking into 1024 + q and subtracting takes seven, and nothing of 32 bits but masks and shifts,
+// which issue twice as fast (2 cycles per wavefront; conversions, packed and three-operand instructions 4).
 struct GQ4K {
-    static constexpr int kRegs = 8;
+    static constexpr int kRegs = 12;
     static constexpr int kTileStep = 4;       // a wavefront's K range starts at a multiple of this many k-tiles
-    static constexpr uint32_t sup_offset(int s) { return (uint32_t)s * 144u; }            // window start of super-tile s
-    static __device__ __forceinline__ uint32_t sup_delta(uint32_t delta, int /*s*/) { return delta; }
     static constexpr int window_bytes(int ktw) { return ktw * 36; }                       // of ktw consecutive k-tiles
     static constexpr uint32_t tile_offset(int kt0) { return (uint32_t)kt0 * 36u; }        // kt0 a multiple of kTileStep
-    static __device__ __forceinline__ void fetch(const uint8_t* rp, int t, int h, uint32_t /*delta*/, uint32_t (&r)[kRegs])
+    static __device__ __forceinline__ void fetch(const uint8_t* rp, int t, int /*h*/, uint32_t /*delta*/, uint32_t (&r)[kRegs])
     {
         rp += (t >> 2) * 144;
         const int j = t & 3;
         const uint4_t hdr = *reinterpret_cast<const uint4_t*>(rp);
-        const uint4_t q = *reinterpret_cast<const uint4_t*>(rp + 16 + j * 32 + h * 16);
+        const uint4_t q0 = *reinterpret_cast<const uint4_t*>(rp + 16 + j * 32), q1 = *reinterpret_cast<const uint4_t*>(rp + 32 + j * 32);
         r[0] = hdr.x; r[1] = hdr.y; r[2] = hdr.z; r[3] = hdr.w;
-        r[4] = q.x; r[5] = q.y; r[6] = q.z; r[7] = q.w;
+        r[4] = q0.x; r[5] = q0.y; r[6] = q0.z; r[7] = q0.w;
+        r[8] = q1.x; r[9] = q1.y; r[10] = q1.z; r[11] = q1.w;
     }
-    // o[0..7]: low nibbles (sub-block 2j, elements 16h..16h+15), o[8..15]: high nibbles (sub-block 2j+1)
     static constexpr uint32_t kLimit = 0x2c00u;      // |d|, |dmin| <= 2^-4: 15 * 63 * d * 2^kWShift stays finite in fp16
     static __device__ __forceinline__ bool out_of_range(uint32_t mark) { return over2(mark, kLimit, kLimit); }
     // (blocks past the end of K or N arrive as zeros, whose scale is in range: `live` is not needed)
-    static __device__ __forceinline__ void dequant(const uint32_t (&r)[kRegs], int j, int /*h*/, uint32_t /*delta*/, bool /*live*/,
+    static __device__ __forceinline__ void dequant(const uint32_t (&r)[kRegs], int t, int h, uint32_t /*delta*/, bool /*live*/,
                                                    uint32_t (&o)[16], uint32_t& bad)
     {
-        const int sh = (j & 1) * 16;
+        const int j = t & 3, sh = (j & 1) * 16;
         const uint32_t a = r[1] >> sh, b = r[2] >> sh, c = r[3] >> sh;
-        const uint32_t sc_lo = a & 0x3f3fu, m_lo = b & 0x3f3fu;
-        const uint32_t sc_hi = (c & 0x0f0fu) | ((a >> 2) & 0x3030u);
-        const uint32_t m_hi = ((c >> 4) & 0x0f0fu) | ((b >> 2) & 0x3030u);
-        const uint32_t sc = (j & 2) ? sc_hi : sc_lo, mn = (j & 2) ? m_hi : m_lo;
+        const uint32_t hi = 0u - (uint32_t)(j >> 1);                    // sub-blocks 4 .. 7: all ones (a mask: k-tiles differ by lane)
+        const uint32_t sc = (((c & 0x0f0fu) | ((a >> 2) & 0x3030u)) & hi) | (a & 0x3f3fu & ~hi);
+        const uint32_t mn = ((((c >> 4) & 0x0f0fu) | ((b >> 2) & 0x3030u)) & hi) | (b & 0x3f3fu & ~hi);
         H2U dm;
         dm.u = r[0];
         mark2(bad, r[0]);
-        const float d = (float)dm.h.x, dmin = (float)dm.h.y * kWUp;
-        const uint32_t s1 = splat(d * kWUp * (float)(sc & 0xffu)), o1 = splat(-(dmin * (float)(mn & 0xffu)));
-        const uint32_t s2 = splat(d * (float)(sc >> 8) * (0.0625f * kWUp)), o2 = splat(-(dmin * (float)(mn >> 8)));
-        const uint32_t magic = 0x64006400u, neg1024 = 0xe400e400u;   // 1024.0, -1024.0
+        const float d = (float)dm.h.x * kWUp, dmin = (float)dm.h.y * kWUp;
+        const uint32_t s = splat(d * (float)((sc >> (8 * h)) & 0xffu)), m = splat(-(dmin * (float)((mn >> (8 * h)) & 0xffu)));
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const uint32_t q = r[4 + i], q8 = q >> 8;
-            // 0x6400 | nibble = 1024 + q (low) or 1024 + 16 q (high): exact after subtracting 1024
-            o[2 * i] = pk_fma(pk_add((q & 0x000f000fu) | magic, neg1024), s1, o1);
-            o[2 * i + 1] = pk_fma(pk_add((q8 & 0x000f000fu) | magic, neg1024), s1, o1);
-            o[8 + 2 * i] = pk_fma(pk_add((q & 0x00f000f0u) | magic, neg1024), s2, o2);
-            o[8 + 2 * i + 1] = pk_fma(pk_add((q8 & 0x00f000f0u) | magic, neg1024), s2, o2);
+        for (int i = 0; i < 8; ++i) {
+            const uint32_t q = (r[4 + i] >> (4 * h)) & 0x0f0f0f0fu;
+            H2U lo, up;
+            lo.h = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(q, 512.f, false);
+            up.h = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(q, 512.f, true);
+            o[2 * i] = pk_fma(lo.u, s, m);
+            o[2 * i + 1] = pk_fma(up.u, s, m);
         }
     }
 };
@@ -750,6 +749,7 @@ struct GLegacy {
     static constexpr int kBlock = kHdr + 16;
     static constexpr bool kMin = TYPE == kTypeQ4_1 || TYPE == kTypeQ5_1;
     static constexpr bool kFive = TYPE == kTypeQ5_0 || TYPE == kTypeQ5_1;
+    static constexpr bool kNatural = TYPE == kTypeQ4_0 || TYPE == kTypeQ4_1;      // activations in natural order, else split nibbles
     static constexpr int kWords = (kBlock + 3) / 4;        // aligned dwords of one block
     static constexpr int kRegs = kWords + 1;
     static constexpr int kSup = 2;                          // four blocks
@@ -787,6 +787,7 @@ struct GLegacy {
             m2 = pk_mul(mbits | (mbits << 16), kWUp2);
         } else {
             mark2(bad, dbits);
+            if (TYPE == kTypeQ4_0) m2 = pk_mul(d2, 0xc800c800u);        // -8 d, exact
         }
         uint32_t qh = 0u;
         if constexpr (kFive) qh = (kHdr & 3) ? __builtin_amdgcn_alignbyte(b[kHdr / 4], b[kHdr / 4 - 1], 2) : b[kHdr / 4 - 1];
@@ -799,6 +800,18 @@ struct GLegacy {
                 // bits 4 w .. 4 w + 3 (elements j) and 16 + 4 w .. (elements j + 16) of qh, one per byte, at bit 4
                 lo |= ((((qh >> (4 * w)) & 0xfu) * 0x00204081u) & 0x01010101u) << 4;
                 hi |= ((((qh >> (16 + 4 * w)) & 0xfu) * 0x00204081u) & 0x01010101u) << 4;
+            }
+            if constexpr (kNatural) {
+                // as Q4_K: nibbles read as fp8; d (q - 8) as d q - 8 d and d q + m are rounded once, by the fused multiply-add
+#pragma unroll
+                for (int s2 = 0; s2 < 2; ++s2) {
+                    H2U vl, vh;
+                    vl.h = s2 ? __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(lo, 512.f, true) : __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(lo, 512.f, false);
+                    vh.h = s2 ? __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(hi, 512.f, true) : __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(hi, 512.f, false);
+                    o[2 * w + s2] = pk_fma(vl.u, d2, m2);
+                    o[8 + 2 * w + s2] = pk_fma(vh.u, d2, m2);
+                }
+                continue;
             }
             uint32_t bias;
             if (TYPE == kTypeIQ4_NL) {
@@ -1193,6 +1206,7 @@ __global__ void __launch_bounds__(NW * 64) gemm_kernel(const GemmArgs A)
 // ------------------------------------------------------------------------------------------
 struct PQ4K {
     typedef GQ4K G;
+    static constexpr int kRegs = 8;
     static constexpr int kParts = 3;                  // header + the k-tile's 32 quant bytes
     static constexpr int kRowBytes = 48;
     static __device__ __forceinline__ uint32_t part_base(int part) { return part == 0 ? 0u : 16u * (uint32_t)part; }
@@ -1204,14 +1218,14 @@ struct PQ4K {
     static __device__ __forceinline__ uint32_t row_window(uint32_t row_start) { return row_start; }
     static __device__ __forceinline__ uint32_t row_delta(uint32_t /*row_start*/) { return 0u; }
     static __device__ __forceinline__ uint32_t delta(uint32_t /*d0*/, int /*kt*/) { return 0u; }
-    static __device__ __forceinline__ void fetch(const uint8_t* rp, int h, uint32_t /*delta*/, uint32_t (&r)[G::kRegs])
+    static __device__ __forceinline__ void fetch(const uint8_t* rp, int h, uint32_t /*delta*/, uint32_t (&r)[kRegs])
     {
         const uint4_t hdr = *reinterpret_cast<const uint4_t*>(rp);
         const uint4_t q = *reinterpret_cast<const uint4_t*>(rp + 16 + h * 16);
         r[0] = hdr.x; r[1] = hdr.y; r[2] = hdr.z; r[3] = hdr.w;
         r[4] = q.x; r[5] = q.y; r[6] = q.z; r[7] = q.w;
     }
-    // The unpacking of one lane's 32 weights of a k-tile (GQ4K::dequant) cut into kMicro small steps that the kernel
+    // The unpacking of one lane's 32 weights of a k-tile cut into kMicro small steps that the kernel
     // places one by one behind its matrix instructions; step I may use what steps < I left in `st` and `o`.
     // Quarter q of `o` (o[4 q .. 4 q + 3], the B operand of k-step q) is complete after step kReady[q].
     static constexpr int kMicro = 17;
@@ -1231,7 +1245,7 @@ struct PQ4K {
     };
     static __device__ __forceinline__ int ready_after(int quarter) { return quarter == 0 ? 10 : quarter == 2 ? 10 : 16; }
     template <int I>
-    static __device__ __forceinline__ void micro(State& st, const uint32_t (&r)[G::kRegs], int j, int /*h*/, uint32_t /*delta*/, bool /*live*/,
+    static __device__ __forceinline__ void micro(State& st, const uint32_t (&r)[kRegs], int j, int /*h*/, uint32_t /*delta*/, bool /*live*/,
                                                  const Consts& K, uint32_t (&o)[16], uint32_t& bad)
     {
         if constexpr (I == 0) {
@@ -1281,6 +1295,7 @@ struct PQ4K {
 // bytes every odd k-tile adds), which GMXFP4's unpacker takes as its byte shift.
 struct PMXFP4 {
     typedef GMXFP4 G;
+    static constexpr int kRegs = G::kRegs;
     static constexpr int kParts = 3;
     static constexpr int kRowBytes = 48;
     static __device__ __forceinline__ uint32_t part_base(int part) { return 16u * (uint32_t)part; }
@@ -1291,7 +1306,7 @@ struct PMXFP4 {
     static __device__ __forceinline__ uint32_t row_window(uint32_t row_start) { return row_start & ~3u; }
     static __device__ __forceinline__ uint32_t row_delta(uint32_t row_start) { return row_start & 3u; }
     static __device__ __forceinline__ uint32_t delta(uint32_t d0, int kt) { return d0 + (((uint32_t)kt & 1u) << 1); }
-    static __device__ __forceinline__ void fetch(const uint8_t* rp, int h, uint32_t delta, uint32_t (&r)[G::kRegs])
+    static __device__ __forceinline__ void fetch(const uint8_t* rp, int h, uint32_t delta, uint32_t (&r)[kRegs])
     {
         G::fetch(rp, 0, h, delta, r);
     }
@@ -1304,7 +1319,7 @@ struct PMXFP4 {
     };
     struct Consts {};
     template <int I>
-    static __device__ __forceinline__ void micro(State& st, const uint32_t (&r)[G::kRegs], int /*j*/, int h, uint32_t delta, bool live,
+    static __device__ __forceinline__ void micro(State& st, const uint32_t (&r)[kRegs], int /*j*/, int h, uint32_t delta, bool live,
                                                  const Consts&, uint32_t (&o)[16], uint32_t& bad)
     {
         if constexpr (I == 0) {
@@ -1329,6 +1344,17 @@ struct PMXFP4 {
         }
     }
 };
+
+// all steps of the unpacking of a lane's 32 weights
+template <typename P, int I = 0>
+__device__ __forceinline__ void unpack_all(typename P::State& st, const uint32_t (&r)[P::kRegs], int j, int h, uint32_t delta, bool live,
+                                           const typename P::Consts& K, uint32_t (&o)[16], uint32_t& bad)
+{
+    if constexpr (I < P::kMicro) {
+        P::template micro<I>(st, r, j, h, delta, live, K, o, bad);
+        unpack_all<P, I + 1>(st, r, j, h, delta, live, K, o, bad);
+    }
+}
 
 template <typename P, int BM, int WN>
 __global__ void __launch_bounds__(128 * WN) gemm_xw_kernel(const GemmArgs A)
@@ -1474,9 +1500,10 @@ __global__ void __launch_bounds__(128 * WN) gemm_xw_kernel(const GemmArgs A)
     }
 #pragma unroll
     for (int u = 0; u < DUTY; ++u) {
-        uint32_t r0[G::kRegs], o0[16];
+        uint32_t r0[P::kRegs], o0[16];
+        typename P::State first;
         P::fetch(rraw + (kt_begin & (ST - 1)) * kRawTile + my_raw + u * 32 * P::kRowBytes, h, P::delta(my_d0[u], kt_begin), r0);
-        G::dequant(r0, P::phase(kt_begin), h, P::delta(my_d0[u], kt_begin), (kt_begin * 2 + h) * 32 < A.K && in_n[u], o0, bad[u]);
+        unpack_all<P>(first, r0, P::phase(kt_begin), h, P::delta(my_d0[u], kt_begin), (kt_begin * 2 + h) * 32 < A.K && in_n[u], typename P::Consts(), o0, bad[u]);
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
             const uint4_t v = {o0[4 * ks], o0[4 * ks + 1], o0[4 * ks + 2], o0[4 * ks + 3]};
@@ -1485,7 +1512,7 @@ __global__ void __launch_bounds__(128 * WN) gemm_xw_kernel(const GemmArgs A)
     }
     __syncthreads();
     half8_t a0[TMW], b0[NB], a1[TMW], b1[NB];
-    uint32_t r[DUTY][G::kRegs];
+    uint32_t r[DUTY][P::kRegs];
 #pragma unroll
     for (int j = 1; j < ST; ++j) {
 #pragma unroll
@@ -2651,12 +2678,20 @@ bool launch_mx(GemmArgs a, int m_tiles, hipStream_t stream, const ChunkScratch& 
 // ------------------------------------------------------------------------------------------
 // At most 32 activation rows per tile (small batches, MoE experts with few tokens; also single rows of formats
 // without a GEMV kernel).  The activations stay in REGISTERS: the eight wavefronts of a workgroup split K between
-// them (KTW k-tiles each), every wavefront keeps the MFMA A operands of its K range for all 32 rows, and the
-// workgroup walks over 32-column weight tiles.  Per tile a wavefront needs only its own K range of the 32 raw
-// weight rows, which it copies itself (global -> LDS, a private ring of buffers, requested RING tiles ahead), so
-// the main loop has no barrier and no activation traffic at all; the eight partial 32 x 32 sums meet in LDS (in
-// the raw buffer the wavefront has just consumed), are added in a fixed order and stored.  A K longer than
-// 8 * KTW k-tiles is cut into chunks whose sums a second kernel adds.
+// them (KTW k-tiles each), every wavefront keeps the MFMA A operands of its K range for all 16 RB rows, and the
+// workgroup walks over 16-column weight tiles.  Per tile a wavefront needs only its own K range of the 16 raw
+// weight rows, which it copies itself (global -> LDS, a private ring of buffers, requested RING tiles ahead); the
+// eight partial sums of a tile meet in LDS and are added in a fixed order, behind the tile's only barrier where two sets of
+// them fit.  A K longer than 8 * KTW k-tiles is cut into chunks whose sums a second kernel adds.
+// The four groups of 16 lanes of a wavefront take different k-tiles (formats of 256-weight blocks) or half k-tiles (32-weight
+// blocks) and not the four k-slices of one: the scales of a block are then worked out once for 64 (32) weights of a lane.
+// What bounds it (leave-out builds, Q4_K 24 x 14336 x 4096, 13.8 us of the launch): unpacking 3.9 and the weights 4.7 on top of each
+// other, the activations 2.3; the tiles' matrix instructions, sums and barriers are most of the rest.  16 columns instead of 32: twice
+// the units for a chip of 256 CUs and half a tile less at the end; LDS that holds twice the K range per wavefront, so that K = 4096 is
+// one chunk in every format.  Whole calls, weights from HBM, us, with 32-column tiles before -> now: Q4_K 8 x 14336 x 4096 20.0 -> 16.9,
+// 24 x 4096 x 4096 13.5 -> 10.7, 24 x 4096 x 14336 24.8 -> 23.4; Q8_0 16 x 14336 x 4096 25.9 -> 22.0, 16 x 4096 x 4096 15.8 -> 11.7, Q6_K
+// 32 x 4096 x 4096 15.1 -> 12.2, Q5_K 32 x 4096 x 4096 15.3 -> 11.4, 48 x 14336 x 4096 33.0 -> 28.3; weights in the memory-side cache:
+// Q4_K 24 x 14336 x 4096 18.3 -> 18.3 (bound by unpacking and sums, not by the stream).
 // ------------------------------------------------------------------------------------------
 // an address that is the same in every lane, for the compiler to keep in scalar registers
 __device__ __forceinline__ uintptr_t uniform_address(uintptr_t a)
@@ -2666,11 +2701,272 @@ __device__ __forceinline__ uintptr_t uniform_address(uintptr_t a)
 }
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-// LDS layout of one wavefront of the register-resident kernel: RING raw buffers of 32 rows x CH 16-byte chunks
+// LDS layout of the register-resident kernel: per wavefront RING raw buffers of 16 rows x CH 16-byte chunks (the bytes of KTW
+// k-tiles plus the up to three bytes between the 4-byte aligned window start and the first block; the unpackers may read a
+// few bytes further, into the next row, and ignore them), then one or two sets of partial sums.
+template <typename G, int KTW, int RB>
+struct SlimLayout {
+    static constexpr int kLds = 160 * 1024;
+    static constexpr int kNeed = (G::window_bytes(KTW) + 15) / 16;
+    static constexpr int SET = 8 * RB * 1024;                            // partial sums of a tile
+    static constexpr int copies_of(int ch) { return (16 * ch + 63) / 64; }
+    static constexpr int sets_of(int ch) { return 16 * copies_of(ch) * 1024 + 2 * SET <= kLds ? 2 : 1; }
+    static constexpr int ring_of(int ch)
+    {
+        const int fit = (kLds - sets_of(ch) * SET) / (8 * copies_of(ch) * 1024);
+        return fit < 4 ? fit : 4;
+    }
+    // an odd chunk count spreads the dword reads of the rows over twice as many LDS banks; taken when it costs no ring depth
+    static constexpr bool kOdd = (kNeed & 1) == 0 && ring_of(kNeed + 1) == ring_of(kNeed) && sets_of(kNeed + 1) == sets_of(kNeed);
+    static constexpr int CH = kNeed + (kOdd ? 1 : 0);
+    static constexpr int DI = copies_of(CH);                             // LDS-direct copies per buffer
+    static constexpr int BUF = DI * 1024;
+    static constexpr int SETS = sets_of(CH);
+    static constexpr int RING = ring_of(CH);
+    static constexpr size_t kBytes = (size_t)8 * RING * BUF + SETS * SET;
+};
+
+typedef float float4_t __attribute__((ext_vector_type(4)));
+
+template <typename G, int KTW, int RB>
+__global__ void __launch_bounds__(512) gemm_slim_kernel(const GemmArgs A)
+{
+    using L = SlimLayout<G, KTW, RB>;
+    constexpr int CH = L::CH, DI = L::DI, BUF = L::BUF, RING = L::RING, SETS = L::SETS;
+    static_assert(KTW % G::kTileStep == 0, "a wavefront's K range must start at a block");
+    // k-tiles of one step of the K loop, and k-halves of them that a lane unpacks itself
+    constexpr int S = G::kTileStep, HALVES = S == 4 ? 2 : 1;
+    static_assert(S == 4 || S == 2, "four lane groups: a k-tile or half a k-tile each");
+    extern __shared__ uint8_t smem[];                                   // 8 wavefronts x RING x BUF, SETS x SET
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int col = lane & 15, g = lane >> 4;
+    const int gt = S == 4 ? g : g >> 1, gh = S == 4 ? 0 : g & 1;         // k-tile of a step and (first) half of this lane
+    uint8_t* const my_buf = smem + wave * RING * BUF;
+    float* const sums = reinterpret_cast<float*>(smem + 8 * RING * BUF);
+
+    const uint32_t row_bytes = (uint32_t)((int64_t)A.w_bytes / A.N);
+    const int nkt = A.Kp / kBK;
+    const int n16 = (A.N + 15) >> 4;
+    const int per_tile = A.k_chunks * n16;                              // units of one row tile
+
+    // grouped launches: the table may end in empty tiles
+    int live_tiles = A.m_tiles;
+    if (A.tile_expert) {
+        int c = 0;
+        for (int i = lane; i < A.m_tiles; i += 64) c += A.tile_rows[i] > 0 ? 1 : 0;
+        for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o);
+        live_tiles = __builtin_amdgcn_readfirstlane(c);
+    }
+    // units = (row tile, K chunk, 16-column tile), column tile fastest; every workgroup takes one contiguous run.  A unit of the last
+    // chunk, which may be short, weighs less: the blocks per wavefront, and about as much as one more for the tile itself.
+    const int chunk_steps = (A.chunk_kt / S + 7) >> 3, last_steps = ((nkt - (A.k_chunks - 1) * A.chunk_kt + S - 1) / S + 7) >> 3;
+    const int64_t front = (int64_t)(A.k_chunks - 1) * n16 * (chunk_steps + 1), weight = front + (int64_t)n16 * (last_steps + 1);
+    auto unit_at = [&](int64_t at) {
+        const int mt = (int)(at / weight);
+        const int rem = (int)(at - mt * weight);
+        return mt * per_tile + (rem < front ? rem / (chunk_steps + 1) : (A.k_chunks - 1) * n16 + (rem - (int)front) / (last_steps + 1));
+    };
+    int u = unit_at(live_tiles * weight * blockIdx.x / gridDim.x);
+    const int u_end = unit_at(live_tiles * weight * (blockIdx.x + 1) / gridDim.x);
+
+    while (u < u_end) {
+        const int mt = u / per_tile, rem = u - mt * per_tile;
+        const int kc = rem / n16, nt0 = rem - kc * n16, cnt = min(n16 - nt0, u_end - u);
+        u += cnt;
+        // the blocks of the chunk, dealt out evenly: at most KTW / S to a wavefront
+        const int blocks = (min(A.chunk_kt, nkt - kc * A.chunk_kt) + S - 1) / S;
+        const int kt0 = kc * A.chunk_kt + S * (wave * (blocks >> 3) + min(wave, blocks & 7));
+        const int kcnt = max(0, min(S * ((blocks >> 3) + (wave < (blocks & 7) ? 1 : 0)), nkt - kt0));      // k-tiles of this wavefront
+        int m0, m_rows;
+        const uint8_t* wbase = A.w;
+        if (A.tile_expert) {
+            m0 = A.tile_row0[mt];
+            m_rows = min(16 * RB, A.tile_rows[mt]);
+            wbase += expert_offset(A, mt);
+        } else {
+            m0 = mt * (16 * RB);
+            m_rows = min(16 * RB, A.M - m0);
+        }
+        // (the expert id comes from memory the kernel also writes to, so the compiler loads it per lane: without the
+        // hint every copy would run in a loop over the distinct descriptors of the wavefront)
+        const uintptr_t wa = uniform_address(reinterpret_cast<uintptr_t>(wbase));
+        const uint32_t base_delta = (uint32_t)(wa & 3);
+        const __amdgpu_buffer_rsrc_t wrs = __builtin_amdgcn_make_buffer_rsrc(
+            reinterpret_cast<void*>(wa & ~(uintptr_t)3), 0, (int)(((uint32_t)A.w_bytes + base_delta + 3u) & ~3u), 0x00020000);
+
+        // result row of this thread in the reduction: accumulator register `wave` of the 4 RB
+        const int ml = 16 * (wave >> 2) + 4 * g + (wave & 3);
+        const bool ok = wave < 4 * RB && ml < m_rows;
+        float sc;
+        int64_t coff;
+        {
+            const int m = m0 + min(ml, m_rows - 1);
+            sc = A.xscale[m];
+            coff = A.partial ? ((int64_t)kc * A.M + m) * A.N : (int64_t)(A.c_rows ? A.c_rows[m] : m) * A.ldc;
+        }
+
+        // Source offsets of the raw copies.  16 rows are a multiple of four bytes, so a row's alignment
+        // inside its window is the same in every column tile.
+        const uint32_t koff = G::tile_offset(kt0);
+        uint32_t w_off[DI];
+#pragma unroll
+        for (int i = 0; i < DI; ++i) {
+            const int q = i * 64 + lane;
+            const int row = q / CH, chunk = q - row * CH;
+            w_off[i] = (row < 16 && 16 * chunk < (kcnt > 0 ? G::window_bytes(kcnt) : 0)) ? ((base_delta + (uint32_t)row * row_bytes + koff) & ~3u) + (uint32_t)chunk * 16u : kDeadOffset;
+        }
+        const uint32_t my_delta = (base_delta + (uint32_t)col * row_bytes + koff) & 3u;
+        auto issue = [&](int i, int b) {                // column tile nt0 + i -> buffer b
+            uint8_t* dst = my_buf + b * BUF;
+            const bool any = i < cnt;
+            const uint32_t so = any ? (uint32_t)(nt0 + i) * 16u * row_bytes : 0u;
+#pragma unroll
+            for (int q = 0; q < DI; ++q) copy16_to_lds(wrs, dst + q * 1024, any ? w_off[q] : kDeadOffset, so);
+        };
+        issue(0, 0);
+
+        // MFMA A operands of this wavefront's K range: rows 16 rb + `col`, the k-tile and k-half of the lane's weights, k-step ks.
+        // Pieces of eight halfs lie row by row (piece_start), so that a load is a few contiguous runs: from rows that followed one
+        // another each was 64 pieces of 16 bytes, and the 256 loads of a workgroup took the address unit about 3 us
+        // (Q4_K 32 x 14336 x 4096 23.2 -> 19.9 us with the kernel of 32-column tiles).  The lanes of missing rows read the last one.
+        half8_t a[KTW / S][HALVES][4][RB];
+        {
+            const uint8_t* const xb = reinterpret_cast<const uint8_t*>(A.x16);
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb) {
+                const int row = m0 + min(16 * rb + col, m_rows - 1);
+                const uint32_t piece = 2u * (uint32_t)piece_halfs(row, A.M);          // bytes to the row's next piece
+                const uint32_t first = 2u * (uint32_t)piece_start(row, A.xld);
+#pragma unroll
+                for (int p = 0; p < KTW / S; ++p) {
+                    const uint32_t at = first + (uint32_t)(min(kt0 + S * p + gt, nkt - 1) * 8 + gh) * piece;
+#pragma unroll
+                    for (int hh = 0; hh < HALVES; ++hh)
+#pragma unroll
+                        for (int ks = 0; ks < 4; ++ks)
+                            a[p][hh][ks][rb] = *reinterpret_cast<const half8_t*>(xb + (at + (uint32_t)(2 * ks + hh) * piece));
+                }
+            }
+        }
+#pragma unroll
+        for (int b = 1; b < RING; ++b) issue(b, b);
+        if (kcnt < KTW) {                               // (k-tiles past the end: neither operand may hold anything)
+            const half8_t zero = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+            for (int p = 0; p < KTW / S; ++p)
+#pragma unroll
+                for (int i = 0; i < HALVES * 4 * RB; ++i)
+                    if (S * p + gt >= kcnt) a[p][i / (4 * RB)][i / RB % 4][i % RB] = zero;
+        }
+        int b = 0;                                      // buffer of column tile i
+        float part[8];                                  // partial sums of the tile before
+        auto read_parts = [&](int i) {
+            if (wave < 4 * RB) {
+                const float* const set = sums + (SETS == 2 ? (i & 1) * (L::SET / 4) : 0);
+#pragma unroll
+                for (int v = 0; v < 8; ++v) part[v] = set[(v * RB * 4 + wave) * 64 + lane];
+            }
+        };
+        float* const dst = A.partial ? A.partial : A.c;
+        auto store_tile_sum = [&](int i) {
+            const int n = (nt0 + i) * 16 + col;
+            if (ok && n < A.N) {
+                float s = 0.f;
+#pragma unroll
+                for (int v = 0; v < 8; ++v) s += part[v];
+                dst[coff + n] = s * sc;
+            }
+        };
+        for (int i = 0; i < cnt; ++i) {
+            // the copies of tile i have landed; those of the RING - 1 tiles after it stay in flight
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"((RING - 1) * DI) : "memory");
+            // the sums of the tile before are read here and added behind the matrix instructions of this one
+            if (SETS == 2 && i > 0) read_parts(i - 1);
+            float4_t acc[RB];
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb) acc[rb] = float4_t{0.f, 0.f, 0.f, 0.f};
+            uint32_t bad = 0u;                          // a scale of this lane's column does not fit the fp16 operands
+            const bool in_n = (nt0 + i) * 16 + col < A.N;
+            const uint8_t* raw = my_buf + b * BUF + col * (CH * 16);
+            // a wavefront with a full K range runs the k-tiles as one branch-free block, so the unpacking of one
+            // k-tile is scheduled into the matrix instructions of the previous one
+            auto k_tiles = [&](auto full_tag) {
+                constexpr bool kFull = decltype(full_tag)::value;
+#pragma unroll
+                for (int p = 0; p < KTW / S; ++p) {
+                    if (kFull || S * p < kcnt) {
+                        const int t = S * p + gt;
+                        const bool in_k = kFull || t < kcnt;
+                        // (whole dwords of the way to step p are left to the address: where a lane's block lies in its dwords is then
+                        // the same in every step, or every other one, and worked out once)
+                        const uint32_t step = G::tile_offset(S * p), delta = my_delta + (step & 3u);
+#pragma unroll
+                        for (int hh = 0; hh < HALVES; ++hh) {
+                            uint32_t r[G::kRegs], o[16];
+                            G::fetch(raw + (step & ~3u), gt, gh + hh, delta, r);
+                            if constexpr (!kFull) {
+#pragma unroll
+                                for (int q = 0; q < G::kRegs; ++q) r[q] = in_k ? r[q] : 0u;
+                            }
+                            G::dequant(r, gt, gh + hh, delta, ((kt0 + t) * 2 + gh + hh) * 32 < A.K && in_n && in_k, o, bad);
+#pragma unroll
+                            for (int ks = 0; ks < 4; ++ks) {
+                                const uint4_t bb = {o[4 * ks], o[4 * ks + 1], o[4 * ks + 2], o[4 * ks + 3]};
+#pragma unroll
+                                for (int rb = 0; rb < RB; ++rb)
+                                    acc[rb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[p][hh][ks][rb], __builtin_bit_cast(half8_t, bb), acc[rb], 0, 0, 0);
+                            }
+                        }
+                    }
+                }
+            };
+            if (kcnt == KTW) k_tiles(std::true_type{});
+            else k_tiles(std::false_type{});
+            // the four lanes of a column saw different blocks and hold different rows of it
+            const uint64_t flagged = __builtin_amdgcn_ballot_w64(G::out_of_range(bad));
+            if (flagged != 0) {
+                const uint64_t two = flagged | (flagged >> 32);
+                const uint32_t cols = (uint32_t)two | (uint32_t)(two >> 16);
+                if ((cols >> col) & 1u) {
+#pragma unroll
+                    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) acc[rb][r] = __uint_as_float(kNaNBits);
+                }
+            }
+            if (i > 0) store_tile_sum(i - 1);
+            // partial sums of this wavefront's K range; the buffer it has just consumed is its own and takes the next copies
+            float* const set = sums + (SETS == 2 ? (i & 1) * (L::SET / 4) : 0);
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) set[(wave * RB * 4 + rb * 4 + r) * 64 + lane] = acc[rb][r];
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            issue(i + RING, b);
+            lds_barrier();
+            // (two sets: a wavefront writes this one again behind the next tile's barrier, which follows the reads)
+            if constexpr (SETS == 1) {
+                read_parts(i);
+                lds_barrier();
+            }
+            b = b + 1 == RING ? 0 : b + 1;
+        }
+        if (SETS == 2) read_parts(cnt - 1);
+        store_tile_sum(cnt - 1);
+        // the next run starts with the first buffer and set: every copy has landed, every sum has been read
+        if (u < u_end) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    }
+}
+
+// The same with 32-column tiles on the 32 x 32 x 16 instruction, the partial sums in the raw buffer that the wavefront has just consumed,
+// two barriers per tile: half as many units, twice the work between barriers (see slim_plan for where it serves).
+// LDS layout of one wavefront: RING raw buffers of 32 rows x CH 16-byte chunks
 // (the bytes of KTW k-tiles plus the up to three bytes between the 4-byte aligned window start and the first
 // block; the unpackers may read a few bytes further, into the next row, and ignore them)
 template <typename G, int KTW>
-struct SlimLayout {
+struct Slim32Layout {
     static constexpr int kNeed = (G::window_bytes(KTW) + 15) / 16;
     static constexpr int buf_of(int ch) { return 32 * ch * 16 > 4096 ? 32 * ch * 16 : 4096; }
     static constexpr int ring_of(int ch) { return 8 * 3 * buf_of(ch) + 1024 <= 160 * 1024 ? 3 : 2; }
@@ -2686,9 +2982,9 @@ struct SlimLayout {
 };
 
 template <typename G, int KTW>
-__global__ void __launch_bounds__(512) gemm_slim_kernel(const GemmArgs A)
+__global__ void __launch_bounds__(512) gemm_slim32_kernel(const GemmArgs A)
 {
-    using L = SlimLayout<G, KTW>;
+    using L = Slim32Layout<G, KTW>;
     constexpr int CH = L::CH, DI = L::DI, BUF = L::BUF, RING = L::RING;
     static_assert(KTW % G::kTileStep == 0, "a wavefront's K range must start at a block");
     extern __shared__ uint8_t smem[];                                   // 8 wavefronts x RING x BUF
@@ -2739,12 +3035,7 @@ __global__ void __launch_bounds__(512) gemm_slim_kernel(const GemmArgs A)
         const __amdgpu_buffer_rsrc_t wrs = __builtin_amdgcn_make_buffer_rsrc(
             reinterpret_cast<void*>(wa & ~(uintptr_t)3), 0, (int)(((uint32_t)A.w_bytes + base_delta + 3u) & ~3u), 0x00020000);
 
-        // MFMA A operands of this wavefront's K range: row `col`, k-half h of every k-step.  Pieces of eight halfs lie row by
-        // row (piece_start), so that a load is one or two contiguous kilobytes: from rows that followed one another each
-        // was 64 pieces of 16 bytes in 32 lines, and the 256 loads of a workgroup took
-        // the address unit about 3 us.  Measured, whole call, us: Q4_K 32 x 14336 x 4096 23.2 -> 19.9, 32 x 4096 x 14336 26.4 -> 23.8,
-        // Q8_0 32 x 2560 x 9728 24.3 -> 21.2, Q5_K 32 x 21504 x 5376 44.4 -> 41.0, MXFP4 32 x 14336 x 4096 21.9 -> 18.2; up to eight
-        // rows the same (the lanes of the missing rows read the last one).
+        // MFMA A operands of this wavefront's K range: row `col`, k-half h of every k-step, in pieces (see gemm_slim_kernel)
         half8_t a[KTW][4];
         {
             const int row = m0 + min(col, m_rows - 1);
@@ -2918,16 +3209,26 @@ bool launch_chunk_sum(const GemmArgs& a, hipStream_t stream)
     return hip_ok(hipGetLastError(), "gemm chunk sum launch");
 }
 
-template <typename G, int KTW>
+// COLS 16: gemm_slim_kernel of RB x 16 rows; 32: gemm_slim32_kernel (RB 2)
+template <typename G, int KTW, int RB, int COLS>
 bool launch_slim(GemmArgs a, int m_tiles, hipStream_t stream, const ChunkScratch& cs)
 {
-    using L = SlimLayout<G, KTW>;
-    auto kern = gemm_slim_kernel<G, KTW>;
-    const size_t lds = (size_t)8 * L::RING * L::BUF + 64;     // the unpackers may read a few bytes past the last row
-    static_assert((size_t)8 * L::RING * L::BUF + 64 <= 160 * 1024, "raw buffers must fit LDS");
+    void (*kern)(GemmArgs);
+    size_t lds;
+    if constexpr (COLS == 16) {
+        using L = SlimLayout<G, KTW, RB>;
+        static_assert(L::RING >= 2 && L::kBytes <= L::kLds, "two raw buffers per wavefront and the partial sums must fit LDS");
+        kern = gemm_slim_kernel<G, KTW, RB>;
+        lds = L::kBytes;
+    } else {
+        using L = Slim32Layout<G, KTW>;
+        static_assert((size_t)8 * L::RING * L::BUF + 64 <= 160 * 1024, "raw buffers must fit LDS");
+        kern = gemm_slim32_kernel<G, KTW>;
+        lds = (size_t)8 * L::RING * L::BUF + 64;     // the unpackers may read a few bytes past the last row
+    }
     if (!cs.need_out && !raise_lds_limit(reinterpret_cast<const void*>(kern), lds)) return false;
     a.m_tiles = m_tiles;
-    a.n_tiles = (a.N + 31) / 32;
+    a.n_tiles = (a.N + COLS - 1) / COLS;
     a.chunk_kt = 8 * KTW;
     a.k_chunks = (a.Kp / kBK + a.chunk_kt - 1) / a.chunk_kt;
     a.partial = nullptr;
@@ -3646,36 +3947,84 @@ bool launch_slim_mx_for(const GemmArgs& a, int m_tiles, hipStream_t stream, cons
     return launch_slim_mx<6, RB>(a, m_tiles, stream, cs);
 }
 
-// k-tiles per wavefront of the register-resident kernel: a multiple of the format's block step, at most what two
-// raw buffers per wavefront fit into LDS; a longer K is cut into chunks of 8 x that many k-tiles
+// Which register-resident kernel serves a launch: columns of its tiles (16: gemm_slim_kernel, 32: gemm_slim32_kernel) and k-tiles per
+// wavefront, a multiple of the format's block step; a longer K is cut into chunks of 8 x that many k-tiles.
+struct SlimPlan {
+    int cols, ktw;
+};
+
 template <typename G, int KTW>
-constexpr bool slim_fits()
+constexpr bool slim32_fits()
 {
-    return (size_t)8 * SlimLayout<G, KTW>::RING * SlimLayout<G, KTW>::BUF + 64 <= 160 * 1024;
+    return (size_t)8 * Slim32Layout<G, KTW>::RING * Slim32Layout<G, KTW>::BUF + 64 <= 160 * 1024;
 }
 
+// 16 columns: up to eight k-tiles per wavefront, as few chunks of even size as that allows (a chunk more is a launch for the sums more:
+// Q8_0 24 x 4096 x 2560 15.1 us with at most four k-tiles, 10.8 with six).
 template <typename G>
 int slim_ktw(int nkt)
 {
-    const int need = (nkt + 7) / 8;
-    const int ktw = (need + G::kTileStep - 1) / G::kTileStep * G::kTileStep;
-    const int limit = slim_fits<G, 8>() ? 8 : slim_fits<G, 6>() && G::kTileStep == 2 ? 6 : 4;
-    return ktw <= limit ? ktw : limit;       // longer K: chunks of 8 * limit k-tiles
+    const int chunks = (nkt + 63) / 64, need = (nkt + 8 * chunks - 1) / (8 * chunks);
+    return std::min(8, (need + G::kTileStep - 1) / G::kTileStep * G::kTileStep);
 }
 
+// 32 columns: what two raw buffers per wavefront leave room for
 template <typename G>
-bool launch_slim_for(const GemmArgs& a, int ktw, int m_tiles, hipStream_t stream, const ChunkScratch& cs)
+int slim32_ktw(int nkt)
+{
+    const int need = (nkt + 7) / 8;
+    const int limit = slim32_fits<G, 8>() ? 8 : slim32_fits<G, 6>() && G::kTileStep == 2 ? 6 : 4;
+    return std::min(limit, (need + G::kTileStep - 1) / G::kTileStep * G::kTileStep);
+}
+
+// 16 columns unless the work between two barriers is too short or larger units fill the chip better (us, 16 / 32 columns):
+//  - more than 16 rows and at most four k-tiles per wavefront (Q6_K 93 x 6327 x 2048 20.8 / 18.5, 331 x 5764 x 1792 39.2 / 35.6);
+//  - several row tiles or chunks whose units of 32 columns are at most one per CU where those of 16 are more, or K beyond 4096
+//    with as few (a workgroup then loads one set of activations: Q6_K 30 x 2609 x 4864 18.1 / 14.2, Q8_0 16 x 317 x 10144 17.1 / 13.7,
+//    Q4_K 92 x 2104 x 2304 15.3 / 12.7, 50 x 368 x 13056 19.6 / 17.5), or results that are added to a residual, by the second launch
+//    in any case, so that chunks cost none (FFN of 53 rows, Q8_0 1536 / 3584: 43.3 / 41.8);
+//  - more than 32 rows of fewer than 1024 columns, which keep the chunks, and with them the workspace, that their plans have had
+//    (Q6_K 67 x 590 x 5632 16.9 / 14.4, but Q8_0 45 x 1001 x 2080 10.9 / 15.4).
+template <typename G>
+SlimPlan slim_plan(int nkt, int M, int N, bool tiles, bool accumulate)
+{
+    const int ktw = slim_ktw<G>(nkt), ktw32 = slim32_ktw<G>(nkt), cus = device_info().num_cus;
+    if (M <= 16 && !tiles && !accumulate && nkt <= 64) return {16, ktw};
+    const int64_t rows = (M + 31) / 32, chunks = (nkt + 8 * ktw - 1) / (8 * ktw), chunks32 = (nkt + 8 * ktw32 - 1) / (8 * ktw32);
+    const int64_t units = rows * chunks * ((N + 15) / 16), units32 = rows * chunks32 * ((N + 31) / 32);
+    const bool few = units32 <= cus && (nkt > 64 || (rows * chunks > 1 && units > cus) || (accumulate && ktw32 < ktw));
+    return ktw <= 4 || few || (M > 32 && N < 1024) ? SlimPlan{32, ktw32} : SlimPlan{16, ktw};
+}
+
+template <typename G, int RB, int COLS>
+bool launch_slim_rows(const GemmArgs& a, int ktw, int m_tiles, hipStream_t stream, const ChunkScratch& cs)
 {
     if constexpr (G::kTileStep == 2) {
-        if (ktw == 2) return launch_slim<G, 2>(a, m_tiles, stream, cs);
-        if constexpr (slim_fits<G, 6>())
-            if (ktw == 6) return launch_slim<G, 6>(a, m_tiles, stream, cs);
+        if (ktw == 2) return launch_slim<G, 2, RB, COLS>(a, m_tiles, stream, cs);
+        if constexpr (COLS == 16 || slim32_fits<G, 6>())
+            if (ktw == 6) return launch_slim<G, 6, RB, COLS>(a, m_tiles, stream, cs);
     }
-    if (ktw == 4) return launch_slim<G, 4>(a, m_tiles, stream, cs);
-    if constexpr (slim_fits<G, 8>())
-        if (ktw == 8) return launch_slim<G, 8>(a, m_tiles, stream, cs);
+    if (ktw == 4) return launch_slim<G, 4, RB, COLS>(a, m_tiles, stream, cs);
+    if constexpr (COLS == 16 || slim32_fits<G, 8>())
+        if (ktw == 8) return launch_slim<G, 8, RB, COLS>(a, m_tiles, stream, cs);
     set_last_error("gemm: no register-resident kernel for this K.");
     return false;
+}
+
+// Up to 16 rows: half the activations and matrix instructions of 32.
+template <typename G>
+bool launch_slim_for(const GemmArgs& a, int m_tiles, hipStream_t stream, const ChunkScratch& cs)
+{
+    const SlimPlan p = slim_plan<G>(a.Kp / kBK, a.M, a.N, a.tile_expert != nullptr, a.accumulate != 0);
+    if (p.cols == 32) return launch_slim_rows<G, 2, 32>(a, p.ktw, m_tiles, stream, cs);
+    if (!a.tile_expert && a.M <= 16) return launch_slim_rows<G, 1, 16>(a, p.ktw, m_tiles, stream, cs);
+    if (p.ktw <= 4) {
+        set_last_error("gemm: no register-resident kernel of 32 rows for this K.");
+        return false;
+    }
+    if constexpr (G::kTileStep == 2)
+        if (p.ktw == 6) return launch_slim<G, 6, 2, 16>(a, m_tiles, stream, cs);
+    return launch_slim<G, 8, 2, 16>(a, m_tiles, stream, cs);
 }
 
 struct WidePlan {
@@ -3768,7 +4117,7 @@ bool launch_for_type(const GemmArgs& a, int bm, int m_tiles, const WidePlan& wid
         set_last_error("gemm: activations in pieces serve the 32-row units of fp16 operands, and these take no others.");
         return false;
     }
-    if (bm == 32 && !a.x_mx) return launch_slim_for<G>(a, slim_ktw<G>(a.Kp / kBK), m_tiles, stream, cs);
+    if (bm == 32 && !a.x_mx) return launch_slim_for<G>(a, m_tiles, stream, cs);
     // Q4_K and MXFP4: the 2 x 4 wavefront layout with the operand exchange through LDS (gemm_xw_kernel); 128-row tiles are
     // 128 x 256.  Q4_K takes it for every launch, MXFP4 for plain ones: the MXFP4 expert tiles of a MoE prefill (128
     // rows) stay on two 128 x 128 workgroups per CU (926 vs 968 us at 2048 tokens).
@@ -3848,24 +4197,24 @@ namespace {
 // about 870 random ones per format over 4 .. 2048 rows, 64 .. 28672 columns and K of 256 .. 21504, a third of them added to a
 // residual.  On 300 further random calls per format the pick took 0.4 % (Q4_K), 0.3 % (Q8_0) and 0.2 % (Q6_K) longer than the
 // fastest candidate on average, more than 4 % longer on 11, 8 and 3 of them, 11 % at most.
-// slim_rows was measured again with the activations in pieces (see gemm_slim_kernel), on 350 (300) calls per format of 2 .. 150
-// rows, 512 .. 21504 columns and K of 1024 .. 14336: with the first fit's value (6.588 / 5.523 / 6.414 for Q4_K / Q8_0 / Q6_K) the
-// pick would be 2.8 / 0.4 / 0.2 % behind there, with this one 0.5 / 0.2 / 0.1 %.  Above 160 rows and under 1024 columns slim_rows_far
-// still serves, the first fit's value or near it: the kernels do not cross at these edges, more had not been measured.  On 3600
-// calls per format since then, 4 .. 2048 rows and 64 columns on, the pick is 1.6 / 0.4 / 1.2 % behind the fastest candidate (Q4_K 1.9
-// with 6.588); slim_rows throughout with a term for the conversion, and gemm_wide_kernel of Q6_K at 0.84 of its k-tile, would make that
-// 0.3 / 0.2 / 0.1 %.
-// The candidates now, us (register-resident / gemm_wide_kernel / 128 rows / 256 rows):
-//   Q4_K  8 x 4096 x 5376 15.8 / 20.6 / - / -,  64 x 828 x 2560 12.4 / 15.9 / - / 28.5,  64 x 9728 x 9728 47.6 / 42.3 / - / 72.6,
+// The register-resident kernel of 16-column tiles was fitted anew, up to 64 rows, on 260 calls per format of 4 .. 420 rows, 300 .. 21504
+// columns and K of 1024 .. 14336: with these constants the pick is 0.05 / 0.07 / 0.00 % behind the faster of it and the best other kernel
+// there.  Above 64 rows, and above 32 under 1024 columns, the costs of the kernel of 32-column tiles before it still draw the line (the
+// far_ constants): the kernels do not cross at these edges, and where that kernel was taken this one serves.
+// The candidates, us (register-resident / gemm_wide_kernel / 128 rows / 256 rows):
+//   Q4_K  24 x 14336 x 4096 19.2 / 22.8 / - / -,  64 x 828 x 2560 12.4 / 15.9 / - / 28.5,  88 x 3078 x 1792 11.2 / 17.5 / - / -,
 //         200 x 4096 x 2560 28.3 / 28.0 / - / 34.8,  257 x 512 x 14336 39.2 / 32.0 / - / 84.9,  480 x 9728 x 9728 (added) - / 142 / - / 124
-//   Q8_0  24 x 14336 x 4096 26.4 / 29.5 / - / -,  64 x 14336 x 4096 33.3 / 34.7 / 39.7 / 46.3,  128 x 9728 x 5376 54.8 / 45.1 / 56.2 / 64.6,
+//   Q8_0  24 x 14336 x 4096 23.9 / 29.5 / - / -,  64 x 14336 x 4096 28.7 / 34.7 / 39.7 / 46.3,  128 x 9728 x 5376 54.8 / 45.1 / 56.2 / 64.6,
 //         400 x 4096 x 4096 - / 41.1 / 41.5 / 48.5,  400 x 9728 x 9728 - / 146 / 173 / 125
-//   Q6_K  64 x 9728 x 9728 54.8 / 52.3 / 78.3 / -,  240 x 9728 x 14336 (added) 230 / 121 / 145 / -,  480 x 14336 x 4096 - / 94.8 / 114 / -
+//   Q6_K  30 x 18504 x 1280 17.8 / 23.5 / - / -,  240 x 9728 x 14336 (added) 230 / 121 / 145 / -,  480 x 14336 x 4096 - / 94.8 / 114 / -
 struct RuleCosts {
-    // register-resident kernel: a call; its activations, per 32 rows and 8 k-tiles per wavefront (slim_rows_far: above 160 rows, or 32
-    // under 1024 columns); a round of units and per k-tile of a wavefront in it; a workgroup whose units cross into another row
-    // tile or K chunk (it loads activations anew)
-    double slim, slim_rows, slim_rows_far, unit, unit_kt, cross, cross_kt;
+    // register-resident kernel: a call; converting a million activations; its activations, per 32 rows and 8 k-tiles per wavefront;
+    // per k-tile of a wavefront in a round of units (up to 16 rows, more); per k-tile where a workgroup's units cross into another
+    // row tile or K chunk (it loads activations anew)
+    double slim, slim_convert, slim_rows, unit_kt_16, unit_kt, cross_kt;
+    // 32-column tiles, above 64 rows, or 32 under 1024 columns: a call, activations (up to 32 rows, or 160 and from 1024 columns on; else), a round of units and
+    // per k-tile in it, a crossing
+    double far_call, far_rows_160, far_rows, far_unit, far_unit_kt, far_cross, far_cross_kt;
     // gemm_wide_kernel: a call, a k-tile of a round and per 32 rows in it, the share of that time that an almost empty round
     // takes, a round
     double wide, wide_kt, wide_kt_rows, wide_fill, wide_round;
@@ -3874,13 +4223,13 @@ struct RuleCosts {
     double sums, sums_rate;                            // the launch that adds K chunks: a call, TB/s of its sums written and read
     double wide_add, tile_add;                         // results added in place: a round, per 32 rows of a tile (one load after the other)
 };
-constexpr RuleCosts kCostsQ4K{6.538, 3.000, 6.000, 0.471, 0.444, 4.440, 0.000, 5.031, 0.423, 0.153, 0.966, 3.404,
+constexpr RuleCosts kCostsQ4K{9.463, 1.784, 0.000, 0.221, 0.241, 0.300, 6.538, 3.000, 6.000, 0.471, 0.444, 4.440, 0.000, 5.031, 0.423, 0.153, 0.966, 3.404,
                               11.108, 1.670, 0.618, 0.032, 0.000, 0.000, 0.000, 0.000,      // (no 128-row tiles)
                               2.367, 4.806, 3.964, 4.582};
-constexpr RuleCosts kCostsQ80{6.249, 2.500, 5.523, 1.221, 0.339, 0.590, 0.891, 5.085, 0.495, 0.148, 1.006, 5.151,
+constexpr RuleCosts kCostsQ80{9.125, 1.025, 1.143, 0.363, 0.333, 0.311, 6.249, 2.500, 5.523, 1.221, 0.339, 0.590, 0.891, 5.085, 0.495, 0.148, 1.006, 5.151,
                               3.152, 1.741, 0.926, 4.675, 4.610, 1.247, 1.492, 1.841,
                               1.697, 5.090, 6.433, 1.591};
-constexpr RuleCosts kCostsQ6K{5.858, 2.500, 6.414, 0.393, 0.658, 2.025, 0.406, 4.411, 1.047, 0.156, 0.890, 6.472,      // (no 256-row tiles)
+constexpr RuleCosts kCostsQ6K{8.854, 1.208, 0.000, 0.366, 0.402, 0.244, 5.858, 2.500, 6.414, 0.393, 0.658, 2.025, 0.406, 4.411, 1.047, 0.156, 0.890, 6.472,      // (no 256-row tiles)
                               0.000, 0.000, 0.000, 0.000, 6.177, 1.561, 0.938, 3.905,
                               3.284, 7.419, 3.358, 1.187};
 constexpr double kNotServed = 1e30;      // a kernel that a format has not, or whose chunk sums do not fit
@@ -3891,17 +4240,28 @@ inline double sums_us(const RuleCosts& c, int k_chunks, int M, int N) { return c
 template <typename G>
 double slim_us(const RuleCosts& c, int M, int N, int nkt, bool accumulate, size_t max_chunk_bytes)
 {
-    const int ktw = slim_ktw<G>(nkt), kc = (nkt + 8 * ktw - 1) / (8 * ktw), cus = device_info().num_cus;
+    const SlimPlan plan = slim_plan<G>(nkt, M, N, false, accumulate);
+    const int ktw = plan.ktw, kc = (nkt + 8 * ktw - 1) / (8 * ktw), cus = device_info().num_cus;
     const bool two_pass = kc > 1 || accumulate;          // (launch_slim adds to a residual in the second launch only)
     if (two_pass && !chunk_sums_fit(kc, M, N, max_chunk_bytes)) return kNotServed;
-    const int64_t segments = (int64_t)((M + 31) / 32) * kc, n32 = (N + 31) / 32, units = segments * n32;
-    // Workgroup b takes the units from floor(units b / cus) on.  Segment i ends inside a workgroup's run unless n32 ((-i cus) mod
+    const double sums = two_pass ? sums_us(c, kc, M, N) : 0.0;
+    // Workgroup b takes the units from floor(units b / cus) on.  Segment i ends inside a workgroup's run unless tiles ((-i cus) mod
     // segments) < cus, and over all i that remainder is at most segments - gcd(segments, cus).
-    const bool crosses = units > cus && n32 * (segments - std::gcd(segments, (int64_t)cus)) >= cus;
-    const double kt = 0.4 * ktw + 0.6 * nkt / (8.0 * kc);      // (wavefronts past the end of K leave theirs to the others)
-    const double rows = M <= 32 || (M <= 160 && N >= 1024) ? c.slim_rows : c.slim_rows_far;
-    return c.slim + rows * std::min(M, 32) * ktw / 256.0 + (double)((units + cus - 1) / cus) * (c.unit + c.unit_kt * kt) +
-           (crosses ? c.cross + c.cross_kt * ktw : 0.0) + (two_pass ? sums_us(c, kc, M, N) : 0.0);
+    auto crosses = [&](int64_t segments, int64_t tiles) { return segments * tiles > cus && tiles * (segments - std::gcd(segments, (int64_t)cus)) >= cus; };
+    // (wavefronts past the end of K leave theirs to the others)
+    if (M > 64 || (M > 32 && N < 1024) || plan.cols == 32) {
+        // (as 32-column tiles, also where those of 16 columns serve)
+        const int far_ktw = slim32_ktw<G>(nkt), far_kc = (nkt + 8 * far_ktw - 1) / (8 * far_ktw);
+        const int64_t segments = (int64_t)((M + 31) / 32) * far_kc, tiles = (N + 31) / 32, units = segments * tiles;
+        const double kt = 0.4 * far_ktw + 0.6 * nkt / (8.0 * far_kc);
+        const double rows = M <= 32 || (M <= 160 && N >= 1024) ? c.far_rows_160 : c.far_rows;
+        return c.far_call + rows * std::min(M, 32) * far_ktw / 256.0 + (double)((units + cus - 1) / cus) * (c.far_unit + c.far_unit_kt * kt) +
+               (crosses(segments, tiles) ? c.far_cross + c.far_cross_kt * far_ktw : 0.0) + (far_kc > 1 || accumulate ? sums_us(c, far_kc, M, N) : 0.0);
+    }
+    const int64_t segments = (int64_t)((M + 31) / 32) * kc, tiles = (N + 15) / 16, units = segments * tiles;
+    const double kt = 0.4 * ktw + 0.6 * nkt / (8.0 * kc);
+    return c.slim + c.slim_convert * M * (nkt * kBK) * 1e-6 + c.slim_rows * std::min(M, 32) * ktw / 256.0 +
+           (double)((units + cus - 1) / cus) * kt * (M <= 16 ? c.unit_kt_16 : c.unit_kt) + (crosses(segments, tiles) ? c.cross_kt * ktw : 0.0) + sums;
 }
 
 // rounds of workgroups x k-tiles; the last round may leave CUs idle
@@ -3945,14 +4305,13 @@ inline double tile_us(const RuleCosts& c, int bm, int M, int N, int nkt, bool ac
                              : c.t128 + rounds_us(tiles * kc, chunk * c.t128_kt, c.t128_fill, c.t128_round + add));
 }
 
-// Few rows stay on the register-resident kernel: all of three and less, and of Q8_0 and Q6_K up to 16, where it was the fastest
-// of all measured calls but one (Q8_0 11 x 8441 x 5120, 8 % behind) while the expected costs are too close to tell.
+// Up to 16 rows stay on the register-resident kernel: it was the fastest of all measured calls but three (at most 8 % behind).
 template <typename G>
 int cheapest_tiles(const RuleCosts& c, int M, int N, int K, bool accumulate, size_t max_chunk_bytes, WidePlan* plan)
 {
     const int nkt = (K + kBK - 1) / kBK;
     const double slim = slim_us<G>(c, M, N, nkt, accumulate, max_chunk_bytes);
-    if (M <= (std::is_same<G, GQ4K>::value ? 3 : 16) && slim < kNotServed) return 32;
+    if (M <= 16 && slim < kNotServed) return 32;
     // (up to 32 rows the other kernel has one row tile, one launch and no sums in the scratch: a near tie goes to it - Q4_K
     // 32 x 4096 x 4096 16.7 vs 18.0 us)
     const double wide = wide_us(c, M, N, nkt, accumulate, max_chunk_bytes, plan) * (M <= 32 ? 1.04 : 1.0);
@@ -4011,14 +4370,14 @@ bool launch_convert(int type, const ConvertSrc& src, int M, int K, void* workspa
                            x_row_halfs(K), chunks, x16, scales);
         return hip_ok(hipGetLastError(), "activation convert launch");
     }
-    if (layout == 2) type = kTypeQ8_0;      // natural order
+    if (layout == 2 || (layout == 3 && type == kTypeQ4_K)) type = kTypeQ8_0;      // natural order
     // three activation orders: the K-quant nibble order, the split-nibble order of the 32-weight blocks, natural
     switch (type) {
     case kTypeQ4_K: case kTypeQ5_K: launch_convert_typed<kTypeQ4_K, SRC>(src, M, K, kp, x16, scales, stream, layout); break;
-    case kTypeMXFP4: case kTypeQ4_0: case kTypeQ4_1: case kTypeQ5_0: case kTypeQ5_1: case kTypeIQ4_NL:
+    case kTypeMXFP4: case kTypeQ5_0: case kTypeQ5_1: case kTypeIQ4_NL:
         launch_convert_typed<kTypeMXFP4, SRC>(src, M, K, kp, x16, scales, stream, layout);
         break;
-    case kTypeQ8_0: case kTypeQ6_K: launch_convert_typed<kTypeQ8_0, SRC>(src, M, K, kp, x16, scales, stream, layout); break;
+    case kTypeQ8_0: case kTypeQ6_K: case kTypeQ4_0: case kTypeQ4_1: launch_convert_typed<kTypeQ8_0, SRC>(src, M, K, kp, x16, scales, stream, layout); break;
     default: set_last_error("gemm: unsupported type."); return false;
     }
     return hip_ok(hipGetLastError(), "activation convert launch");

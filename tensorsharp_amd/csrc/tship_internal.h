@@ -154,7 +154,7 @@ struct GemmPlan {
     int wide_tm, k_chunks, chunk_kt;     // gemm_wide_kernel: rows per tile / 32, K chunks, k-tiles per chunk
     int x_layout;                        // of the converted activations: 0 fp16 in the format's unpack order, 1 MX fp6 pairs (MXFP4 on
                                          // the block-scaled matrix instruction), 2 fp16 in natural order (Q4_K on gemm_wide_kernel),
-                                         // 3 as 0 in pieces of eight, row by row (the 32-row units of fp16 operands)
+                                         // 3 as 0 (Q4_K: as 2) in pieces of eight, row by row (the 32-row units of fp16 operands)
     size_t chunk_bytes;                  // scratch for the sums of K chunks (0 for most shapes)
 };
 // max_chunk_bytes: what the launch will be given; kernels and K chunks whose sums do not fit are passed over
