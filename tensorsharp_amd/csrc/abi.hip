@@ -391,9 +391,11 @@ MatmulPlan plan_matmul(int type, int M, int64_t K, int64_t N, bool norm, bool ac
 // result (+)= f(m1) * W^T with f = identity or RMSNorm(eps) * norm_w, as `plan` (of the same call) says.  All pointers are
 // device pointers; `ws` has ws_bytes >= plan.total() bytes.  silu (calls that convert their activations only): the rows of m1 are
 // (gate | up) of 2 K floats, f(m1) = silu(gate) * up.
+// leave / take (calls that convert their activations and run as one slice only): the sums of the product's K chunks are left to the call
+// that reads the result next and takes them.
 bool run_matmul_device_ws(const MatmulPlan& plan, const TSHipTensorView2D& result, const TSHipTensorView2D& m1, const void* w, int type,
                           int64_t K, int64_t N, hipStream_t stream, void* ws, size_t ws_bytes, const float* norm_w, float eps, bool accumulate,
-                          bool silu = false)
+                          bool silu = false, PendingSums* leave = nullptr, const PendingSums* take = nullptr)
 {
     const size_t rs = row_size(type, K);
     if (!check_device_operands(m1, w, type)) return false;
@@ -461,11 +463,14 @@ bool run_matmul_device_ws(const MatmulPlan& plan, const TSHipTensorView2D& resul
             const bool whole = m == plan.m_step && n == std::min<int64_t>(N, plan.n_step);
             const GemmPlan g = whole ? plan.gemm : plan_gemm(type, m, (int)n, (int)K, accumulate, chunk_bytes);
             if (g.x_layout != converted) {
-                if (!launch_convert_x(type, x, m1.stride0, nullptr, m, (int)K, ws, stream, norm_w, eps, g.x_layout, silu)) return false;
+                const bool ok = take && take->chunks > 0
+                                    ? launch_convert_x_sums(type, *take, const_cast<float*>(x), m1.stride0, m, (int)K, ws, stream, norm_w, eps, g.x_layout)
+                                    : launch_convert_x(type, x, m1.stride0, nullptr, m, (int)K, ws, stream, norm_w, eps, g.x_layout, silu);
+                if (!ok) return false;
                 converted = g.x_layout;
             }
             if (!launch_gemm(type, g, wb + (size_t)n0 * rs, (int64_t)(rs * (size_t)n), ws, out + (int64_t)m0 * result.stride0 + n0,
-                             result.stride0, m, (int)n, (int)K, stream, accumulate, chunk_ws, chunk_bytes))
+                             result.stride0, m, (int)n, (int)K, stream, accumulate, chunk_ws, chunk_bytes, leave))
                 return false;
         }
     }
@@ -537,7 +542,7 @@ FfnPlan plan_ffn(int M, int gu_type, int dn_type, int hidden, int half)
 
 bool run_ffn_swiglu_device(const FfnPlan& plan, const TSHipTensorView2D& residual, const TSHipTensorView2D& input, const float* norm_w,
                            float eps, const void* gate_up, int gu_type, const void* down, int dn_type, int hidden, int half,
-                           hipStream_t stream, char* ws)
+                           hipStream_t stream, char* ws, const PendingSums* take = nullptr)
 {
     const int M = input.dim0;
     const size_t gu_bytes = plan.gu_bytes, act_bytes = plan.act_bytes, mm_bytes = plan.mm_bytes;
@@ -569,7 +574,8 @@ bool run_ffn_swiglu_device(const FfnPlan& plan, const TSHipTensorView2D& residua
         return true;
     }
     const TSHipTensorView2D gu_view{gu, M, 2 * half, 2 * half, 1, (int64_t)((size_t)M * 2 * half * sizeof(float))};
-    if (!run_matmul_device_ws(plan.gu, gu_view, input, gate_up, gu_type, hidden, 2 * half, stream, mm_ws, mm_bytes, norm_w, eps, false)) return false;
+    if (!run_matmul_device_ws(plan.gu, gu_view, input, gate_up, gu_type, hidden, 2 * half, stream, mm_ws, mm_bytes, norm_w, eps, false, false, nullptr, take))
+        return false;
     if (gates_in_conversion(plan, M)) {
         const TSHipTensorView2D gate_view{gu, M, half, 2 * half, 1, gu_view.raw_bytes};
         return run_matmul_device_ws(plan.dn, residual, gate_view, down, dn_type, half, hidden, stream, mm_ws, mm_bytes, nullptr, 0.f, true, true);
@@ -1262,8 +1268,20 @@ bool run_outproj_ffn_device(const OutprojFfnPlan& plan, const TSHipTensorView2D&
                             const WeightDesc& od, const float* norm_w, float eps, const void* gu, int gu_type, const void* dn, int dn_type,
                             int half, hipStream_t stream, char* ws)
 {
-    if (!run_matmul_device_ws(plan.out, residual, input, out_w, od.type, od.ne0, od.ne1, stream, ws, plan.total(), nullptr, 0.f, true)) return false;
-    return run_ffn_swiglu_device(plan.ffn, residual, residual, norm_w, eps, gu, gu_type, dn, dn_type, residual.dim1, half, stream, ws);
+    // The chunk sums of the projection are added to the residual rows by the conversion that reads them for the FFN, where both calls are
+    // one conversion and one product, nothing refuses the rows in between, and the sums do not lie where that conversion writes.
+    const int M = input.dim0, hidden = residual.dim1;
+    const MatmulPlan &op = plan.out, &gp = plan.ffn.gu;
+    const bool aligned = ((reinterpret_cast<uintptr_t>(residual.data) | reinterpret_cast<uintptr_t>(norm_w) | reinterpret_cast<uintptr_t>(gu)) & 15) == 0 &&
+                         (residual.stride0 & 3) == 0;
+    const bool one = op.converts && gp.converts && M <= op.m_step && M <= gp.m_step && od.ne1 <= op.n_step && 2 * (int64_t)half <= gp.n_step;
+    const bool defer = aligned && one && residual.stride0 >= hidden && op.total() <= plan.ffn.gu_bytes + plan.ffn.act_bytes &&
+                       convert_sums_fits(gu_type, gp.gemm.x_layout, hidden);
+    PendingSums sums{nullptr, 0};
+    if (!run_matmul_device_ws(op, residual, input, out_w, od.type, od.ne0, od.ne1, stream, ws, plan.total(), nullptr, 0.f, true, false,
+                              defer ? &sums : nullptr))
+        return false;
+    return run_ffn_swiglu_device(plan.ffn, residual, residual, norm_w, eps, gu, gu_type, dn, dn_type, hidden, half, stream, ws, &sums);
 }
 
 bool validate_outproj_router(const TSHipTensorView2D& residual, const TSHipTensorView2D& input, const WeightDesc& out_w, const void* norm_w,

@@ -139,8 +139,13 @@ struct ConvertSrc {
     const float* bias;       // kSrcSwiglu: optional [experts x 2 K] bias, picked through expert_of
     const int* expert_of;
     float alpha, limit;
+    // kSrcSums: x plus the sums of K chunks that a product has left, sums[chunk][row][K]; the rows are stored back
+    const float* sums;
+    int sum_chunks;
+    float* rows;
 };
-constexpr int kSrcPlain = 0, kSrcSwiglu = 1, kSrcSilu = 2;
+constexpr int kSrcPlain = 0, kSrcSwiglu = 1, kSrcSilu = 2, kSrcSums = 3;
+constexpr int kSumsHold = 2, kSumsThreads = 1024;      // kSrcSums: rows of up to 8192 elements
 
 // SwiGLU of the gpt-oss experts (ggml-cpu/ops.cpp swiglu_oai: x = min(gate, limit), y = clamp(up, +-limit),
 // x / (1 + exp(-alpha x)) * (y + 1))
@@ -172,12 +177,13 @@ __global__ void __launch_bounds__(THREADS) convert_x_kernel(const ConvertSrc S, 
     const int m = piece_rows ? xcd * (piece_rows >> 3) + min(xcd, piece_rows & 7) + ((int)blockIdx.x >> 3) : (int)blockIdx.x;
     const int tid = threadIdx.x;
     const float* src = S.x + (int64_t)(S.row_map ? S.row_map[m] : m) * S.ldx;
-    const float* norm_w = SRC == kSrcPlain ? S.norm_w : nullptr;
+    const float* norm_w = SRC == kSrcPlain || SRC == kSrcSums ? S.norm_w : nullptr;
     const float* bias = (SRC == kSrcSwiglu && S.bias) ? S.bias + (int64_t)S.expert_of[m] * 2 * K : nullptr;
     __shared__ float red[THREADS / 64];
     __shared__ double redd[THREADS / 64];
     const int k4 = K >> 2;                       // K is a multiple of 32
-    constexpr int kHeld = kCvtHold * THREADS * 4;
+    constexpr int kHold = SRC == kSrcSums ? kSumsHold : kCvtHold;
+    constexpr int kHeld = kHold * THREADS * 4;
     // element k of the row as it enters the product (before the optional RMSNorm)
     auto raw4 = [&](int q) -> float4 {
         if (SRC == kSrcSwiglu) {
@@ -202,11 +208,38 @@ __global__ void __launch_bounds__(THREADS) convert_x_kernel(const ConvertSrc S, 
         return src[k];
     };
     auto held = [&](int i) -> int { return tid + i * THREADS; };      // which float4 of the row register i holds
-    float4 hold[kCvtHold];
+    float4 hold[kHold];
 #pragma unroll
-    for (int i = 0; i < kCvtHold; ++i) {
+    for (int i = 0; i < kHold; ++i) {
         const int q = held(i);
         hold[i] = q < k4 ? raw4(q) : float4{0.f, 0.f, 0.f, 0.f};
+    }
+    if (SRC == kSrcSums) {
+        // Added here, in the order of gemm_chunk_sum4_kernel, and stored by the one thread that holds them (the launcher sees to it that
+        // a row fits its registers): a launch less, and the rows are read once.  Bound: latency, so the requests of four chunks travel
+        // together, on 1024 threads (200 rows of 4096, sums and conversion: 10.8 us as two launches, 9.3 chunk by chunk on 256 threads, 7.6).
+        // Output projection and FFN, us: 200 rows of 4096 / 14336 169.9 -> 168.0, 100 of 4096 / 8192 (Q8_0) 110.4 -> 107.1, 53 of 1536 /
+        // 3584 41.7 -> 40.6; 400 of 4096 / 14336 the same.
+        const float4* p = reinterpret_cast<const float4*>(S.sums + (int64_t)m * K);
+        const int64_t step = (int64_t)gridDim.x * k4;
+        for (int kc = 0; kc < S.sum_chunks; kc += 4, p += 4 * step) {
+            float4 part[4][kHold];
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+#pragma unroll
+                for (int i = 0; i < kHold; ++i)
+                    if (kc + c < S.sum_chunks && held(i) < k4) part[c][i] = p[c * step + held(i)];
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+#pragma unroll
+                for (int i = 0; i < kHold; ++i)
+                    if (kc + c < S.sum_chunks && held(i) < k4)
+                        hold[i] = float4{hold[i].x + part[c][i].x, hold[i].y + part[c][i].y, hold[i].z + part[c][i].z, hold[i].w + part[c][i].w};
+        }
+        float4* rows = reinterpret_cast<float4*>(S.rows + (int64_t)m * S.ldx);
+#pragma unroll
+        for (int i = 0; i < kHold; ++i)
+            if (held(i) < k4) rows[held(i)] = hold[i];
     }
     // optional RMSNorm prologue (ggml-cpu/ops.cpp:3646-3695: sum of squares in double, scale = 1/sqrtf(mean + eps),
     // then the multiply by the norm weight: (x * scale) * w)
@@ -214,7 +247,7 @@ __global__ void __launch_bounds__(THREADS) convert_x_kernel(const ConvertSrc S, 
     if (norm_w) {
         double ss = 0.0;
 #pragma unroll
-        for (int i = 0; i < kCvtHold; ++i)
+        for (int i = 0; i < kHold; ++i)
             ss += (double)(hold[i].x * hold[i].x) + (double)(hold[i].y * hold[i].y) + (double)(hold[i].z * hold[i].z) +
                   (double)(hold[i].w * hold[i].w);
         for (int k = kHeld + tid; k < K; k += THREADS) ss += (double)(src[k] * src[k]);
@@ -226,7 +259,7 @@ __global__ void __launch_bounds__(THREADS) convert_x_kernel(const ConvertSrc S, 
         for (int i = 0; i < THREADS / 64; ++i) tot += redd[i];
         rms = 1.0f / sqrtf((float)(tot / (double)K) + S.eps);
 #pragma unroll
-        for (int i = 0; i < kCvtHold; ++i) {
+        for (int i = 0; i < kHold; ++i) {
             const int q = held(i);
             if (q < k4) {
                 const float4 wv = reinterpret_cast<const float4*>(norm_w)[q];
@@ -237,7 +270,7 @@ __global__ void __launch_bounds__(THREADS) convert_x_kernel(const ConvertSrc S, 
     auto tail_value = [&](int k) { return norm_w ? (src[k] * rms) * norm_w[k] : raw1(k); };
     float amax = 0.f;
 #pragma unroll
-    for (int i = 0; i < kCvtHold; ++i)
+    for (int i = 0; i < kHold; ++i)
         amax = fmaxf(amax, fmaxf(fmaxf(fabsf(hold[i].x), fabsf(hold[i].y)), fmaxf(fabsf(hold[i].z), fabsf(hold[i].w))));
     for (int k = kHeld + tid; k < K; k += THREADS) amax = fmaxf(amax, fabsf(tail_value(k)));
     for (int o = 32; o > 0; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o));
@@ -264,7 +297,7 @@ __global__ void __launch_bounds__(THREADS) convert_x_kernel(const ConvertSrc S, 
     // activations 16 further on, which the lane four to the right (left) holds - the pair swaps them and each stores
     // one half of the 16 bytes.
 #pragma unroll
-    for (int i = 0; i < kCvtHold; ++i) {
+    for (int i = 0; i < kHold; ++i) {
         const int q = tid + i * THREADS;
         const float4 v = float4{hold[i].x * inv, hold[i].y * inv, hold[i].z * inv, hold[i].w * inv};
         uint2 o;
@@ -858,6 +891,7 @@ struct GemmArgs {
     // register-resident kernel with K cut into chunks: chunk kc of a row tile writes its sums (already scaled) to
     // partial[kc][activation row][column]; a second kernel adds the chunks in order into c
     float* partial;          // null: one chunk, results go straight to c
+    PendingSums* pending;    // host: where the sums are left to the caller instead (it adds them to c)
     int k_chunks;
     int chunk_kt;            // k-tiles per chunk (8 wavefronts x KTW)
     int x_pieces;            // the activations are in pieces, row by row (piece_start): gemm_slim_kernel
@@ -3198,6 +3232,10 @@ __global__ void __launch_bounds__(256) gemm_chunk_sum4_kernel(const float* __res
 // c[row] (+)= the chunk sums of a launch whose K was cut into chunks
 bool launch_chunk_sum(const GemmArgs& a, hipStream_t stream)
 {
+    if (a.pending) {
+        *a.pending = PendingSums{a.partial, a.k_chunks};
+        return true;
+    }
     const bool vec = (a.N & 3) == 0 && (a.ldc & 3) == 0 && (reinterpret_cast<uintptr_t>(a.c) & 15) == 0 &&
                      (reinterpret_cast<uintptr_t>(a.partial) & 15) == 0;
     if (vec)
@@ -4347,6 +4385,10 @@ template <int TYPE, int SRC>
 void launch_convert_typed(const ConvertSrc& src, int M, int K, int kp, _Float16* x16, float* scales, hipStream_t stream, int layout)
 {
     const int ldo = x_row_halfs(K), piece_rows = layout == 3 ? M : 0;
+    if constexpr (SRC == kSrcSums) {
+        hipLaunchKernelGGL((convert_x_kernel<TYPE, kSumsThreads, SRC>), dim3(M), dim3(kSumsThreads), 0, stream, src, K, kp, ldo, x16, scales, piece_rows);
+        return;
+    }
     // short rows: 256 threads hold the whole row and eight workgroups share a CU
     if (K <= 256 * kCvtHold * 4)
         hipLaunchKernelGGL((convert_x_kernel<TYPE, 256, SRC>), dim3(M), dim3(256), 0, stream, src, K, kp, ldo, x16, scales, piece_rows);
@@ -4365,9 +4407,11 @@ bool launch_convert(int type, const ConvertSrc& src, int M, int K, void* workspa
             set_last_error("gemm: the MX activation layout is for MXFP4 weights.");
             return false;
         }
-        const int chunks = (kp / 32 + kMxCvtBlocks - 1) / kMxCvtBlocks;
-        hipLaunchKernelGGL((convert_x_mx_kernel<SRC>), dim3((unsigned)((int64_t)M * chunks)), dim3(kMxCvtBlocks), 0, stream, src, K, kp,
-                           x_row_halfs(K), chunks, x16, scales);
+        if constexpr (SRC != kSrcSums) {
+            const int chunks = (kp / 32 + kMxCvtBlocks - 1) / kMxCvtBlocks;
+            hipLaunchKernelGGL((convert_x_mx_kernel<SRC>), dim3((unsigned)((int64_t)M * chunks)), dim3(kMxCvtBlocks), 0, stream, src, K, kp,
+                               x_row_halfs(K), chunks, x16, scales);
+        }
         return hip_ok(hipGetLastError(), "activation convert launch");
     }
     if (layout == 2 || (layout == 3 && type == kTypeQ4_K)) type = kTypeQ8_0;      // natural order
@@ -4396,6 +4440,26 @@ bool launch_convert_x(int type, const float* x, int64_t ldx, const int* row_map,
     src.eps = eps;
     return silu ? launch_convert<kSrcSilu>(type, src, M, K, workspace, stream, layout)
                 : launch_convert<kSrcPlain>(type, src, M, K, workspace, stream, layout);
+}
+
+bool convert_sums_fits(int type, int x_layout, int K) { return x_layout != 1 && type != kTypeMXFP4 && K % 4 == 0 && K <= kSumsThreads * kSumsHold * 4; }
+
+bool launch_convert_x_sums(int type, const PendingSums& sums, float* rows, int64_t ld, int M, int K, void* workspace, hipStream_t stream,
+                           const float* norm_w, float eps, int layout)
+{
+    if (!convert_sums_fits(type, layout, K)) {
+        set_last_error("gemm: no conversion of this layout adds the sums of K chunks.");
+        return false;
+    }
+    ConvertSrc src{};
+    src.x = rows;
+    src.ldx = ld;
+    src.norm_w = norm_w;
+    src.eps = eps;
+    src.sums = sums.partial;
+    src.sum_chunks = sums.chunks;
+    src.rows = rows;
+    return launch_convert<kSrcSums>(type, src, M, K, workspace, stream, layout);
 }
 
 bool launch_convert_x_swiglu(int type, const float* gate_up, const float* bias, const int* expert_of, float alpha, float limit,
@@ -4510,11 +4574,13 @@ GemmPlan plan_gemm(int type, int M, int N, int K, bool accumulate, size_t max_ch
 }
 
 bool launch_gemm(int type, const GemmPlan& plan, const void* w, int64_t w_bytes, const void* workspace, float* c, int64_t ldc, int M, int N,
-                 int K, hipStream_t stream, bool accumulate, void* chunk_ws, size_t chunk_ws_bytes)
+                 int K, hipStream_t stream, bool accumulate, void* chunk_ws, size_t chunk_ws_bytes, PendingSums* pending)
 {
     const ChunkScratch cs{static_cast<float*>(chunk_ws), chunk_ws ? chunk_ws_bytes : 0, nullptr};
     GemmArgs a{};
-    return gemm_args(&a, w, w_bytes, workspace, c, ldc, M, N, K, plan.x_layout) && gemm_dispatch_plan(type, a, plan, stream, accumulate, cs);
+    if (!gemm_args(&a, w, w_bytes, workspace, c, ldc, M, N, K, plan.x_layout)) return false;
+    a.pending = pending;
+    return gemm_dispatch_plan(type, a, plan, stream, accumulate, cs);
 }
 
 bool launch_gemm_tiles(int type, const GemmTiles& tiles, const void* w, int64_t w_bytes, const void* workspace, float* c, int64_t ldc,

@@ -160,6 +160,17 @@ struct GemmPlan {
 // max_chunk_bytes: what the launch will be given; kernels and K chunks whose sums do not fit are passed over
 GemmPlan plan_gemm(int type, int M, int N, int K, bool accumulate, size_t max_chunk_bytes = ~(size_t)0);
 
+// The sums of a product's K chunks that its launch has left in its scratch, partial[chunk][row][column] (chunks 0: none, the results are
+// complete), for the conversion that reads the rows next to add.
+struct PendingSums {
+    const float* partial;
+    int chunks;
+};
+// rows += the sums (stored), then converted as launch_convert_x does with norm_w
+bool convert_sums_fits(int type, int x_layout, int K);
+bool launch_convert_x_sums(int type, const PendingSums& sums, float* rows, int64_t ld, int M, int K, void* workspace, hipStream_t stream,
+                           const float* norm_w, float eps, int layout);
+
 // fp32 activations -> workspace (fp16 in the weight format's unpack order + per-row scales);
 // row_map (device, optional) gathers source rows.
 // norm_w (device, optional) applies RMSNorm first: x <- x / sqrt(mean(x^2) + eps) * norm_w.
@@ -197,7 +208,7 @@ bool launch_gemm_swiglu_mx(const void* w, const void* workspace, void* workspace
 // chunk_ws (device): where the sums of K chunks go, plan.chunk_bytes of them (with less, 128- and 256-row tiles run with whole K
 // and the other kernels fail: plan_gemm takes the bound).  Nothing is allocated.
 bool launch_gemm(int type, const GemmPlan& plan, const void* w, int64_t w_bytes, const void* workspace, float* c, int64_t ldc, int M, int N,
-                 int K, hipStream_t stream, bool accumulate, void* chunk_ws, size_t chunk_ws_bytes);
+                 int K, hipStream_t stream, bool accumulate, void* chunk_ws, size_t chunk_ws_bytes, PendingSums* pending = nullptr);
 // the same by tile tables: c[row] with row = c_rows ? c_rows[m] : m
 bool launch_gemm_tiles(int type, const GemmTiles& tiles, const void* w, int64_t w_bytes, const void* workspace, float* c, int64_t ldc,
                        const int* c_rows, int M, int N, int K, hipStream_t stream, void* chunk_ws, size_t chunk_ws_bytes, int x_layout);
