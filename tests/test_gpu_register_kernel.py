@@ -14,7 +14,8 @@ pytestmark = pytest.mark.gpu
 FORMATS = {"q4_0": (2, 32), "q4_1": (3, 32), "q5_0": (6, 32), "q5_1": (7, 32), "q8_0": (8, 32), "q4_k": (12, 256), "q5_k": (13, 256),
            "q6_k": (14, 256), "iq4_nl": (20, 32)}
 # rows, columns, K in units of 256 (formats of 32-weight blocks: 32 less, an odd number of blocks)
-SHAPES = [(4, 64, 1), (16, 65, 3), (17, 4097, 9), (32, 79, 16), (33, 1041, 17), (16, 300, 18), (24, 4100, 23), (61, 1027, 33)]
+SHAPES = [(4, 64, 1), (16, 65, 3), (17, 4097, 9), (32, 79, 16), (33, 1041, 17), (16, 300, 18), (24, 4100, 23), (61, 1027, 33),
+          (7, 129, 10), (12, 200, 16), (20, 70, 3), (40, 200, 8), (40, 200, 11)]
 
 
 @pytest.mark.parametrize("name", sorted(FORMATS))
