@@ -23,6 +23,7 @@
 // are then rounded to fp16 operands (Q4_K: d*sc and dmin*m rounded to fp16 first); the contraction
 // is TensorSharp.Models/ModelBase.cs:924-991 with fp32 accumulation on the matrix cores.
 #include "tship_internal.h"
+#include "unit_runs.h"
 
 #include <algorithm>
 #include <mutex>
@@ -2795,17 +2796,10 @@ __global__ void __launch_bounds__(512) gemm_slim_kernel(const GemmArgs A)
         for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o);
         live_tiles = __builtin_amdgcn_readfirstlane(c);
     }
-    // units = (row tile, K chunk, 16-column tile), column tile fastest; every workgroup takes one contiguous run.  A unit of the last
-    // chunk, which may be short, weighs less: the blocks per wavefront, and about as much as one more for the tile itself.
-    const int chunk_steps = (A.chunk_kt / S + 7) >> 3, last_steps = ((nkt - (A.k_chunks - 1) * A.chunk_kt + S - 1) / S + 7) >> 3;
-    const int64_t front = (int64_t)(A.k_chunks - 1) * n16 * (chunk_steps + 1), weight = front + (int64_t)n16 * (last_steps + 1);
-    auto unit_at = [&](int64_t at) {
-        const int mt = (int)(at / weight);
-        const int rem = (int)(at - mt * weight);
-        return mt * per_tile + (rem < front ? rem / (chunk_steps + 1) : (A.k_chunks - 1) * n16 + (rem - (int)front) / (last_steps + 1));
-    };
-    int u = unit_at(live_tiles * weight * blockIdx.x / gridDim.x);
-    const int u_end = unit_at(live_tiles * weight * (blockIdx.x + 1) / gridDim.x);
+    // a unit weighs the blocks per wavefront, and about as much as one more for the tile itself
+    const UnitRuns runs{live_tiles, A.k_chunks, n16, ((A.chunk_kt / S + 7) >> 3) + 1, (((nkt - (A.k_chunks - 1) * A.chunk_kt + S - 1) / S + 7) >> 3) + 1};
+    int u = runs.first(blockIdx.x, gridDim.x);
+    const int u_end = runs.first(blockIdx.x + 1, gridDim.x);
 
     while (u < u_end) {
         const int mt = u / per_tile, rem = u - mt * per_tile;
