@@ -893,6 +893,7 @@ struct GemmArgs {
     int64_t expert_stride;   // bytes between experts
     const int64_t* expert_off;  // optional [experts]: byte offset of each expert from w instead (experts held by pointer)
     int accumulate;          // c += ... instead of c = ...
+    int by_tiles;            // host: a launch by tile tables, also where its size is asked for and there are none yet
     // register-resident kernel with K cut into chunks: chunk kc of a row tile writes its sums (already scaled) to
     // partial[kc][activation row][column]; a second kernel adds the chunks in order into c
     float* partial;          // null: one chunk, results go straight to c
@@ -2327,7 +2328,7 @@ bool launch_tiles(GemmArgs a, int m_tiles, hipStream_t stream, const ChunkScratc
     a.k_chunks = 1;
     a.chunk_kt = (nkt + 3) / 4 * 4;
     a.partial = nullptr;
-    if (!a.tile_expert) {
+    if (!a.by_tiles) {
         const int per_cu = std::max(1, (int)((160 * 1024) / (lds + 512)));
         // measured: about 1.7 us per k-tile of a 256 x 256 tile when all CUs are busy
         a.k_chunks = pick_k_chunks(a.m_tiles * a.n_tiles, nkt, device_info().num_cus * per_cu, (int64_t)a.M * a.N,
@@ -2372,7 +2373,7 @@ bool launch_xw(GemmArgs a, int m_tiles, hipStream_t stream, const ChunkScratch& 
     a.k_chunks = 1;
     a.chunk_kt = (nkt + 3) / 4 * 4;
     a.partial = nullptr;
-    if (!a.tile_expert) {
+    if (!a.by_tiles) {
         a.k_chunks = pick_k_chunks(a.m_tiles * a.n_tiles, nkt, device_info().num_cus, (int64_t)a.M * a.N, 1.7 * BM * BN / 65536.0);
         if (a.k_chunks > 1) {
             a.chunk_kt = ((nkt + a.k_chunks - 1) / a.k_chunks + 3) / 4 * 4;
@@ -4049,9 +4050,9 @@ bool launch_slim_rows(const GemmArgs& a, int ktw, int m_tiles, hipStream_t strea
 template <typename G>
 bool launch_slim_for(const GemmArgs& a, int m_tiles, hipStream_t stream, const ChunkScratch& cs)
 {
-    const SlimPlan p = slim_plan<G>(a.Kp / kBK, a.M, a.N, a.tile_expert != nullptr, a.accumulate != 0);
+    const SlimPlan p = slim_plan<G>(a.Kp / kBK, a.M, a.N, a.by_tiles != 0, a.accumulate != 0);
     if (p.cols == 32) return launch_slim_rows<G, 2, 32>(a, p.ktw, m_tiles, stream, cs);
-    if (!a.tile_expert && a.M <= 16) return launch_slim_rows<G, 1, 16>(a, p.ktw, m_tiles, stream, cs);
+    if (!a.by_tiles && a.M <= 16) return launch_slim_rows<G, 1, 16>(a, p.ktw, m_tiles, stream, cs);
     if (p.ktw <= 4) {
         set_last_error("gemm: no register-resident kernel of 32 rows for this K.");
         return false;
@@ -4160,21 +4161,21 @@ bool launch_for_type(const GemmArgs& a, int bm, int m_tiles, const WidePlan& wid
         if (bm == 128) return launch_xw<PQ4K, 128, 4>(a, m_tiles, stream, cs);
     } else if constexpr (std::is_same<G, GMXFP4>::value) {
         if (a.x_mx) {
-            if (bm == 256 && !a.tile_expert) return launch_mx<256>(a, m_tiles, stream, cs);
-            if (bm == 128 && !a.tile_expert) return launch_mx<128>(a, m_tiles, stream, cs);
+            if (bm == 256 && !a.by_tiles) return launch_mx<256>(a, m_tiles, stream, cs);
+            if (bm == 128 && !a.by_tiles) return launch_mx<128>(a, m_tiles, stream, cs);
             // a plain small batch whose K fits one chunk, in 48-row units where those are at most two thirds as many as
             // 32-row units (33 .. 48, 65 .. 96, 129 .. 144 rows): a unit less is a pass less over the weights, and a 48-row
             // pass costs a little more than a 32-row one (32 x 184320 x 2880 65 us; 48 rows 77 instead of 97, 96 rows 132
             // instead of 164, but 128 rows 208 instead of 186)
-            if (bm == 32 && !a.tile_expert && !a.accumulate && a.Kp / kBK <= 48 && 3 * ((a.M + 47) / 48) <= 2 * ((a.M + 31) / 32))
+            if (bm == 32 && !a.by_tiles && !a.accumulate && a.Kp / kBK <= 48 && 3 * ((a.M + 47) / 48) <= 2 * ((a.M + 31) / 32))
                 return launch_slim_mx48<0>(a, (a.M + 47) / 48, stream, cs);
             if (bm == 32) return launch_slim_mx_for<1>(a, m_tiles, stream, cs);
             if (bm == 48) return launch_slim_mx48<0>(a, m_tiles, stream, cs);
             set_last_error("gemm: the MX activation layout serves 32- and 48-row units and plain launches of 128- and 256-row tiles.");
             return false;
         }
-        if (bm == 256 && !a.tile_expert) return launch_xw<PMXFP4, 256, 4>(a, m_tiles, stream, cs);
-        if (bm == 128 && !a.tile_expert) return launch_xw<PMXFP4, 128, 4>(a, m_tiles, stream, cs);
+        if (bm == 256 && !a.by_tiles) return launch_xw<PMXFP4, 256, 4>(a, m_tiles, stream, cs);
+        if (bm == 128 && !a.by_tiles) return launch_xw<PMXFP4, 128, 4>(a, m_tiles, stream, cs);
         if (bm == 128) return launch_tiles<G, 128, 2, 4>(a, m_tiles, stream, cs);
     } else {
         if constexpr (2 * 256 * kXRow + 2 * 256 * G::kRawRow + 1024 <= 160 * 1024) {
@@ -4528,10 +4529,10 @@ bool gemm_dispatch_plan(int type, GemmArgs a, const GemmPlan& plan, hipStream_t 
     return gemm_dispatch(type, a, plan.bm, plan.bm == kWideTiles ? 1 : (a.M + plan.bm - 1) / plan.bm, wide, stream, cs);
 }
 
-// only tiles->bm and tiles->count matter when nothing is launched
 bool gemm_dispatch_tiles(int type, GemmArgs a, const int* c_rows, const GemmTiles& tiles, hipStream_t stream, const ChunkScratch& cs)
 {
     a.c_rows = c_rows;
+    a.by_tiles = 1;
     a.tile_expert = tiles.expert;
     a.tile_row0 = tiles.row0;
     a.tile_rows = tiles.rows;

@@ -195,6 +195,24 @@ def test_scratch_of_gated_rows_is_not_reserved_where_the_conversion_forms_them(s
         assert need <= got / 1.25 < need + 4 * M * F, (got / 1.25, need)
 
 
+TILE_SCRATCH = """
+w = space(max(H, F) * max(H, F) // 32 * 34)
+x, r = space(4 * M * H).view(np.float32), space(4 * M * H).view(np.float32)
+e, up, down = (C.c_void_p * n)(*[w.ctypes.data] * n), (8, H, F, F * H // 32 * 34), (8, F, H, F * H // 32 * 34)
+assert L.TSHip_MoEExpertsSwiGLUForwardF32Device(view(r, M, H), view(x, M, H), n, e, e, e, *up, *up, *down, (C.c_float * n)(*[1] * n)), L.TSHip_GetLastError()
+out.append(log())
+"""
+
+
+@pytest.mark.parametrize("n,M,H,F", [(2, 200, 4096, 512), (3, 300, 4096, 512), (2, 161, 512, 4096)])
+def test_expert_sets_on_128_row_tiles_reserve_no_chunk_sums(stub, n, M, H, F):
+    """Launches by tile tables run with whole K; the size of their scratch is asked for before the tables are there."""
+    (log,) = stub(TILE_SCRATCH, n=n, M=M, H=H, F=F)
+    (got,) = [int(l[1]) for l in log if l[0] == "malloc"]
+    need = n * M * (8 * F + 4 * H + 2 * H + 2 * F)                          # (gate | up), the results, the converted rows of both
+    assert need <= got / 1.25 < need + n * M * 64 + (1 << 16), (got / 1.25, need)
+
+
 def test_only_stamped_launches_leave_the_split_kernel(stub):
     """While a timeline buffer is set, plain launches of few and long rows run unsplit; those with the RMSNorm are not stamped."""
     on = "assert L.TSHip_SetGemvTimeline(C.c_void_p(4096), 1 << 20)\n"
