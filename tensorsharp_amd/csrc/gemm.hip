@@ -4012,23 +4012,52 @@ int slim32_ktw(int nkt)
     return std::min(limit, (need + G::kTileStep - 1) / G::kTileStep * G::kTileStep);
 }
 
-// 16 columns unless the work between two barriers is too short or larger units fill the chip better (us, 16 / 32 columns):
-//  - more than 16 rows and at most four k-tiles per wavefront (Q6_K 93 x 6327 x 2048 20.8 / 18.5, 331 x 5764 x 1792 39.2 / 35.6);
-//  - several row tiles or chunks whose units of 32 columns are at most one per CU where those of 16 are more, or K beyond 4096
-//    with as few (a workgroup then loads one set of activations: Q6_K 30 x 2609 x 4864 18.1 / 14.2, Q8_0 16 x 317 x 10144 17.1 / 13.7,
-//    Q4_K 92 x 2104 x 2304 15.3 / 12.7, 50 x 368 x 13056 19.6 / 17.5), or results that are added to a residual, by the second launch
-//    in any case, so that chunks cost none (FFN of 53 rows, Q8_0 1536 / 3584: 43.3 / 41.8);
-//  - more than 32 rows of fewer than 1024 columns, which keep the chunks, and with them the workspace, that their plans have had
-//    (Q6_K 67 x 590 x 5632 16.9 / 14.4, but Q8_0 45 x 1001 x 2080 10.9 / 15.4).
+// Whether workgroups that take the units from floor(units b / cus) on cross into another segment (row tile and K chunk) of `tiles` units.
+// Segment i ends inside a workgroup's run unless tiles ((-i cus) mod segments) < cus, and over all i that remainder is at most
+// segments - gcd(segments, cus).
+inline bool runs_cross(int64_t segments, int64_t tiles)
+{
+    const int cus = device_info().num_cus;
+    return segments * tiles > cus && tiles * (segments - std::gcd(segments, (int64_t)cus)) >= cus;
+}
+
+inline bool chunk_sums_fit(int k_chunks, int M, int N, size_t max_bytes) { return (size_t)k_chunks * M * N * sizeof(float) <= max_bytes; }
+
+// The kernel that is expected to take less: 16 columns where that spares the launch for the sums, else by the k-tiles of the workgroup
+// that has most of them and the activations it loads anew where its run crosses into another row tile or K chunk.  In hundredths of a
+// us, fitted to 6500 whole calls of the ten formats on both kernels (4 .. 420 rows, 256 .. 21504 columns, K of 1024 .. 21504, weights
+// from HBM and from the memory-side cache): the pick is 0.5 % behind the faster one on average, more than 4 % behind on 320 of them.
+// Either kernel alone would be 2 (16) and 9 % (32) behind.  us, 16 / 32 columns:
+//   Q6_K 23 x 5120 x 6144 25.4 / 19.6, Q8_0 27 x 2560 x 14336 (added) 29.8 / 24.7, MXFP4 26 x 4096 x 14336 28.7 / 22.5 (runs that cross),
+//   Q4_K 24 x 14336 x 4096 18.4 / 20.3, Q8_0 24 x 4096 x 2560 10.8 / 15.1 (one launch).
+// Up to 16 rows: half the matrix instructions of 32, so less per k-tile; with at most four k-tiles per wavefront the tile's sums and
+// barrier weigh more, and twice as many tiles of 16 columns lose (Q6_K 13 x 8192 x 1024 9.8 / 9.4; 3 against 2 win, 0.94).
+// More than 32 rows of fewer than 1024 columns keep the chunks, and with them the workspace, of the 32-column kernel.
+// max_bytes: of the chunk sums; a kernel whose sums do not fit gives way to one whose sums do.  row_tiles may count empty tiles of a table.
 template <typename G>
-SlimPlan slim_plan(int nkt, int M, int N, bool tiles, bool accumulate)
+SlimPlan slim_plan(int nkt, int M, int N, int row_tiles, bool by_tiles, bool accumulate, size_t max_bytes)
 {
     const int ktw = slim_ktw<G>(nkt), ktw32 = slim32_ktw<G>(nkt), cus = device_info().num_cus;
-    if (M <= 16 && !tiles && !accumulate && nkt <= 64) return {16, ktw};
-    const int64_t rows = (M + 31) / 32, chunks = (nkt + 8 * ktw - 1) / (8 * ktw), chunks32 = (nkt + 8 * ktw32 - 1) / (8 * ktw32);
-    const int64_t units = rows * chunks * ((N + 15) / 16), units32 = rows * chunks32 * ((N + 31) / 32);
-    const bool few = units32 <= cus && (nkt > 64 || (rows * chunks > 1 && units > cus) || (accumulate && ktw32 < ktw));
-    return ktw <= 4 || few || (M > 32 && N < 1024) ? SlimPlan{32, ktw32} : SlimPlan{16, ktw};
+    const bool rows16 = M <= 16 && !by_tiles;
+    // (at most four k-tiles and 32 rows: no kernel of 16 columns; Q6_K 93 x 6327 x 2048 20.8 / 18.5, 331 x 5764 x 1792 39.2 / 35.6)
+    if ((ktw <= 4 && !rows16) || (M > 32 && N < 1024)) return {32, ktw32};
+    const int chunks = (nkt + 8 * ktw - 1) / (8 * ktw), chunks32 = (nkt + 8 * ktw32 - 1) / (8 * ktw32);
+    const bool sums = chunks > 1 || accumulate, sums32 = chunks32 > 1 || accumulate;
+    const bool fits = !sums || chunk_sums_fit(chunks, M, N, max_bytes), fits32 = !sums32 || chunk_sums_fit(chunks32, M, N, max_bytes);
+    if (!fits32) return {16, ktw};
+    if (!fits) return {32, ktw32};
+    if (sums32 && !sums) return {16, ktw};
+    // k-tiles of a wavefront in a unit: of a whole chunk, of the last one
+    auto unit_kt = [](int kt) { return ((kt + G::kTileStep - 1) / G::kTileStep + 7) / 8 * G::kTileStep; };
+    const int full = unit_kt(std::min(8 * ktw, nkt)), last = unit_kt(nkt - (chunks - 1) * 8 * ktw), full32 = unit_kt(std::min(8 * ktw32, nkt));
+    const int64_t tiles = (N + 15) / 16, segments = (int64_t)row_tiles * chunks, units = segments * tiles;
+    const int64_t tiles32 = (N + 31) / 32, segments32 = (int64_t)row_tiles * chunks32, rounds32 = (segments32 * tiles32 + cus - 1) / cus;
+    int64_t kt = full;
+    if (units > cus)         // (dealt out by weight where the last chunk is shorter: at most a unit above the average)
+        kt = last == full ? (units + cus - 1) / cus * full : row_tiles * tiles * ((chunks - 1) * full + last) / cus + full;
+    const int64_t cost = kt * (!rows16 ? 29 : ktw <= 4 ? 24 : 17) + (units > cus && segments > 1 ? 22 * ktw : 0);
+    const int64_t cost32 = rounds32 * full32 * 46 + (runs_cross(segments32, tiles32) ? 58 : 0);
+    return cost <= cost32 ? SlimPlan{16, ktw} : SlimPlan{32, ktw32};
 }
 
 template <typename G, int RB, int COLS>
@@ -4050,13 +4079,9 @@ bool launch_slim_rows(const GemmArgs& a, int ktw, int m_tiles, hipStream_t strea
 template <typename G>
 bool launch_slim_for(const GemmArgs& a, int m_tiles, hipStream_t stream, const ChunkScratch& cs)
 {
-    const SlimPlan p = slim_plan<G>(a.Kp / kBK, a.M, a.N, a.by_tiles != 0, a.accumulate != 0);
+    const SlimPlan p = slim_plan<G>(a.Kp / kBK, a.M, a.N, m_tiles, a.by_tiles != 0, a.accumulate != 0, cs.bytes);
     if (p.cols == 32) return launch_slim_rows<G, 2, 32>(a, p.ktw, m_tiles, stream, cs);
     if (!a.by_tiles && a.M <= 16) return launch_slim_rows<G, 1, 16>(a, p.ktw, m_tiles, stream, cs);
-    if (p.ktw <= 4) {
-        set_last_error("gemm: no register-resident kernel of 32 rows for this K.");
-        return false;
-    }
     if constexpr (G::kTileStep == 2)
         if (p.ktw == 6) return launch_slim<G, 6, 2, 16>(a, m_tiles, stream, cs);
     return launch_slim<G, 8, 2, 16>(a, m_tiles, stream, cs);
@@ -4269,20 +4294,16 @@ constexpr RuleCosts kCostsQ6K{8.854, 1.208, 0.000, 0.366, 0.402, 0.244, 5.858, 2
                               3.284, 7.419, 3.358, 1.187};
 constexpr double kNotServed = 1e30;      // a kernel that a format has not, or whose chunk sums do not fit
 
-inline bool chunk_sums_fit(int k_chunks, int M, int N, size_t max_bytes) { return (size_t)k_chunks * M * N * sizeof(float) <= max_bytes; }
 inline double sums_us(const RuleCosts& c, int k_chunks, int M, int N) { return c.sums + (double)k_chunks * M * N * 8e-6 / c.sums_rate; }
 
 template <typename G>
 double slim_us(const RuleCosts& c, int M, int N, int nkt, bool accumulate, size_t max_chunk_bytes)
 {
-    const SlimPlan plan = slim_plan<G>(nkt, M, N, false, accumulate);
+    const SlimPlan plan = slim_plan<G>(nkt, M, N, (M + 31) / 32, false, accumulate, max_chunk_bytes);
     const int ktw = plan.ktw, kc = (nkt + 8 * ktw - 1) / (8 * ktw), cus = device_info().num_cus;
     const bool two_pass = kc > 1 || accumulate;          // (launch_slim adds to a residual in the second launch only)
     if (two_pass && !chunk_sums_fit(kc, M, N, max_chunk_bytes)) return kNotServed;
     const double sums = two_pass ? sums_us(c, kc, M, N) : 0.0;
-    // Workgroup b takes the units from floor(units b / cus) on.  Segment i ends inside a workgroup's run unless tiles ((-i cus) mod
-    // segments) < cus, and over all i that remainder is at most segments - gcd(segments, cus).
-    auto crosses = [&](int64_t segments, int64_t tiles) { return segments * tiles > cus && tiles * (segments - std::gcd(segments, (int64_t)cus)) >= cus; };
     // (wavefronts past the end of K leave theirs to the others)
     if (M > 64 || (M > 32 && N < 1024) || plan.cols == 32) {
         // (as 32-column tiles, also where those of 16 columns serve)
@@ -4291,12 +4312,12 @@ double slim_us(const RuleCosts& c, int M, int N, int nkt, bool accumulate, size_
         const double kt = 0.4 * far_ktw + 0.6 * nkt / (8.0 * far_kc);
         const double rows = M <= 32 || (M <= 160 && N >= 1024) ? c.far_rows_160 : c.far_rows;
         return c.far_call + rows * std::min(M, 32) * far_ktw / 256.0 + (double)((units + cus - 1) / cus) * (c.far_unit + c.far_unit_kt * kt) +
-               (crosses(segments, tiles) ? c.far_cross + c.far_cross_kt * far_ktw : 0.0) + (far_kc > 1 || accumulate ? sums_us(c, far_kc, M, N) : 0.0);
+               (runs_cross(segments, tiles) ? c.far_cross + c.far_cross_kt * far_ktw : 0.0) + (far_kc > 1 || accumulate ? sums_us(c, far_kc, M, N) : 0.0);
     }
     const int64_t segments = (int64_t)((M + 31) / 32) * kc, tiles = (N + 15) / 16, units = segments * tiles;
     const double kt = 0.4 * ktw + 0.6 * nkt / (8.0 * kc);
     return c.slim + c.slim_convert * M * (nkt * kBK) * 1e-6 + c.slim_rows * std::min(M, 32) * ktw / 256.0 +
-           (double)((units + cus - 1) / cus) * kt * (M <= 16 ? c.unit_kt_16 : c.unit_kt) + (crosses(segments, tiles) ? c.cross_kt * ktw : 0.0) + sums;
+           (double)((units + cus - 1) / cus) * kt * (M <= 16 ? c.unit_kt_16 : c.unit_kt) + (runs_cross(segments, tiles) ? c.cross_kt * ktw : 0.0) + sums;
 }
 
 // rounds of workgroups x k-tiles; the last round may leave CUs idle
@@ -4561,8 +4582,9 @@ GemmPlan plan_gemm(int type, int M, int N, int K, bool accumulate, size_t max_ch
     if (type == kTypeQ4_K && p.bm == kWideTiles) p.x_layout = 2;
     if (type == kTypeMXFP4 && K <= 1024 * kCvtHold * 4 && (p.bm >= 128 || (int64_t)N * K >= ((int64_t)64 << 20))) p.x_layout = 1;
     if (p.bm == 32 && p.x_layout == 0) p.x_layout = 3;
-    // the launcher's own dry run, with no bound, so that it makes the choices it would make with the reported bytes at hand
-    const ChunkScratch cs{nullptr, ~(size_t)0, &p.chunk_bytes};
+    // the launcher's own dry run, so that it makes the choices it would make with the reported bytes at hand; the register-resident
+    // kernels choose by the bound, the others are not given one
+    const ChunkScratch cs{nullptr, p.bm == 32 ? max_chunk_bytes : ~(size_t)0, &p.chunk_bytes};
     GemmArgs a{};
     const int64_t w_bytes = block_bytes(type) * (K / block_elems(type)) * N;
     if (!gemm_args(&a, nullptr, w_bytes, nullptr, nullptr, N, M, N, K, p.x_layout) || !gemm_dispatch_plan(type, a, p, nullptr, accumulate, cs))
