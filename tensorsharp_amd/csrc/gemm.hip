@@ -2754,9 +2754,9 @@ struct SlimLayout {
         const int fit = (kLds - sets_of(ch) * SET) / (8 * copies_of(ch) * 1024);
         return fit < 4 ? fit : 4;
     }
-    // an odd chunk count spreads the dword reads of the rows over twice as many LDS banks; taken when it costs no ring depth
-    static constexpr bool kOdd = (kNeed & 1) == 0 && ring_of(kNeed + 1) == ring_of(kNeed) && sets_of(kNeed + 1) == sets_of(kNeed);
-    static constexpr int CH = kNeed + (kOdd ? 1 : 0);
+    // An odd chunk count: the dword reads of the 16 rows spread over all LDS banks.  An even one would begin rows in the same banks, 16 chunks
+    // (Q4_1, six k-tiles; a fourth buffer fitted then) all of them: 11 x 4096 x 8608 21.1 / 18.9 us, 13 x 7046 x 2880 13.2 / 11.8.
+    static constexpr int CH = kNeed | 1;
     static constexpr int DI = copies_of(CH);                             // LDS-direct copies per buffer
     static constexpr int BUF = DI * 1024;
     static constexpr int SETS = sets_of(CH);
@@ -2772,6 +2772,7 @@ __global__ void __launch_bounds__(512) gemm_slim_kernel(const GemmArgs A)
     using L = SlimLayout<G, KTW, RB>;
     constexpr int CH = L::CH, DI = L::DI, BUF = L::BUF, RING = L::RING, SETS = L::SETS;
     static_assert(KTW % G::kTileStep == 0, "a wavefront's K range must start at a block");
+    static_assert(CH % 2 == 1, "rows of an even chunk count begin in the same LDS banks");
     // k-tiles of one step of the K loop, and k-halves of them that a lane unpacks itself
     constexpr int S = G::kTileStep, HALVES = S == 4 ? 2 : 1;
     static_assert(S == 4 || S == 2, "four lane groups: a k-tile or half a k-tile each");
