@@ -4405,7 +4405,13 @@ void launch_convert_typed(const ConvertSrc& src, int M, int K, int kp, _Float16*
 {
     const int ldo = x_row_halfs(K), piece_rows = layout == 3 ? M : 0;
     if constexpr (SRC == kSrcSums) {
-        hipLaunchKernelGGL((convert_x_kernel<TYPE, kSumsThreads, SRC>), dim3(M), dim3(kSumsThreads), 0, stream, src, K, kp, ldo, x16, scales, piece_rows);
+        // As few threads as hold the row (1024 for one row of 256 .. 2048 elements leave most of them idle, and two rows to a CU).  Output
+        // projection and FFN, us, sums by a launch of their own / 1024 / 256 threads: 445 rows of 256 / 6144 50.1 / 51.4 / 49.1, 323 of
+        // 1024 / 4352 71.4 / 72.2 / 70.5, 12 of 1024 / 2560 29.7 / 29.2 / 28.4, 49 of 2048 / 7424 47.5 / 46.9 / 46.5.
+        if (K <= 256 * kSumsHold * 4)
+            hipLaunchKernelGGL((convert_x_kernel<TYPE, 256, SRC>), dim3(M), dim3(256), 0, stream, src, K, kp, ldo, x16, scales, piece_rows);
+        else
+            hipLaunchKernelGGL((convert_x_kernel<TYPE, kSumsThreads, SRC>), dim3(M), dim3(kSumsThreads), 0, stream, src, K, kp, ldo, x16, scales, piece_rows);
         return;
     }
     // short rows: 256 threads hold the whole row and eight workgroups share a CU
