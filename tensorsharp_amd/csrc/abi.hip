@@ -703,7 +703,7 @@ ExpertSetLayout expert_set_layout(int M, int n, const ExpertFfn* ex, int H, int 
     return L;
 }
 
-// One linear of a tiled expert set: per block type one tile-table GEMM over the members whose weight has that type.
+// One linear of a tiled expert set: a tile-table GEMM per run of members whose weights share a block type.
 // x: fp32 source rows (ldx; silu: (gate | up) rows of 2 K floats), gathered through row_map when given; the members' results go to rows slot * M .. of c.
 struct ExpertLinear {
     const void* w[kMaxExpertSet];
@@ -722,18 +722,13 @@ bool run_expert_linear_tiled(const ExpertSetLayout& L, char* ws, int n, int M, c
     int64_t* offs = reinterpret_cast<int64_t*>(ws + L.tbl_off + 3 * tile_bytes);
     int* row_map = reinterpret_cast<int*>(ws + L.tbl_off + 3 * tile_bytes + al((size_t)n * 8));
     const int rows = n * M;
-    bool handled[kMaxExpertSet] = {};
-    for (int first = 0; first < n; ++first) {
-        if (handled[first]) continue;
+    for (int first = 0, end; first < n; first = end) {
         const int t = lin.type[first];
-        // base pointer: the lowest address among the type's members, so that every offset is >= 0
+        // the members from here on that share the type; base pointer: the lowest address among them, so that every offset is >= 0
         uintptr_t base = reinterpret_cast<uintptr_t>(lin.w[first]);
-        for (int e = first; e < n; ++e)
-            if (lin.type[e] == t) base = std::min(base, reinterpret_cast<uintptr_t>(lin.w[e]));
+        for (end = first + 1; end < n && lin.type[end] == t; ++end) base = std::min(base, reinterpret_cast<uintptr_t>(lin.w[end]));
         ExpertTileSpec spec{};
-        for (int e = first; e < n; ++e) {
-            if (lin.type[e] != t) continue;
-            handled[e] = true;
+        for (int e = first; e < end; ++e) {
             spec.off[spec.count] = (int64_t)(reinterpret_cast<uintptr_t>(lin.w[e]) - base);
             spec.slot[spec.count] = e;
             ++spec.count;
@@ -743,6 +738,8 @@ bool run_expert_linear_tiled(const ExpertSetLayout& L, char* ws, int n, int M, c
         if (!launch_convert_x(t, x, ldx, gather ? row_map : nullptr, rows, K, ws + x_off, stream, nullptr, 0.f, layout, silu)) return false;
         GemmTiles tiles{t_expert, t_row0, t_rows, spec.count * per, L.bm, (int64_t)(row_size(t, K) * (size_t)out_features)};
         tiles.expert_off = offs;
+        tiles.first_row = first * M;
+        tiles.row_count = (end - first) * M;
         if (!launch_gemm_tiles(t, tiles, reinterpret_cast<const void*>(base), tiles.expert_stride, ws + x_off, c, ldc, nullptr, rows,
                                out_features, K, stream, L.chunk_bytes ? ws + L.chunk_off : nullptr, L.chunk_bytes, layout))
             return false;

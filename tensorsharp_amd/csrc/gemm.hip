@@ -897,6 +897,7 @@ struct GemmArgs {
     // register-resident kernel with K cut into chunks: chunk kc of a row tile writes its sums (already scaled) to
     // partial[kc][activation row][column]; a second kernel adds the chunks in order into c
     float* partial;          // null: one chunk, results go straight to c
+    int sum_row0, sum_rows;  // host: the rows that the second kernel adds (0 rows: all M)
     PendingSums* pending;    // host: where the sums are left to the caller instead (it adds them to c)
     int k_chunks;
     int chunk_kt;            // k-tiles per chunk (8 wavefronts x KTW)
@@ -1027,8 +1028,6 @@ struct ChunkScratch {
     size_t* need_out;
 };
 inline float* chunk_scratch(const ChunkScratch& cs, size_t bytes) { return bytes <= cs.bytes ? cs.ptr : nullptr; }
-__global__ void gemm_chunk_sum_kernel(const float* __restrict__ partial, int k_chunks, int M, int N, const int* __restrict__ c_rows,
-                                      float* __restrict__ c, int64_t ldc, int accumulate);
 bool launch_chunk_sum(const GemmArgs& a, hipStream_t stream);
 
 // BM x 256 x 64 tiles, eight wavefronts, each owning all BM rows of 32 output columns.
@@ -3194,14 +3193,14 @@ __global__ void __launch_bounds__(512) gemm_slim32_kernel(const GemmArgs A)
     }
 }
 
-// c[row][n] (+)= sum over the K chunks of partial[kc][m][n], chunks added in order
-__global__ void __launch_bounds__(256) gemm_chunk_sum_kernel(const float* __restrict__ partial, int k_chunks, int M, int N,
+// c[row][n] (+)= sum over the K chunks of partial[kc][m][n] for rows m < rows of a chunk's M, chunks added in order
+__global__ void __launch_bounds__(256) gemm_chunk_sum_kernel(const float* __restrict__ partial, int k_chunks, int M, int N, int rows,
                                                              const int* __restrict__ c_rows, float* __restrict__ c, int64_t ldc,
                                                              int accumulate)
 {
     const int n = blockIdx.x * 256 + threadIdx.x;
     if (n >= N) return;
-    for (int m = blockIdx.y; m < M; m += gridDim.y) {
+    for (int m = blockIdx.y; m < rows; m += gridDim.y) {
         float* out = c + (int64_t)(c_rows ? c_rows[m] : m) * ldc + n;
         float s = accumulate ? *out : 0.f;
         for (int kc = 0; kc < k_chunks; ++kc) s += partial[((int64_t)kc * M + m) * N + n];
@@ -3210,13 +3209,13 @@ __global__ void __launch_bounds__(256) gemm_chunk_sum_kernel(const float* __rest
 }
 
 // the same, four columns per thread (N, ldc multiples of 4, c 16-byte aligned)
-__global__ void __launch_bounds__(256) gemm_chunk_sum4_kernel(const float* __restrict__ partial, int k_chunks, int M, int N,
+__global__ void __launch_bounds__(256) gemm_chunk_sum4_kernel(const float* __restrict__ partial, int k_chunks, int M, int N, int rows,
                                                               const int* __restrict__ c_rows, float* __restrict__ c, int64_t ldc,
                                                               int accumulate)
 {
     const int n = (blockIdx.x * 256 + threadIdx.x) * 4;
     if (n >= N) return;
-    for (int m = blockIdx.y; m < M; m += gridDim.y) {
+    for (int m = blockIdx.y; m < rows; m += gridDim.y) {
         float4* out = reinterpret_cast<float4*>(c + (int64_t)(c_rows ? c_rows[m] : m) * ldc + n);
         float4 s = accumulate ? *out : float4{0.f, 0.f, 0.f, 0.f};
         for (int kc = 0; kc < k_chunks; ++kc) {
@@ -3234,14 +3233,18 @@ bool launch_chunk_sum(const GemmArgs& a, hipStream_t stream)
         *a.pending = PendingSums{a.partial, a.k_chunks};
         return true;
     }
-    const bool vec = (a.N & 3) == 0 && (a.ldc & 3) == 0 && (reinterpret_cast<uintptr_t>(a.c) & 15) == 0 &&
-                     (reinterpret_cast<uintptr_t>(a.partial) & 15) == 0;
+    const int rows = a.sum_rows > 0 ? a.sum_rows : a.M;
+    const float* partial = a.partial + (int64_t)a.sum_row0 * a.N;
+    const int* c_rows = a.c_rows ? a.c_rows + a.sum_row0 : nullptr;
+    float* c = a.c_rows ? a.c : a.c + a.sum_row0 * a.ldc;
+    const bool vec = (a.N & 3) == 0 && (a.ldc & 3) == 0 && (reinterpret_cast<uintptr_t>(c) & 15) == 0 &&
+                     (reinterpret_cast<uintptr_t>(partial) & 15) == 0;
     if (vec)
-        hipLaunchKernelGGL(gemm_chunk_sum4_kernel, dim3((a.N / 4 + 255) / 256, std::min(a.M, 65535)), dim3(256), 0, stream, a.partial,
-                           a.k_chunks, a.M, a.N, a.c_rows, a.c, a.ldc, a.accumulate);
+        hipLaunchKernelGGL(gemm_chunk_sum4_kernel, dim3((a.N / 4 + 255) / 256, std::min(rows, 65535)), dim3(256), 0, stream, partial,
+                           a.k_chunks, a.M, a.N, rows, c_rows, c, a.ldc, a.accumulate);
     else
-        hipLaunchKernelGGL(gemm_chunk_sum_kernel, dim3((a.N + 255) / 256, std::min(a.M, 65535)), dim3(256), 0, stream, a.partial,
-                           a.k_chunks, a.M, a.N, a.c_rows, a.c, a.ldc, a.accumulate);
+        hipLaunchKernelGGL(gemm_chunk_sum_kernel, dim3((a.N + 255) / 256, std::min(rows, 65535)), dim3(256), 0, stream, partial,
+                           a.k_chunks, a.M, a.N, rows, c_rows, c, a.ldc, a.accumulate);
     return hip_ok(hipGetLastError(), "gemm chunk sum launch");
 }
 
@@ -4561,6 +4564,8 @@ bool gemm_dispatch_tiles(int type, GemmArgs a, const int* c_rows, const GemmTile
 {
     a.c_rows = c_rows;
     a.by_tiles = 1;
+    a.sum_row0 = tiles.first_row;
+    a.sum_rows = tiles.row_count;
     a.tile_expert = tiles.expert;
     a.tile_row0 = tiles.row0;
     a.tile_rows = tiles.rows;

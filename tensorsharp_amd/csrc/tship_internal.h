@@ -193,6 +193,9 @@ struct GemmTiles {
     int bm;
     int64_t expert_stride;
     const int64_t* expert_off = nullptr;   // device table, optional
+    // the rows that the tiles cover, where these are not all M (0 rows: all): sums of K chunks are added for no others, whose results
+    // are another launch's
+    int first_row = 0, row_count = 0;
 };
 
 // The gate_up GEMM of MXFP4 gpt-oss experts on 32-row tiles with the down projection's activations as its result:

@@ -220,3 +220,21 @@ def test_only_stamped_launches_leave_the_split_kernel(stub):
     for plain, norm in (stub(GEMV_LINEAR, cases=cases), stub(on + GEMV_LINEAR, cases=cases)):
         assert len(launches(norm, "gemv_split_kernel")) == 1
     assert not launches(plain, "gemv_split_kernel")
+
+
+TWO_TYPES = """
+w, blocks = space(max(H, I) * max(H, I) // 32 * 34), {8: 34, 2: 18}
+x, r = space(4 * M * H).view(np.float32), space(4 * M * H).view(np.float32)
+shape = lambda t: (t, H, I, I * H // 32 * blocks[t], t, H, I, I * H // 32 * blocks[t], t, I, H, H * I // 32 * blocks[t])
+e, p = (C.c_void_p * n)(*[w.ctypes.data] * n), C.c_void_p(w.ctypes.data)
+assert L.TSHip_MoEExpertsSwiGLUResidualF32Device(view(r, M, H), view(x, M, H), n, e, e, e, *shape(8), (C.c_float * n)(*[1] * n), 1, p, p, p, *shape(2), 1.0), L.TSHip_GetLastError()
+out.append(log())
+"""
+
+
+def test_sums_of_an_expert_set_of_two_types_are_added_for_the_rows_of_each(stub):
+    """Gate, up and down projections of four routed Q8_0 experts and a shared Q4_0 one, K in chunks: the sums of one type's launch are
+    added to its members' rows only, the others' rows are another launch's results."""
+    n, M = 4, 20
+    (log,) = stub(TWO_TYPES, n=n, M=M, H=8192, I=8192)
+    assert [int(l[3]) for l in launches(log, "gemm_chunk_sum")] == 3 * [n * M, M], launches(log, "gemm_chunk_sum")
