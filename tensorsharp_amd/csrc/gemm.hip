@@ -5,7 +5,7 @@
 //      magnitude overflows or underflows fp16), written in the k-order in which the weight
 //      format unpacks (so the dequantizer never has to shuffle lanes), zero-padded to a
 //      multiple of the k-tile.  Optionally gathers rows through an index (MoE).
-//   2. by size (gemm_tile_m) gemm_slim_kernel / gemm_slim32_kernel (32 rows per tile: activations in registers, K split over the wavefronts,
+//   2. by size (gemm_tile_m) gemm_slim_kernel / gemm_slim32_kernel (16 or 32 rows per tile: activations in registers, K split over the wavefronts,
 //      long K in chunks), gemm_wide_kernel (32 .. 128 rows x 256 columns, K in chunks that fill the chip) or
 //      gemm_xw_kernel / gemm_kernel (128 / 256 rows per tile).  gemm_kernel:
 //      BM x 256 x 64 tiles, eight wavefronts, each owning 32 output columns.  The fp16
@@ -861,7 +861,7 @@ struct GLegacy {
                 hi = (__builtin_amdgcn_perm(t3, t2, shh) & mh) | (__builtin_amdgcn_perm(t1, t0, shh) & ~mh);
                 bias = 0xe480e480u;                          // -(1024 + 128)
             } else {
-                bias = kMin ? 0xe400e400u : kFive ? 0xe410e410u : 0xe408e408u;   // -1024, -(1024 + 16), -(1024 + 8)
+                bias = kMin ? 0xe400e400u : 0xe410e410u;     // -1024, -(1024 + 16)
             }
 #pragma unroll
             for (int s2 = 0; s2 < 4; ++s2) {
@@ -1330,6 +1330,9 @@ struct PQ4K {
     }
 };
 
+// MXFP4: a k-tile is two 17-byte blocks = 34 bytes of a row that is only byte aligned.  The copied window is the 48 bytes from
+// (row start & ~3) + (34 kt & ~3): the blocks begin 0 .. 5 bytes into it (the row's own misalignment, and two bytes in every odd
+// k-tile), which GMXFP4's unpacker takes as its byte shift.
 struct PMXFP4 {
     typedef GMXFP4 G;
     static constexpr int kRegs = G::kRegs;
@@ -2725,10 +2728,11 @@ bool launch_mx(GemmArgs a, int m_tiles, hipStream_t stream, const ChunkScratch& 
 // What bounds it (leave-out builds, Q4_K 24 x 14336 x 4096, 13.8 us of the launch): unpacking 3.9 and the weights 4.7 on top of each
 // other, the activations 2.3; the tiles' matrix instructions, sums and barriers are most of the rest.  16 columns instead of 32: twice
 // the units for a chip of 256 CUs and half a tile less at the end; LDS that holds twice the K range per wavefront, so that K = 4096 is
-// one chunk in every format.  Whole calls, weights from HBM, us, with 32-column tiles before -> now: Q4_K 8 x 14336 x 4096 20.0 -> 16.9,
-// 24 x 4096 x 4096 13.5 -> 10.7, 24 x 4096 x 14336 24.8 -> 23.4; Q8_0 16 x 14336 x 4096 25.9 -> 22.0, 16 x 4096 x 4096 15.8 -> 11.7, Q6_K
-// 32 x 4096 x 4096 15.1 -> 12.2, Q5_K 32 x 4096 x 4096 15.3 -> 11.4, 48 x 14336 x 4096 33.0 -> 28.3; weights in the memory-side cache:
-// Q4_K 24 x 14336 x 4096 18.3 -> 18.3 (bound by unpacking and sums, not by the stream).
+// one chunk in every format.  Whole calls, weights from HBM, us, tiles of 32 / 16 columns: Q4_K 8 x 14336 x 4096 18.3 / 18.1, 24 x 4096 x
+// 4096 13.1 / 11.4; Q8_0 16 x 14336 x 4096 25.5 / 23.1, 16 x 4096 x 4096 14.0 / 12.1, 16 x 9728 x 2560 20.2 / 15.4; Q6_K 32 x 4096 x 4096
+// 14.0 / 12.8; Q5_K 32 x 4096 x 4096 13.2 / 11.8, 48 x 14336 x 4096 31.9 / 28.5.  Bound by unpacking and sums more than by the stream, and
+// lost, where a CU has three or four tiles of a cheap format: Q4_K 24 x 14336 x 4096 19.3 / 20.1, from the memory-side cache 16.1 / 17.2
+// (slim_plan picks).
 // ------------------------------------------------------------------------------------------
 // an address that is the same in every lane, for the compiler to keep in scalar registers
 __device__ __forceinline__ uintptr_t uniform_address(uintptr_t a)
@@ -4032,10 +4036,11 @@ inline bool chunk_sums_fit(int k_chunks, int M, int N, size_t max_bytes) { retur
 // us, fitted to 6500 whole calls of the ten formats on both kernels (4 .. 420 rows, 256 .. 21504 columns, K of 1024 .. 21504, weights
 // from HBM and from the memory-side cache): the pick is 0.5 % behind the faster one on average, more than 4 % behind on 320 of them.
 // Either kernel alone would be 2 (16) and 9 % (32) behind.  us, 16 / 32 columns:
-//   Q6_K 23 x 5120 x 6144 25.4 / 19.6, Q8_0 27 x 2560 x 14336 (added) 29.8 / 24.7, MXFP4 26 x 4096 x 14336 28.7 / 22.5 (runs that cross),
-//   Q4_K 24 x 14336 x 4096 18.4 / 20.3, Q8_0 24 x 4096 x 2560 10.8 / 15.1 (one launch).
+//   Q6_K 23 x 5120 x 6144 25.6 / 19.8, Q8_0 27 x 2560 x 14336 (added) 30.0 / 24.9, MXFP4 26 x 4096 x 14336 28.7 / 23.0 (runs that cross);
+//   Q8_0 24 x 4096 x 2560 11.2 / 13.4, Q6_K 10 x 2800 x 4096 11.4 / 13.3 (the launch for the sums spared);
+//   Q4_K 24 x 4096 x 4096 11.4 / 13.1, 24 x 14336 x 4096 20.1 / 19.3 (one tile of 16 columns per CU, and three to four).
 // Up to 16 rows: half the matrix instructions of 32, so less per k-tile; with at most four k-tiles per wavefront the tile's sums and
-// barrier weigh more, and twice as many tiles of 16 columns lose (Q6_K 13 x 8192 x 1024 9.8 / 9.4; 3 against 2 win, 0.94).
+// barrier weigh more, and twice as many tiles of 16 columns lose (Q6_K 13 x 8192 x 1024 10.2 / 9.8; 3 against 2 win, 0.94).
 // More than 32 rows of fewer than 1024 columns keep the chunks, and with them the workspace, of the 32-column kernel.
 // max_bytes: of the chunk sums; a kernel whose sums do not fit gives way to one whose sums do.  row_tiles may count empty tiles of a table.
 template <typename G>
@@ -4261,16 +4266,18 @@ namespace {
 // about 870 random ones per format over 4 .. 2048 rows, 64 .. 28672 columns and K of 256 .. 21504, a third of them added to a
 // residual.  On 300 further random calls per format the pick took 0.4 % (Q4_K), 0.3 % (Q8_0) and 0.2 % (Q6_K) longer than the
 // fastest candidate on average, more than 4 % longer on 11, 8 and 3 of them, 11 % at most.
-// The register-resident kernel of 16-column tiles was fitted anew, up to 64 rows, on 260 calls per format of 4 .. 420 rows, 300 .. 21504
-// columns and K of 1024 .. 14336: with these constants the pick is 0.05 / 0.07 / 0.00 % behind the faster of it and the best other kernel
-// there.  Above 64 rows, and above 32 under 1024 columns, the costs of the kernel of 32-column tiles before it still draw the line (the
-// far_ constants): the kernels do not cross at these edges, and where that kernel was taken this one serves.
+// The register-resident kernel of 16-column tiles was fitted by itself, up to 64 rows, on 260 calls per format of 4 .. 420 rows, 300 .. 21504
+// columns and K of 1024 .. 14336.  Above 64 rows, above 32 under 1024 columns, and where tiles of 32 columns serve (slim_plan), the costs of
+// that kernel draw the line (the far_ constants), whichever of the two is launched: they are the upper ones of the two, so rows go to the
+// other kernels too early if at all.  On 650 further calls per format the pick is 4.4 / 1.6 / 1.4 % (Q4_K / Q8_0 / Q6_K) behind the fastest of
+// the two and gemm_wide_kernel from 17 to 64 rows, 4.6 / 3.9 / 1.4 % above, most of it under 1024 columns (Q4_K 34 x 844 x 2560 15.6 us, 10.0
+// on tiles of 16 columns), and 0.5 % up to 16.
 // The candidates, us (register-resident / gemm_wide_kernel / 128 rows / 256 rows):
-//   Q4_K  24 x 14336 x 4096 19.2 / 22.8 / - / -,  64 x 828 x 2560 12.4 / 15.9 / - / 28.5,  88 x 3078 x 1792 11.2 / 17.5 / - / -,
-//         200 x 4096 x 2560 28.3 / 28.0 / - / 34.8,  257 x 512 x 14336 39.2 / 32.0 / - / 84.9,  480 x 9728 x 9728 (added) - / 142 / - / 124
-//   Q8_0  24 x 14336 x 4096 23.9 / 29.5 / - / -,  64 x 14336 x 4096 28.7 / 34.7 / 39.7 / 46.3,  128 x 9728 x 5376 54.8 / 45.1 / 56.2 / 64.6,
+//   Q4_K  24 x 14336 x 4096 19.4 / 25.0 / - / 38.2,  64 x 828 x 2560 11.9 / 15.8 / - / 28.3,  88 x 3078 x 1792 11.6 / 17.2 / - / 29.0,
+//         200 x 4096 x 2560 24.9 / 28.2 / - / 36.3,  257 x 512 x 14336 39.2 / 32.0 / - / 84.9,  480 x 9728 x 9728 (added) - / 142 / - / 124
+//   Q8_0  24 x 14336 x 4096 24.8 / 28.9 / 36.4 / 43.0,  64 x 14336 x 4096 29.9 / 33.9 / 39.0 / 45.5,  128 x 9728 x 5376 54.8 / 45.1 / 56.2 / 64.6,
 //         400 x 4096 x 4096 - / 41.1 / 41.5 / 48.5,  400 x 9728 x 9728 - / 146 / 173 / 125
-//   Q6_K  30 x 18504 x 1280 17.8 / 23.5 / - / -,  240 x 9728 x 14336 (added) 230 / 121 / 145 / -,  480 x 14336 x 4096 - / 94.8 / 114 / -
+//   Q6_K  30 x 18504 x 1280 17.8 / 23.4 / 31.5 / -,  240 x 9728 x 14336 (added) 230 / 121 / 145 / -,  480 x 14336 x 4096 - / 94.8 / 114 / -
 struct RuleCosts {
     // register-resident kernel: a call; converting a million activations; its activations, per 32 rows and 8 k-tiles per wavefront;
     // per k-tile of a wavefront in a round of units (up to 16 rows, more); per k-tile where a workgroup's units cross into another
@@ -4372,8 +4379,7 @@ int cheapest_tiles(const RuleCosts& c, int M, int N, int K, bool accumulate, siz
     const int nkt = (K + kBK - 1) / kBK;
     const double slim = slim_us<G>(c, M, N, nkt, accumulate, max_chunk_bytes);
     if (M <= 16 && slim < kNotServed) return 32;
-    // (up to 32 rows the other kernel has one row tile, one launch and no sums in the scratch: a near tie goes to it - Q4_K
-    // 32 x 4096 x 4096 16.7 vs 18.0 us)
+    // (up to 32 rows a near tie goes to the register-resident kernel: Q4_K 25 x 14383 x 5120 28.0 vs 28.3 us)
     const double wide = wide_us(c, M, N, nkt, accumulate, max_chunk_bytes, plan) * (M <= 32 ? 1.04 : 1.0);
     // (128-row tiles of Q4_K: never the cheapest)
     const double t128 = std::is_same<G, GQ4K>::value ? kNotServed : tile_us(c, 128, M, N, nkt, accumulate, max_chunk_bytes);
@@ -4388,7 +4394,8 @@ int gemm_tile_m(int type, int M, int N, int K, bool accumulate, size_t max_chunk
     if (type == kTypeQ4_K) return cheapest_tiles<GQ4K>(kCostsQ4K, M, N, K, accumulate, max_chunk_bytes, wide);
     if (type == kTypeQ8_0) return cheapest_tiles<GQ80>(kCostsQ80, M, N, K, accumulate, max_chunk_bytes, wide);
     if (type == kTypeQ6_K) return cheapest_tiles<GQ6K>(kCostsQ6K, M, N, K, accumulate, max_chunk_bytes, wide);
-    // (drawn while the register-resident kernel read its activations from whole rows; not measured since)
+    // (drawn while the register-resident kernel was of 32-column tiles and read its activations from whole rows; the tile kernels have not
+    // been measured against the present ones here)
     if (M <= 128) return 32;
     if (type == kTypeMXFP4 && M <= 512 && ((M + 127) / 128) * ((N + 127) / 128) <= 128) return 32;
     // 128- or 256-row tiles by rounds of workgroups x time per k-tile of a round (measured per k-tile: a 256 x 256 tile

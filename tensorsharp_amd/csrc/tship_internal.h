@@ -215,7 +215,8 @@ bool launch_gemm(int type, const GemmPlan& plan, const void* w, int64_t w_bytes,
 // the same by tile tables: c[row] with row = c_rows ? c_rows[m] : m
 bool launch_gemm_tiles(int type, const GemmTiles& tiles, const void* w, int64_t w_bytes, const void* workspace, float* c, int64_t ldc,
                        const int* c_rows, int M, int N, int K, hipStream_t stream, void* chunk_ws, size_t chunk_ws_bytes, int x_layout);
-// bytes of chunk_ws such a launch uses; only tiles.bm and tiles.count are read
+// bytes of chunk_ws such a launch uses (of the tiles, only bm and the count: there need be no tables yet); a launch of fewer tiles does with
+// as much, by the kernel whose sums fit if not by the same one
 size_t gemm_tiles_ws_bytes(int type, const GemmTiles& tiles, int M, int N, int K, int x_layout);
 // the kernels address one weight (or one launch's converted activations) with 32-bit offsets
 constexpr int64_t kMaxOperandBytes = ((int64_t)1 << 31) - 64;
