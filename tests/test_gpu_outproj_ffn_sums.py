@@ -7,12 +7,13 @@ test_outproj_ffn_launches.py: which of these shapes leave the sums to the conver
 import pytest
 
 pytestmark = pytest.mark.gpu
-T = {"q4_0": 2, "q8_0": 8, "q4_k": 12, "q5_k": 13, "q6_k": 14, "iq4_nl": 20, "mxfp4": 39}
+T = {"q4_0": 2, "q5_0": 6, "q8_0": 8, "q4_k": 12, "q5_k": 13, "q6_k": 14, "iq4_nl": 20, "mxfp4": 39}
 ROWS = [4, 20, 53, 200, 333]
 # output projection, gate / up, hidden, attention width, FFN half width, columns between the residual's rows
 SHAPES = [("q8_0", "q8_0", 1536, 1536, 3584, 0), ("q4_k", "q4_k", 4096, 4096, 14336, 0), ("q4_k", "q5_k", 2048, 5120, 8192, 4),
           ("q6_k", "iq4_nl", 768, 5120, 4096, 8), ("q6_k", "q4_0", 1024, 4096, 6144, 0), ("q4_k", "q4_k", 2304, 2304, 8192, 12),
-          ("mxfp4", "q8_0", 1024, 6144, 4096, 8), ("q8_0", "q6_k", 2048, 2048, 6144, 0)]
+          ("mxfp4", "q8_0", 1024, 6144, 4096, 8), ("q8_0", "q6_k", 2048, 2048, 6144, 0), ("q4_k", "q4_k", 1024, 1536, 14336, 0),
+          ("q8_0", "q5_k", 2304, 2304, 6144, 0), ("q8_0", "q5_0", 2304, 2304, 6144, 4)]
 # the sums lie where the conversion writes; rows that do not fit its registers; activations in block-scaled pairs, which it does not form
 REFUSED = [("q4_k", "q4_k", 4096, 4096, 2048, 0), ("q4_k", "q4_k", 8448, 512, 8192, 0), ("q4_k", "mxfp4", 1024, 4096, 4096, 0)]
 
