@@ -897,6 +897,7 @@ struct GemmArgs {
     // register-resident kernel with K cut into chunks: chunk kc of a row tile writes its sums (already scaled) to
     // partial[kc][activation row][column]; a second kernel adds the chunks in order into c
     float* partial;          // null: one chunk, results go straight to c
+    int slim_cols;           // host: columns of the register-resident kernel's tiles as planned (0: not yet)
     int sum_row0, sum_rows;  // host: the rows that the second kernel adds (0 rows: all M)
     PendingSums* pending;    // host: where the sums are left to the caller instead (it adds them to c)
     int k_chunks;
@@ -1026,6 +1027,7 @@ struct ChunkScratch {
     float* ptr;
     size_t bytes;
     size_t* need_out;
+    int* cols_out = nullptr;      // the columns that a register-resident kernel is planned with
 };
 inline float* chunk_scratch(const ChunkScratch& cs, size_t bytes) { return bytes <= cs.bytes ? cs.ptr : nullptr; }
 bool launch_chunk_sum(const GemmArgs& a, hipStream_t stream);
@@ -4031,41 +4033,42 @@ inline bool runs_cross(int64_t segments, int64_t tiles)
 
 inline bool chunk_sums_fit(int k_chunks, int M, int N, size_t max_bytes) { return (size_t)k_chunks * M * N * sizeof(float) <= max_bytes; }
 
-// The kernel that is expected to take less: 16 columns where that spares the launch for the sums, else by the k-tiles of the workgroup
-// that has most of them and the activations it loads anew where its run crosses into another row tile or K chunk.  In hundredths of a
-// us, fitted to 6500 whole calls of the ten formats on both kernels (4 .. 420 rows, 256 .. 21504 columns, K of 1024 .. 21504, weights
-// from HBM and from the memory-side cache): the pick is 0.5 % behind the faster one on average, more than 4 % behind on 320 of them.
-// Either kernel alone would be 2 (16) and 9 % (32) behind.  us, 16 / 32 columns:
+// Whether there is a kernel of 16 columns: none of 32 rows with at most four k-tiles per wavefront, whose tiles are too little work between
+// two barriers (Q6_K 93 x 6327 x 2048 20.8 us, 18.5 on 32 columns, 331 x 5764 x 1792 39.2 / 35.6).
+inline bool has_slim16(int ktw, int M, bool by_tiles) { return ktw > 4 || (M <= 16 && !by_tiles); }
+
+// The kernel that is expected to take less, by the run of units that takes longest: its k-tiles and tiles, the activations it loads anew
+// where it crosses into another row tile or K chunk, the launch that adds the chunks, and the activations that a workgroup begins with.
+// Hundredths of a us, fitted to 16200 whole calls of the ten formats on both kernels (4 .. 420 rows, 256 .. 21504 columns, K of 1024 ..
+// 21504, weights from HBM and from the memory-side cache): the pick is 0.22 % behind the faster one on average, more than 4 % behind on 1.7 %
+// of them.  Either kernel alone would be 2 (16) and 9 % (32) behind.  Against the kernel of 32 columns before there was another, on 6900
+// further calls: 0.912 of its time, more than 4 % more on 45 of them (10 % at most).  us, 16 / 32 columns:
 //   Q6_K 23 x 5120 x 6144 25.6 / 19.8, Q8_0 27 x 2560 x 14336 (added) 30.0 / 24.9, MXFP4 26 x 4096 x 14336 28.7 / 23.0 (runs that cross);
 //   Q8_0 24 x 4096 x 2560 11.2 / 13.4, Q6_K 10 x 2800 x 4096 11.4 / 13.3 (the launch for the sums spared);
-//   Q4_K 24 x 4096 x 4096 11.4 / 13.1, 24 x 14336 x 4096 20.1 / 19.3 (one tile of 16 columns per CU, and three to four).
-// Up to 16 rows: half the matrix instructions of 32, so less per k-tile; with at most four k-tiles per wavefront the tile's sums and
-// barrier weigh more, and twice as many tiles of 16 columns lose (Q6_K 13 x 8192 x 1024 10.2 / 9.8; 3 against 2 win, 0.94).
+//   Q4_K 24 x 4096 x 4096 11.4 / 13.1, 24 x 14336 x 4096 20.1 / 19.3 (one tile of 16 columns per CU, and three to four);
+//   Q4_K 40 x 2340 x 5120 15.8 / 18.9 (a short last chunk).
 // More than 32 rows of fewer than 1024 columns keep the chunks, and with them the workspace, of the 32-column kernel.
 // max_bytes: of the chunk sums; a kernel whose sums do not fit gives way to one whose sums do.  row_tiles may count empty tiles of a table.
 template <typename G>
 SlimPlan slim_plan(int nkt, int M, int N, int row_tiles, bool by_tiles, bool accumulate, size_t max_bytes)
 {
     const int ktw = slim_ktw<G>(nkt), ktw32 = slim32_ktw<G>(nkt), cus = device_info().num_cus;
-    const bool rows16 = M <= 16 && !by_tiles;
-    // (at most four k-tiles and 32 rows: no kernel of 16 columns; Q6_K 93 x 6327 x 2048 20.8 / 18.5, 331 x 5764 x 1792 39.2 / 35.6)
-    if ((ktw <= 4 && !rows16) || (M > 32 && N < 1024)) return {32, ktw32};
+    if (!has_slim16(ktw, M, by_tiles) || (M > 32 && N < 1024)) return {32, ktw32};
     const int chunks = (nkt + 8 * ktw - 1) / (8 * ktw), chunks32 = (nkt + 8 * ktw32 - 1) / (8 * ktw32);
     const bool sums = chunks > 1 || accumulate, sums32 = chunks32 > 1 || accumulate;
     const bool fits = !sums || chunk_sums_fit(chunks, M, N, max_bytes), fits32 = !sums32 || chunk_sums_fit(chunks32, M, N, max_bytes);
     if (!fits32) return {16, ktw};
     if (!fits) return {32, ktw32};
-    if (sums32 && !sums) return {16, ktw};
-    // k-tiles of a wavefront in a unit: of a whole chunk, of the last one
-    auto unit_kt = [](int kt) { return ((kt + G::kTileStep - 1) / G::kTileStep + 7) / 8 * G::kTileStep; };
-    const int full = unit_kt(std::min(8 * ktw, nkt)), last = unit_kt(nkt - (chunks - 1) * 8 * ktw), full32 = unit_kt(std::min(8 * ktw32, nkt));
-    const int64_t tiles = (N + 15) / 16, segments = (int64_t)row_tiles * chunks, units = segments * tiles;
-    const int64_t tiles32 = (N + 31) / 32, segments32 = (int64_t)row_tiles * chunks32, rounds32 = (segments32 * tiles32 + cus - 1) / cus;
-    int64_t kt = full;
-    if (units > cus)         // (dealt out by weight where the last chunk is shorter: at most a unit above the average)
-        kt = last == full ? (units + cus - 1) / cus * full : row_tiles * tiles * ((chunks - 1) * full + last) / cus + full;
-    const int64_t cost = kt * (!rows16 ? 29 : ktw <= 4 ? 24 : 17) + (units > cus && segments > 1 ? 22 * ktw : 0);
-    const int64_t cost32 = rounds32 * full32 * 46 + (runs_cross(segments32, tiles32) ? 58 : 0);
+    constexpr int S = G::kTileStep;
+    // steps of a wavefront in a unit: of a whole chunk, of the last one
+    auto steps = [](int kt) { return ((kt + S - 1) / S + 7) / 8; };
+    const int whole = steps(std::min(8 * ktw, nkt)), last = steps(nkt - (chunks - 1) * 8 * ktw);
+    const UnitRuns runs{row_tiles, chunks, (N + 15) / 16, whole + 1, last + 1};
+    const int64_t rows = std::min(M, 32), tiles32 = (N + 31) / 32, segments32 = (int64_t)row_tiles * chunks32;
+    const int64_t rounds32 = (segments32 * tiles32 + cus - 1) / cus, full32 = steps(std::min(8 * ktw32, nkt)) * S;
+    const int64_t cost = runs.longest(cus, whole * S, last * S, M <= 16 && !by_tiles ? 12 : 19, M <= 16 && !by_tiles ? 67 : 69, 30 * ktw) +
+                         (sums ? 187 + (int64_t)chunks * M * N * 90 / 1000000 : 0) + 162 * rows * ktw / 256;
+    const int64_t cost32 = rounds32 * (full32 * 35 + 110) + (runs_cross(segments32, tiles32) ? 19 * ktw32 : 0) + (sums32 ? 187 : 0) + 159 * rows * ktw32 / 256;
     return cost <= cost32 ? SlimPlan{16, ktw} : SlimPlan{32, ktw32};
 }
 
@@ -4088,7 +4091,10 @@ bool launch_slim_rows(const GemmArgs& a, int ktw, int m_tiles, hipStream_t strea
 template <typename G>
 bool launch_slim_for(const GemmArgs& a, int m_tiles, hipStream_t stream, const ChunkScratch& cs)
 {
-    const SlimPlan p = slim_plan<G>(a.Kp / kBK, a.M, a.N, m_tiles, a.by_tiles != 0, a.accumulate != 0, cs.bytes);
+    const int nkt = a.Kp / kBK;
+    const SlimPlan p = a.slim_cols == 0 ? slim_plan<G>(nkt, a.M, a.N, m_tiles, a.by_tiles != 0, a.accumulate != 0, cs.bytes)
+                                        : SlimPlan{a.slim_cols, a.slim_cols == 32 ? slim32_ktw<G>(nkt) : slim_ktw<G>(nkt)};
+    if (cs.cols_out) *cs.cols_out = p.cols;
     if (p.cols == 32) return launch_slim_rows<G, 2, 32>(a, p.ktw, m_tiles, stream, cs);
     if (!a.by_tiles && a.M <= 16) return launch_slim_rows<G, 1, 16>(a, p.ktw, m_tiles, stream, cs);
     if constexpr (G::kTileStep == 2)
@@ -4267,11 +4273,11 @@ namespace {
 // residual.  On 300 further random calls per format the pick took 0.4 % (Q4_K), 0.3 % (Q8_0) and 0.2 % (Q6_K) longer than the
 // fastest candidate on average, more than 4 % longer on 11, 8 and 3 of them, 11 % at most.
 // The register-resident kernel of 16-column tiles was fitted by itself, up to 64 rows, on 260 calls per format of 4 .. 420 rows, 300 .. 21504
-// columns and K of 1024 .. 14336.  Above 64 rows, above 32 under 1024 columns, and where tiles of 32 columns serve (slim_plan), the costs of
-// that kernel draw the line (the far_ constants), whichever of the two is launched: they are the upper ones of the two, so rows go to the
-// other kernels too early if at all.  On 650 further calls per format the pick is 4.4 / 1.6 / 1.4 % (Q4_K / Q8_0 / Q6_K) behind the fastest of
-// the two and gemm_wide_kernel from 17 to 64 rows, 4.6 / 3.9 / 1.4 % above, most of it under 1024 columns (Q4_K 34 x 844 x 2560 15.6 us, 10.0
-// on tiles of 16 columns), and 0.5 % up to 16.
+// columns and K of 1024 .. 14336, and draws the line there also where tiles of 32 columns serve, which take less then (slim_plan).  Above 64
+// rows, above 32 under 1024 columns, and where there is no kernel of 16 columns, the costs of the one of 32 draw it (the far_ constants).
+// On 750 further calls per format the pick is 0.3 / 0.6 / 0.4 % (Q4_K / Q8_0 / Q6_K) behind the fastest of the two and gemm_wide_kernel up to
+// 16 rows, 0.8 / 0.6 / 0.3 % up to 64 and 2.7 / 1.6 / 1.9 % up to 420; above 32 rows of fewer than 1024 columns 10 / 0.7 / 0.2 % (Q4_K 34 x 844
+// x 2560 15.6 us, 10.0 on tiles of 16 columns: the plans and the workspace of these calls are older than that kernel).
 // The candidates, us (register-resident / gemm_wide_kernel / 128 rows / 256 rows):
 //   Q4_K  24 x 14336 x 4096 19.4 / 25.0 / - / 38.2,  64 x 828 x 2560 11.9 / 15.8 / - / 28.3,  88 x 3078 x 1792 11.6 / 17.2 / - / 29.0,
 //         200 x 4096 x 2560 24.9 / 28.2 / - / 36.3,  257 x 512 x 14336 39.2 / 32.0 / - / 84.9,  480 x 9728 x 9728 (added) - / 142 / - / 124
@@ -4310,21 +4316,23 @@ inline double sums_us(const RuleCosts& c, int k_chunks, int M, int N) { return c
 template <typename G>
 double slim_us(const RuleCosts& c, int M, int N, int nkt, bool accumulate, size_t max_chunk_bytes)
 {
-    const SlimPlan plan = slim_plan<G>(nkt, M, N, (M + 31) / 32, false, accumulate, max_chunk_bytes);
-    const int ktw = plan.ktw, kc = (nkt + 8 * ktw - 1) / (8 * ktw), cus = device_info().num_cus;
-    const bool two_pass = kc > 1 || accumulate;          // (launch_slim adds to a residual in the second launch only)
-    if (two_pass && !chunk_sums_fit(kc, M, N, max_chunk_bytes)) return kNotServed;
-    const double sums = two_pass ? sums_us(c, kc, M, N) : 0.0;
+    const int ktw = slim_ktw<G>(nkt), kc = (nkt + 8 * ktw - 1) / (8 * ktw), cus = device_info().num_cus;
+    const int far_ktw = slim32_ktw<G>(nkt), far_kc = (nkt + 8 * far_ktw - 1) / (8 * far_ktw);
+    const bool only32 = (M > 32 && N < 1024) || !has_slim16(ktw, M, false);
+    // (launch_slim adds to a residual in the second launch only)
+    const bool two_pass = kc > 1 || accumulate, far_two_pass = far_kc > 1 || accumulate;
+    const bool fits = !two_pass || chunk_sums_fit(kc, M, N, max_chunk_bytes), far_fits = !far_two_pass || chunk_sums_fit(far_kc, M, N, max_chunk_bytes);
+    if (only32 ? !far_fits : !fits && !far_fits) return kNotServed;
     // (wavefronts past the end of K leave theirs to the others)
-    if (M > 64 || (M > 32 && N < 1024) || plan.cols == 32) {
+    if (M > 64 || only32) {
         // (as 32-column tiles, also where those of 16 columns serve)
-        const int far_ktw = slim32_ktw<G>(nkt), far_kc = (nkt + 8 * far_ktw - 1) / (8 * far_ktw);
         const int64_t segments = (int64_t)((M + 31) / 32) * far_kc, tiles = (N + 31) / 32, units = segments * tiles;
         const double kt = 0.4 * far_ktw + 0.6 * nkt / (8.0 * far_kc);
         const double rows = M <= 32 || (M <= 160 && N >= 1024) ? c.far_rows_160 : c.far_rows;
         return c.far_call + rows * std::min(M, 32) * far_ktw / 256.0 + (double)((units + cus - 1) / cus) * (c.far_unit + c.far_unit_kt * kt) +
-               (runs_cross(segments, tiles) ? c.far_cross + c.far_cross_kt * far_ktw : 0.0) + (far_kc > 1 || accumulate ? sums_us(c, far_kc, M, N) : 0.0);
+               (runs_cross(segments, tiles) ? c.far_cross + c.far_cross_kt * far_ktw : 0.0) + (far_two_pass ? sums_us(c, far_kc, M, N) : 0.0);
     }
+    const double sums = two_pass ? sums_us(c, kc, M, N) : 0.0;
     const int64_t segments = (int64_t)((M + 31) / 32) * kc, tiles = (N + 15) / 16, units = segments * tiles;
     const double kt = 0.4 * ktw + 0.6 * nkt / (8.0 * kc);
     return c.slim + c.slim_convert * M * (nkt * kBK) * 1e-6 + c.slim_rows * std::min(M, 32) * ktw / 256.0 +
@@ -4563,6 +4571,7 @@ bool gemm_dispatch_plan(int type, GemmArgs a, const GemmPlan& plan, hipStream_t 
         return false;
     }
     a.accumulate = accumulate ? 1 : 0;
+    a.slim_cols = plan.slim_cols;
     const WidePlan wide{plan.wide_tm, plan.k_chunks, plan.chunk_kt};
     return gemm_dispatch(type, a, plan.bm, plan.bm == kWideTiles ? 1 : (a.M + plan.bm - 1) / plan.bm, wide, stream, cs);
 }
@@ -4603,7 +4612,7 @@ GemmPlan plan_gemm(int type, int M, int N, int K, bool accumulate, size_t max_ch
     if (p.bm == 32 && p.x_layout == 0) p.x_layout = 3;
     // the launcher's own dry run, so that it makes the choices it would make with the reported bytes at hand; the register-resident
     // kernels choose by the bound, the others are not given one
-    const ChunkScratch cs{nullptr, p.bm == 32 ? max_chunk_bytes : ~(size_t)0, &p.chunk_bytes};
+    const ChunkScratch cs{nullptr, p.bm == 32 ? max_chunk_bytes : ~(size_t)0, &p.chunk_bytes, &p.slim_cols};
     GemmArgs a{};
     const int64_t w_bytes = block_bytes(type) * (K / block_elems(type)) * N;
     if (!gemm_args(&a, nullptr, w_bytes, nullptr, nullptr, N, M, N, K, p.x_layout) || !gemm_dispatch_plan(type, a, p, nullptr, accumulate, cs))

@@ -152,6 +152,7 @@ size_t gemm_workspace_bytes(int M, int K);
 struct GemmPlan {
     int bm;                              // rows of activations per tile: 32, 128 or 256, 0 where gemm_wide_kernel runs, -1 no kernel
     int wide_tm, k_chunks, chunk_kt;     // gemm_wide_kernel: rows per tile / 32, K chunks, k-tiles per chunk
+    int slim_cols;                       // register-resident kernels of fp16 operands: columns per tile
     int x_layout;                        // of the converted activations: 0 fp16 in the format's unpack order, 1 MX fp6 pairs (MXFP4 on
                                          // the block-scaled matrix instruction), 2 fp16 in natural order (Q4_K on gemm_wide_kernel),
                                          // 3 as 0 (Q4_K: as 2) in pieces of eight, row by row (the 32-row units of fp16 operands)

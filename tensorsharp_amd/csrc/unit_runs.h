@@ -22,6 +22,37 @@ struct UnitRuns {
         const int tile = (int)(at / weight), rest = (int)(at - tile * weight);
         return tile * per_tile + (rest < front ? rest / chunk_weight : (k_chunks - 1) * n_tiles + (rest - (int)front) / last_weight);
     }
+
+    // What the run that takes longest costs: per_kt for each k-tile of a wavefront (`full` in a unit, `last` in those of the last K chunk),
+    // per_unit for each unit, per_cross for each further row tile or K chunk that the run enters.  Looked at are the runs inside one chunk
+    // and those across its edges (twelve of them, evenly spread, where there are more).
+    constexpr int64_t longest(int grid, int full, int last, int per_kt, int per_unit, int per_cross) const
+    {
+        const int64_t whole = (int64_t)full * per_kt + per_unit, end = (int64_t)last * per_kt + per_unit;
+        const int segments = row_tiles * k_chunks, edges = segments - 1;
+        if ((int64_t)segments * n_tiles <= grid) return k_chunks > 1 ? whole : end;
+        const int64_t weight = (int64_t)n_tiles * ((int64_t)(k_chunks - 1) * chunk_weight + last_weight), total = row_tiles * weight;
+        const int64_t n_end = (total + (int64_t)grid * last_weight - 1) / ((int64_t)grid * last_weight);
+        int64_t worst = end * (n_end < n_tiles ? n_end : n_tiles);
+        if (k_chunks > 1) {
+            const int64_t n = (total + (int64_t)grid * chunk_weight - 1) / ((int64_t)grid * chunk_weight), cost = whole * (n < n_tiles ? n : n_tiles);
+            if (cost > worst) worst = cost;
+        }
+        for (int i = 0; i < (edges < 12 ? edges : 12); ++i) {
+            const int s = 1 + (edges <= 12 ? i : (int)((int64_t)i * edges / 12));            // the edge in front of segment s
+            const int64_t before = (s / k_chunks * weight + (int64_t)(s % k_chunks) * n_tiles * chunk_weight) * grid;
+            if (before % total == 0) continue;                                                // (a run begins there)
+            const int b = (int)(before / total), lo = first(b, grid), hi = first(b + 1, grid);
+            int64_t cost = -(int64_t)per_cross;
+            for (int u = lo, next = lo; u < hi; u = next) {
+                const int segment = u / n_tiles;
+                next = (segment + 1) * n_tiles < hi ? (segment + 1) * n_tiles : hi;
+                cost += (next - u) * (segment % k_chunks == k_chunks - 1 ? end : whole) + per_cross;
+            }
+            if (cost > worst) worst = cost;
+        }
+        return worst;
+    }
 };
 
 }  // namespace tship

@@ -63,3 +63,13 @@ def test_expert_stages_launch_the_kernels_they_are_for(stub):  # noqa: F811
     for name in ("q4_k", "q5_k", "q6_k", "q8_0"):
         assert (16, 8, 32) in seen[name] and any(k[0] == 32 for k in seen[name])
     assert (16, 6, 32) in seen["q8_0"] & seen["q4_0"]
+
+
+@pytest.mark.parametrize("name,M,N,K,columns", [
+    ("q4_k", 40, 2340, 5120, 16), ("q4_k", 53, 2195, 5120, 16), ("q4_k", 24, 4096, 4096, 16), ("q8_0", 24, 4096, 2560, 16), ("q8_0", 108, 1024, 6080, 16),
+    ("q4_k", 24, 14336, 4096, 32), ("q4_k", 29, 4096, 14336, 32), ("q6_k", 23, 5120, 6144, 32), ("mxfp4", 26, 4096, 14336, 32), ("q8_0", 21, 5120, 14848, 32)])
+def test_the_faster_kernel_is_launched(stub, name, M, N, K, columns):  # noqa: F811
+    """Calls that take 4 to 25 % longer on the other one."""
+    t, per = FORMATS[name]
+    (log,) = stub(PRODUCT, cases=[(t, per, BYTES[t], M, N, K)])
+    assert [k[0] for k in kernels(log)] == [columns], log

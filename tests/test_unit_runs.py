@@ -12,6 +12,10 @@ extern "C" int first(int rows, int chunks, int columns, int chunk, int last, int
 {
     return tship::UnitRuns{rows, chunks, columns, chunk, last}.first(b, grid);
 }
+extern "C" long long longest(int rows, int chunks, int columns, int chunk, int last, int grid, int kt, int unit, int cross)
+{
+    return tship::UnitRuns{rows, chunks, columns, chunk, last}.longest(grid, 4 * (chunk - 1), 4 * (last - 1), kt, unit, cross);
+}
 """
 
 
@@ -21,7 +25,10 @@ def first(tmp_path_factory):
     (out / "runs.cpp").write_text(SOURCE)
     lib = str(out / "libruns.so")
     subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-I" + os.path.join(ROOT, "tensorsharp_amd", "csrc"), str(out / "runs.cpp"), "-o", lib], check=True)
-    return C.CDLL(lib).first
+    got = C.CDLL(lib)
+    got.longest.restype = C.c_longlong
+    got.first.longest = got.longest
+    return got.first
 
 
 # (row tiles, K chunks, column tiles, weight of a unit of a whole chunk, of the last chunk)
@@ -53,3 +60,17 @@ def test_runs_weigh_about_the_same(first, case):
     runs = [(first(*case, b, 256), first(*case, b + 1, 256)) for b in range(256)]
     if total < 10 ** 6:
         assert max(sum(weigh(u) for u in range(*r)) for r in runs) <= total / 256 + chunk
+
+
+@pytest.mark.parametrize("case", [c for c in CASES if 0 < c[0] * c[1] * c[2] < 10 ** 5] + [(2, 2, 147, 3, 2), (1, 4, 256, 3, 2), (3, 1, 418, 3, 3), (5, 7, 33, 4, 2)])
+@pytest.mark.parametrize("kt,unit,cross", [(19, 69, 240), (12, 67, 120), (1, 0, 0)])
+def test_the_longest_run(first, case, kt, unit, cross):
+    """Against all runs, where every edge is looked at: no run costs more, and what is said is at most one unit above the one that does most."""
+    rows, chunks, columns, chunk, last = case
+    cost = lambda u: kt * 4 * ((last if u // columns % chunks == chunks - 1 else chunk) - 1) + unit
+    runs = [range(first(*case, b, 256), first(*case, b + 1, 256)) for b in range(256)]
+    most = max(sum(map(cost, r)) + cross * (r[-1] // columns - r[0] // columns) for r in runs if len(r))
+    got = first.longest(*case, 256, kt, unit, cross)
+    assert got <= most + kt * 4 * (chunk - 1) + unit
+    if rows * chunks <= 13:
+        assert got >= most
